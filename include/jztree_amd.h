@@ -239,6 +239,18 @@ int jzt_knn_node2node_ex(jzt_stream_t stream, const int32_t* parent_ilist_spl, c
                          int64_t size_parents, int64_t size_nodes, int64_t parent_ilist_size,
                          int64_t node_ilist_size, int k, float boxsize, int dim, int dtype);
 
+/* jzt_knn_node2node_ex with scratch (jzt_knn_node2node_tmp_bytes bytes): parents with long lists and
+ * long lists themselves are queued there and get larger workgroups.  tmp may be NULL.
+ * parent_rmax2 (may be NULL): the parents' guaranteed radius^2, where the children's search starts. */
+size_t jzt_knn_node2node_tmp_bytes(int64_t size_parents, int64_t node_ilist_size);
+int jzt_knn_node2node_tmp(jzt_stream_t stream, const int32_t* parent_ilist_spl, const int32_t* parent_ilist_isrc,
+                          const float* parent_ilist_r2, const int32_t* parent_spl, const void* nodes,
+                          const int32_t* nodes_npart, const float* parent_rmax2, const float* node_r2_in, float* node_rmax2,
+                          int32_t* node_ilist_spl, int32_t* node_ilist_isrc, float* node_ilist_r2,
+                          int64_t size_parents, int64_t size_nodes, int64_t parent_ilist_size,
+                          int64_t node_ilist_size, int k, float boxsize, int dim, int dtype, void* tmp,
+                          size_t tmp_bytes);
+
 
 /* Regularization's extra leaf splits (tree.py:236-243 of the reference, one kernel here):
  * flags[i] = flags[i] | (lvl[i] >= *lvl_max && i <= *npart) as 0/1 bytes, i < n; lvl_max and npart

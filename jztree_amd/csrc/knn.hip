@@ -2,11 +2,12 @@
 //
 // KnnNode2Node (knn.cuh:435-694): for every child node Q of a parent, walk the parent's
 //   r2-sorted interaction list and
-//     FindRmax     accumulate (maxdist2, npart) bins until >= k particles are guaranteed; the
-//                  bin radius (times 1 + 2^-16) bounds the k-th neighbour of every point in Q
-//     Count/Insert every child T of the listed parents with mindist2(Q,T) <= rmax2(Q)
-//     SegmentSort  each node's list ascending by (r2, src)
-//   One wave64 workgroup per parent; its children sit in lanes; source children are staged in LDS.
+//     find      the smallest maxdist2 within which >= k particles are guaranteed; that radius
+//               (times 1 + 2^-16) bounds the k-th neighbour of every point in Q
+//     count,    then, after a scan of the counts, list every child T of the listed parents with
+//     insert    mindist2(Q,T) <= rmax2(Q)
+//     sort      each node's list ascending by (r2, src)
+//   node_tiles.h has the work split.
 //
 // KnnLeaf2Leaf (knn.cuh:203-356): one wave64 per query leaf, one query per lane.  The leaf's
 //   interaction list is walked in ascending r2 and stops once no lane could still accept
@@ -20,6 +21,7 @@
 #include "util.h"
 #include "knn_common.h"
 #include "knn_nd.h"
+#include "node_tiles.h"
 #include "../../include/jztree_amd.h"
 
 namespace jzt {
@@ -55,312 +57,444 @@ __device__ __forceinline__ Vec<D, T> add(const Vec<D, T>& a, const Vec<D, T>& b)
 }
 
 // ------------------------------------------------------------------------------------------------
-// per-lane bins of (r2, count) for the guaranteed radius (knn.cuh:106-191, same semantics)
+// guaranteed k-neighbour radius of a node, and the nodes within it
 // ------------------------------------------------------------------------------------------------
-template <int KB> struct RmaxBins {
-  float r2s[KB];
-  int cts[KB];
-  int total, target;
-  __device__ __forceinline__ RmaxBins(int tgt) {
-#pragma unroll
-    for (int i = 0; i < KB; i++) {
-      r2s[i] = INFINITY;
-      cts[i] = 0;
-    }
-    total = 0;
-    target = tgt;
-  }
-  __device__ __forceinline__ float max_r2(int count) const {
-    bool active = true;
-    int sum = 0;
-    float r2 = INFINITY;
-#pragma unroll
-    for (int i = 0; i < KB; i++) {
-      sum += cts[i];
-      r2 = (active && sum >= count) ? r2s[i] : r2;
-      active = sum < count;
-    }
-    return r2;
-  }
-  __device__ __forceinline__ void insert_add(float r2, int num) {
-    total += num;
-    bool active = true;
-#pragma unroll
-    for (int i = 0; i < KB; i++) {
-      bool a = active && (r2s[i] >= r2);
-      cts[i] = a ? cts[i] + num : cts[i];
-      active = active && !a;
-    }
-  }
-  __device__ __forceinline__ void insert_shift(float r2, int num) {
-    total = total + num - cts[KB - 1];
-    bool active = true;
-#pragma unroll
-    for (int i = KB - 2; i >= 0; i--) {
-      bool take = active && (r2 < r2s[i]);
-      r2s[i + 1] = active ? (take ? r2s[i] : r2) : r2s[i + 1];
-      cts[i + 1] = active ? (take ? cts[i] : num) : cts[i + 1];
-      active = take;
-    }
-    r2s[0] = active ? r2 : r2s[0];
-    cts[0] = active ? num : cts[0];
-  }
-  __device__ __forceinline__ void consider(float r2, int num) {
-    if (r2 > r2s[KB - 1]) return;
-    bool need_add = (cts[KB - 1] > 0) && (total + num - cts[KB - 1] < target);
-    need_add |= r2 == r2s[KB - 1];
-    if (need_add) insert_add(r2, num);
-    else insert_shift(r2, num);
-  }
+// The guaranteed radius^2 of a child Q is the smallest R such that the nodes T with maxdist2(Q, T) <= R
+// hold at least k particles (knn.cuh:106-191 keeps 8 to 32 bins of (maxdist2, count) per child and
+// merges the rest; here the selection is exact).  A node that holds k particles itself starts at its
+// own squared diagonal.  Candidates below the current radius go into the child's LDS buffer; a wave
+// then sums, for every buffered entry, the particles of the entries up to it, and the smallest entry
+// that reaches k is the new radius; entries beyond it are dropped.
+//
+// Cost: about 40 VALU instructions per child pair, and the latency of the list walk (entry, children
+// range, node) where a parent has few pairs.  KnnNode2Node of 2^24 clustered points, leaf 48, k = 32: the
+// leaf plane (8e8 child pairs, 1.4e8 list entries) takes 3.0 ms for the radii and counts and 1.2 ms for the
+// lists, the top plane (1.5e8 pairs) 0.7 and 0.3 ms; one wave per parent, walking its list entry by entry,
+// took 18.2 and 12.0 ms for the two planes without the list sort.
+constexpr int kNodeKeep = 64;   // entries a child keeps after a reduction
+constexpr int kNodeLazy = 32;   // new entries that trigger one
+
+template <int D, typename T> struct NodeChild {
+  Vec<D, T> c, e;
 };
 
-#ifndef JZT_RMAX_GROUP
-#define JZT_RMAX_GROUP 16
-#endif
-constexpr int kRmaxGroup = JZT_RMAX_GROUP;  // children per lane group of k_find_rmax_groups (8, 16 or 32)
-static_assert(kRmaxGroup == 8 || kRmaxGroup == 16 || kRmaxGroup == 32, "lane group size");
+template <int NT> struct RadiusLds {
+  static constexpr int kCap = kNodeKeep + kNodeLazy + NT;
+  float r[kNodeChildren][kCap];
+  int w[kNodeChildren][kCap];
+  int n[kNodeChildren];       // entries in the buffer
+  int kept[kNodeChildren];    // of them left by the last reduction
+};
 
-template <int KB, int D, typename T>
-__global__ __launch_bounds__(64) void k_find_rmax(const int32_t* __restrict__ pil_spl, const int32_t* __restrict__ pil_src,
-                                                  const float* __restrict__ pil_r2, const int32_t* __restrict__ parent_spl,
-                                                  const T* __restrict__ nodes, const int32_t* __restrict__ npart,
-                                                  float* __restrict__ rmax_out, int k, T boxsize, int64_t pil_size, int64_t nitems,
-                                                  int skip_le) {
-  __shared__ Vec<D, T> s_x[64];
-  __shared__ Vec<D, T> s_e[64];
-  __shared__ int s_n[64];
-  const int lane = threadIdx.x;
-  const int64_t nact_ = active_items(parent_spl, nitems);
-  for (int pq = blockIdx.x; pq < nact_; pq += gridDim.x) {
-    const int q0 = parent_spl[pq], q1 = parent_spl[pq + 1];
-    if (q1 - q0 <= skip_le) continue;  // done by k_find_rmax_groups
-    const int e0 = pil_spl[pq], e1 = (int)min((int64_t)pil_spl[pq + 1], pil_size);
-    for (int qoff = q0; qoff < q1; qoff += 64) {
-      const int iq = min(qoff + lane, q1 - 1);
-      NodeT<D, T> nq = load_node<D, T>(nodes, iq);
-      Vec<D, T> eq = lvl_half_ext<D, T>(nq.level);
-      RmaxBins<KB> bins(k);
-      float rmax2 = INFINITY;
-      for (int e = e0; e < e1; e++) {
-        const int pt = pil_src[e];
-        const float r2t = pil_r2[e];
-        if (!wave_any(r2t <= rmax2)) break;
-        const int t0 = parent_spl[pt], t1 = parent_spl[pt + 1];
-        for (int toff = t0; toff < t1; toff += 64) {
-          const int it = toff + lane;
-          if (it < t1) {
-            NodeT<D, T> nt = load_node<D, T>(nodes, it);
-            s_x[lane] = nt.cent;
-            s_e[lane] = lvl_half_ext<D, T>(nt.level);
-            s_n[lane] = npart[it];
-          }
-          __syncthreads();
-          const int nl = min(t1 - toff, 64);
-          for (int j = 0; j < nl; j++) {
-            float r2 = (float)maxdist2<D, T>(s_x[j], nq.cent, add<D, T>(eq, s_e[j]), boxsize);
-            bins.consider(r2, s_n[j]);
-          }
-          __syncthreads();
-        }
-        rmax2 = bins.max_r2(k) * kRmaxSlack;
-      }
-      if (qoff + lane < q1) rmax_out[iq] = rmax2;
-    }
-  
+// Smallest radius^2 among the wave's entries (radius r, w particles; w = 0: none) up to which they hold at
+// least k particles; +inf if they hold fewer.  `in`: the lanes with an entry.  Every entry is broadcast
+// with readlane and added where it does not lie beyond the lane's own: about six instructions per
+// entry and no wait for LDS (broadcast from LDS, the same loop waited 64 times for a read).
+__device__ __forceinline__ float wave_select(float r, int w, uint64_t in, int k) {
+  int sum = 0;
+  for (uint64_t b = in; b; b &= b - 1ull) {
+    const int j = __builtin_ctzll(b);
+    const float rj = rdlane(r, j);
+    const int wj = rdlane(w, j);
+    sum += rj <= r ? wj : 0;
   }
+  return wave_minf(w > 0 && sum >= k ? r : INFINITY);
 }
 
-// FindRmax for parents with at most G children, 64 / G of them per wave: lane group g (G lanes)
-// takes parent base + g, lane j of the group its child j.  Each group does exactly what
-// k_find_rmax does for such a parent -- the same entries in list order, the same break test (no
-// child of the parent reaches the next entry), the same targets in order -- so every child's bins
-// see the same sequence and the radii are identical; only the lanes are shared.  The loop is
-// wave-uniform: each step every unfinished group stages (up to G targets of) its current entry
-// in its own LDS slice, and its lanes consider them.
-template <int KB, int D, typename T, int G>
-__global__ __launch_bounds__(64) void k_find_rmax_groups(const int32_t* __restrict__ pil_spl,
-                                                         const int32_t* __restrict__ pil_src,
-                                                         const float* __restrict__ pil_r2,
-                                                         const int32_t* __restrict__ parent_spl,
-                                                         const T* __restrict__ nodes, const int32_t* __restrict__ npart,
-                                                         float* __restrict__ rmax_out, int k, T boxsize,
-                                                         int64_t pil_size, int64_t nitems) {
-  constexpr int NG = 64 / G;
-  __shared__ Vec<D, T> s_x[64];
-  __shared__ Vec<D, T> s_e[64];
-  __shared__ int s_n[64];
-  const int lane = threadIdx.x, g = lane / G, j = lane - g * G;
-  const uint64_t gmask = (G == 64 ? ~0ull : ((1ull << G) - 1ull)) << (g * G);
-  const int64_t nact_ = active_items(parent_spl, nitems);
-  const int64_t nwaves = (nact_ + NG - 1) / NG;
-  for (int64_t wv = blockIdx.x; wv < nwaves; wv += gridDim.x) {
-    const int64_t pq = wv * NG + g;
-    int q0 = 0, nc = 0, e = 0, e1 = 0;
-    if (pq < nact_) {
-      q0 = parent_spl[pq];
-      nc = parent_spl[pq + 1] - q0;
-      e = pil_spl[pq];
-      e1 = (int)min((int64_t)pil_spl[pq + 1], pil_size);
-    }
-    // a group with more than G children (k_find_rmax's) or none has nothing to do
-    bool gdone = nc <= 0 || nc > G;
-    const bool valid = !gdone && j < nc;
-    const int iq = q0 + min(j, max(nc - 1, 0));
-    NodeT<D, T> nq = load_node<D, T>(nodes, valid ? iq : 0);
-    const Vec<D, T> eq = lvl_half_ext<D, T>(nq.level);
-    RmaxBins<KB> bins(k);
-    float rmax2 = INFINITY;
-    int toff = 0, t1 = 0;  // current entry's target range; toff >= t1: fetch the next entry
-    while (__ballot(!gdone) != 0ull) {
-      if (!gdone && toff >= t1) {
-        bool go = e < e1;
-        if (go) {
-          const float r2t = pil_r2[e];
-          go = (__ballot(valid && r2t <= rmax2) & gmask) != 0ull;
-        }
-        if (go) {
-          const int pt = pil_src[e];
-          toff = parent_spl[pt];
-          t1 = parent_spl[pt + 1];
-          e++;
-        } else {
-          gdone = true;
-        }
-      }
-      const int it = toff + j;
-      if (!gdone && it < t1 && j < G) {
-        NodeT<D, T> nt = load_node<D, T>(nodes, it);
-        s_x[lane] = nt.cent;
-        s_e[lane] = lvl_half_ext<D, T>(nt.level);
-        s_n[lane] = npart[it];
-      }
-      __syncthreads();
-      if (!gdone) {
-        const int nl = min(t1 - toff, G);
-        if (valid) {
-          for (int jj = 0; jj < nl; jj++) {
-            const int sl = g * G + jj;
-            float r2 = (float)maxdist2<D, T>(s_x[sl], nq.cent, add<D, T>(eq, s_e[sl]), boxsize);
-            bins.consider(r2, s_n[sl]);
-          }
-        }
-        toff += G;
-        if (toff >= t1) rmax2 = bins.max_r2(k) * kRmaxSlack;  // the entry is done
-      }
-      __syncthreads();
-    }
-    if (valid) rmax_out[iq] = rmax2;
+// One wave reduces the buffer of child c: returns the smallest radius^2 that its entries guarantee
+// (+inf if they hold fewer than k particles) and compacts the buffer to the entries below it and one
+// entry for the radius itself.  At most k entries stay (every entry holds a particle); with k > kNodeKeep
+// they are merged in order, each group taking its largest radius, which is still guaranteed.
+template <int NT> __device__ __forceinline__ float node_radius_reduce(RadiusLds<NT>& s, int c, int k) {
+  constexpr int E = (RadiusLds<NT>::kCap + 63) / 64;
+  const int lane = threadIdx.x & 63;
+  const int m = __builtin_amdgcn_readfirstlane(s.n[c]);
+  float r[E];
+  int w[E];
+#pragma unroll
+  for (int i = 0; i < E; i++) {
+    const int me = i * 64 + lane;
+    r[i] = me < m ? s.r[c][me] : INFINITY;
+    w[i] = me < m ? s.w[c][me] : 0;
   }
-}
-
-// One wave per parent node; its children are staged in LDS, and for every entry of the parent's
-// list the children of that entry are staged too.  Lanes take (child, target) pairs: with nt targets
-// staged, lane l tests child c0 + l / nt against target l % nt, so a parent with 8 children and an
-// entry with 8 targets keeps all 64 lanes busy (one lane per child would leave 56 idle).  A child's
-// hits in one step are lanes of one contiguous block: counted with a ballot, and in the insert pass
-// placed at the child's running offset plus the rank of the hit in its block.  The order inside a
-// node's list is therefore not the reference's, but every list is sorted by (r2, src) afterwards
-// (pairs are unique), so the lists are identical.
-template <int PASS, int D, typename T>
-__global__ __launch_bounds__(64) void k_count_insert(const int32_t* __restrict__ pil_spl, const int32_t* __restrict__ pil_src,
-                                                     const float* __restrict__ pil_r2,
-                                                     const int32_t* __restrict__ parent_spl, const T* __restrict__ nodes,
-                                                     const float* __restrict__ rmax2, int32_t* __restrict__ count_out,
-                                                     const int32_t* __restrict__ out_spl, int32_t* __restrict__ out_src,
-                                                     float* __restrict__ out_r2, int64_t nmax, T boxsize,
-                                                     int64_t pil_size, int64_t nitems) {
-  __shared__ Vec<D, T> s_qc[64], s_qe[64], s_tc[64], s_te[64];
-  __shared__ float s_qr[64];
-  __shared__ int64_t s_run[64];  // per child: hits so far (count pass) or next output slot (insert pass)
-  const int lane = threadIdx.x;
+  float best = INFINITY;
+  if (m <= 64) {
+    best = wave_select(r[0], w[0], m == 64 ? ~0ull : (1ull << m) - 1ull, k);
+  } else {
+    int sum[E];
+#pragma unroll
+    for (int i = 0; i < E; i++) sum[i] = 0;
+#pragma unroll
+    for (int i2 = 0; i2 < E; i2++) {
+      for (int j = 0; j < min(64, m - i2 * 64); j++) {
+        const float rj = rdlane(r[i2], j);
+        const int wj = rdlane(w[i2], j);
+#pragma unroll
+        for (int i = 0; i < E; i++) sum[i] += rj <= r[i] ? wj : 0;
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < E; i++)
+      if (w[i] > 0 && sum[i] >= k) best = fminf(best, r[i]);
+    best = wave_minf(best);
+  }
+  // entries that stay: strictly below the radius
+  int kept = 0;
   const uint64_t lt_mask = (1ull << lane) - 1ull;
-  const int64_t nact_ = active_items(parent_spl, nitems);
-  for (int pq = blockIdx.x; pq < nact_; pq += gridDim.x) {
-    const int q0 = parent_spl[pq], q1 = parent_spl[pq + 1];
-    const int e0 = pil_spl[pq], e1 = (int)min((int64_t)pil_spl[pq + 1], pil_size);
-    for (int qoff = q0; qoff < q1; qoff += 64) {
-      const int nc = min(q1 - qoff, 64);
-      float rq = -INFINITY;
-      if (lane < nc) {
-        const NodeT<D, T> nq = load_node<D, T>(nodes, qoff + lane);
-        s_qc[lane] = nq.cent;
-        s_qe[lane] = lvl_half_ext<D, T>(nq.level);
-        rq = rmax2[qoff + lane];
-        s_qr[lane] = rq;
-        s_run[lane] = (PASS == 1) ? (int64_t)out_spl[qoff + lane] : 0;
+#pragma unroll
+  for (int i = 0; i < E; i++) {
+    const bool keep = w[i] > 0 && r[i] < best;
+    const uint64_t b = __ballot(keep);
+    if (keep) {
+      const int o = kept + __popcll(b & lt_mask);
+      s.r[c][o] = r[i];
+      s.w[c][o] = w[i];
+    }
+    kept += __popcll(b);
+  }
+  if (best < INFINITY) {
+    if (lane == 0) {
+      s.r[c][kept] = best;
+      s.w[c][kept] = k;
+    }
+    kept++;
+  }
+  if (kept > kNodeKeep) {
+    // merge groups of q entries that are consecutive in (radius, slot) order
+    const int q = (kept + kNodeKeep - 1) / kNodeKeep;
+    int slot[E];
+    bool top[E];
+#pragma unroll
+    for (int i = 0; i < E; i++) {
+      const int me = i * 64 + lane;
+      int rank = 0;
+      r[i] = me < kept ? s.r[c][me] : INFINITY;
+      w[i] = me < kept ? s.w[c][me] : 0;
+      if (i * 64 < kept) {
+        for (int j = 0; j < kept; j++) {
+          const float rj = s.r[c][j];
+          rank += (rj < r[i] || (rj == r[i] && j < me)) ? 1 : 0;
+        }
       }
-      const float rq_max = wave_maxf(rq);
+      slot[i] = rank / q;
+      top[i] = rank % q == q - 1 || rank == kept - 1;
+    }
+    const int groups = (kept + q - 1) / q;
+    if (lane < groups) s.w[c][lane] = 0;  // groups <= kNodeKeep = 64
+#pragma unroll
+    for (int i = 0; i < E; i++) {
+      if (i * 64 + lane < kept) {
+        atomicAdd(&s.w[c][slot[i]], w[i]);
+        if (top[i]) s.r[c][slot[i]] = r[i];
+      }
+    }
+    kept = groups;
+  }
+  if (lane == 0) {
+    s.n[c] = kept;
+    s.kept[c] = kept;
+  }
+  return best;
+}
+
+// RADIUS: find the guaranteed radii (written to rmax2, slack included), else read them from rmax2; in both
+// cases count, for every child, the children of the listed parents within its radius.
+template <bool RADIUS, int NT, int D, typename T>
+__global__ __launch_bounds__(NT) void k_node_count(
+    const int32_t* __restrict__ pil_spl, const int32_t* __restrict__ pil_src, const float* __restrict__ pil_r2,
+    const int32_t* __restrict__ parent_spl, const T* __restrict__ nodes, const int32_t* __restrict__ npart,
+    const float* __restrict__ parent_rmax2, float* __restrict__ rmax2, int32_t* __restrict__ count_out, int k, T boxsize, int64_t pil_size, int64_t nitems,
+    NodeQueue queue) {
+  __shared__ TileLds<NT> s_t;
+  __shared__ NodeChild<D, T> s_q[kNodeChildren];
+  __shared__ float s_R[kNodeChildren];
+  __shared__ int s_cnt[kNodeChildren];
+  __shared__ typename std::conditional<RADIUS, RadiusLds<NT>, int>::type s_b;
+  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+  const uint64_t lt_mask = (1ull << lane) - 1ull;
+  // one-wave workgroups take all parents but those with long lists, the larger ones the queue's
+  const int64_t nact = NT == 64 ? active_items(parent_spl, nitems) : min((int64_t)queue.q[0], queue.most);
+  const NodeGroups ng = NT == 64 ? node_groups(nact) : NodeGroups{4, kNodeChildren};
+  for (int64_t item = blockIdx.x; item < nact * ng.groups; item += gridDim.x) {
+    const int grp = (int)(item / nact), ip = (int)(item - grp * nact);  // see node_groups
+    const int pq = NT == 64 ? ip : queue.q[1 + ip];
+    const int q1 = parent_spl[pq + 1];
+    const int e0 = pil_spl[pq], e1 = (int)min((int64_t)pil_spl[pq + 1], pil_size);
+    if (NT == 64 && queue.is_long(e1 - e0)) {
+      if (grp == 0 && tid == 0) queue.push(pq);
+      continue;
+    }
+    for (int q0 = parent_spl[pq] + grp * ng.width; q0 < q1; q0 += ng.groups * ng.width) {
+      const int nc = min(q1 - q0, ng.width);
+      __syncthreads();  // the previous round's readers are done
+      if (tid < nc) {
+        const NodeT<D, T> nq = load_node<D, T>(nodes, q0 + tid);
+        NodeChild<D, T> q;
+        q.c = nq.cent;
+        q.e = lvl_half_ext<D, T>(nq.level);
+        s_q[tid] = q;
+        s_cnt[tid] = 0;
+        if constexpr (RADIUS) {
+          s_b.n[tid] = 0;
+          s_b.kept[tid] = 0;
+          // radii known before any list entry: the parent's (it holds for every point of the parent) and,
+          // if the node holds k particles itself, its squared diagonal
+          float r0 = parent_rmax2 ? parent_rmax2[pq] : INFINITY;
+          if (npart[q0 + tid] >= k) r0 = fminf(r0, (float)maxdist2<D, T>(q.c, q.c, add<D, T>(q.e, q.e), boxsize));
+          s_R[tid] = r0;
+        } else {
+          s_R[tid] = rmax2[q0 + tid];
+        }
+      }
       __syncthreads();
-      for (int e = e0; e < e1; e++) {
-        const float r2t = pil_r2[e];
-        if (!(r2t <= rq_max)) break;  // entries ascend by r2; no child reaches this one or any later
-        const int pt = pil_src[e];
-        const int t0 = parent_spl[pt], t1 = parent_spl[pt + 1];
-        for (int toff = t0; toff < t1; toff += 64) {
-          const int nt = min(t1 - toff, 64);
-          if (lane < nt) {
-            const NodeT<D, T> ntn = load_node<D, T>(nodes, toff + lane);
-            s_tc[lane] = ntn.cent;
-            s_te[lane] = lvl_half_ext<D, T>(ntn.level);
-          }
-          __syncthreads();
-          const int cstep = nt >= 32 ? 1 : 64 / nt;
-          const int my_c = lane / nt, my_t = lane - my_c * nt;
-          const uint64_t block = (nt == 64 ? ~0ull : ((1ull << nt) - 1ull)) << (my_c * nt);
-          for (int c0 = 0; c0 < nc; c0 += cstep) {
-            const int c = c0 + my_c;
-            const bool active = my_c < cstep && c < nc;
-            bool hit = false;
-            float r2 = 0.f;
-            if (active) {
-              const Vec<D, T> ew = add<D, T>(s_qe[c], s_te[my_t]);
-              r2 = (float)mindist2<D, T>(s_tc[my_t], s_qc[c], ew, boxsize);
-              hit = r2 <= s_qr[c];
-              // Touching nodes are listed with a negative radius, -1 / maxdist2: they sort before every
-              // node at a positive distance, the node itself first among them (smallest maxdist2), and
-              // a consumer's "r2 <= k-th distance" test keeps them even when the k-th distance is
-              // exactly 0 (k or more copies of a point): such a node may hold copies with smaller ids.
-              // (A tiny positive radius, 1e-10 * maxdist2, failed that test and lost those ties.)
-              if (PASS == 1 && hit && r2 == 0.f)
-                r2 = -1.0f / fmaxf((float)maxdist2<D, T>(s_tc[my_t], s_qc[c], ew, boxsize), 1e-30f);
+      if constexpr (RADIUS) {
+        bool first = true;
+        for (int eb = e0; eb < e1; eb += NT) {
+          float rtop = s_R[0];
+          for (int c = 1; c < nc; c++) rtop = fmaxf(rtop, s_R[c]);
+          rtop *= kRmaxSlack;
+          const int ne = min(NT, e1 - eb);
+          int t0 = 0, cnt = 0, tot;
+          float r2t = INFINITY;
+          if (tid < ne) {
+            r2t = pil_r2[eb + tid];
+            if (r2t <= rtop) {
+              const int pt = pil_src[eb + tid];
+              t0 = parent_spl[pt];
+              cnt = parent_spl[pt + 1] - t0;
             }
-            const uint64_t hits = __ballot(hit) & block;
-            if (PASS == 1 && hit) {
-              const int64_t o = s_run[c] + __popcll(hits & lt_mask);
-              if (o < nmax) {
-                out_r2[o] = r2;
-                out_src[o] = toff + my_t;
+          }
+          const int pre = block_excl_scan<NT>(cnt, s_t.scan, &tot);
+          s_t.pre[tid] = pre;
+          s_t.off[tid] = t0 - pre;
+          int act = __syncthreads_count(tid < ne && r2t <= rtop);  // entries ascend by r2: a prefix
+          int lim = tot;
+          for (int base = 0; base < lim;) {
+            // the first tile (the node, its siblings and its nearest neighbours) is a short one:
+            // its reduction gives a radius that keeps nearly all later targets out of the buffer
+            const int width = first ? 64 : NT;
+            const int j = base + tid;
+            const bool valid = tid < width && j < lim;
+            const int e = tile_entry<NT>(s_t, ne, valid ? j : 0);
+            int np = 0;
+            NodeChild<D, T> t;
+            if (valid) {
+              const int it = j + s_t.off[e];
+              const NodeT<D, T> nt = load_node<D, T>(nodes, it);
+              t.c = nt.cent;
+              t.e = lvl_half_ext<D, T>(nt.level);
+              np = npart[it];
+            }
+            for (int c = 0; c < nc; c++) {
+              bool cand = false;
+              float r2 = 0.f;
+              if (np > 0) {
+                r2 = (float)maxdist2<D, T>(t.c, s_q[c].c, add<D, T>(s_q[c].e, t.e), boxsize);
+                cand = r2 < s_R[c];
+              }
+              uint64_t hits = __ballot(cand);
+              if (hits) {
+                if (first) {  // one wave holds the whole first tile: select before anything is stored
+                  const float rn = wave_select(cand ? r2 : INFINITY, cand ? np : 0, hits, k);
+                  cand = cand && (r2 < rn || rn == INFINITY);
+                  hits = __ballot(cand);
+                  if (rn < INFINITY) {
+                    if (lane == 0) {
+                      s_R[c] = rn;
+                      s_b.r[c][0] = rn;
+                      s_b.w[c][0] = k;
+                      s_b.n[c] = 1;
+                    }
+                  }
+                }
+                int o = 0;
+                if (lane == 0) o = atomicAdd(&s_b.n[c], __popcll(hits));
+                o = __builtin_amdgcn_readfirstlane(o) + __popcll(hits & lt_mask);
+                if (cand) {
+                  s_b.r[c][o] = r2;
+                  s_b.w[c][o] = np;
+                }
+                if (first && lane == 0) s_b.kept[c] = s_b.n[c];
               }
             }
-            if (active && my_t == 0 && hits) s_run[c] += __popcll(hits);
+            __syncthreads();
+            bool any = false;
+            for (int c = 0; c < nc; c++) any |= first || s_b.n[c] - s_b.kept[c] >= kNodeLazy;
+            __syncthreads();  // all have read the fills before the reductions change them
+            if (any) {
+              for (int c = w; c < nc; c += NT / 64) {
+                if (s_b.n[c] > s_b.kept[c]) {
+                  const float rn = node_radius_reduce(s_b, c, k);
+                  if (lane == 0) s_R[c] = fminf(s_R[c], rn);
+                }
+              }
+              __syncthreads();
+              rtop = s_R[0];
+              for (int c = 1; c < nc; c++) rtop = fmaxf(rtop, s_R[c]);
+              rtop *= kRmaxSlack;
+              act = __syncthreads_count(tid < ne && r2t <= rtop);
+              lim = act < ne ? min(lim, s_t.pre[act]) : lim;
+            }
+            base += width;
+            first = false;
           }
+          const bool more = act == ne;
           __syncthreads();
+          if (!more) break;
         }
+        for (int c = w; c < nc; c += NT / 64) {
+          float rn = INFINITY;
+          if (s_b.n[c] > s_b.kept[c]) rn = node_radius_reduce(s_b, c, k);
+          if (lane == 0) {
+            rn = fminf(s_R[c], rn) * kRmaxSlack;
+            s_R[c] = rn;
+            rmax2[q0 + c] = rn;
+          }
+        }
+        __syncthreads();
       }
-      if (PASS == 0 && lane < nc) count_out[qoff + lane] = (int32_t)s_run[lane];
+      float rtop = s_R[0];
+      for (int c = 1; c < nc; c++) rtop = fmaxf(rtop, s_R[c]);
+      for_target_tiles<NT>(
+          s_t, e0, e1,
+          [&](int e, int& t0, int& cnt) {
+            const bool in = pil_r2[e] <= rtop;
+            if (in) {
+              const int pt = pil_src[e];
+              t0 = parent_spl[pt];
+              cnt = parent_spl[pt + 1] - t0;
+            }
+            return in;
+          },
+          [&](bool valid, int it) {
+            const NodeT<D, T> nt = load_node<D, T>(nodes, it);
+            const Vec<D, T> te = lvl_half_ext<D, T>(nt.level);
+            for (int c = 0; c < nc; c++) {
+              const float r2 = (float)mindist2<D, T>(nt.cent, s_q[c].c, add<D, T>(s_q[c].e, te), boxsize);
+              const uint64_t hits = __ballot(valid && r2 <= s_R[c]);
+              if (hits && lane == 0) atomicAdd(&s_cnt[c], __popcll(hits));
+            }
+          });
+      if (tid < nc) count_out[q0 + tid] = s_cnt[tid];
+    }
+  }
+}
+
+// The same pairs as k_node_count's, written to the children's lists.  A child's slots are handed out by
+// an LDS counter, a wave's hits at a time, so the order inside a list is arbitrary; every list is sorted by
+// (r2, src) afterwards and its pairs are unique, so the lists do not depend on it.
+template <int NT, int D, typename T>
+__global__ __launch_bounds__(NT) void k_node_insert(
+    const int32_t* __restrict__ pil_spl, const int32_t* __restrict__ pil_src, const float* __restrict__ pil_r2,
+    const int32_t* __restrict__ parent_spl, const T* __restrict__ nodes, const float* __restrict__ rmax2,
+    const int32_t* __restrict__ out_spl, int32_t* __restrict__ out_src, float* __restrict__ out_r2, int64_t nmax,
+    T boxsize, int64_t pil_size, int64_t nitems, NodeQueue queue) {
+  __shared__ TileLds<NT> s_t;
+  __shared__ NodeChild<D, T> s_q[kNodeChildren];
+  __shared__ float s_R[kNodeChildren];
+  __shared__ int s_run[kNodeChildren];  // hits so far
+  __shared__ int s_out[kNodeChildren];  // first list slot
+  const int tid = threadIdx.x, lane = tid & 63;
+  const uint64_t lt_mask = (1ull << lane) - 1ull;
+  // one-wave workgroups take all parents but those with long lists, the larger ones the queue's
+  const int64_t nact = NT == 64 ? active_items(parent_spl, nitems) : min((int64_t)queue.q[0], queue.most);
+  const NodeGroups ng = NT == 64 ? node_groups(nact) : NodeGroups{4, kNodeChildren};
+  for (int64_t item = blockIdx.x; item < nact * ng.groups; item += gridDim.x) {
+    const int grp = (int)(item / nact), ip = (int)(item - grp * nact);  // see node_groups
+    const int pq = NT == 64 ? ip : queue.q[1 + ip];
+    const int q1 = parent_spl[pq + 1];
+    const int e0 = pil_spl[pq], e1 = (int)min((int64_t)pil_spl[pq + 1], pil_size);
+    if (NT == 64 && queue.is_long(e1 - e0)) {
+      continue;
+    }
+    for (int q0 = parent_spl[pq] + grp * ng.width; q0 < q1; q0 += ng.groups * ng.width) {
+      const int nc = min(q1 - q0, ng.width);
       __syncthreads();
+      if (tid < nc) {
+        const NodeT<D, T> nq = load_node<D, T>(nodes, q0 + tid);
+        NodeChild<D, T> q;
+        q.c = nq.cent;
+        q.e = lvl_half_ext<D, T>(nq.level);
+        s_q[tid] = q;
+        s_R[tid] = rmax2[q0 + tid];
+        s_run[tid] = 0;
+        s_out[tid] = out_spl[q0 + tid];
+      }
+      __syncthreads();
+      float rtop = s_R[0];
+      for (int c = 1; c < nc; c++) rtop = fmaxf(rtop, s_R[c]);
+      for_target_tiles<NT>(
+          s_t, e0, e1,
+          [&](int e, int& t0, int& cnt) {
+            const bool in = pil_r2[e] <= rtop;
+            if (in) {
+              const int pt = pil_src[e];
+              t0 = parent_spl[pt];
+              cnt = parent_spl[pt + 1] - t0;
+            }
+            return in;
+          },
+          [&](bool valid, int it) {
+            const NodeT<D, T> nt = load_node<D, T>(nodes, it);
+            const Vec<D, T> te = lvl_half_ext<D, T>(nt.level);
+            for (int c = 0; c < nc; c++) {
+              const Vec<D, T> ew = add<D, T>(s_q[c].e, te);
+              float r2 = (float)mindist2<D, T>(nt.cent, s_q[c].c, ew, boxsize);
+              const bool hit = valid && r2 <= s_R[c];
+              const uint64_t hits = __ballot(hit);
+              if (hits) {
+                int o = 0;
+                if (lane == 0) o = atomicAdd(&s_run[c], __popcll(hits));
+                const int64_t slot =
+                    (int64_t)s_out[c] + __builtin_amdgcn_readfirstlane(o) + __popcll(hits & lt_mask);
+                // Touching nodes are listed with a negative radius, -1 / maxdist2: they sort before every
+                // node at a positive distance, the node itself first among them (smallest maxdist2), and
+                // a consumer's "r2 <= k-th distance" test keeps them even when the k-th distance is
+                // exactly 0 (k or more copies of a point): such a node may hold copies with smaller ids.
+                // (A tiny positive radius, 1e-10 * maxdist2, failed that test and lost those ties.)
+                if (hit && r2 == 0.f)
+                  r2 = -1.0f / fmaxf((float)maxdist2<D, T>(nt.cent, s_q[c].c, ew, boxsize), 1e-30f);
+                if (hit && slot < nmax) {
+                  out_r2[slot] = r2;
+                  out_src[slot] = it;
+                }
+              }
+            }
+          });
     }
   }
 }
 
 // ------------------------------------------------------------------------------------------------
-// segmented sort by (key, val): bitonic network with only ascending comparators (the first stage of
-// each merge compares mirrored pairs), so lengths need not be powers of two (virtual +inf tail)
+// segmented sort by (key, val)
 // ------------------------------------------------------------------------------------------------
+// A (key, val) pair is one double whose high word is the key's own bits: keys are floats, so the
+// exponent field of the double never reaches 0x7ff (float infinity and NaN patterns are ordinary
+// doubles), and the double order is the float total order; below zero the order of the low word is
+// reversed, so val is stored complemented there.  Denormal doubles are kept by the FP64 mode.  A
+// compare-exchange is then one FP64 compare (or v_min_f64 + v_max_f64) instead of a 64-bit integer one.
 constexpr int kSegThreads = 256;
-constexpr int kSegLds = 4096;  // entries held in LDS (32 KB)
+constexpr int kSegLds = 4096;        // entries a workgroup of kSegThreads sorts in LDS (32 KB)
+constexpr int kSegBigThreads = 1024;
+constexpr int kSegBigLds = 16384;    // entries a workgroup of kSegBigThreads sorts in LDS (128 KB)
+constexpr int kWaveSortMax = 1024;   // entries one wave sorts in registers
 
-__device__ __forceinline__ uint64_t kv_pack(float k, int32_t v) {
-  uint32_t kb = __float_as_uint(k);
-  kb = (kb & 0x80000000u) ? ~kb : (kb | 0x80000000u);  // total order of IEEE floats
-  return ((uint64_t)kb << 32) | (uint32_t)v;
+__device__ __forceinline__ double kv_pack(float k, int32_t v) {
+  const uint32_t kb = __float_as_uint(k);
+  const uint32_t lo = (kb >> 31) ? ~(uint32_t)v : (uint32_t)v;
+  return __longlong_as_double((long long)(((uint64_t)kb << 32) | lo));
 }
-__device__ __forceinline__ float kv_key(uint64_t p) {
-  uint32_t kb = (uint32_t)(p >> 32);
-  kb = (kb & 0x80000000u) ? (kb & 0x7fffffffu) : ~kb;
-  return __uint_as_float(kb);
+__device__ __forceinline__ float kv_key(double p) {
+  return __uint_as_float((uint32_t)((uint64_t)__double_as_longlong(p) >> 32));
 }
+__device__ __forceinline__ int32_t kv_val(double p) {
+  const uint64_t b = (uint64_t)__double_as_longlong(p);
+  return (int32_t)((b >> 63) ? ~(uint32_t)b : (uint32_t)b);
+}
+__device__ __forceinline__ double kv_last() { return __longlong_as_double(0x7fefffffffffffffll); }  // above every pair
 
+// Bitonic network with only ascending comparators (the first stage of each merge compares mirrored
+// pairs), so lengths need not be powers of two (virtual +inf tail).
 template <typename Arr>
 __device__ __forceinline__ void bitonic_sort_asc(Arr a, int len) {
   int np2 = 1;
@@ -372,7 +506,7 @@ __device__ __forceinline__ void bitonic_sort_asc(Arr a, int len) {
       int i = blk * size + off;
       int j = blk * size + size - 1 - off;
       if (j < len) {
-        uint64_t x = a.load(i), y = a.load(j);
+        const double x = a.load(i), y = a.load(j);
         if (y < x) {
           a.store(i, y);
           a.store(j, x);
@@ -386,7 +520,7 @@ __device__ __forceinline__ void bitonic_sort_asc(Arr a, int len) {
         int i = blk * 2 * stride + off;
         int j = i + stride;
         if (j < len) {
-          uint64_t x = a.load(i), y = a.load(j);
+          const double x = a.load(i), y = a.load(j);
           if (y < x) {
             a.store(i, y);
             a.store(j, x);
@@ -399,132 +533,169 @@ __device__ __forceinline__ void bitonic_sort_asc(Arr a, int len) {
 }
 
 struct LdsArr {
-  uint64_t* p;
-  __device__ __forceinline__ uint64_t load(int i) const { return p[i]; }
-  __device__ __forceinline__ void store(int i, uint64_t x) const { p[i] = x; }
+  double* p;
+  __device__ __forceinline__ double load(int i) const { return p[i]; }
+  __device__ __forceinline__ void store(int i, double x) const { p[i] = x; }
 };
 // (key, val) pairs sorted in place in global memory
 struct GlobalKV {
   float* k;
   int32_t* v;
-  __device__ __forceinline__ uint64_t load(int i) const { return kv_pack(k[i], v[i]); }
-  __device__ __forceinline__ void store(int i, uint64_t x) const {
+  __device__ __forceinline__ double load(int i) const { return kv_pack(k[i], v[i]); }
+  __device__ __forceinline__ void store(int i, double x) const {
     k[i] = kv_key(x);
-    v[i] = (int32_t)(uint32_t)x;
+    v[i] = kv_val(x);
   }
 };
 
 // ---- wave-level segment sort ---------------------------------------------------------------
-// One wave per segment of up to 64*E entries, the keys in registers: entry i*64 + lane lives in
-// lane `lane`, register i.  Bitonic stages with stride >= 64 compare registers inside a lane,
-// smaller strides exchange with a lane shuffle; no barriers, no LDS.
-constexpr int kWaveSortMax = 1024;
+// One wave per segment of up to 64*E entries, entry lane*E + i in register i of lane `lane`: the
+// short strides, which a bitonic network uses most, stay inside a lane (v_min_f64 / v_max_f64), and
+// the lane strides go through DPP and, from 16 on, permlane swaps, so nothing waits for LDS
+// (exchanged with ds_bpermute, entry i*64 + lane, the sort was bound by LDS: 2.0 ms for the
+// 548,000 lists of 257 entries of 2^24 clustered points at leaf 48, 0.97 now).
+template <int CTRL> __device__ __forceinline__ uint32_t dpp(uint32_t x) {
+  return (uint32_t)__builtin_amdgcn_mov_dpp((int)x, CTRL, 0xf, 0xf, true);
+}
+// lane l's value of lane l ^ M, for M = 1, 2, 4, 8, 16, 32 (strides) and 3, 7, 15, 31, 63 (mirrors)
+template <int M> __device__ __forceinline__ uint32_t lane_xor(uint32_t x) {
+  if constexpr (M == 1) return dpp<0xB1>(x);         // quad_perm 1,0,3,2
+  else if constexpr (M == 2) return dpp<0x4E>(x);    // quad_perm 2,3,0,1
+  else if constexpr (M == 3) return dpp<0x1B>(x);    // quad_perm 3,2,1,0
+  else if constexpr (M == 7) return dpp<0x141>(x);   // row_half_mirror
+  else if constexpr (M == 15) return dpp<0x140>(x);  // row_mirror
+  else if constexpr (M == 8) return dpp<0x128>(x);   // row_ror:8
+  else if constexpr (M == 4) return lane_xor<3>(lane_xor<7>(x));
+  else if constexpr (M == 16) {
+    const auto r = __builtin_amdgcn_permlane16_swap(x, x, false, false);
+    return (__lane_id() & 16) ? r[0] : r[1];
+  } else if constexpr (M == 32) {
+    const auto r = __builtin_amdgcn_permlane32_swap(x, x, false, false);
+    return (__lane_id() & 32) ? r[0] : r[1];
+  } else if constexpr (M == 31) return lane_xor<16>(lane_xor<15>(x));
+  else return lane_xor<32>(lane_xor<31>(x));  // 63
+}
+template <int M> __device__ __forceinline__ double lane_xor(double v) {
+  const uint64_t b = (uint64_t)__double_as_longlong(v);
+  const uint32_t lo = lane_xor<M>((uint32_t)b), hi = lane_xor<M>((uint32_t)(b >> 32));
+  return __longlong_as_double((long long)(((uint64_t)hi << 32) | lo));
+}
+// keeps the smaller of v and o where `low`, else the larger (v and o differ or are both padding)
+__device__ __forceinline__ double keep_side(double v, double o, bool low) { return (o < v) == low ? o : v; }
 
-__device__ __forceinline__ uint64_t shfl_xor_u64(uint64_t x, int m) {
-  const int lo = __shfl_xor((int)(uint32_t)x, m, 64), hi = __shfl_xor((int)(uint32_t)(x >> 32), m, 64);
-  return ((uint64_t)(uint32_t)hi << 32) | (uint32_t)lo;
+__device__ __forceinline__ void kv_order(double& a, double& b) {
+  const double lo = __builtin_fmin(a, b), hi = __builtin_fmax(a, b);
+  a = lo;
+  b = hi;
 }
 
-template <int E>
-__device__ __forceinline__ void wave_bitonic_sort(uint64_t (&v)[E], int lane) {
-  constexpr int N = 64 * E;
+// entries x ^ S for register strides S < E (the whole wave is in blocks of 2S)
+template <int E, int S> __device__ __forceinline__ void half_clean(double (&v)[E], int lane) {
+  if constexpr (S < E) {
 #pragma unroll
-  for (int size = 2; size <= N; size <<= 1) {
+    for (int i = 0; i < E; i++)
+      if (!(i & S)) kv_order(v[i], v[i | S]);
+  } else {
+    const bool low = (lane & (S / E)) == 0;
 #pragma unroll
-    for (int stride = size / 2; stride > 0; stride >>= 1) {
-      if (stride >= 64) {
-        const int rs = stride / 64;
-#pragma unroll
-        for (int i = 0; i < E; i++) {
-          const int j = i ^ rs;
-          if (j > i) {
-            const bool asc = ((i * 64 + lane) & size) == 0;
-            const uint64_t a = v[i], b = v[j];
-            const bool sw = asc ? (b < a) : (a < b);
-            v[i] = sw ? b : a;
-            v[j] = sw ? a : b;
-          }
-        }
-      } else {
-#pragma unroll
-        for (int i = 0; i < E; i++) {
-          const uint64_t o = shfl_xor_u64(v[i], stride);
-          const bool asc = ((i * 64 + lane) & size) == 0;
-          const bool lower = (lane & stride) == 0;
-          const bool take_min = lower == asc;
-          const bool o_less = o < v[i];
-          v[i] = (take_min == o_less) ? o : v[i];
-        }
-      }
-    }
+    for (int i = 0; i < E; i++) v[i] = keep_side(v[i], lane_xor<S / E>(v[i]), low);
   }
+  if constexpr (S > 1) half_clean<E, S / 2>(v, lane);
+}
+// merges sorted blocks of SIZE/2 entries into sorted blocks of SIZE, from SIZE = 2 up to 64 * E
+template <int E, int SIZE> __device__ __forceinline__ void wave_merge(double (&v)[E], int lane) {
+  if constexpr (SIZE <= E) {
+#pragma unroll
+    for (int i = 0; i < E; i++) {
+      const int j = i ^ (SIZE - 1);
+      if (j > i) kv_order(v[i], v[j]);
+    }
+  } else {
+    constexpr int M = SIZE / E - 1;  // mirrored partner: lane ^ M, register E - 1 - i
+    const bool low = (lane & (SIZE / E / 2)) == 0;
+    double o[E];
+#pragma unroll
+    for (int i = 0; i < E; i++) o[i] = lane_xor<M>(v[E - 1 - i]);
+#pragma unroll
+    for (int i = 0; i < E; i++) v[i] = keep_side(v[i], o[i], low);
+  }
+  if constexpr (SIZE > 2) half_clean<E, SIZE / 4>(v, lane);
+  if constexpr (SIZE < 64 * E) wave_merge<E, SIZE * 2>(v, lane);
 }
 
 template <int E>
 __device__ __forceinline__ void wave_sort_segment(float* key, int32_t* val, const float* key_in, const int32_t* val_in,
                                                   int64_t b, int len, int lane) {
-  uint64_t v[E];
+  double v[E];
 #pragma unroll
   for (int i = 0; i < E; i++) {
-    const int idx = i * 64 + lane;
-    v[i] = idx < len ? kv_pack(key_in[b + idx], val_in[b + idx]) : ~0ull;
+    const int idx = i * 64 + lane;  // any assignment will do before the sort: the coalesced one
+    v[i] = idx < len ? kv_pack(key_in[b + idx], val_in[b + idx]) : kv_last();
   }
-  wave_bitonic_sort<E>(v, lane);
+  wave_merge<E, 2>(v, lane);
 #pragma unroll
   for (int i = 0; i < E; i++) {
-    const int idx = i * 64 + lane;
+    const int idx = lane * E + i;
     if (idx < len) {
       key[b + idx] = kv_key(v[i]);
-      val[b + idx] = (int32_t)(uint32_t)v[i];
+      val[b + idx] = kv_val(v[i]);
     }
   }
 }
 
+// Segments too long for one wave: n, then their indices (a segment of more than kWaveSortMax entries
+// each, so nmax / kWaveSortMax of them at most).  Null: the long-segment kernels look at every segment.
+inline int64_t seg_queue_words(int64_t nmax) { return nmax / kWaveSortMax + 1; }
+
 // Segments of up to kWaveSortMax entries, one wave each (in place allowed: a wave reads its whole
-// segment into registers before writing); longer ones are left to k_segment_sort.
+// segment into registers before writing); longer ones are queued for k_segment_sort.
 __global__ __launch_bounds__(64) void k_segment_sort_wave(const int32_t* __restrict__ spl, float* key, int32_t* val,
-                                                          const float* key_in, const int32_t* val_in, int64_t nmax, int64_t nitems) {
+                                                          const float* key_in, const int32_t* val_in, int64_t nmax,
+                                                          int64_t nitems, int32_t* __restrict__ queue) {
   const int64_t nact_ = active_items(spl, nitems);
-  for (int seg = blockIdx.x; seg < nact_; seg += gridDim.x) {
-    const int lane = threadIdx.x;
+  const int lane = threadIdx.x;
+  for (int64_t seg = blockIdx.x; seg < nact_; seg += gridDim.x) {
     int64_t b = spl[seg], e = spl[seg + 1];
     if (e > nmax) e = nmax;
     if (b >= e) continue;
     const int64_t len = e - b;
-    if (len > kWaveSortMax) continue;
+    if (len > kWaveSortMax) {
+      if (queue && lane == 0) queue[1 + atomicAdd(queue, 1)] = (int32_t)seg;
+      continue;
+    }
     if (len <= 64) wave_sort_segment<1>(key, val, key_in, val_in, b, (int)len, lane);
     else if (len <= 128) wave_sort_segment<2>(key, val, key_in, val_in, b, (int)len, lane);
     else if (len <= 256) wave_sort_segment<4>(key, val, key_in, val_in, b, (int)len, lane);
     else if (len <= 512) wave_sort_segment<8>(key, val, key_in, val_in, b, (int)len, lane);
     else wave_sort_segment<16>(key, val, key_in, val_in, b, (int)len, lane);
-  
   }
 }
 
-// One workgroup per segment.  Segments up to kSegLds entries are sorted in LDS; longer ones in
+// One workgroup per segment of more than LO entries: up to CAP in LDS; longer ones, where BIG, in
 // place in the output arrays (global memory, visible within the workgroup across barriers).
-__global__ __launch_bounds__(kSegThreads) void k_segment_sort(const int32_t* __restrict__ spl, float* key,
-                                                              int32_t* val, const float* key_in, const int32_t* val_in,
-                                                              int64_t nmax, int skip_short, int64_t nitems) {
-  __shared__ uint64_t s_a[kSegLds];
-  const int64_t nact_ = active_items(spl, nitems);
-  for (int seg = blockIdx.x; seg < nact_; seg += gridDim.x) {
+template <int NT, int LO, int CAP, bool BIG>
+__global__ __launch_bounds__(NT) void k_segment_sort(const int32_t* __restrict__ spl, float* key, int32_t* val,
+                                                     const float* key_in, const int32_t* val_in, int64_t nmax,
+                                                     int64_t nitems, const int32_t* __restrict__ queue) {
+  __shared__ double s_a[CAP];
+  const int64_t nseg = queue ? (int64_t)queue[0] : active_items(spl, nitems);
+  for (int64_t it = blockIdx.x; it < nseg; it += gridDim.x) {
+    const int64_t seg = queue ? (int64_t)queue[1 + it] : it;
     int64_t b = spl[seg], e = spl[seg + 1];
     if (e > nmax) e = nmax;
-    if (b >= e) continue;
+    if (e - b <= LO || (!BIG && e - b > CAP)) continue;
     const int len = (int)(e - b);
-    if (len <= kWaveSortMax && skip_short) continue;  // done by k_segment_sort_wave
-    if (len <= kSegLds) {
-      for (int i = threadIdx.x; i < len; i += blockDim.x) s_a[i] = kv_pack(key_in[b + i], val_in[b + i]);
+    if (len <= CAP) {
+      for (int i = threadIdx.x; i < len; i += NT) s_a[i] = kv_pack(key_in[b + i], val_in[b + i]);
       __syncthreads();
       bitonic_sort_asc(LdsArr{s_a}, len);
-      for (int i = threadIdx.x; i < len; i += blockDim.x) {
+      for (int i = threadIdx.x; i < len; i += NT) {
         key[b + i] = kv_key(s_a[i]);
-        val[b + i] = (int32_t)(uint32_t)s_a[i];
+        val[b + i] = kv_val(s_a[i]);
       }
     } else {
       if (key != key_in) {
-        for (int i = threadIdx.x; i < len; i += blockDim.x) {
+        for (int i = threadIdx.x; i < len; i += NT) {
           key[b + i] = key_in[b + i];
           val[b + i] = val_in[b + i];
         }
@@ -533,7 +704,6 @@ __global__ __launch_bounds__(kSegThreads) void k_segment_sort(const int32_t* __r
       bitonic_sort_asc(GlobalKV{key + b, val + b}, len);
     }
     __syncthreads();  // the next segment reuses s_a
-  
   }
 }
 
@@ -702,16 +872,30 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(W))) void k_
   }
 }
 
-// Sort each segment by (key, val): segments up to kWaveSortMax entries one wave each in registers,
-// longer ones by a workgroup (LDS up to kSegLds entries, else in place in global memory).
+// Sort each segment by (key, val): segments of up to kWaveSortMax entries one wave each in registers,
+// longer ones by a workgroup (in LDS up to kSegBigLds entries, else in place in global memory).
+// queue (seg_queue_words(nmax) words, or null): the long segments, found by the first kernel.  A segment
+// has no more than max_len entries, so kernels for longer ones than that are not launched.  Lists of 4096
+// to 16384 entries (the nodes around a void; 200 of 548,000 at 2^24, leaf 48) are sorted in 128 KB of LDS:
+// in global memory they took 3.1 ms together, 0.9 now.
 int segment_sort(hipStream_t s, const int32_t* spl, float* key, int32_t* val, const float* key_in,
-                 const int32_t* val_in, int64_t nseg, int64_t nmax, const char* what) {
+                 const int32_t* val_in, int64_t nseg, int64_t nmax, int64_t max_len, int32_t* queue, const char* what) {
   if (nseg <= 0) return 0;
-  hipLaunchKernelGGL(k_segment_sort_wave, dim3(grid_for(nseg)), dim3(64), 0, s, spl, key, val, key_in, val_in, nmax, nseg);
+  if (queue && max_len > kWaveSortMax && fill_u32(s, queue, 0u, 1)) return 1;
+  // four times the waves that the chip holds: workgroups stride over the segments
+  const unsigned gw = (unsigned)(nseg < 32768 ? nseg : 32768);
+  hipLaunchKernelGGL(k_segment_sort_wave, dim3(gw), dim3(64), 0, s, spl, key, val, key_in, val_in, nmax, nseg,
+                     max_len > kWaveSortMax ? queue : nullptr);
   if (check_launch(what)) return 1;
-  // the two kernels touch disjoint segments
-  hipLaunchKernelGGL(k_segment_sort, dim3(grid_for(nseg)), dim3(kSegThreads), 0, s, spl, key, val, key_in, val_in, nmax,
-                     1, nseg);
+  // the kernels touch disjoint segments; without a queue their workgroups go over all of them
+  if (max_len > kWaveSortMax)
+    hipLaunchKernelGGL((k_segment_sort<kSegThreads, kWaveSortMax, kSegLds, false>),
+                       dim3((unsigned)(nseg < 4096 ? nseg : 4096)), dim3(kSegThreads), 0, s, spl, key, val, key_in,
+                       val_in, nmax, nseg, queue);
+  if (max_len > kSegLds)
+    hipLaunchKernelGGL((k_segment_sort<kSegBigThreads, kSegLds, kSegBigLds, true>),
+                       dim3((unsigned)(nseg < 1024 ? nseg : 1024)), dim3(kSegBigThreads), 0, s, spl, key, val, key_in,
+                       val_in, nmax, nseg, queue);
   return check_launch(what);
 }
 
@@ -766,44 +950,52 @@ __global__ void k_segment_max(const int32_t* __restrict__ spl, const float* __re
 
 template <int D, typename T>
 int node2node_impl(hipStream_t s, const int32_t* pil_spl, const int32_t* pil_src, const float* pil_r2,
-                   const int32_t* parent_spl, const void* nodes, const int32_t* npart, const float* rmax2_in,
+                   const int32_t* parent_spl, const void* nodes, const int32_t* npart, const float* parent_rmax2,
+                   const float* rmax2_in,
                    float* rmax2, int32_t* il_spl, int32_t* il_src, float* il_r2, int64_t size_parents,
-                   int64_t size_nodes, int64_t pil_size, int64_t il_size, int k, float boxsize) {
+                   int64_t size_nodes, int64_t pil_size, int64_t il_size, int k, float boxsize, void* tmp,
+                   size_t tmp_bytes) {
   const T* nd = (const T*)nodes;
   if (fill_u32(s, il_spl, 0u, size_nodes + 1)) return 1;
   if (size_parents <= 0) return 0;
-  dim3 g(grid_for(size_parents)), b(64);
+  const dim3 g(node_grid(size_parents, 64)), b(64), gl(node_grid(size_parents, kNodeThreads)), bl(kNodeThreads);
+  // without room for the queue, one-wave workgroups run the long lists too
+  const bool split = tmp && tmp_bytes >= 4 * (size_t)node_queue_words(size_parents);
+  const NodeQueue queue{split ? (int32_t*)tmp : nullptr, size_parents};
+  if (split && fill_u32(s, tmp, 0u, 1)) return 1;
+#define JZT_NODE_COUNT(RADIUS)                                                                                        \
+  do {                                                                                                                \
+    hipLaunchKernelGGL((k_node_count<RADIUS, 64, D, T>), g, b, 0, s, pil_spl, pil_src, pil_r2, parent_spl, nd, npart, \
+                       parent_rmax2, rmax2, il_spl + 1, k, (T)boxsize, pil_size, size_parents, queue);                              \
+    if (split)                                                                                                        \
+      hipLaunchKernelGGL((k_node_count<RADIUS, kNodeThreads, D, T>), gl, bl, 0, s, pil_spl, pil_src, pil_r2,          \
+                         parent_spl, nd, npart, parent_rmax2, rmax2, il_spl + 1, k, (T)boxsize, pil_size,             \
+                         size_parents, queue);                                                                        \
+  } while (0)
   if (rmax2_in) {
     if (size_nodes > 0)
       hipLaunchKernelGGL(k_scale_rmax2, dim3((unsigned)div_up(size_nodes, 256)), dim3(256), 0, s, rmax2_in, rmax2,
                          size_nodes);
+    JZT_NODE_COUNT(false);
   } else {
-    // parents with at most kRmaxGroup children: several per wave; the others: one wave each
-    constexpr int G = kRmaxGroup;
-    dim3 gg(grid_for(div_up(size_parents, 64 / G)));
-#define JZT_FIND_RMAX(KB)                                                                                           \
-  do {                                                                                                              \
-    hipLaunchKernelGGL((k_find_rmax_groups<KB, D, T, G>), gg, b, 0, s, pil_spl, pil_src, pil_r2, parent_spl, nd,   \
-                       npart, rmax2, k, (T)boxsize, pil_size, size_parents);                                        \
-    hipLaunchKernelGGL((k_find_rmax<KB, D, T>), g, b, 0, s, pil_spl, pil_src, pil_r2, parent_spl, nd, npart, rmax2, \
-                       k, (T)boxsize, pil_size, size_parents, G);                                                   \
-  } while (0)
-    if (k <= 16) JZT_FIND_RMAX(8);
-    else if (k <= 32) JZT_FIND_RMAX(16);
-    else JZT_FIND_RMAX(32);
-#undef JZT_FIND_RMAX
+    JZT_NODE_COUNT(true);
   }
-  if (check_launch("KnnNode2Node FindRmax")) return 1;
-  hipLaunchKernelGGL((k_count_insert<0, D, T>), g, b, 0, s, pil_spl, pil_src, pil_r2, parent_spl, nd, rmax2, il_spl + 1,
-                     (const int32_t*)nullptr, (int32_t*)nullptr, (float*)nullptr, il_size, (T)boxsize, pil_size, size_parents);
+#undef JZT_NODE_COUNT
+  if (check_launch("KnnNode2Node count")) return 1;
   // inclusive scan of the counts in place; the scan temp lives in the (not yet written) list
   if (scan_tmp_words(size_nodes) > il_size) return fail("KnnNode2Node: interaction list too small for scan temp");
   if (scan_i32(s, il_spl + 1, il_spl + 1, size_nodes, true, il_src)) return 1;
-  hipLaunchKernelGGL((k_count_insert<1, D, T>), g, b, 0, s, pil_spl, pil_src, pil_r2, parent_spl, nd, rmax2,
-                     (int32_t*)nullptr, il_spl, il_src, il_r2, il_size, (T)boxsize, pil_size, size_parents);
+  hipLaunchKernelGGL((k_node_insert<64, D, T>), g, b, 0, s, pil_spl, pil_src, pil_r2, parent_spl, nd, rmax2, il_spl,
+                     il_src, il_r2, il_size, (T)boxsize, pil_size, size_parents, queue);
+  if (split)
+    hipLaunchKernelGGL((k_node_insert<kNodeThreads, D, T>), gl, bl, 0, s, pil_spl, pil_src, pil_r2, parent_spl, nd, rmax2,
+                       il_spl, il_src, il_r2, il_size, (T)boxsize, pil_size, size_parents, queue);
   if (check_launch("KnnNode2Node insert")) return 1;
   // sort each node's list by (r2, src) in place
-  return segment_sort(s, il_spl, il_r2, il_src, il_r2, il_src, size_nodes, il_size, "KnnNode2Node sort");
+  // (a list names every node at most once)
+  const size_t qoff = align256(4 * (size_t)node_queue_words(size_parents));
+  int32_t* sq = tmp && tmp_bytes >= qoff + 4 * (size_t)seg_queue_words(il_size) ? (int32_t*)((char*)tmp + qoff) : nullptr;
+  return segment_sort(s, il_spl, il_r2, il_src, il_r2, il_src, size_nodes, il_size, size_nodes, sq, "KnnNode2Node sort");
 }
 
 template <int D>
@@ -878,6 +1070,10 @@ extern "C" int jzt_knn_node2node(jzt_stream_t stream, const int32_t* parent_ilis
                               size_parents, size_nodes, parent_ilist_size, node_ilist_size, k, boxsize, dim, dtype);
 }
 
+extern "C" size_t jzt_knn_node2node_tmp_bytes(int64_t size_parents, int64_t node_ilist_size) {
+  return align256(4 * (size_t)node_queue_words(size_parents)) + 4 * (size_t)seg_queue_words(node_ilist_size);
+}
+
 extern "C" int jzt_knn_node2node_ex(jzt_stream_t stream, const int32_t* parent_ilist_spl,
                                     const int32_t* parent_ilist_isrc, const float* parent_ilist_r2,
                                     const int32_t* parent_spl, const void* nodes, const int32_t* nodes_npart,
@@ -885,13 +1081,26 @@ extern "C" int jzt_knn_node2node_ex(jzt_stream_t stream, const int32_t* parent_i
                                     int32_t* node_ilist_isrc, float* node_ilist_r2, int64_t size_parents,
                                     int64_t size_nodes, int64_t parent_ilist_size, int64_t node_ilist_size, int k,
                                     float boxsize, int dim, int dtype) {
+  return jzt_knn_node2node_tmp(stream, parent_ilist_spl, parent_ilist_isrc, parent_ilist_r2, parent_spl, nodes,
+                               nodes_npart, nullptr, node_r2_in, node_rmax2, node_ilist_spl, node_ilist_isrc, node_ilist_r2,
+                               size_parents, size_nodes, parent_ilist_size, node_ilist_size, k, boxsize, dim, dtype,
+                               nullptr, 0);
+}
+
+extern "C" int jzt_knn_node2node_tmp(jzt_stream_t stream, const int32_t* parent_ilist_spl,
+                                    const int32_t* parent_ilist_isrc, const float* parent_ilist_r2,
+                                    const int32_t* parent_spl, const void* nodes, const int32_t* nodes_npart,
+                                    const float* parent_rmax2, const float* node_r2_in, float* node_rmax2, int32_t* node_ilist_spl,
+                                    int32_t* node_ilist_isrc, float* node_ilist_r2, int64_t size_parents,
+                                    int64_t size_nodes, int64_t parent_ilist_size, int64_t node_ilist_size, int k,
+                                    float boxsize, int dim, int dtype, void* tmp, size_t tmp_bytes) {
   hipStream_t s = (hipStream_t)stream;
   if (k < 1) return fail("KnnNode2Node: k must be >= 1");
   // dims 2-10, float or double node geometry (_generate_ffi.py:9-21)
 #define JZT_N2N(D, T)                                                                                              \
   return node2node_impl<D, T>(s, parent_ilist_spl, parent_ilist_isrc, parent_ilist_r2, parent_spl, nodes,         \
-                              nodes_npart, node_r2_in, node_rmax2, node_ilist_spl, node_ilist_isrc, node_ilist_r2, \
-                              size_parents, size_nodes, parent_ilist_size, node_ilist_size, k, boxsize)
+                              nodes_npart, parent_rmax2, node_r2_in, node_rmax2, node_ilist_spl, node_ilist_isrc, node_ilist_r2, \
+                              size_parents, size_nodes, parent_ilist_size, node_ilist_size, k, boxsize, tmp, tmp_bytes)
 #define JZT_N2N_DIM(D)                  \
   case D:                               \
     if (dtype == JZT_F32) JZT_N2N(D, float); \
@@ -976,5 +1185,6 @@ extern "C" int jzt_segment_sort(jzt_stream_t stream, const int32_t* spl, const f
                                 float* key_out, int32_t* val_out, int64_t size_segs, int64_t size_keys) {
   hipStream_t s = (hipStream_t)stream;
   if (size_segs <= 0) return 0;
-  return segment_sort(s, spl, key_out, val_out, key, val, size_segs, size_keys, "SegmentSort");
+  return segment_sort(s, spl, key_out, val_out, key, val, size_segs, size_keys, size_keys, nullptr,
+                      "SegmentSort");
 }

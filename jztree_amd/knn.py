@@ -96,12 +96,15 @@ _knn_leaf2leaf.jit = _knn_leaf2leaf
 
 
 def _knn_node2node_ilist(ilist: InteractionList, spl_parent, node_data: PosLvlNum, k: int = 32,
-                         boxsize: float = 0., with_radii: bool = False, rmax2_in=None, overflow: list | None = None):
+                         boxsize: float = 0., with_radii: bool = False, rmax2_in=None, overflow: list | None = None,
+                         parent_rmax2=None):
     """knn.py:62-110 -> KnnNode2Node.
 
     rmax2_in (extension): search radius^2 per node instead of the guaranteed k-neighbour radius;
     each list then holds every node within rmax2_in * (1 + 2^-16).  overflow (extension): instead of
-    raising on a too small list, append the device flag "list overflowed" to this list."""
+    raising on a too small list, append the device flag "list overflowed" to this list.
+    parent_rmax2 (extension): the parents' radius^2 from the plane above (with_radii), from which the
+    search for the children's starts."""
     boxsize = 0. if boxsize is None else boxsize
     assert ilist.ispl.shape[0] == spl_parent.shape[0]
     assert ilist.isrc.shape == ilist.rad2.shape
@@ -115,10 +118,12 @@ def _knn_node2node_ilist(ilist: InteractionList, spl_parent, node_data: PosLvlNu
     npart = node_data.npart.to(torch.int32).contiguous()
     r2in = None if rmax2_in is None else rmax2_in.to(torch.float32).contiguous()
     assert r2in is None or r2in.shape[0] >= size
-    L.call("jzt_knn_node2node_ex", L.stream(), L.ptr(ilist.ispl), L.ptr(ilist.isrc), L.ptr(ilist.rad2),
-           L.ptr(spl_parent.contiguous()), L.ptr(poslvl), L.ptr(npart), L.ptr(r2in), L.ptr(radii), L.ptr(ispl),
+    nb = L.LIB.jzt_knn_node2node_tmp_bytes(spl_parent.shape[0] - 1, ilist.size())
+    tmp = _tmp(nb, dev)
+    L.call("jzt_knn_node2node_tmp", L.stream(), L.ptr(ilist.ispl), L.ptr(ilist.isrc), L.ptr(ilist.rad2),
+           L.ptr(spl_parent.contiguous()), L.ptr(poslvl), L.ptr(npart), L.ptr(parent_rmax2), L.ptr(r2in), L.ptr(radii), L.ptr(ispl),
            L.ptr(il), L.ptr(ilr2), spl_parent.shape[0] - 1, size, ilist.size(), ilist.size(), int(k),
-           float(boxsize), node_data.pos.shape[-1], L.dtype_code(node_data.pos.dtype))
+           float(boxsize), node_data.pos.shape[-1], L.dtype_code(node_data.pos.dtype), L.ptr(tmp), nb)
     if overflow is not None:  # the caller checks (and handles) overflow itself
         overflow.append(ispl[-1] > il.numel())
     else:
@@ -148,7 +153,8 @@ def _knn_dual_walk(th: TreeHierarchy, k: int, boxsize: float | None = None,
         parent_spl = spl_n2n.get(level + 1, size + 1)
         node_data = PosLvlNum(pos=th.geom_cent.get(level, size), lvl=th.lvl.get(level, size),
                               npart=th.npart(level, size=size, ptype=0))
-        ilist, rmax2 = _knn_node2node_ilist(ilist, parent_spl, node_data, k=k, boxsize=boxsize, with_radii=True)
+        ilist, rmax2 = _knn_node2node_ilist(ilist, parent_spl, node_data, k=k, boxsize=boxsize, with_radii=True,
+                                            parent_rmax2=rmax2)
     if return_parents:
         return ilist, rmax2, spl_n2n.get(stop_level, size + 1)
     return ilist
