@@ -2,6 +2,8 @@
 
 Segment sort: lengths around the powers of two of the one-wave sort (64 to 1024 entries), of the LDS sorts
 (4096, 16384) and beyond, negative keys, equal keys, against numpy's lexicographic order.
+FofNode2Node at every number of children per work item, against the oracle.
+FofNode2Node: joined nodes and lists against all pairs, at every number of children per work item.
 Node lists: every child's radius against the exact weighted selection and every list against all pairs,
 with parents whose lists are short (one wave) and long (queued), fewer and more than 64 particles of
 candidates per child, one and several children per work item."""
@@ -118,3 +120,69 @@ def test_node_lists_against_all_pairs(dev, nparents, kids, k, box):
         pos = rr >= 0
         assert np.allclose(rr[pos], dmin[i][got[pos]], rtol=2.0 ** -18, atol=0)
         assert (dmin[i][got[~pos]] <= 1e-12).all()
+
+
+@pytest.mark.parametrize("nparents,kids", [(3, 9), (130, 20), (300, 12), (1100, 3)])  # every width of a work item
+def test_fof_node_passes_against_all_pairs(dev, nparents, kids):
+    """FofNode2Node on a dense parent list: nodes joined by guaranteed pairs share the smallest index of their
+    set, and the lists hold every other pair that may link, each parent pair once."""
+    import jztree_amd as jz
+    from jztree_amd.data import InteractionList
+    from jztree_amd.fof import PosLvl, _fof_node2node
+    rng = np.random.default_rng(nparents)
+    dim, f32 = 3, np.float32
+    nch = rng.integers(0, kids + 1, size=nparents)
+    nch[0] = kids
+    spl = np.concatenate([[0], np.cumsum(nch)]).astype(np.int32)
+    n = int(spl[-1])
+    parent = np.repeat(np.arange(nparents), nch)
+    lvl = rng.integers(-24, -12, size=n).astype(np.int32)
+    cent = rng.random((n, dim)).astype(f32)
+    cent[: n // 2] *= f32(0.1)
+    rlink = 0.02
+    t = lambda a: torch.from_numpy(a).to(dev)
+    size_il = max(n * n, nparents * nparents, 64)
+    il = torch.zeros(size_il, dtype=torch.int32, device=dev)
+    il[: nparents * nparents] = t(np.tile(np.arange(nparents, dtype=np.int32), nparents))
+    dense = InteractionList(t((np.arange(nparents + 1) * nparents).astype(np.int32)), il)
+    ig, out = _fof_node2node(dense, t(spl), PosLvl(t(cent), t(lvl)), torch.arange(n, dtype=torch.int32, device=dev),
+                             rlink=rlink, boxsize=1.0)
+    jz.checks.flush()
+    ig, ispl, src = ig.cpu().numpy()[:n], out.ispl.cpu().numpy(), out.isrc.cpu().numpy()
+    e = _half_ext(lvl, dim).astype(f32)
+    d = cent[None] - cent[:, None]
+    d = np.where(d < -f32(0.5), d + f32(1), d)
+    d = np.where(d >= f32(0.5), d - f32(1), d)
+    w = e[:, None] + e[None]
+
+    def norm2(v):
+        r = np.zeros(v.shape[:-1], dtype=f32)
+        for i in range(dim):
+            x = v[..., i].astype(np.float64)
+            r = (x * x + r).astype(f32)
+        return r.astype(np.float64)
+
+    dmin, dmax = norm2(np.maximum(np.abs(d) - w, f32(0))), norm2(np.abs(d) + w)
+    diag = norm2(e) * 4
+    r2 = float(f32(rlink * rlink))
+    tol = 2.0 ** -20  # float32 sums of three fused steps
+    once = parent[None] >= parent[:, None]
+    bound = np.maximum(dmax, diag[None])
+    surely = once & (bound <= r2 * (1 - 2.0 ** -16) * (1 - tol))
+    maybe = once & (bound <= r2 * (1 - 2.0 ** -16) * (1 + tol))
+    assert (surely == maybe).all()  # no pair at the edge of the test
+    root = np.arange(n)
+    for i, j in zip(*np.nonzero(surely)):
+        a, b = root[i], root[j]
+        if a != b:
+            root[root == max(a, b)] = min(a, b)
+    assert np.array_equal(ig, root)
+    rest = once & ~surely & ((root[:, None] != root[None]) | np.eye(n, dtype=bool))
+    need = rest & (dmin < r2 * (1 + 2.0 ** -16) * (1 - tol))
+    may = rest & (dmin <= r2 * (1 + 2.0 ** -16) * (1 + tol))
+    got = np.zeros((n, n), dtype=bool)
+    for i in range(n):
+        assert len(np.unique(src[ispl[i]:ispl[i + 1]])) == ispl[i + 1] - ispl[i]
+        got[i, src[ispl[i]:ispl[i + 1]]] = True
+    assert not (need & ~got).any() and not (got & ~may).any()
+    assert need.any()
