@@ -210,9 +210,10 @@ class CapturedSets:
         nsets = len(self.off) - 1
         self.r2set = _r2_per_set(rlink, nsets, dev)
         cfg_tree = cfg_tree if cfg_tree is not None else KNNConfig().tree
-        args = (k, self.r2set, boxsize, cfg_tree, alloc_fac_ilist_knn, alloc_fac_ilist_fof)
-        self._step = lambda: _pipeline_core(self.pos, self.off, *args)
-        self._g = Captured(self._step)
+        # no reference to self in the captured callable: the object, and with it the graph, is then freed
+        # when its last user drops it and not by a later garbage collection (see Captured)
+        args = (self.pos, self.off, k, self.r2set, boxsize, cfg_tree, alloc_fac_ilist_knn, alloc_fac_ilist_fof)
+        self._g = Captured(lambda: _pipeline_core(*args))
         self.graph = self._g.graph
         self.out = self._g.out
         self.node_counts = self._g.node_counts

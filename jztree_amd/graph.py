@@ -15,6 +15,7 @@ tensors the callable closes over: copy new data into them (same shapes) between 
 """
 from __future__ import annotations
 
+import gc
 from typing import Any, Callable
 
 import torch
@@ -42,12 +43,20 @@ class Captured:
             torch.cuda.synchronize()
         self.graph = torch.cuda.CUDAGraph(keep_graph=True)
         checks.clear()
+        # No garbage collection while the stream is capturing: freeing another graph then (one held by
+        # a reference cycle) synchronises the device in its destructor, which a capture does not
+        # permit, and the error ends the process.
+        collecting = gc.isenabled()
+        gc.disable()
         try:
             with checks.deferred(), torch.cuda.graph(self.graph):
                 self.out = fn()
         except BaseException:
             checks.clear()
             raise
+        finally:
+            if collecting:
+                gc.enable()
         self._conds = checks.take()
         counts = torch.zeros(4, dtype=torch.int64)
         L.call("jzt_graph_count_nodes", self.graph.raw_cuda_graph(), counts.data_ptr())

@@ -58,3 +58,28 @@ def test_captured_knn_learned_fof_replays(dev, boxsize):
             assert torch.equal(a, b), f"replay {rep} (input {which}): {name} differ from the eager call"
         _ = torch.cumsum(inputs[1][:, 0], 0)  # eager work between replays
         torch.cuda.synchronize()
+
+
+def test_captured_objects_are_freed_without_garbage_collection(dev):
+    """A captured graph held by a reference cycle would be freed by a later collection, possibly within
+    another capture, where its destructor's device synchronisation is an error that ends the process."""
+    import gc
+    import weakref
+    import jztree_amd as jz
+    x = torch.rand((600, 3), device=dev)
+    was = gc.isenabled()
+    gc.disable()
+    try:
+        g = jz.batch.CapturedSets(x, [256, 344], k=4, rlink=0.05, boxsize=1.0)
+        assert not gc.isenabled()  # as it was before
+        g.run(x)
+        torch.cuda.synchronize()
+        ref, inner = weakref.ref(g), weakref.ref(g._g)
+        del g
+        assert ref() is None and inner() is None
+    finally:
+        if was:
+            gc.enable()
+    seen = []
+    jz.graph.Captured(lambda: seen.append(gc.isenabled()) or torch.zeros(4, device=dev))
+    assert seen == [was, False] and gc.isenabled() == was  # the eager run, then the capture
