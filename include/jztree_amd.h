@@ -199,6 +199,13 @@ int jzt_regularization_level(jzt_stream_t stream, const int32_t* lvl, const int3
 int jzt_dense_ilist(jzt_stream_t stream, const int32_t* nnodes, int ngroup, int32_t* spl_super, int32_t* ispl,
                     int64_t size_super, int32_t* ilist, float* r2, int64_t size_ilist, int32_t* nsuper);
 
+/* jzt_dense_ilist with the node count read as node_spl[plane + 1] - node_spl[plane], and two checks (extension):
+ * err[0] = the list does not fit into size_ilist, err[1] = nsuper + 1 more splits after *nfilled do not fit
+ * into `space` slots. */
+int jzt_dense_ilist_top(jzt_stream_t stream, const int32_t* node_spl, int plane, int ngroup, int32_t* spl_super,
+                        int32_t* ispl, int64_t size_super, int32_t* ilist, float* r2, int64_t size_ilist,
+                        int32_t* nsuper, const int32_t* nfilled, int64_t space, uint8_t* err);
+
 /* jzt_dense_ilist_sets: jzt_dense_ilist for a batch (no counterpart in the reference).  node_set
  * (int32, non-decreasing over the first *nnodes entries, values in [0, nsets)) names the set of
  * each top-plane node.  The c_s nodes of set s form ceil(c_s/ngroup) super-nodes (numbered set
@@ -241,7 +248,8 @@ int jzt_knn_node2node_ex(jzt_stream_t stream, const int32_t* parent_ilist_spl, c
 
 /* jzt_knn_node2node_ex with scratch (jzt_knn_node2node_tmp_bytes bytes): parents with long lists and
  * long lists themselves are queued there and get larger workgroups.  tmp may be NULL.
- * parent_rmax2 (may be NULL): the parents' guaranteed radius^2, where the children's search starts. */
+ * parent_rmax2 (may be NULL): the parents' guaranteed radius^2, where the children's search starts.
+ * overflow (may be NULL): receives whether the lists need more than node_ilist_size entries. */
 size_t jzt_knn_node2node_tmp_bytes(int64_t size_parents, int64_t node_ilist_size);
 int jzt_knn_node2node_tmp(jzt_stream_t stream, const int32_t* parent_ilist_spl, const int32_t* parent_ilist_isrc,
                           const float* parent_ilist_r2, const int32_t* parent_spl, const void* nodes,
@@ -249,7 +257,7 @@ int jzt_knn_node2node_tmp(jzt_stream_t stream, const int32_t* parent_ilist_spl, 
                           int32_t* node_ilist_spl, int32_t* node_ilist_isrc, float* node_ilist_r2,
                           int64_t size_parents, int64_t size_nodes, int64_t parent_ilist_size,
                           int64_t node_ilist_size, int k, float boxsize, int dim, int dtype, void* tmp,
-                          size_t tmp_bytes);
+                          size_t tmp_bytes, uint8_t* overflow);
 
 
 /* Regularization's extra leaf splits (tree.py:236-243 of the reference, one kernel here):
@@ -383,6 +391,31 @@ int jzt_adam_step(jzt_stream_t stream, float* w, uint16_t* wq, float* m, float* 
                   float lr, float beta1, float beta2, float eps, int step);
 int jzt_to_bf16(jzt_stream_t stream, const float* w, uint16_t* wq, int64_t n);
 
+/* The hierarchy of z-sorted positions in one call (extension; tree.py:189-262 and :600-829 of the reference are the
+ * steps): leaf splits, plane activity, packed split arrays, node levels and centres.
+ * set_id (size_part, non-decreasing) with leaf_set (alloc_size - 1, output), or both NULL: a batch of sets.
+ * The filled rows are *npart (device), else npart_host, else (npart NULL, npart_host < 0) the rows whose first
+ * coordinate is not NaN; rows with a NaN come last.  node_sizes (host, nplanes): largest node per plane.
+ * Outputs: leaf_spl, n2l, n2n (alloc_size each), level_spl, prop_spl (nplanes + 1), n2l_fill, n2n_fill, lvl_fill,
+ * cent_fill (nplanes), lvl and cent (alloc_size - nplanes rows), counts = {leaf splits found, nplanes},
+ * err = {leaf splits exceed alloc_size, node splits exceed it}. */
+size_t jzt_build_tree_tmp_bytes(int64_t size_part, int64_t alloc_size, int nplanes, int dim, int dtype, int regularize);
+int jzt_build_tree(jzt_stream_t stream, const void* posz, const int32_t* set_id, const int32_t* npart,
+                   int64_t npart_host, int64_t size_part, int dim, int dtype, const int32_t* node_sizes, int nplanes,
+                   int64_t alloc_size, int regularize, float max_volume_fac, float min_percentile, int32_t* leaf_spl,
+                   int32_t* n2l, int32_t* n2n, int32_t* level_spl, int32_t* n2l_fill, int32_t* n2n_fill, int32_t* lvl,
+                   void* cent, int32_t* prop_spl, int32_t* lvl_fill, void* cent_fill, int32_t* counts,
+                   int32_t* leaf_set, uint8_t* err, void* tmp, size_t tmp_bytes);
+
+/* Per plane p (extension): child splits out_spl (nplanes, size_nodes + 1), padded with the plane's fill value, and
+ * for the plane's nodes out_nodes (dim + 1 columns; the level bits last), out_lvl and out_npart (size_nodes + 1 rows per
+ * plane); rows past the nodes are not written. */
+int jzt_plane_tables(jzt_stream_t stream, const int32_t* n2n, const int32_t* n2l, const int32_t* level_spl,
+                     const int32_t* n2n_fill, const int32_t* n2l_fill, const int32_t* lvl, const void* cent,
+                     const int32_t* prop_spl, const int32_t* leaf_spl, int64_t size_leaf_spl, int nplanes,
+                     int64_t size_nodes, int dim, int dtype, int32_t* out_spl, void* out_nodes, int32_t* out_lvl,
+                     int32_t* out_npart);
+
 /* ------------------------------------------------------------------------------------------ */
 /* friends-of-friends                                                                           */
 /* ------------------------------------------------------------------------------------------ */
@@ -400,6 +433,14 @@ int jzt_fof_node2node(jzt_stream_t stream, const int32_t* parent_ilist_spl, cons
                       int32_t* node_igroup, int32_t* node_ilist_spl, int32_t* node_ilist, int64_t size_parent,
                       int64_t size_node, int64_t parent_ilist_size, int64_t size_node_ilist, float r2link,
                       float boxsize, int dim, int dtype);
+
+/* FofNode2Node of one linking length (parent_r2link NULL) or one per parent, without clearing the unused part of
+ * node_ilist (extension).  overflow (may be NULL): whether the lists need more than size_node_ilist entries. */
+int jzt_fof_node2node_ex(jzt_stream_t stream, const int32_t* parent_ilist_spl, const int32_t* parent_ilist,
+                         const int32_t* parent_spl, const float* parent_r2link, const void* nodes,
+                         const int32_t* node_igroup_in, int32_t* node_igroup, int32_t* node_ilist_spl,
+                         int32_t* node_ilist, int64_t size_parent, int64_t size_node, int64_t parent_ilist_size,
+                         int64_t size_node_ilist, float r2link, float boxsize, int dim, int dtype, uint8_t* overflow);
 
 /* FofLeaf2Leaf -- replaces ffi target "FofLeaf2Leaf" (generated/ffi_fof.cu:277-406, host
  * fof.cuh:349-379, caller fof.py:153-169).  part_igroup = min z-index of each particle's group. */

@@ -57,7 +57,14 @@ _SIGNATURES = {
                               _f32, _i32, _i32], _i32),
     "jzt_knn_node2node_tmp_bytes": ([_i64, _i64], _sz),
     "jzt_knn_node2node_tmp": ([_p, _p, _p, _p, _p, _p, _p, _p, _p, _p, _p, _p, _p, _i64, _i64, _i64, _i64, _i32,
-                               _f32, _i32, _i32, _p, _sz], _i32),
+                               _f32, _i32, _i32, _p, _sz, _p], _i32),
+    "jzt_dense_ilist_top": ([_p, _p, _i32, _i32, _p, _p, _i64, _p, _p, _i64, _p, _p, _i64, _p], _i32),
+    "jzt_build_tree_tmp_bytes": ([_i64, _i64, _i32, _i32, _i32, _i32], _sz),
+    "jzt_build_tree": ([_p, _p, _p, _p, _i64, _i64, _i32, _i32, _p, _i32, _i64, _i32, _f32, _f32, _p, _p, _p, _p, _p,
+                        _p, _p, _p, _p, _p, _p, _p, _p, _p, _p, _sz], _i32),
+    "jzt_plane_tables": ([_p, _p, _p, _p, _p, _p, _p, _p, _p, _p, _i64, _i32, _i64, _i32, _i32, _p, _p, _p, _p], _i32),
+    "jzt_fof_node2node_ex": ([_p, _p, _p, _p, _p, _p, _p, _p, _p, _p, _i64, _i64, _i64, _i64, _f32, _f32, _i32, _i32,
+                              _p], _i32),
     "jzt_segment_max_f32": ([_p, _p, _p, _i64, _p, _i64, _f32], _i32),
     "jzt_flags_or_level": ([_p, _p, _p, _i64, _p, _p], _i32),
     "jzt_plane_cap": ([_p, _p, _p, _i64, _p, _p, _p, _i64, _i32, _i32, _p], _i32),

@@ -64,13 +64,24 @@ def flush():
     evaluate(take())
 
 
-def evaluate(items: list):
-    """Raise RuntimeError for the first of the given recorded conditions that holds."""
-    if not items:
-        return
-    conds = torch.stack([c.to(torch.bool) for c, _, _ in items]).cpu()
-    bad = [i for i in range(len(items)) if bool(conds[i])]
+def flush_with(flag: torch.Tensor) -> bool:
+    """flush(), and the value of a further device flag, with the same read-back."""
+    return evaluate(take(), flag)
+
+
+def evaluate(items: list, flag: torch.Tensor | None = None) -> bool:
+    """Raise RuntimeError for the first of the given recorded conditions that holds; returns the value of
+    `flag`, read back with them (False without one).  Message values may be callables, evaluated on
+    failure only."""
+    conds = [c.to(torch.bool) for c, _, _ in items]
+    if flag is not None:
+        conds.append(flag.reshape(()).to(torch.bool))
+    if not conds:
+        return False
+    conds = torch.stack(conds).tolist()
+    bad = [i for i in range(len(items)) if conds[i]]
     if bad:
         _, msg, values = items[bad[0]]
-        vals = {k: (v.item() if torch.is_tensor(v) else v) for k, v in values.items()}
+        vals = {k: (v() if callable(v) else v.item() if torch.is_tensor(v) else v) for k, v in values.items()}
         raise RuntimeError(msg.format(**vals))
+    return bool(conds[-1]) if flag is not None else False

@@ -134,19 +134,21 @@ __global__ __launch_bounds__(64) void k_fof_node(const int32_t* __restrict__ pil
                                                  const int32_t* __restrict__ spl, const T* __restrict__ nodes,
                                                  const int32_t* __restrict__ il_spl, int32_t* ig, int32_t* __restrict__ count,
                                                  int32_t* __restrict__ il, float r2link, const float* __restrict__ r2v,
-                                                 T boxsize, int64_t il_size, int64_t pil_size, int64_t nitems) {
+                                                 T boxsize, int64_t il_size, int64_t pil_size, int64_t nitems, int nnodes,
+                                                 uint8_t* __restrict__ overflow) {
   __shared__ TileLds<64> s_t;
   __shared__ NodeX<D, T> s_q[kNodeChildren];
   __shared__ int s_qg[kNodeChildren];
   __shared__ int s_run[kNodeChildren];  // per child: hits so far
   __shared__ int s_out[kNodeChildren];  // first list slot
   const int lane = threadIdx.x;
+  if (PASS == 2 && overflow && blockIdx.x == 0 && lane == 0) *overflow = (int64_t)il_spl[nnodes] > il_size ? 1 : 0;
   const uint64_t lt_mask = (1ull << lane) - 1ull;
   const int64_t nact = active_items(spl, nitems);
   const NodeGroups ng = node_groups(nact);
   for (int64_t item = blockIdx.x; item < nact * ng.groups; item += gridDim.x) {
     const int grp = (int)(item / nact), pq = (int)(item - grp * nact);
-    const int q1 = spl[pq + 1];
+    const int q1 = min(spl[pq + 1], nnodes);
     const int e0 = pil_spl[pq], e1 = (int)min((int64_t)pil_spl[pq + 1], pil_size);
     const float r2 = r2v ? r2v[pq] : r2link;
     const T rl_hi = (T)r2 * (T)kSlackHi, rl_lo = (T)r2 * (T)kSlackLo;
@@ -166,7 +168,7 @@ __global__ __launch_bounds__(64) void k_fof_node(const int32_t* __restrict__ pil
             const int pt = pil[e];
             if (pt >= pq) {  // each parent pair once
               t0 = spl[pt];
-              cnt = spl[pt + 1] - t0;
+              cnt = max(min(spl[pt + 1], nnodes) - t0, 0);
             }
             return true;
           },
@@ -572,27 +574,33 @@ int node2child_impl(hipStream_t s, const int32_t* pig, const uint8_t* local, con
 template <int D, typename T>
 int fof_node_impl(hipStream_t s, const int32_t* pil_spl, const int32_t* pil, const int32_t* pspl, const void* nodes,
                   const int32_t* ig_in, int32_t* ig, int32_t* il_spl, int32_t* il, int64_t size_parent, int64_t size_node,
-                  int64_t pil_size, int64_t il_size, float r2link, const float* r2v, float boxsize) {
+                  int64_t pil_size, int64_t il_size, float r2link, const float* r2v, float boxsize, bool zero_list,
+                  uint8_t* overflow) {
   const T* nd = (const T*)nodes;
+  if (size_parent <= 0 && overflow) return fail("FofNode2Node: no parents");
   if (fill_u32(s, il_spl, 0u, size_node + 1)) return 1;
-  if (fill_u32(s, il, 0u, il_size)) return 1;
+  if (zero_list && fill_u32(s, il, 0u, il_size)) return 1;
+  if (size_node >= INT32_MAX) return fail("FofNode2Node: too many nodes");
   if (ig != ig_in && hipMemcpyAsync(ig, ig_in, (size_t)size_node * 4, hipMemcpyDeviceToDevice, s) != hipSuccess)
     return fail("FofNode2Node: copy failed");
   if (size_parent > 0) {
     dim3 g(node_grid(size_parent, 64)), b(64);
     hipLaunchKernelGGL((k_fof_node<0, D, T>), g, b, 0, s, pil_spl, pil, pspl, nd, (const int32_t*)nullptr, ig,
-                       (int32_t*)nullptr, (int32_t*)nullptr, r2link, r2v, (T)boxsize, il_size, pil_size, size_parent);
+                       (int32_t*)nullptr, (int32_t*)nullptr, r2link, r2v, (T)boxsize, il_size, pil_size, size_parent,
+                       (int)size_node, overflow);
     hipLaunchKernelGGL(k_contract, dim3((unsigned)div_up(size_node, 256)), dim3(256), 0, s, ig, size_node);
     hipLaunchKernelGGL((k_fof_node<1, D, T>), g, b, 0, s, pil_spl, pil, pspl, nd, (const int32_t*)nullptr, ig,
-                       il_spl + 1, (int32_t*)nullptr, r2link, r2v, (T)boxsize, il_size, pil_size, size_parent);
+                       il_spl + 1, (int32_t*)nullptr, r2link, r2v, (T)boxsize, il_size, pil_size, size_parent,
+                       (int)size_node, overflow);
     if (check_launch("FofNode2Node link/count")) return 1;
   }
   if (scan_tmp_words(size_node) > il_size) return fail("FofNode2Node: interaction list too small for scan temp");
   if (scan_i32(s, il_spl + 1, il_spl + 1, size_node, true, il)) return 1;
-  if (fill_u32(s, il, 0u, scan_tmp_words(size_node))) return 1;
+  if (zero_list && fill_u32(s, il, 0u, scan_tmp_words(size_node))) return 1;
   if (size_parent > 0) {
     hipLaunchKernelGGL((k_fof_node<2, D, T>), dim3(node_grid(size_parent, 64)), dim3(64), 0, s, pil_spl, pil, pspl, nd,
-                       il_spl, ig, (int32_t*)nullptr, il, r2link, r2v, (T)boxsize, il_size, pil_size, size_parent);
+                       il_spl, ig, (int32_t*)nullptr, il, r2link, r2v, (T)boxsize, il_size, pil_size, size_parent,
+                       (int)size_node, overflow);
   }
   return check_launch("FofNode2Node insert");
 }
@@ -659,7 +667,7 @@ extern "C" int jzt_fof_node2node(jzt_stream_t stream, const int32_t* parent_ilis
                                  float boxsize, int dim, int dtype) {
   JZT_DISPATCH2(fof_node_impl, (hipStream_t)stream, parent_ilist_spl, parent_ilist, parent_spl, nodes, node_igroup_in,
                 node_igroup, node_ilist_spl, node_ilist, size_parent, size_node, parent_ilist_size, size_node_ilist,
-                r2link, (const float*)nullptr, boxsize);
+                r2link, (const float*)nullptr, boxsize, true, (uint8_t*)nullptr);
 }
 
 extern "C" int jzt_fof_node2node_sets(jzt_stream_t stream, const int32_t* parent_ilist_spl, const int32_t* parent_ilist,
@@ -671,7 +679,18 @@ extern "C" int jzt_fof_node2node_sets(jzt_stream_t stream, const int32_t* parent
   if (parent_r2link == nullptr) return fail("FofNode2Node (sets): parent_r2link is required");
   JZT_DISPATCH2(fof_node_impl, (hipStream_t)stream, parent_ilist_spl, parent_ilist, parent_spl, nodes, node_igroup_in,
                 node_igroup, node_ilist_spl, node_ilist, size_parent, size_node, parent_ilist_size, size_node_ilist,
-                0.f, parent_r2link, boxsize);
+                0.f, parent_r2link, boxsize, true, (uint8_t*)nullptr);
+}
+
+extern "C" int jzt_fof_node2node_ex(jzt_stream_t stream, const int32_t* parent_ilist_spl, const int32_t* parent_ilist,
+                                    const int32_t* parent_spl, const float* parent_r2link, const void* nodes,
+                                    const int32_t* node_igroup_in, int32_t* node_igroup, int32_t* node_ilist_spl,
+                                    int32_t* node_ilist, int64_t size_parent, int64_t size_node,
+                                    int64_t parent_ilist_size, int64_t size_node_ilist, float r2link, float boxsize,
+                                    int dim, int dtype, uint8_t* overflow) {
+  JZT_DISPATCH2(fof_node_impl, (hipStream_t)stream, parent_ilist_spl, parent_ilist, parent_spl, nodes, node_igroup_in,
+                node_igroup, node_ilist_spl, node_ilist, size_parent, size_node, parent_ilist_size, size_node_ilist,
+                r2link, parent_r2link, boxsize, false, overflow);
 }
 
 extern "C" int jzt_fof_leaf2leaf(jzt_stream_t stream, const int32_t* ilist_spl, const int32_t* ilist,

@@ -204,7 +204,7 @@ __global__ __launch_bounds__(NT) void k_node_count(
     const int32_t* __restrict__ pil_spl, const int32_t* __restrict__ pil_src, const float* __restrict__ pil_r2,
     const int32_t* __restrict__ parent_spl, const T* __restrict__ nodes, const int32_t* __restrict__ npart,
     const float* __restrict__ parent_rmax2, float* __restrict__ rmax2, int32_t* __restrict__ count_out, int k, T boxsize, int64_t pil_size, int64_t nitems,
-    NodeQueue queue) {
+    int nnodes, NodeQueue queue) {
   __shared__ TileLds<NT> s_t;
   __shared__ NodeChild<D, T> s_q[kNodeChildren];
   __shared__ float s_R[kNodeChildren];
@@ -218,7 +218,7 @@ __global__ __launch_bounds__(NT) void k_node_count(
   for (int64_t item = blockIdx.x; item < nact * ng.groups; item += gridDim.x) {
     const int grp = (int)(item / nact), ip = (int)(item - grp * nact);  // see node_groups
     const int pq = NT == 64 ? ip : queue.q[1 + ip];
-    const int q1 = parent_spl[pq + 1];
+    const int q1 = min(parent_spl[pq + 1], nnodes);
     const int e0 = pil_spl[pq], e1 = (int)min((int64_t)pil_spl[pq + 1], pil_size);
     if (NT == 64 && queue.is_long(e1 - e0)) {
       if (grp == 0 && tid == 0) queue.push(pq);
@@ -261,7 +261,7 @@ __global__ __launch_bounds__(NT) void k_node_count(
             if (r2t <= rtop) {
               const int pt = pil_src[eb + tid];
               t0 = parent_spl[pt];
-              cnt = parent_spl[pt + 1] - t0;
+              cnt = max(min(parent_spl[pt + 1], nnodes) - t0, 0);
             }
           }
           const int pre = block_excl_scan<NT>(cnt, s_t.scan, &tot);
@@ -362,7 +362,7 @@ __global__ __launch_bounds__(NT) void k_node_count(
             if (in) {
               const int pt = pil_src[e];
               t0 = parent_spl[pt];
-              cnt = parent_spl[pt + 1] - t0;
+              cnt = max(min(parent_spl[pt + 1], nnodes) - t0, 0);
             }
             return in;
           },
@@ -388,12 +388,13 @@ __global__ __launch_bounds__(NT) void k_node_insert(
     const int32_t* __restrict__ pil_spl, const int32_t* __restrict__ pil_src, const float* __restrict__ pil_r2,
     const int32_t* __restrict__ parent_spl, const T* __restrict__ nodes, const float* __restrict__ rmax2,
     const int32_t* __restrict__ out_spl, int32_t* __restrict__ out_src, float* __restrict__ out_r2, int64_t nmax,
-    T boxsize, int64_t pil_size, int64_t nitems, NodeQueue queue) {
+    T boxsize, int64_t pil_size, int64_t nitems, int nnodes, uint8_t* __restrict__ overflow, NodeQueue queue) {
   __shared__ TileLds<NT> s_t;
   __shared__ NodeChild<D, T> s_q[kNodeChildren];
   __shared__ float s_R[kNodeChildren];
   __shared__ int s_run[kNodeChildren];  // hits so far
   __shared__ int s_out[kNodeChildren];  // first list slot
+  if (NT == 64 && overflow && blockIdx.x == 0 && threadIdx.x == 0) *overflow = (int64_t)out_spl[nnodes] > nmax ? 1 : 0;
   const int tid = threadIdx.x, lane = tid & 63;
   const uint64_t lt_mask = (1ull << lane) - 1ull;
   // one-wave workgroups take all parents but those with long lists, the larger ones the queue's
@@ -402,7 +403,7 @@ __global__ __launch_bounds__(NT) void k_node_insert(
   for (int64_t item = blockIdx.x; item < nact * ng.groups; item += gridDim.x) {
     const int grp = (int)(item / nact), ip = (int)(item - grp * nact);  // see node_groups
     const int pq = NT == 64 ? ip : queue.q[1 + ip];
-    const int q1 = parent_spl[pq + 1];
+    const int q1 = min(parent_spl[pq + 1], nnodes);
     const int e0 = pil_spl[pq], e1 = (int)min((int64_t)pil_spl[pq + 1], pil_size);
     if (NT == 64 && queue.is_long(e1 - e0)) {
       continue;
@@ -430,7 +431,7 @@ __global__ __launch_bounds__(NT) void k_node_insert(
             if (in) {
               const int pt = pil_src[e];
               t0 = parent_spl[pt];
-              cnt = parent_spl[pt + 1] - t0;
+              cnt = max(min(parent_spl[pt + 1], nnodes) - t0, 0);
             }
             return in;
           },
@@ -954,10 +955,11 @@ int node2node_impl(hipStream_t s, const int32_t* pil_spl, const int32_t* pil_src
                    const float* rmax2_in,
                    float* rmax2, int32_t* il_spl, int32_t* il_src, float* il_r2, int64_t size_parents,
                    int64_t size_nodes, int64_t pil_size, int64_t il_size, int k, float boxsize, void* tmp,
-                   size_t tmp_bytes) {
+                   size_t tmp_bytes, uint8_t* overflow) {
   const T* nd = (const T*)nodes;
   if (fill_u32(s, il_spl, 0u, size_nodes + 1)) return 1;
-  if (size_parents <= 0) return 0;
+  if (size_nodes >= INT32_MAX) return fail("KnnNode2Node: too many nodes");
+  if (size_parents <= 0) return overflow ? fail("KnnNode2Node: no parents") : 0;
   const dim3 g(node_grid(size_parents, 64)), b(64), gl(node_grid(size_parents, kNodeThreads)), bl(kNodeThreads);
   // without room for the queue, one-wave workgroups run the long lists too
   const bool split = tmp && tmp_bytes >= 4 * (size_t)node_queue_words(size_parents);
@@ -966,11 +968,11 @@ int node2node_impl(hipStream_t s, const int32_t* pil_spl, const int32_t* pil_src
 #define JZT_NODE_COUNT(RADIUS)                                                                                        \
   do {                                                                                                                \
     hipLaunchKernelGGL((k_node_count<RADIUS, 64, D, T>), g, b, 0, s, pil_spl, pil_src, pil_r2, parent_spl, nd, npart, \
-                       parent_rmax2, rmax2, il_spl + 1, k, (T)boxsize, pil_size, size_parents, queue);                              \
+                       parent_rmax2, rmax2, il_spl + 1, k, (T)boxsize, pil_size, size_parents, (int)size_nodes, queue);             \
     if (split)                                                                                                        \
       hipLaunchKernelGGL((k_node_count<RADIUS, kNodeThreads, D, T>), gl, bl, 0, s, pil_spl, pil_src, pil_r2,          \
                          parent_spl, nd, npart, parent_rmax2, rmax2, il_spl + 1, k, (T)boxsize, pil_size,             \
-                         size_parents, queue);                                                                        \
+                         size_parents, (int)size_nodes, queue);                                                       \
   } while (0)
   if (rmax2_in) {
     if (size_nodes > 0)
@@ -986,10 +988,11 @@ int node2node_impl(hipStream_t s, const int32_t* pil_spl, const int32_t* pil_src
   if (scan_tmp_words(size_nodes) > il_size) return fail("KnnNode2Node: interaction list too small for scan temp");
   if (scan_i32(s, il_spl + 1, il_spl + 1, size_nodes, true, il_src)) return 1;
   hipLaunchKernelGGL((k_node_insert<64, D, T>), g, b, 0, s, pil_spl, pil_src, pil_r2, parent_spl, nd, rmax2, il_spl,
-                     il_src, il_r2, il_size, (T)boxsize, pil_size, size_parents, queue);
+                     il_src, il_r2, il_size, (T)boxsize, pil_size, size_parents, (int)size_nodes, overflow, queue);
   if (split)
     hipLaunchKernelGGL((k_node_insert<kNodeThreads, D, T>), gl, bl, 0, s, pil_spl, pil_src, pil_r2, parent_spl, nd, rmax2,
-                       il_spl, il_src, il_r2, il_size, (T)boxsize, pil_size, size_parents, queue);
+                       il_spl, il_src, il_r2, il_size, (T)boxsize, pil_size, size_parents, (int)size_nodes, overflow,
+                       queue);
   if (check_launch("KnnNode2Node insert")) return 1;
   // sort each node's list by (r2, src) in place
   // (a list names every node at most once)
@@ -1084,7 +1087,7 @@ extern "C" int jzt_knn_node2node_ex(jzt_stream_t stream, const int32_t* parent_i
   return jzt_knn_node2node_tmp(stream, parent_ilist_spl, parent_ilist_isrc, parent_ilist_r2, parent_spl, nodes,
                                nodes_npart, nullptr, node_r2_in, node_rmax2, node_ilist_spl, node_ilist_isrc, node_ilist_r2,
                                size_parents, size_nodes, parent_ilist_size, node_ilist_size, k, boxsize, dim, dtype,
-                               nullptr, 0);
+                               nullptr, 0, nullptr);
 }
 
 extern "C" int jzt_knn_node2node_tmp(jzt_stream_t stream, const int32_t* parent_ilist_spl,
@@ -1093,14 +1096,15 @@ extern "C" int jzt_knn_node2node_tmp(jzt_stream_t stream, const int32_t* parent_
                                     const float* parent_rmax2, const float* node_r2_in, float* node_rmax2, int32_t* node_ilist_spl,
                                     int32_t* node_ilist_isrc, float* node_ilist_r2, int64_t size_parents,
                                     int64_t size_nodes, int64_t parent_ilist_size, int64_t node_ilist_size, int k,
-                                    float boxsize, int dim, int dtype, void* tmp, size_t tmp_bytes) {
+                                    float boxsize, int dim, int dtype, void* tmp, size_t tmp_bytes,
+                                     uint8_t* overflow) {
   hipStream_t s = (hipStream_t)stream;
   if (k < 1) return fail("KnnNode2Node: k must be >= 1");
   // dims 2-10, float or double node geometry (_generate_ffi.py:9-21)
 #define JZT_N2N(D, T)                                                                                              \
   return node2node_impl<D, T>(s, parent_ilist_spl, parent_ilist_isrc, parent_ilist_r2, parent_spl, nodes,         \
                               nodes_npart, parent_rmax2, node_r2_in, node_rmax2, node_ilist_spl, node_ilist_isrc, node_ilist_r2, \
-                              size_parents, size_nodes, parent_ilist_size, node_ilist_size, k, boxsize, tmp, tmp_bytes)
+                              size_parents, size_nodes, parent_ilist_size, node_ilist_size, k, boxsize, tmp, tmp_bytes, overflow)
 #define JZT_N2N_DIM(D)                  \
   case D:                               \
     if (dtype == JZT_F32) JZT_N2N(D, float); \

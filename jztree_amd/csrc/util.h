@@ -34,6 +34,13 @@ int fill_u32(hipStream_t s, void* p, uint32_t v, int64_t n);
 int where_flags_i8(hipStream_t s, const int8_t* flags, int64_t n, int32_t* out, int64_t size, int32_t fill,
                    const int32_t* fill_dev, int32_t* count_out, int32_t* tmp);
 
+// exclusive scan of n words in place by one workgroup; the total goes to p[n]
+void scan_tiles_i32(hipStream_t s, int32_t* p, int64_t n);
+
+// flags[i] |= lvl[i] >= *lvl_max && i <= *npart, as 0/1 bytes
+int flags_or_level_i8(hipStream_t s, int8_t* flags, const int32_t* lvl, int64_t n, const int32_t* lvl_max,
+                      const int32_t* npart);
+
 // wave64 inclusive prefix sum of an int (all 64 lanes active)
 __device__ __forceinline__ int wave_incl_scan(int v) {
   int lane = __lane_id();

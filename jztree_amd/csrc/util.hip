@@ -101,6 +101,10 @@ int scan_i32(hipStream_t s, const int32_t* in, int32_t* out, int64_t n, bool inc
   return check_launch("scan_i32");
 }
 
+void scan_tiles_i32(hipStream_t s, int32_t* p, int64_t n) {
+  hipLaunchKernelGGL(k_scan_tiles, dim3(1), dim3(kScanThreads), 0, s, p, n);
+}
+
 // Compaction of int8 flags: where(flags != 0) in index order, as two passes over the flags (the
 // flags are read as 16-byte vectors, 16 per thread, kWhereTile per workgroup): per-tile counts,
 // their exclusive scan, then each tile writes its indices at its offset plus the in-tile rank.
@@ -172,10 +176,14 @@ int where_flags_i8(hipStream_t s, const int8_t* flags, int64_t n, int32_t* out, 
 // device): super-node splits spl_super[i] = min(i*ngroup, nn) and list splits
 // ispl[i] = min(i*nsuper, nint) for i <= size_super, entries ilist[j] = j % nsuper (and r2[j] = 0)
 // for j < min(nint, size_ilist); entries past the list are not touched (readers stop at ispl).
-__global__ void k_dense_ilist(const int32_t* __restrict__ nn_dev, int ngroup, int32_t* __restrict__ spl_super,
+// nn = nn_dev[0], less nn_base[0] when given; err (optional): the list does not fit, the super-nodes' splits do not
+// fit into `space` slots after nfilled[0] others.
+__global__ void k_dense_ilist(const int32_t* __restrict__ nn_dev, const int32_t* __restrict__ nn_base, int ngroup,
+                              int32_t* __restrict__ spl_super,
                               int32_t* __restrict__ ispl, int64_t size_super, int32_t* __restrict__ ilist,
-                              float* __restrict__ r2, int64_t size_ilist, int32_t* __restrict__ nsuper_out) {
-  const int64_t nn = nn_dev[0] > 0 ? nn_dev[0] : 0;
+                              float* __restrict__ r2, int64_t size_ilist, int32_t* __restrict__ nsuper_out,
+                              const int32_t* __restrict__ nfilled, int64_t space, uint8_t* __restrict__ err) {
+  const int64_t nn = max(nn_dev[0] - (nn_base ? nn_base[0] : 0), 0);
   const int64_t nsuper = (nn + ngroup - 1) / ngroup;
   const int64_t nint = nsuper * nsuper;
   const int64_t tid = (int64_t)blockIdx.x * blockDim.x + threadIdx.x, st = (int64_t)gridDim.x * blockDim.x;
@@ -188,7 +196,13 @@ __global__ void k_dense_ilist(const int32_t* __restrict__ nn_dev, int ngroup, in
     ilist[j] = (int32_t)(j % nsuper);
     if (r2) r2[j] = 0.f;
   }
-  if (tid == 0) nsuper_out[0] = (int32_t)nsuper;
+  if (tid == 0) {
+    nsuper_out[0] = (int32_t)nsuper;
+    if (err) {
+      err[0] = nint > size_ilist ? 1 : 0;
+      err[1] = nfilled && (int64_t)nfilled[0] + nsuper + 1 > space ? 1 : 0;
+    }
+  }
 }
 
 // Dense top-plane lists of a batch: the top nodes of set s (node_set non-decreasing over the first
@@ -303,6 +317,12 @@ __global__ void k_flags_or_level(int8_t* __restrict__ flags, const int32_t* __re
   flags[i] = (flags[i] != 0 || extra) ? 1 : 0;
 }
 
+int flags_or_level_i8(hipStream_t s, int8_t* flags, const int32_t* lvl, int64_t n, const int32_t* lvl_max,
+                      const int32_t* npart) {
+  hipLaunchKernelGGL(k_flags_or_level, dim3((unsigned)div_up(n, 256)), dim3(256), 0, s, flags, lvl, n, lvl_max, npart);
+  return check_launch("FlagsOrLevel");
+}
+
 // leaf kNN waves per EU (K <= 32), onesweep keys per thread, XCD-aware order of the leaf kernels
 static int g_tune[kTuneCount] = {4, 12, 1};
 int tune_get(int knob) { return (knob >= 0 && knob < kTuneCount) ? __atomic_load_n(&g_tune[knob], __ATOMIC_RELAXED) : 0; }
@@ -363,15 +383,31 @@ extern "C" int jzt_get_tuning(int knob) { return jzt::tune_get(knob); }
 extern "C" const char* jzt_last_error(void) { return jzt::g_err.c_str(); }
 extern "C" int jzt_abi_version(void) { return JZT_ABI_VERSION; }
 
+static int dense_ilist(hipStream_t s, const int32_t* nn, const int32_t* nn_base, int ngroup, int32_t* spl_super,
+                       int32_t* ispl, int64_t size_super, int32_t* ilist, float* r2, int64_t size_ilist, int32_t* nsuper,
+                       const int32_t* nfilled, int64_t space, uint8_t* err) {
+  using namespace jzt;
+  if (ngroup < 1) return fail("DenseIlist: ngroup must be >= 1");
+  // only the nsuper^2 live entries are written, far fewer than the allocation
+  const int64_t blocks = div_up(size_super + 1 > size_ilist ? size_super + 1 : size_ilist, 256);
+  hipLaunchKernelGGL(k_dense_ilist, dim3((unsigned)(blocks < 2048 ? (blocks > 0 ? blocks : 1) : 2048)), dim3(256), 0, s, nn,
+                     nn_base, ngroup, spl_super, ispl, size_super, ilist, r2, size_ilist, nsuper, nfilled, space, err);
+  return check_launch("DenseIlist");
+}
+
 extern "C" int jzt_dense_ilist(jzt_stream_t stream, const int32_t* nnodes, int ngroup, int32_t* spl_super,
                                int32_t* ispl, int64_t size_super, int32_t* ilist, float* r2, int64_t size_ilist,
                                int32_t* nsuper) {
-  using namespace jzt;
-  if (ngroup < 1) return fail("DenseIlist: ngroup must be >= 1");
-  const int64_t work = size_super + 1 > size_ilist ? size_super + 1 : size_ilist;
-  hipLaunchKernelGGL(k_dense_ilist, dim3(grid_for(div_up(work, 256))), dim3(256), 0, (hipStream_t)stream, nnodes,
-                     ngroup, spl_super, ispl, size_super, ilist, r2, size_ilist, nsuper);
-  return check_launch("DenseIlist");
+  return dense_ilist((hipStream_t)stream, nnodes, nullptr, ngroup, spl_super, ispl, size_super, ilist, r2, size_ilist,
+                     nsuper, nullptr, 0, nullptr);
+}
+
+extern "C" int jzt_dense_ilist_top(jzt_stream_t stream, const int32_t* node_spl, int plane, int ngroup,
+                                   int32_t* spl_super, int32_t* ispl, int64_t size_super, int32_t* ilist, float* r2,
+                                   int64_t size_ilist, int32_t* nsuper, const int32_t* nfilled, int64_t space,
+                                   uint8_t* err) {
+  return dense_ilist((hipStream_t)stream, node_spl + plane + 1, node_spl + plane, ngroup, spl_super, ispl, size_super,
+                     ilist, r2, size_ilist, nsuper, nfilled, space, err);
 }
 
 extern "C" size_t jzt_dense_ilist_sets_tmp_bytes(int64_t nsets) { return (size_t)3 * 8 * (size_t)(nsets + 1); }
@@ -390,7 +426,7 @@ extern "C" int jzt_dense_ilist_sets(jzt_stream_t stream, const int32_t* nnodes, 
   hipStream_t s = (hipStream_t)stream;
   hipLaunchKernelGGL(k_dense_sets_prep, dim3(1), dim3(256), 0, s, nnodes, node_set, nsets, ngroup, F, S, I);
   const int64_t work = size_super + 1 > size_ilist ? size_super + 1 : size_ilist;
-  hipLaunchKernelGGL(k_dense_sets_fill, dim3(grid_for(div_up(work, 256))), dim3(256), 0, s, nnodes, nsets, ngroup, F, S,
+  hipLaunchKernelGGL(k_dense_sets_fill, dim3((unsigned)min(max(div_up(work, 256), (int64_t)1), (int64_t)2048)), dim3(256), 0, s, nnodes, nsets, ngroup, F, S,
                      I, spl_super, ispl, size_super, ilist, r2, size_ilist, nsuper);
   return check_launch("DenseIlistSets");
 }
@@ -431,7 +467,5 @@ extern "C" int jzt_flags_or_level(jzt_stream_t stream, int8_t* flags, const int3
   using namespace jzt;
   if (n <= 0) return 0;
   if (!flags || !lvl || !lvl_max || !npart) return fail("FlagsOrLevel: null argument");
-  hipLaunchKernelGGL(k_flags_or_level, dim3((unsigned)div_up(n, 256)), dim3(256), 0, (hipStream_t)stream, flags, lvl,
-                     n, lvl_max, npart);
-  return check_launch("FlagsOrLevel");
+  return flags_or_level_i8((hipStream_t)stream, flags, lvl, n, lvl_max, npart);
 }

@@ -20,7 +20,7 @@ from .checks import raise_if
 from .config import FofCatalogueConfig, FofConfig
 from .data import (FofCatalogue, InteractionList, PackedArray, TreeHierarchy, count_not_nan, get_pos,
                    tree_map_by_len, verify_ilist)
-from .tree import _tmp, build_tree_hierarchy, top_dense_interaction_list, zsort
+from .tree import _tmp, build_tree_hierarchy, plane_tables, top_plane_lists, zsort
 
 
 @dataclass
@@ -28,8 +28,11 @@ class PosLvl:
     """Node positions and levels (data.py:199-212)."""
     pos: torch.Tensor
     lvl: torch.Tensor
+    rows: torch.Tensor | None = None  # pos_lvl(), when it is there already
 
     def pos_lvl(self) -> torch.Tensor:
+        if self.rows is not None:
+            return self.rows
         if self.pos.dtype == torch.float32:
             lvl_t = self.lvl.to(torch.int32).view(torch.float32)
         else:
@@ -45,6 +48,7 @@ class FofNodeData:
     igroup: torch.Tensor
     spl: torch.Tensor
     cent: torch.Tensor | None = None
+    rows: torch.Tensor | None = None  # centre and level rows (PosLvl.pos_lvl), when they are there already
 
 
 def _r2link(rlink: float) -> float:
@@ -68,19 +72,15 @@ def _fof_node2node(ilist: InteractionList, spl_parent, node_data: PosLvl, node_i
     ig = node_igroup.to(torch.int32).contiguous()
     il_spl = torch.empty(size + 1, dtype=torch.int32, device=dev)
     il = torch.empty(ilist.size(), dtype=torch.int32, device=dev)
-    if torch.is_tensor(rlink):  # r2link per parent node (batches of sets)
-        L.call("jzt_fof_node2node_sets", L.stream(), L.ptr(ilist.ispl), L.ptr(ilist.isrc),
-               L.ptr(spl_parent.contiguous()), L.ptr(_r2_items(rlink, spl_parent.shape[0] - 1)),
-               L.ptr(node_data.pos_lvl()), L.ptr(ig), L.ptr(ig), L.ptr(il_spl), L.ptr(il), spl_parent.shape[0] - 1,
-               size, ilist.size(), ilist.size(), float(boxsize or 0.), node_data.pos.shape[-1],
-               L.dtype_code(node_data.pos.dtype))
-    else:
-        L.call("jzt_fof_node2node", L.stream(), L.ptr(ilist.ispl), L.ptr(ilist.isrc), L.ptr(spl_parent.contiguous()),
-               L.ptr(node_data.pos_lvl()), L.ptr(ig), L.ptr(ig), L.ptr(il_spl), L.ptr(il), spl_parent.shape[0] - 1,
-               size, ilist.size(), ilist.size(), _r2link(rlink), float(boxsize or 0.), node_data.pos.shape[-1],
-               L.dtype_code(node_data.pos.dtype))
+    over = torch.empty(1, dtype=torch.bool, device=dev)
+    per_parent = torch.is_tensor(rlink)  # r2link per parent node (batches of sets)
+    r2v = _r2_items(rlink, spl_parent.shape[0] - 1) if per_parent else None
+    L.call("jzt_fof_node2node_ex", L.stream(), L.ptr(ilist.ispl), L.ptr(ilist.isrc), L.ptr(spl_parent.contiguous()),
+           L.ptr(r2v), L.ptr(node_data.pos_lvl()), L.ptr(ig), L.ptr(ig), L.ptr(il_spl), L.ptr(il),
+           spl_parent.shape[0] - 1, size, ilist.size(), ilist.size(), 0. if per_parent else _r2link(rlink),
+           float(boxsize or 0.), node_data.pos.shape[-1], L.dtype_code(node_data.pos.dtype), L.ptr(over))
     node_ilist = verify_ilist(InteractionList(il_spl, il))
-    raise_if(node_ilist.nfilled() > il.numel(),
+    raise_if(over[0],
              "The interaction list allocation is too small. (need: {n1} have: {n2})\n"
              "Hint: Increase alloc_fac_ilist", n1=node_ilist.nfilled(), n2=il.numel())
     return ig, node_ilist
@@ -130,27 +130,24 @@ def _fof_dual_walk(th: TreeHierarchy, rlink: float, boxsize: float = 0., alloc_f
     r2link_set (extension, batch forests): float32 r2link of every set, used in place of rlink."""
     nplanes = th.num_planes()
     size = th.size()
-    spl, ilist, nsup = top_dense_interaction_list(th, int(th.size_leaves * alloc_fac_ilist))
+    spl, ilist = top_plane_lists(th, int(th.size_leaves * alloc_fac_ilist))
     if r2link_set is not None:
         assert th.leaf_set is not None
         r2_plane = [r2link_set[s.long()].contiguous() for s in _plane_node_sets(th, spl)]
     dev = spl.device
+    tables = plane_tables(th)
+    n2c = tables.spl + [spl]
     igroup = torch.arange(size, dtype=torch.int32, device=dev)
-    spl_n2n = th.ispl_n2n.append(spl, nsup + 1, fill_value=spl[-1], resize=True)
-    raise_if(spl_n2n.nfilled() > spl_n2n.size(), "No space for top-level splits\nHint: Increase alloc_fac_nodes.")
-    max_lvl = th.info().max_lvl()
-    nlvl = th.lvl.append(torch.full_like(igroup, max_lvl), nsup, max_lvl, resize=True)
+    lvl = torch.full_like(igroup, th.info().max_lvl())  # of the super-nodes
     dim = th.geom_cent.data.shape[-1]
-    for i in range(nplanes):
-        level = nplanes - 1 - i
-        parent_spl = spl_n2n.get(level + 1, size + 1)
+    for level in reversed(range(nplanes)):
         rl = rlink if r2link_set is None else r2_plane[level + 1]
-        igroup = _node_to_child_label(igroup, nlvl.get(level + 1, size), parent_spl, num=th.num(level), rlink=rl,
-                                      dim=dim, dtype=th.geom_cent.data.dtype)
-        node_data = PosLvl(pos=th.geom_cent.get(level, size), lvl=nlvl.get(level, size))
-        igroup, ilist = _fof_node2node(ilist, parent_spl, node_data, igroup, rlink=rl, boxsize=boxsize)
-    node_data = FofNodeData(nlvl.get(0, size), igroup, spl_n2n.get(0, size + 1), cent=th.geom_cent.get(0, size))
-    return node_data, ilist
+        # (num of fof.py:133 masks nothing here: only children below the parents' last split are written)
+        igroup = _node_to_child_label(igroup, lvl, n2c[level + 1], rlink=rl, dim=dim, dtype=th.geom_cent.data.dtype)
+        rows, lvl = tables.nodes[level], tables.lvl[level]
+        igroup, ilist = _fof_node2node(ilist, n2c[level + 1], PosLvl(pos=rows[:, :-1], lvl=lvl, rows=rows), igroup,
+                                       rlink=rl, boxsize=boxsize)
+    return FofNodeData(lvl, igroup, n2c[0], cent=rows[:, :-1], rows=rows), ilist
 
 
 def _fof_leaf2leaf(leaf_data: FofNodeData, ilist: InteractionList, posz, rlink: float, boxsize: float = 0.,
@@ -172,7 +169,7 @@ def _fof_leaf2leaf(leaf_data: FofNodeData, ilist: InteractionList, posz, rlink: 
                L.ptr(posz.contiguous()), L.ptr(part_igroup), L.ptr(out), len(leaf_data.spl) - 1, len(posz),
                float(boxsize or 0.), posz.shape[-1], L.dtype_code(posz.dtype))
     elif leaf_data.cent is not None and leaf_data.cent.dtype == posz.dtype:
-        cells = PosLvl(pos=leaf_data.cent, lvl=leaf_data.lvl).pos_lvl()
+        cells = PosLvl(pos=leaf_data.cent, lvl=leaf_data.lvl, rows=leaf_data.rows).pos_lvl()
         L.call("jzt_fof_leaf2leaf_cells", L.stream(), L.ptr(ilist.ispl), L.ptr(ilist.isrc), ilist.size(),
                L.ptr(leaf_data.spl.contiguous()), L.ptr(posz.contiguous()), L.ptr(cells), L.ptr(part_igroup),
                L.ptr(out), len(leaf_data.spl) - 1, len(posz), _r2link(rlink), float(boxsize or 0.), posz.shape[-1],

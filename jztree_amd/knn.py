@@ -20,7 +20,7 @@ from .checks import raise_if
 from .config import KNNConfig
 from .data import InteractionList, Pos, RankIdx, TreeHierarchy, get_num, get_num_total, get_pos, tree_map_by_len
 from .tools import inverse_of_splits, masked_inverse
-from .tree import (_tmp, f32_view, top_dense_interaction_list, zsort_and_tree, zsort_and_tree_multi_type,
+from .tree import (_tmp, f32_view, plane_tables, top_plane_lists, zsort_and_tree, zsort_and_tree_multi_type,
                    zsort_and_tree_origin)
 
 
@@ -30,9 +30,17 @@ class PosLvlNum:
     pos: torch.Tensor
     lvl: torch.Tensor
     npart: torch.Tensor
+    rows: torch.Tensor | None = None  # pos_lvl(), when it is there already
+
+    @classmethod
+    def of_plane(cls, tables, level: int) -> "PosLvlNum":
+        rows = tables.nodes[level]
+        return cls(pos=rows[:, :-1], lvl=tables.lvl[level], npart=tables.npart[level], rows=rows)
 
     def pos_lvl(self) -> torch.Tensor:
         """(size, dim+1): positions with the level bit-cast into the last column."""
+        if self.rows is not None:
+            return self.rows
         if self.pos.dtype == torch.float32:
             lvl_t = self.lvl.to(torch.int32).view(torch.float32)
         else:
@@ -120,14 +128,15 @@ def _knn_node2node_ilist(ilist: InteractionList, spl_parent, node_data: PosLvlNu
     assert r2in is None or r2in.shape[0] >= size
     nb = L.LIB.jzt_knn_node2node_tmp_bytes(spl_parent.shape[0] - 1, ilist.size())
     tmp = _tmp(nb, dev)
+    over = torch.empty(1, dtype=torch.bool, device=dev)
     L.call("jzt_knn_node2node_tmp", L.stream(), L.ptr(ilist.ispl), L.ptr(ilist.isrc), L.ptr(ilist.rad2),
            L.ptr(spl_parent.contiguous()), L.ptr(poslvl), L.ptr(npart), L.ptr(parent_rmax2), L.ptr(r2in), L.ptr(radii), L.ptr(ispl),
            L.ptr(il), L.ptr(ilr2), spl_parent.shape[0] - 1, size, ilist.size(), ilist.size(), int(k),
-           float(boxsize), node_data.pos.shape[-1], L.dtype_code(node_data.pos.dtype), L.ptr(tmp), nb)
+           float(boxsize), node_data.pos.shape[-1], L.dtype_code(node_data.pos.dtype), L.ptr(tmp), nb, L.ptr(over))
     if overflow is not None:  # the caller checks (and handles) overflow itself
-        overflow.append(ispl[-1] > il.numel())
+        overflow.append(over[0])
     else:
-        raise_if(ispl[-1] > il.numel(),
+        raise_if(over[0],
                  "The interaction list allocation is too small. (need: {n1}, have: {n2})\n"
                  "Hint: increase alloc_fac_ilist", n1=ispl[-1], n2=il.numel())
     if with_radii:
@@ -143,20 +152,15 @@ def _knn_dual_walk(th: TreeHierarchy, k: int, boxsize: float | None = None,
     With return_parents, also returns (rmax2 of the plane's nodes or None at the top, the
     node-to-child splits of that plane)."""
     nlevels = th.num_planes()
-    size = th.size()
-    spl, ilist, nsup = top_dense_interaction_list(th, int(th.size_leaves * alloc_fac_ilist), with_r2=True)
-    spl_n2n = th.ispl_n2n.append(spl, nsup + 1, fill_value=spl[-1], resize=True)
-    raise_if(spl_n2n.nfilled() > spl_n2n.size(), "No space for top-level splits\nHint: Increase alloc_fac_nodes.")
+    spl, ilist = top_plane_lists(th, int(th.size_leaves * alloc_fac_ilist), with_r2=True)
+    tables = plane_tables(th)
+    n2c = tables.spl + [spl]
     rmax2 = None
-    for i in range(nlevels - stop_level):
-        level = nlevels - i - 1
-        parent_spl = spl_n2n.get(level + 1, size + 1)
-        node_data = PosLvlNum(pos=th.geom_cent.get(level, size), lvl=th.lvl.get(level, size),
-                              npart=th.npart(level, size=size, ptype=0))
-        ilist, rmax2 = _knn_node2node_ilist(ilist, parent_spl, node_data, k=k, boxsize=boxsize, with_radii=True,
-                                            parent_rmax2=rmax2)
+    for level in reversed(range(stop_level, nlevels)):
+        ilist, rmax2 = _knn_node2node_ilist(ilist, n2c[level + 1], PosLvlNum.of_plane(tables, level), k=k,
+                                            boxsize=boxsize, with_radii=True, parent_rmax2=rmax2)
     if return_parents:
-        return ilist, rmax2, spl_n2n.get(stop_level, size + 1)
+        return ilist, rmax2, n2c[stop_level]
     return ilist
 
 
@@ -259,20 +263,15 @@ def _knn_radius_walk(th: TreeHierarchy, k: int, radii: list, boxsize: float = 0.
     keep_plane1: also return (the plane-1 lists, plane-1 -> leaf splits) -- with a one-plane tree
     the dense top-level list and its super-node splits."""
     nlevels = th.num_planes()
-    size = th.size()
-    spl, ilist, nsup = top_dense_interaction_list(th, int(th.size_leaves * alloc_fac_ilist), with_r2=True)
-    spl_n2n = th.ispl_n2n.append(spl, nsup + 1, fill_value=spl[-1], resize=True)
-    raise_if(spl_n2n.nfilled() > spl_n2n.size(), "No space for top-level splits\nHint: Increase alloc_fac_nodes.")
+    spl, ilist = top_plane_lists(th, int(th.size_leaves * alloc_fac_ilist), with_r2=True)
+    tables = plane_tables(th)
+    n2c = tables.spl + [spl]
     plane1 = None
-    for i in range(nlevels):
-        level = nlevels - i - 1
-        parent_spl = spl_n2n.get(level + 1, size + 1)
+    for level in reversed(range(nlevels)):
         if level == 0:
-            plane1 = (ilist, parent_spl)
-        node_data = PosLvlNum(pos=th.geom_cent.get(level, size), lvl=th.lvl.get(level, size),
-                              npart=th.npart(level, size=size, ptype=0))
-        ilist = _knn_node2node_ilist(ilist, parent_spl, node_data, k=k, boxsize=boxsize, rmax2_in=radii[level],
-                                     overflow=overflow)
+            plane1 = (ilist, n2c[1])
+        ilist = _knn_node2node_ilist(ilist, n2c[level + 1], PosLvlNum.of_plane(tables, level), k=k, boxsize=boxsize,
+                                     rmax2_in=radii[level], overflow=overflow)
     if keep_plane1:
         return ilist, plane1
     return ilist
@@ -413,12 +412,12 @@ def _knn_leaf_start_bound(ilist: InteractionList, spl, posz, k: int, boxsize, le
     xQ = posz if xQ is None else xQ
     nq = len(xQ)
     size = len(splQ) - 1
-    init = (leaf_r2.to(torch.float64) * (1.0 + 2.0 ** -10)).to(torch.float32).contiguous()
+    init = leaf_r2.to(torch.float32).contiguous() * (1.0 + 2.0 ** -10)  # a float32 factor: rounded once
     rnn, inn, retry = _knn_leaf2leaf(ilist, spl, posz, k=k, boxsize=boxsize, splQ=splQ, xQ=xQ, src_ids=src_ids,
                                      dst_rows=dst_rows, init_r2=init)
-    # eagerly the redo runs only when a query came up short (one read-back); under graph capture
+    # eagerly the redo runs only when a query came up short (read back with the recorded conditions); under graph capture
     # it always runs, and every leaf without a short query skips it (negative radius)
-    if checks.is_deferred() or bool((retry != 0).any()):
+    if checks.is_deferred() or checks.flush_with(retry.any()):
         # per leaf: does it hold a flagged query (a segment maximum over the query splits; a
         # scatter of every flag onto its leaf costs an atomic per query)
         short = torch.empty(size, dtype=torch.float32, device=xQ.device)

@@ -383,6 +383,82 @@ def _define_split_hierarchy(posz, node_sizes, alloc_size, npart=None, ptype=None
     return ispl, ispl_per_type, ispl_n2l, ispl_n2n
 
 
+# most planes and the position dtypes of the one-call hierarchy build
+_BUILD_PLANES = 32
+_BUILD_DTYPES = (torch.float32, torch.float64)
+
+
+def _build_hierarchy(posz, node_sizes, alloc_size, npart, cfg_reg: RegularizationConfig | None,
+                     set_id: torch.Tensor | None):
+    """_define_split_hierarchy and the node geometry of build_tree_hierarchy in one library call
+    (jzt_build_tree), for one particle type: the same arrays.  npart: None = count the rows whose
+    first coordinate is not NaN.  Returns (leaf splits, n2l, n2n, lvl, geom_cent, leaf_set)."""
+    n, dim = posz.shape
+    dev = posz.device
+    posz = posz.contiguous()
+    nl = len(node_sizes)
+    A = alloc_size
+    i32 = lambda *shape: torch.empty(shape, dtype=torch.int32, device=dev)
+    ispl, n2l, n2n, lvl = i32(A), i32(A), i32(A), i32(A - nl)
+    level_spl, prop_spl = i32(nl + 1), i32(nl + 1)
+    n2l_fill, n2n_fill, lvl_fill, counts = i32(nl), i32(nl), i32(nl), i32(2)
+    cent = torch.empty((A - nl, dim), dtype=posz.dtype, device=dev)
+    cent_fill = torch.empty(nl, dtype=posz.dtype, device=dev)
+    err = torch.empty(2, dtype=torch.bool, device=dev)
+    leaf_set = None if set_id is None else i32(A - 1)
+    npart_dev = npart.reshape(1).to(device=dev, dtype=torch.int32) if torch.is_tensor(npart) else None
+    npart_host = -1 if npart is None or npart_dev is not None else int(npart)
+    dt = L.dtype_code(posz.dtype)
+    reg = cfg_reg is not None
+    nb = L.LIB.jzt_build_tree_tmp_bytes(n, A, nl, dim, dt, int(reg))
+    tmp = _tmp(nb, dev)
+    sizes = np.asarray(node_sizes, dtype=np.int32)
+    L.call("jzt_build_tree", L.stream(), L.ptr(posz), L.ptr(set_id), L.ptr(npart_dev), npart_host, n, dim, dt,
+           sizes.ctypes.data, nl, A, int(reg), float(cfg_reg.max_volume_fac) if reg else 0.,
+           float(cfg_reg.regularize_percentile) if reg else 0., L.ptr(ispl), L.ptr(n2l), L.ptr(n2n),
+           L.ptr(level_spl), L.ptr(n2l_fill), L.ptr(n2n_fill), L.ptr(lvl), L.ptr(cent), L.ptr(prop_spl),
+           L.ptr(lvl_fill), L.ptr(cent_fill), L.ptr(counts), L.ptr(leaf_set), L.ptr(err), L.ptr(tmp), nb)
+    raise_if(err[0],
+             "Tree-Leaf allocation too small: filled={filled} size={size}.\n"
+             "Hint: Increase alloc_fac_nodes or max_leaf_size", filled=counts[0], size=A)
+    raise_if(err[1],
+             "Tree-node allocation too small: filled={filled} size={size}.\n"
+             "Hint: Increase alloc_fac_nodes, max_leaf_size or coarse_fac", filled=level_spl[-1], size=A)
+    levels = counts[1:]
+    return (ispl, PackedArray(n2l, level_spl, n2l_fill, levels), PackedArray(n2n, level_spl, n2n_fill, levels),
+            PackedArray(lvl, prop_spl, lvl_fill, levels), PackedArray(cent, prop_spl, cent_fill, levels), leaf_set)
+
+
+@dataclasses.dataclass
+class PlaneTables:
+    """What the dual walks read per plane (lists indexed by plane, rows past a plane's nodes undefined):
+    spl = child splits (size + 1, padded), nodes = centre with the level's bits in the last column,
+    lvl, npart (type 0)."""
+    spl: list
+    nodes: list
+    lvl: list
+    npart: list
+
+
+def plane_tables(th: TreeHierarchy) -> PlaneTables:
+    """The tables of every plane, in one kernel (jzt_plane_tables); the values are those of
+    ispl_n2n.get, geom_cent.get, lvl.get and th.npart."""
+    size = th.size()
+    nl = th.num_planes()
+    cent = th.geom_cent.data.contiguous()
+    dev, dim = cent.device, cent.shape[-1]
+    c32 = lambda t: t.to(torch.int32).contiguous()
+    spl = c32(th.splits_leaf_to_part(0))
+    out = torch.empty((3, nl, size + 1), dtype=torch.int32, device=dev)
+    nodes = torch.empty((nl, size + 1, dim + 1), dtype=cent.dtype, device=dev)
+    L.call("jzt_plane_tables", L.stream(), L.ptr(c32(th.ispl_n2n.data)), L.ptr(c32(th.ispl_n2l.data)),
+           L.ptr(c32(th.ispl_n2n.ispl)), L.ptr(c32(th.ispl_n2n.fill_values)), L.ptr(c32(th.ispl_n2l.fill_values)),
+           L.ptr(c32(th.lvl.data)), L.ptr(cent), L.ptr(c32(th.lvl.ispl)), L.ptr(spl), spl.numel(), nl, size, dim,
+           L.dtype_code(cent.dtype), L.ptr(out[0]), L.ptr(nodes), L.ptr(out[1]), L.ptr(out[2]))
+    return PlaneTables(list(out[0].unbind(0)), list(nodes[:, :size].unbind(0)), list(out[1, :, :size].unbind(0)),
+                       list(out[2, :, :size].unbind(0)))
+
+
 def center_of_mass(ispl: torch.Tensor, pos: torch.Tensor, mass, kahan_summation: bool = True):
     """tree.py:479-499 -> CenterOfMass: mass-weighted centre and total mass of the points in every
     range [ispl[i], ispl[i+1]) (NaN for empty ranges).  mass: per point, or a scalar (broadcast as
@@ -430,10 +506,23 @@ def build_tree_hierarchy(partz, cfg_tree: TreeConfig, lvl_bound=None, ptype=None
     posz = get_pos(partz)
     npart_tot = get_num_total(partz, default_to_length=True)
     np_per_dev = npart_tot
-    npart = get_num(partz, default_to_nancount=True)
     node_sizes = _define_tree_level_node_sizes(npart_tot, cfg_tree)
     alloc_size = _estimate_node_number(np_per_dev, cfg_tree.max_leaf_size, cfg_tree.alloc_fac_nodes)
+    size_leaves = _estimate_node_number(np_per_dev, cfg_tree.max_leaf_size)
+    # one particle type is built by one library call; several types count their particles per node
+    # apart and keep the steps below, as does anything that call does not take
+    if (ptype is None and lvl_bound is None and posz.is_cuda and posz.dtype in _BUILD_DTYPES and len(posz) > 0
+            and len(node_sizes) <= _BUILD_PLANES and len(node_sizes) < alloc_size):
+        npart = get_num(partz, default_to_nancount=True) if getattr(partz, "num", None) is not None else None
+        ispl_l2p, ispl_n2l, ispl_n2n, lvl, geom_cent, leaf_set = _build_hierarchy(
+            posz, node_sizes, alloc_size, npart, cfg_tree.regularization if set_id is None else None,
+            None if set_id is None else set_id.contiguous())
+        nmass_cent, nmass = (_get_tree_mass_centers(partz, ispl_n2n, lvl.ispl) if cfg_tree.mass_centered
+                             else (None, None))
+        return TreeHierarchy(size_leaves, ispl_n2n, ispl_n2l, ispl_l2p.reshape(1, -1), lvl, geom_cent, mass=nmass,
+                             mass_cent=nmass_cent, leaf_set=leaf_set, nsets=int(nsets))
 
+    npart = get_num(partz, default_to_nancount=True)
     if set_id is None:
         ispl_l2p, ispl_per_type, ispl_n2l, ispl_n2n = _define_split_hierarchy(
             posz, node_sizes, alloc_size, npart=npart, ptype=ptype, num_types=num_types, lvl_bound=lvl_bound,
@@ -456,7 +545,6 @@ def build_tree_hierarchy(partz, cfg_tree: TreeConfig, lvl_bound=None, ptype=None
     nmass_cent, nmass = None, None
     if cfg_tree.mass_centered:
         nmass_cent, nmass = _get_tree_mass_centers(partz, ispl_n2n, prop_array_spl)
-    size_leaves = _estimate_node_number(np_per_dev, cfg_tree.max_leaf_size)
     return TreeHierarchy(size_leaves, ispl_n2n, ispl_n2l, ispl_per_type, lvl, geom_cent, mass=nmass,
                          mass_cent=nmass_cent, leaf_set=leaf_set, nsets=int(nsets))
 
@@ -631,6 +719,30 @@ def grouped_dense_interaction_list(nnodes, size_ilist: int, ngroup: int = 32, si
 
 
 grouped_dense_interaction_list.jit = grouped_dense_interaction_list
+
+
+def top_plane_lists(th: TreeHierarchy, size_ilist: int, ngroup: int = 32, with_r2: bool = False):
+    """top_dense_interaction_list for a walk: (super-node splits, list), with the check that the splits would
+    fit behind the packed ones (ispl_n2n.append, tree.py:868-930 and knn.py:151-153)."""
+    size = th.size()
+    no_space = "No space for top-level splits\nHint: Increase alloc_fac_nodes."
+    filled = th.ispl_n2n.ispl
+    if th.leaf_set is not None or th.lvl.ispl.dtype != torch.int32 or filled.dtype != torch.int32:
+        spl, ilist, nsup = top_dense_interaction_list(th, size_ilist, ngroup=ngroup, with_r2=with_r2)
+        raise_if(filled[-1] + (nsup + 1) > th.ispl_n2n.size(), no_space)
+        return spl, ilist
+    dev = th.lvl.data.device
+    i32 = lambda m: torch.empty(m, dtype=torch.int32, device=dev)
+    spl, ispl, ilist, nsuper = i32(size + 1), i32(size + 1), i32(size_ilist), i32(1)
+    r2 = torch.empty(size_ilist, dtype=torch.float32, device=dev) if with_r2 else None
+    err = torch.empty(2, dtype=torch.bool, device=dev)
+    L.call("jzt_dense_ilist_top", L.stream(), L.ptr(th.lvl.ispl.contiguous()), th.num_planes() - 1, int(ngroup),
+           L.ptr(spl), L.ptr(ispl), size, L.ptr(ilist), L.ptr(r2), size_ilist, L.ptr(nsuper), L.ptr(filled[-1:]),
+           th.ispl_n2n.size(), L.ptr(err))
+    raise_if(err[0], "Cannot fit {n} interactions into interaction list with size {size}\nHint: Increase alloc_fac_ilist",
+             n=lambda: int(nsuper) ** 2, size=size_ilist)
+    raise_if(err[1], no_space)
+    return spl, verify_ilist(InteractionList(ispl=ispl, isrc=ilist, rad2=r2))
 
 
 def top_dense_interaction_list(th: TreeHierarchy, size_ilist: int, ngroup: int = 32, with_r2: bool = False):
