@@ -48,8 +48,8 @@ int jzt_abi_version(void);
  * host thread launches.
  *   JZT_TUNE_LEAF_WAVES  waves per EU the leaf kNN kernel is compiled for when k <= 32 (1, 2, 4;
  *                        default 4): the register budget per lane against occupancy
- *   JZT_TUNE_SORT_KPT    keys per thread of the onesweep radix passes (8, 12, 16; default 12):
- *                        tile = 256 * kpt keys
+ *   JZT_TUNE_SORT_KPT    keys per thread of the onesweep radix passes (8, 12, 16; default 12, which
+ *                        means 8 below 2^23 keys): tile = threads * kpt keys
  *   JZT_TUNE_XCD         order of the query leaves in the kNN and FoF leaf kernels (0, 1; default
  *                        1): 1 gives each of the 8 XCDs a contiguous eighth of the z-ordered
  *                        leaves, so that neighbouring leaves share an L2; 0 deals consecutive
@@ -76,9 +76,8 @@ int jzt_pos_zorder_sort(jzt_stream_t stream, const void* pos_in, void* pos_out, 
  * allocate device memory (code under HIP graph capture, tight serving loops, harnesses that
  * forbid hipMalloc): same inputs, outputs and order as jzt_pos_zorder_sort, but the scratch is a
  * fixed 64 MiB device array inside the library (one per device, held until the process ends), so
- * nothing is allocated and no tmp buffer is passed.  n is limited to what fits that array
- * (jzt_zsort_tmp_bytes(n, dim, dtype) <= 64 MiB: up to 1,427,456 points for f32 3D,
- * 1,137,141 for f64 3D); larger n fails
+ * nothing is allocated and no tmp buffer is passed.  n is limited (up to 1,427,456 points for f32 3D,
+ * 1,137,141 for f64 3D; always enough for jzt_zsort_tmp_bytes); larger n fails
  * with a message.  Calls that overlap on one device share the array and race: serialise them. */
 int jzt_pos_zorder_sort_noalloc(jzt_stream_t stream, const void* pos_in, void* pos_out, void* id_out, int64_t n,
                                 int dim, int dtype);
@@ -100,6 +99,12 @@ int jzt_pos_zorder_sort_segmented(jzt_stream_t stream, const void* pos_in, void*
  * point per leaf; the index of the neighbouring leaf with the smaller level difference to x. */
 int jzt_search_sorted_z(jzt_stream_t stream, const void* posz_have, const void* posz_query, int64_t n_have,
                         int64_t n_query, int dim, int dtype, int leaf_search, int32_t* indices);
+
+/* Gradient of the sort -- replaces the scatter of tree.py:111-138: out[id[i]] = rows[i] for n rows of
+ * `width` elements of elem_bytes (4 with int32 id, 8 with int64 id).  id is a permutation (entries out
+ * of [0, n) are skipped). */
+int jzt_unsort_rows(jzt_stream_t stream, const void* rows, const void* id, int64_t n, int width, int elem_bytes,
+                    void* out);
 
 /* SegmentSort -- replaces ffi target "SegmentSort" (generated/ffi_knn.cu:412-423, knn.cuh:700-722,
  * caller knn.py:112-127).  Sorts (key, val) within segments spl[i]..spl[i+1] by (key, val). */

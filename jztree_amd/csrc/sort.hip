@@ -4,12 +4,14 @@
 // (math.cuh:381-402).  Here the order is computed with an LSD radix sort of a 64-bit Morton key:
 //
 //   1. bounds: max exponent of the finite coordinates, any negative, any inf  (read 12 B/pt)
-//   2. keygen: 63-bit interleaved key + input index; fused 8x256 digit histograms (r12 w12 B/pt)
+//   2. keygen: 63-bit interleaved key; fused 8x256 digit histograms          (r12 w8 B/pt)
 //   3. digit offsets: exclusive scan of the 8 histograms (1 workgroup)
 //   4. 8 onesweep passes (8-bit digits): dynamic tile ids, LDS ranking with wave64 ballots,
-//      decoupled look-back on per-tile digit counts, LDS-staged coalesced scatter (r12 w12 B/pt)
-//   5. fix-up: runs of equal keys are re-ordered with the exact comparator (rare)
-//   6. gather: pos_out = pos_in[idx], id_out = idx                           (r4+12 w12+4 B/pt)
+//      decoupled look-back on per-tile digit counts, LDS-staged coalesced scatter (r12 w12 B/pt;
+//      the first pass reads no indices)
+//   5. finish: pos_out = pos_in[idx], id_out = idx; members of a short run of equal keys write to
+//      their place by the exact comparator                                   (r12+12 w12+4 B/pt)
+//   6. long runs of equal keys, sorted and written by a workgroup each (rare)
 //
 // Key construction.  For coordinates whose largest finite exponent is Lt, each dim contributes a
 // B-bit code (B = 63/dim, i.e. 21 for 3D): the fixed-point bits of |x| at levels Lt-B+1 .. Lt.
@@ -30,10 +32,8 @@
 namespace jzt {
 namespace {
 
-constexpr int kSortThreads = 256;  // 4 waves
-constexpr int kSortWaves = kSortThreads / 64;
-constexpr int kKPTMin = 8;                        // keys per thread: 8, 12 (default) or 16, tuned at run
-                                                  // time; look-back state is sized for the smallest tile
+constexpr int kSortTileMin = 256 * 8;  // smallest tile of a pass (see onesweep()); the look-back
+                                       // state is sized for it
 constexpr int kRadix = 256;
 constexpr int kPasses = 8;
 constexpr uint32_t kFlagAgg = 1u << 30, kFlagInc = 2u << 30, kCountMask = (1u << 30) - 1;
@@ -215,6 +215,9 @@ __device__ __forceinline__ void bounds_value(T x, uint32_t& emax, uint32_t& neg,
 // The coordinates are read as 16-byte vectors, four per thread in flight (a single 4-byte load
 // per iteration left the kernel waiting on memory latency: 0.36 ms for 2^26 3-D points); an
 // unaligned array or the tail past the last whole vector is read value by value.
+// Atomics on the one meta line take about 11 ns each, one after the other: one per wave of 4096
+// workgroups made 188 us, whatever the size.  Now a workgroup adds what is new to the line only
+// (a stale read costs an atomic, no more): 6 us at 1.25e7 values.
 template <typename T>
 __global__ __launch_bounds__(256) void k_bounds(const T* __restrict__ pos, int64_t nval, uint32_t* meta) {
   constexpr int V = 16 / (int)sizeof(T);  // values per vector
@@ -244,16 +247,15 @@ __global__ __launch_bounds__(256) void k_bounds(const T* __restrict__ pos, int64
     for (int c = 0; c < V; c++) bounds_value<T>(e[c], emax, neg, inf);
   }
   for (int64_t j = nvec * V + tid; j < nval; j += st) bounds_value<T>(pos[j], emax, neg, inf);
-  // wave reductions then one atomic per wave
-  for (int o = 32; o > 0; o >>= 1) {
-    emax = max(emax, (uint32_t)__shfl_xor((int)emax, o, 64));
-    neg |= (uint32_t)__shfl_xor((int)neg, o, 64);
-    inf |= (uint32_t)__shfl_xor((int)inf, o, 64);
-  }
-  if ((threadIdx.x & 63) == 0) {
-    atomicMax(&meta[0], emax);
-    if (neg) atomicOr(&meta[1], 1u);
-    if (inf) atomicOr(&meta[2], 1u);
+  __shared__ uint32_t s_e[4];
+  for (int o = 32; o > 0; o >>= 1) emax = max(emax, (uint32_t)__shfl_xor((int)emax, o, 64));
+  if ((threadIdx.x & 63) == 0) s_e[threadIdx.x >> 6] = emax;
+  const int any_neg = __syncthreads_or((int)neg), any_inf = __syncthreads_or((int)inf);
+  if (threadIdx.x == 0) {
+    emax = max(max(s_e[0], s_e[1]), max(s_e[2], s_e[3]));
+    if (emax > ld_acq(&meta[0])) atomicMax(&meta[0], emax);
+    if (any_neg && !ld_acq(&meta[1])) atomicOr(&meta[1], 1u);
+    if (any_inf && !ld_acq(&meta[2])) atomicOr(&meta[2], 1u);
   }
 }
 
@@ -289,8 +291,7 @@ template <typename T> __device__ __forceinline__ int top_level_from_meta(const u
 // ---------------------------------------------------------------------------------------------
 template <int D, typename T>
 __global__ __launch_bounds__(256) void k_keygen(const T* __restrict__ pos, int64_t n, const uint32_t* __restrict__ meta,
-                                                uint64_t* __restrict__ keys, uint32_t* __restrict__ vals,
-                                                uint32_t* __restrict__ hist) {
+                                                uint64_t* __restrict__ keys, uint32_t* __restrict__ hist) {
   __shared__ uint32_t sh[kPasses][kRadix];
   for (int i = threadIdx.x; i < kPasses * kRadix; i += blockDim.x) (&sh[0][0])[i] = 0;
   __syncthreads();
@@ -313,7 +314,6 @@ __global__ __launch_bounds__(256) void k_keygen(const T* __restrict__ pos, int64
     for (int d = 0; d < D; d++) x[d] = pos[i * D + d];
     uint64_t k = morton_key<D, T>(x, Lt, general);
     keys[i] = k;
-    vals[i] = (uint32_t)i;
 #pragma unroll
     for (int p = 0; p < kPasses; p++) atomicAdd(&sh[p][(k >> (8 * p)) & 255u], 1u);
   }
@@ -340,43 +340,51 @@ __global__ __launch_bounds__(256) void k_hist_scan(uint32_t* hist) {
 // ---------------------------------------------------------------------------------------------
 // 4. onesweep pass
 // ---------------------------------------------------------------------------------------------
-template <int KPT>
-__global__ __launch_bounds__(kSortThreads) void k_onesweep(const uint64_t* __restrict__ kin,
-                                                           const uint32_t* __restrict__ vin,
-                                                           uint64_t* __restrict__ kout, uint32_t* __restrict__ vout,
-                                                           int64_t n, int shift,
-                                                           const uint32_t* __restrict__ bucket_off,
-                                                           uint32_t* lookback, uint32_t* tile_counter) {
-  __shared__ uint32_t s_wcnt[kSortWaves][kRadix];
+// One tile of THREADS * KPT pairs per workgroup; vin = nullptr: the values are the indices.
+//
+// Bound by HBM at large n (24 B moved per pair and pass), by the look-back's latency at small n: all
+// tiles start together, so a tile walks back over the aggregates of those before it, one read of about
+// 0.7 us after the other, until it meets a tile that is further along (about sqrt(2 * tile) steps).
+// kLookback rows are therefore read at once, and tiles grow with n: fewer rows to walk over, and the
+// tile's share of a digit, written in one piece, fills whole cache lines.
+constexpr int kLookback = 8;
+
+template <int THREADS, int KPT>
+__global__ __launch_bounds__(THREADS) void k_onesweep(const uint64_t* __restrict__ kin,
+                                                      const uint32_t* __restrict__ vin, uint64_t* __restrict__ kout,
+                                                      uint32_t* __restrict__ vout, int64_t n, int shift,
+                                                      const uint32_t* __restrict__ bucket_off, uint32_t* lookback,
+                                                      uint32_t* tile_counter) {
+  constexpr int kWaves = THREADS / 64, kTile = THREADS * KPT;
+  static_assert(THREADS >= kRadix, "a thread per digit");
+  __shared__ uint32_t s_wcnt[kWaves][kRadix];
   __shared__ uint32_t s_lstart[kRadix];
   __shared__ uint32_t s_gbase[kRadix];
-  __shared__ uint64_t s_keys[(kSortThreads * KPT)];
-  __shared__ int s_scan[kSortThreads / 64];
+  __shared__ uint64_t s_keys[kTile];
+  __shared__ int s_scan[kWaves];
   __shared__ uint32_t s_tile;
 
   const int tid = threadIdx.x, w = tid >> 6, lane = tid & 63;
   if (tid == 0) s_tile = atomicAdd(tile_counter, 1u);
-  for (int i = tid; i < kSortWaves * kRadix; i += kSortThreads) (&s_wcnt[0][0])[i] = 0;
+  for (int i = tid; i < kWaves * kRadix; i += THREADS) (&s_wcnt[0][0])[i] = 0;
   __syncthreads();
   const uint32_t tile = s_tile;
-  const int64_t base = (int64_t)tile * (kSortThreads * KPT);
+  const int64_t base = (int64_t)tile * kTile;
   const int64_t wbase = base + (int64_t)w * 64 * KPT;
 
   uint64_t key[KPT];
   uint32_t val[KPT];  // loaded with the keys, so the tile waits for global memory once
-  uint32_t dig[KPT];
   uint32_t rank[KPT];
 #pragma unroll
   for (int r = 0; r < KPT; r++) {
-    int64_t idx = wbase + r * 64 + lane;
+    const int64_t idx = wbase + r * 64 + lane;
     key[r] = idx < n ? kin[idx] : ~0ull;
-    val[r] = idx < n ? vin[idx] : 0u;
-    dig[r] = (uint32_t)(key[r] >> shift) & 255u;
+    val[r] = vin ? (idx < n ? vin[idx] : 0u) : (uint32_t)idx;
   }
   const uint64_t lt_mask = (1ull << lane) - 1ull;
 #pragma unroll
   for (int r = 0; r < KPT; r++) {
-    uint32_t d = dig[r];
+    const uint32_t d = (uint32_t)(key[r] >> shift) & 255u;
     uint64_t m = ~0ull;
 #pragma unroll
     for (int b = 0; b < 8; b++) {
@@ -391,55 +399,66 @@ __global__ __launch_bounds__(kSortThreads) void k_onesweep(const uint64_t* __res
   }
   __syncthreads();
 
-  // per-digit tile totals and per-wave exclusive offsets (thread tid owns digit tid)
+  // per-digit tile totals and per-wave exclusive offsets (thread tid < 256 owns digit tid)
   const int d = tid;
-  uint32_t total = 0;
+  uint32_t total = 0, excl = 0;
+  if (tid < kRadix) {
 #pragma unroll
-  for (int ww = 0; ww < kSortWaves; ww++) {
-    uint32_t c = s_wcnt[ww][d];
-    s_wcnt[ww][d] = total;
-    total += c;
-  }
-  // decoupled look-back across tiles, one digit per thread
-  uint32_t* lb = lookback + (int64_t)tile * kRadix;
-  uint32_t excl = 0;
-  if (tile == 0) {
-    st_rel(&lb[d], kFlagInc | total);
-  } else {
-    st_rel(&lb[d], kFlagAgg | total);
-    int64_t j = (int64_t)tile - 1;
-    while (true) {
-      uint32_t v = ld_acq(&lookback[j * kRadix + d]);
-      uint32_t f = v & ~kCountMask;
-      if (f == 0) continue;
-      excl += v & kCountMask;
-      if (f == kFlagInc) break;
-      j--;
+    for (int ww = 0; ww < kWaves; ww++) {
+      uint32_t c = s_wcnt[ww][d];
+      s_wcnt[ww][d] = total;
+      total += c;
     }
-    st_rel(&lb[d], kFlagInc | (excl + total));
+    // decoupled look-back across tiles, one digit per thread
+    uint32_t* lb = lookback + (int64_t)tile * kRadix;
+    if (tile == 0) {
+      st_rel(&lb[d], kFlagInc | total);
+    } else {
+      st_rel(&lb[d], kFlagAgg | total);
+      int64_t j = (int64_t)tile - 1;
+      bool done = false;
+      while (!done) {
+        uint32_t v[kLookback];
+#pragma unroll
+        for (int u = 0; u < kLookback; u++) v[u] = ld_acq(&lookback[max(j - u, (int64_t)0) * kRadix + d]);
+        // up to the first row that is not there yet; tile 0's is inclusive, so the walk ends there
+        bool go = true;
+#pragma unroll
+        for (int u = 0; u < kLookback; u++) {
+          go = go && !done && (v[u] & ~kCountMask) != 0;
+          if (go) {
+            excl += v[u] & kCountMask;
+            done = (v[u] & kFlagInc) != 0;
+            j--;
+          }
+        }
+      }
+      st_rel(&lb[d], kFlagInc | (excl + total));
+    }
   }
   int tot;
-  uint32_t lstart = (uint32_t)block_excl_scan<kSortThreads>((int)total, s_scan, &tot);
-  s_lstart[d] = lstart;
-  s_gbase[d] = bucket_off[d] + excl - lstart;
+  const uint32_t lstart = (uint32_t)block_excl_scan<THREADS>((int)total, s_scan, &tot);
+  if (tid < kRadix) {
+    s_lstart[d] = lstart;
+    s_gbase[d] = bucket_off[d] + excl - lstart;
+  }
   __syncthreads();
 
   // scatter keys into LDS in tile-local digit order (each key's local slot kept for its value)
-  uint32_t slot[KPT];
 #pragma unroll
   for (int r = 0; r < KPT; r++) {
-    uint32_t dd = dig[r];
-    slot[r] = s_lstart[dd] + s_wcnt[w][dd] + rank[r];
-    s_keys[slot[r]] = key[r];
+    const uint32_t dd = (uint32_t)(key[r] >> shift) & 255u;
+    rank[r] += s_lstart[dd] + s_wcnt[w][dd];
+    s_keys[rank[r]] = key[r];
   }
   __syncthreads();
   // write out in local order; a slot's digit comes from its key, its global index is kept for
-  // the value pass (slot i = tid + r * kSortThreads)
-  const int tile_n = (int)((n - base) < (kSortThreads * KPT) ? (n - base) : (kSortThreads * KPT));
+  // the value pass (slot i = tid + r * THREADS)
+  const int tile_n = (int)((n - base) < kTile ? (n - base) : kTile);
   uint32_t gidx[KPT];
 #pragma unroll
   for (int r = 0; r < KPT; r++) {
-    const int i = tid + r * kSortThreads;
+    const int i = tid + r * THREADS;
     gidx[r] = 0xffffffffu;
     if (i < tile_n) {
       const uint64_t kk = s_keys[i];
@@ -450,41 +469,82 @@ __global__ __launch_bounds__(kSortThreads) void k_onesweep(const uint64_t* __res
   __syncthreads();
   uint32_t* s_vals = reinterpret_cast<uint32_t*>(s_keys);
 #pragma unroll
-  for (int r = 0; r < KPT; r++) s_vals[slot[r]] = val[r];
+  for (int r = 0; r < KPT; r++) s_vals[rank[r]] = val[r];
   __syncthreads();
 #pragma unroll
   for (int r = 0; r < KPT; r++) {
-    const int i = tid + r * kSortThreads;
+    const int i = tid + r * THREADS;
     if (i < tile_n && gidx[r] < (uint64_t)n) vout[gidx[r]] = s_vals[i];
   }
 }
 
 // ---------------------------------------------------------------------------------------------
-// 5. fix-up of equal-key runs (exact comparator, then index)
+// 5., 6. finish: equal-key runs (exact comparator, then index) and the gather
 // ---------------------------------------------------------------------------------------------
-__global__ __launch_bounds__(256) void k_run_flags(const uint64_t* __restrict__ keys, int64_t n,
-                                                   int8_t* __restrict__ flags) {
-  int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  const uint64_t k = keys[i];
-  flags[i] = (i + 1 < n && keys[i + 1] == k && (i == 0 || keys[i - 1] != k)) ? 1 : 0;
-}
-
 template <int D, typename T>
 __device__ __forceinline__ bool idx_less(const T* __restrict__ pos, uint32_t a, uint32_t b) {
   int c = exact_cmp<D, T>(pos + (int64_t)a * D, pos + (int64_t)b * D);
   return (c < 0) || (c == 0 && a < b);
 }
 
-// One workgroup per run of equal keys (grid-stride over the run list).  The run's end is found by
+template <int D, typename T>
+__device__ __forceinline__ void finish_row(const T* __restrict__ pos, uint32_t v, int64_t dst, int64_t n,
+                                           T* __restrict__ pos_out, typename IntOf<T>::type* __restrict__ id_out) {
+  if (v >= (uint64_t)n) v = 0;  // unreachable for a valid permutation; keeps a logic error in bounds
+#pragma unroll
+  for (int d = 0; d < D; d++) pos_out[dst * D + d] = pos[(int64_t)v * D + d];
+  id_out[dst] = (typename IntOf<T>::type)v;
+}
+
+// One row per thread.  A row whose key no neighbour has goes where it stands; the members of a run of
+// up to kShortRun equal keys (of the same set, with setk) each count those before them; the starts of
+// longer runs are listed for k_long_runs.  Bound by the random reads of pos (a cache line for every
+// 12 or 24 bytes).  Flags, compaction, fix-up and gather as steps of their own took 6 launches and
+// wrote and read a flag per row: 120 us instead of 95 at 4.2e6 points.
+constexpr int kShortRun = 16;
+
+template <int D, typename T>
+__global__ __launch_bounds__(256) void k_finish(const uint64_t* __restrict__ keys, const uint32_t* __restrict__ vals,
+                                                const int32_t* __restrict__ setk, int64_t n,
+                                                const T* __restrict__ pos, T* __restrict__ pos_out,
+                                                typename IntOf<T>::type* __restrict__ id_out,
+                                                int32_t* __restrict__ runs, int32_t* nruns, int64_t max_runs) {
+  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= n) return;
+  const uint64_t k = keys[i];
+  const int32_t sk = setk ? setk[i] : 0;
+  auto same = [&](int64_t j) { return keys[j] == k && (!setk || setk[j] == sk); };
+  const uint32_t v = vals[i];
+  int64_t dst = i;
+  const bool prev = i > 0 && same(i - 1), next = i + 1 < n && same(i + 1);
+  if (prev || next) {
+    int64_t a = i, b = i + 1;  // the run is [a, b), looked at up to kShortRun rows either way
+    while (a > 0 && i - a < kShortRun && same(a - 1)) a--;
+    while (b < n && b - i <= kShortRun && same(b)) b++;
+    if (b - a > kShortRun) {
+      if (!prev) {
+        const int32_t at = atomicAdd(nruns, 1);
+        if (at < max_runs) runs[at] = (int32_t)i;
+      }
+      return;
+    }
+    dst = a;
+    for (int64_t j = a; j < b; j++) dst += j != i && idx_less<D, T>(pos, vals[j], v);
+  }
+  finish_row<D, T>(pos, v, dst, n, pos_out, id_out);
+}
+
+// One workgroup per listed run (grid-stride over the list).  The run's end is found by
 // a strided parallel search, sortedness by (exact order, index) is checked pairwise, and unsorted
 // runs are put in order by a bitonic network (ascending comparators only, so any length works)
 // applied in place to the run's indices in global memory.
 template <int D, typename T>
-__global__ __launch_bounds__(256) void k_fix_runs(const uint64_t* __restrict__ keys, uint32_t* vals, int64_t n,
-                                                  const T* __restrict__ pos, const int32_t* __restrict__ runs,
-                                                  const int32_t* __restrict__ nruns_p, int64_t max_runs,
-                                                  const int32_t* __restrict__ setk) {
+__global__ __launch_bounds__(256) void k_long_runs(const uint64_t* __restrict__ keys, uint32_t* vals, int64_t n,
+                                                   const T* __restrict__ pos, T* __restrict__ pos_out,
+                                                   typename IntOf<T>::type* __restrict__ id_out,
+                                                   const int32_t* __restrict__ runs,
+                                                   const int32_t* __restrict__ nruns_p, int64_t max_runs,
+                                                   const int32_t* __restrict__ setk) {
   __shared__ unsigned long long s_end;
   const int64_t nruns = min((int64_t)nruns_p[0], max_runs);
   for (int64_t r = blockIdx.x; r < nruns; r += gridDim.x) {
@@ -538,62 +598,79 @@ __global__ __launch_bounds__(256) void k_fix_runs(const uint64_t* __restrict__ k
         }
       }
     }
+    for (int64_t j = start + threadIdx.x; j < end; j += blockDim.x)
+      finish_row<D, T>(pos, vals[j], j, n, pos_out, id_out);
     __syncthreads();
   }
 }
 
-// ---------------------------------------------------------------------------------------------
-// 6. gather
-// ---------------------------------------------------------------------------------------------
 template <int D, typename T>
-__global__ __launch_bounds__(256) void k_gather(const T* __restrict__ pos, const uint32_t* __restrict__ vals, int64_t n,
-                                                T* __restrict__ pos_out, typename IntOf<T>::type* __restrict__ id_out) {
-  int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  uint32_t v = vals[i];
-  if (v >= (uint64_t)n) v = 0;  // unreachable for a valid permutation; keeps a logic error in bounds
-#pragma unroll
-  for (int d = 0; d < D; d++) pos_out[i * D + d] = pos[(int64_t)v * D + d];
-  id_out[i] = (typename IntOf<T>::type)v;
+int finish(hipStream_t s, const uint64_t* keys, uint32_t* vals, const int32_t* setk, int64_t n, const T* pos,
+           T* pos_out, typename IntOf<T>::type* id_out, int32_t* runs, int32_t* nruns) {
+  const int64_t max_runs = n / (kShortRun + 1) + 1;  // none shorter is listed
+  hipLaunchKernelGGL((k_finish<D, T>), dim3((unsigned)div_up(n, 256)), dim3(256), 0, s, keys, vals, setk, n, pos,
+                     pos_out, id_out, runs, nruns, max_runs);
+  if (n > kShortRun)
+    hipLaunchKernelGGL((k_long_runs<D, T>), dim3((unsigned)std::min(max_runs, (int64_t)512)), dim3(256), 0, s, keys,
+                       vals, n, pos, pos_out, id_out, runs, nruns, max_runs, setk);
+  return check_launch("zsort finish");
 }
 
-// one onesweep pass with the tuned tile (keys per thread); look-back slots are `stride` tiles apart
-int onesweep(hipStream_t s, const uint64_t* ki, const uint32_t* vi, uint64_t* ko, uint32_t* vo, int64_t n, int shift,
-             const uint32_t* bucket, uint32_t* lookback, uint32_t* counter) {
-  const int kpt = tune_get(kTuneSortKpt);
-  if (kpt == 8)
-    hipLaunchKernelGGL(k_onesweep<8>, dim3((unsigned)div_up(n, kSortThreads * 8)), dim3(kSortThreads), 0, s, ki, vi, ko,
-                       vo, n, shift, bucket, lookback, counter);
-  else if (kpt == 16)
-    hipLaunchKernelGGL(k_onesweep<16>, dim3((unsigned)div_up(n, kSortThreads * 16)), dim3(kSortThreads), 0, s, ki, vi,
-                       ko, vo, n, shift, bucket, lookback, counter);
-  else
-    hipLaunchKernelGGL(k_onesweep<12>, dim3((unsigned)div_up(n, kSortThreads * 12)), dim3(kSortThreads), 0, s, ki, vi,
-                       ko, vo, n, shift, bucket, lookback, counter);
+// Tile of a pass over n pairs.  More threads per tile mean fewer look-back rows and longer writes,
+// fewer tiles than compute units leave the chip idle.  Whole sort of float 3-D points, us, with tiles of
+// 256 x 8 / 512 x 8 / 1024 x 8 / 1024 x 12 pairs:
+//   65,536 points 94 / 101 / 128 / 158      2^20 255 / 219 / 235 / 260      2^22 623 / 502 / 481 / 499
+//   2^24 2077 / 1713 / 1601 / 1573          2^26 8200 / 6820 / 6348 / 5847
+// (256 x 12 with one look-back row at a time: 130, 530, 810, 2600, 7800.)  A tuned number of keys per
+// thread other than the default takes the place of 8 and 12.
+struct SortTile {
+  int threads, kpt;
+  int64_t tiles;
+};
+SortTile sort_tile(int64_t n) {
+  const int tuned = tune_get(kTuneSortKpt);
+  const int kpt = tuned != 12 ? tuned : n < (int64_t)1 << 23 ? 8 : 12;
+  const int threads = n < (int64_t)1 << 18 ? 256 : n < (int64_t)1 << 21 ? 512 : 1024;
+  return {threads, kpt, div_up(n, (int64_t)threads * kpt)};
+}
+
+// one onesweep pass; look-back rows are st.tiles apart from pass to pass
+int onesweep(hipStream_t s, const SortTile& st, const uint64_t* ki, const uint32_t* vi, uint64_t* ko, uint32_t* vo,
+             int64_t n, int shift, const uint32_t* bucket, uint32_t* lookback, uint32_t* counter) {
+#define JZT_SWEEP(TH, K)                                                                                        \
+  if (st.threads == TH && st.kpt == K)                                                                          \
+    hipLaunchKernelGGL((k_onesweep<TH, K>), dim3((unsigned)st.tiles), dim3(TH), 0, s, ki, vi, ko, vo, n, shift, \
+                       bucket, lookback, counter)
+  JZT_SWEEP(256, 8);
+  JZT_SWEEP(256, 12);
+  JZT_SWEEP(256, 16);
+  JZT_SWEEP(512, 8);
+  JZT_SWEEP(512, 12);
+  JZT_SWEEP(512, 16);
+  JZT_SWEEP(1024, 8);
+  JZT_SWEEP(1024, 12);
+  JZT_SWEEP(1024, 16);
+#undef JZT_SWEEP
   return 0;
 }
 
 struct SortLayout {
-  size_t keys0, vals0, keys1, vals1, hist, meta, lookback, poscopy, runflags, runtmp, runs, nruns, total;
-  int64_t ntiles;
+  size_t keys0, vals0, keys1, vals1, hist, meta, lookback, poscopy, runs, total;
 };
 
 SortLayout sort_layout(int64_t n, int dim, int dtype) {
   SortLayout L;
   size_t o = 0;
-  L.ntiles = div_up(n > 0 ? n : 1, kSortThreads * kKPTMin);  // look-back stride of every pass
+  const int64_t ntiles = div_up(n > 0 ? n : 1, kSortTileMin);
   L.keys0 = o; o = align256(o + 8 * (size_t)n);
   L.vals0 = o; o = align256(o + 4 * (size_t)n);
   L.keys1 = o; o = align256(o + 8 * (size_t)n);
   L.vals1 = o; o = align256(o + 4 * (size_t)n);
   L.hist = o; o += 4 * (size_t)kPasses * kRadix;
-  L.meta = o; o += 4 * 16;
-  L.lookback = o; o = align256(o + 4 * (size_t)kPasses * L.ntiles * kRadix);
+  L.meta = o; o += 4 * 32;  // bounds, number of long runs (4), tile counters (8..15, set passes 16, 17)
+  L.lookback = o; o = align256(o + 4 * (size_t)(kPasses + 2) * ntiles * kRadix);
   L.poscopy = o; o = align256(o + (size_t)n * dim * ((dtype == JZT_F64 || dtype == JZT_I64) ? 8 : 4));
-  L.runflags = o; o = align256(o + (size_t)n);
-  L.runtmp = o; o = align256(o + 4 * (size_t)(scan_tmp_words(n) + n));
-  L.runs = o; o = align256(o + 4 * (size_t)(n / 2 + 1));
-  L.nruns = o; o = align256(o + 4);
+  L.runs = o; o = align256(o + 4 * (size_t)(n / (kShortRun + 1) + 1));
   L.total = o;
   return L;
 }
@@ -608,8 +685,9 @@ int zsort_impl(hipStream_t s, const T* pos_in, T* pos_out, typename IntOf<T>::ty
   uint32_t* hist = (uint32_t*)(tmp + L.hist);
   uint32_t* meta = (uint32_t*)(tmp + L.meta);
   uint32_t* lookback = (uint32_t*)(tmp + L.lookback);
+  const SortTile st = sort_tile(n);
   // zero histograms, meta (incl. tile counters) and look-back state in one fill
-  if (fill_u32(s, hist, 0u, (int64_t)((L.poscopy - L.hist) / 4))) return 1;
+  if (fill_u32(s, hist, 0u, (int64_t)((L.lookback - L.hist) / 4) + kPasses * st.tiles * kRadix)) return 1;
   const T* src = pos_in;
   if ((const void*)pos_in == (const void*)pos_out) {
     T* cp = (T*)(tmp + L.poscopy);
@@ -617,37 +695,26 @@ int zsort_impl(hipStream_t s, const T* pos_in, T* pos_out, typename IntOf<T>::ty
       return fail("zsort: copy of aliased input failed");
     src = cp;
   }
-  int64_t blocks = div_up(n * D, 256);
-  if (blocks > 4096) blocks = 4096;
+  int64_t blocks = div_up(n * D, 256 * 16);
+  if (blocks > 2048) blocks = 2048;
   if constexpr (std::is_integral<T>::value)
     hipLaunchKernelGGL((k_bounds_int<T>), dim3((unsigned)blocks), dim3(256), 0, s, src, n * D, meta);
   else
     hipLaunchKernelGGL((k_bounds<T>), dim3((unsigned)blocks), dim3(256), 0, s, src, n * D, meta);
   blocks = div_up(n, 256);
   if (blocks > 2048) blocks = 2048;
-  hipLaunchKernelGGL((k_keygen<D, T>), dim3((unsigned)blocks), dim3(256), 0, s, src, n, meta, k0, v0, hist);
+  hipLaunchKernelGGL((k_keygen<D, T>), dim3((unsigned)blocks), dim3(256), 0, s, src, n, meta, k0, hist);
   hipLaunchKernelGGL(k_hist_scan, dim3(1), dim3(256), 0, s, hist);
   if (check_launch("zsort keygen")) return 1;
   for (int p = 0; p < kPasses; p++) {
     const uint64_t* ki = (p & 1) ? k1 : k0;
-    const uint32_t* vi = (p & 1) ? v1 : v0;
+    const uint32_t* vi = p == 0 ? nullptr : (p & 1) ? v1 : v0;
     uint64_t* ko = (p & 1) ? k0 : k1;
     uint32_t* vo = (p & 1) ? v0 : v1;
-    onesweep(s, ki, vi, ko, vo, n, 8 * p,
-                       hist + p * kRadix, lookback + (int64_t)p * L.ntiles * kRadix, meta + 8 + p);
+    onesweep(s, st, ki, vi, ko, vo, n, 8 * p, hist + p * kRadix, lookback + p * st.tiles * kRadix, meta + 8 + p);
   }
   if (check_launch("zsort onesweep")) return 1;
-  // fix-up of equal-key runs
-  int8_t* rflags = (int8_t*)(tmp + L.runflags);
-  int32_t* runs = (int32_t*)(tmp + L.runs);
-  int32_t* nruns = (int32_t*)(tmp + L.nruns);
-  const int64_t max_runs = n / 2 + 1;
-  hipLaunchKernelGGL(k_run_flags, dim3((unsigned)div_up(n, 256)), dim3(256), 0, s, k0, n, rflags);
-  if (where_flags_i8(s, rflags, n, runs, max_runs, 0, nullptr, nruns, (int32_t*)(tmp + L.runtmp))) return 1;
-  hipLaunchKernelGGL((k_fix_runs<D, T>), dim3(1024), dim3(256), 0, s, k0, v0, n, src, runs, nruns, max_runs,
-                     (const int32_t*)nullptr);
-  hipLaunchKernelGGL((k_gather<D, T>), dim3((unsigned)div_up(n, 256)), dim3(256), 0, s, src, v0, n, pos_out, id_out);
-  return check_launch("zsort gather");
+  return finish<D, T>(s, k0, v0, nullptr, n, src, pos_out, id_out, (int32_t*)(tmp + L.runs), (int32_t*)meta + 4);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -748,8 +815,7 @@ template <int D, typename T>
 __global__ __launch_bounds__(256) void k_keygen_seg(const T* __restrict__ pos, int64_t n,
                                                     const int32_t* __restrict__ setid,
                                                     const uint32_t* __restrict__ metas, uint64_t* __restrict__ keys,
-                                                    uint64_t* __restrict__ keys_orig, uint32_t* __restrict__ vals,
-                                                    uint32_t* __restrict__ hist) {
+                                                    uint64_t* __restrict__ keys_orig, uint32_t* __restrict__ hist) {
   __shared__ uint32_t sh[kPasses][kRadix];
   for (int i = threadIdx.x; i < kPasses * kRadix; i += blockDim.x) (&sh[0][0])[i] = 0;
   __syncthreads();
@@ -763,7 +829,6 @@ __global__ __launch_bounds__(256) void k_keygen_seg(const T* __restrict__ pos, i
     const uint64_t k = morton_key<D, T>(x, Lt, general);
     keys[i] = k;
     keys_orig[i] = k;
-    vals[i] = (uint32_t)i;
 #pragma unroll
     for (int p = 0; p < kPasses; p++) atomicAdd(&sh[p][(k >> (8 * p)) & 255u], 1u);
   }
@@ -800,18 +865,6 @@ __global__ void k_final_keys(const uint32_t* __restrict__ vals, const uint64_t* 
   kf[i] = keys_orig[v];
   setk[i] = setid[v];
 }
-__global__ __launch_bounds__(256) void k_run_flags_seg(const uint64_t* __restrict__ keys,
-                                                       const int32_t* __restrict__ setk, int64_t n,
-                                                       int8_t* __restrict__ flags) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  const uint64_t k = keys[i];
-  const int32_t sk = setk[i];
-  const bool next = i + 1 < n && keys[i + 1] == k && setk[i + 1] == sk;
-  const bool prev = i > 0 && keys[i - 1] == k && setk[i - 1] == sk;
-  flags[i] = (next && !prev) ? 1 : 0;
-}
-
 struct SegLayout {
   SortLayout base;
   size_t setid, setk, korig, metas, total;
@@ -844,7 +897,9 @@ int zsort_seg_impl(hipStream_t s, const T* pos_in, T* pos_out, typename IntOf<T>
   int32_t* setid = (int32_t*)(tmp + SL.setid);
   uint64_t* korig = (uint64_t*)(tmp + SL.korig);
   uint32_t* metas = (uint32_t*)(tmp + SL.metas);
-  if (fill_u32(s, hist, 0u, (int64_t)((L.poscopy - L.hist) / 4))) return 1;
+  const SortTile st = sort_tile(n);
+  // the set passes have look-back rows of their own; their histograms take the place of the first two
+  if (fill_u32(s, hist, 0u, (int64_t)((L.lookback - L.hist) / 4) + (kPasses + 2) * st.tiles * kRadix)) return 1;
   if (fill_u32(s, metas, 0u, 3 * nsets)) return 1;
   const T* src = pos_in;
   if ((const void*)pos_in == (const void*)pos_out) {
@@ -856,36 +911,31 @@ int zsort_seg_impl(hipStream_t s, const T* pos_in, T* pos_out, typename IntOf<T>
   const unsigned gb = (unsigned)std::min(div_up(n, 256), (int64_t)2048);
   hipLaunchKernelGGL(k_set_ids, dim3(gb), dim3(256), 0, s, off, nsets, n, setid);
   hipLaunchKernelGGL((k_bounds_seg<D, T>), dim3(gb), dim3(256), 0, s, src, n, setid, metas);
-  hipLaunchKernelGGL((k_keygen_seg<D, T>), dim3(gb), dim3(256), 0, s, src, n, setid, metas, k0, korig, v0, hist);
+  hipLaunchKernelGGL((k_keygen_seg<D, T>), dim3(gb), dim3(256), 0, s, src, n, setid, metas, k0, korig, hist);
   hipLaunchKernelGGL(k_hist_scan, dim3(1), dim3(256), 0, s, hist);
   if (check_launch("zsort_segmented keygen")) return 1;
   for (int p = 0; p < kPasses; p++) {
     const uint64_t* ki = (p & 1) ? k1 : k0;
-    const uint32_t* vi = (p & 1) ? v1 : v0;
+    const uint32_t* vi = p == 0 ? nullptr : (p & 1) ? v1 : v0;
     uint64_t* ko = (p & 1) ? k0 : k1;
     uint32_t* vo = (p & 1) ? v0 : v1;
-    onesweep(s, ki, vi, ko, vo, n, 8 * p,
-                       hist + p * kRadix, lookback + (int64_t)p * L.ntiles * kRadix, meta + 8 + p);
+    onesweep(s, st, ki, vi, ko, vo, n, 8 * p, hist + p * kRadix, lookback + p * st.tiles * kRadix, meta + 8 + p);
   }
   if (check_launch("zsort_segmented onesweep")) return 1;
-  // stable set passes: (set key, value) from (k1, v0); histograms, look-back and tile counters of
-  // Morton passes 0 and 1 are reused after clearing
+  // stable set passes: (set key, value) from (k1, v0)
   const int npass_set = nsets > 256 ? 2 : 1;
+  uint32_t* lookback_set = lookback + kPasses * st.tiles * kRadix;
   if (fill_u32(s, hist, 0u, 2 * kRadix)) return 1;
-  if (fill_u32(s, lookback, 0u, 2 * L.ntiles * kRadix)) return 1;
-  if (fill_u32(s, meta + 8, 0u, 2)) return 1;
   hipLaunchKernelGGL(k_set_hist, dim3((unsigned)std::min(div_up(nsets, 256), (int64_t)1024)), dim3(256), 0, s, off, nsets,
                      hist);
   hipLaunchKernelGGL(k_hist_scan, dim3(1), dim3(256), 0, s, hist);  // scans all 8 rows; rows 0-1 matter
   hipLaunchKernelGGL(k_set_keys, dim3((unsigned)div_up(n, 256)), dim3(256), 0, s, v0, setid, n, k1);
   const uint32_t* vfinal = v0;
   {
-    onesweep(s, k1, v0, k0, v1, n, 0, hist,
-                       lookback, meta + 8);
+    onesweep(s, st, k1, v0, k0, v1, n, 0, hist, lookback_set, meta + 16);
     vfinal = v1;
     if (npass_set == 2) {
-      onesweep(s, k0, v1, k1, v0, n, 8,
-                         hist + kRadix, lookback + (int64_t)L.ntiles * kRadix, meta + 9);
+      onesweep(s, st, k0, v1, k1, v0, n, 8, hist + kRadix, lookback_set + st.tiles * kRadix, meta + 17);
       vfinal = v0;
     }
   }
@@ -894,15 +944,7 @@ int zsort_seg_impl(hipStream_t s, const T* pos_in, T* pos_out, typename IntOf<T>
   uint64_t* kf = (vf == v1) ? k1 : k0;  // the key buffer not holding set keys any more
   int32_t* setk = (int32_t*)(tmp + SL.setk);
   hipLaunchKernelGGL(k_final_keys, dim3((unsigned)div_up(n, 256)), dim3(256), 0, s, vf, korig, setid, n, kf, setk);
-  int8_t* rflags = (int8_t*)(tmp + L.runflags);
-  int32_t* runs = (int32_t*)(tmp + L.runs);
-  int32_t* nruns = (int32_t*)(tmp + L.nruns);
-  const int64_t max_runs = n / 2 + 1;
-  hipLaunchKernelGGL(k_run_flags_seg, dim3((unsigned)div_up(n, 256)), dim3(256), 0, s, kf, setk, n, rflags);
-  if (where_flags_i8(s, rflags, n, runs, max_runs, 0, nullptr, nruns, (int32_t*)(tmp + L.runtmp))) return 1;
-  hipLaunchKernelGGL((k_fix_runs<D, T>), dim3(1024), dim3(256), 0, s, kf, vf, n, src, runs, nruns, max_runs, setk);
-  hipLaunchKernelGGL((k_gather<D, T>), dim3((unsigned)div_up(n, 256)), dim3(256), 0, s, src, vf, n, pos_out, id_out);
-  return check_launch("zsort_segmented gather");
+  return finish<D, T>(s, kf, vf, setk, n, src, pos_out, id_out, (int32_t*)(tmp + L.runs), (int32_t*)meta + 4);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -918,8 +960,8 @@ int zsort_seg_impl(hipStream_t s, const T* pos_in, T* pos_out, typename IntOf<T>
 
 __global__ __launch_bounds__(256) void k_label_keys(const int32_t* __restrict__ igroup,
                                                     const int32_t* __restrict__ npart_dev, int64_t n, int npass,
-                                                    uint64_t* __restrict__ keys, uint32_t* __restrict__ vals,
-                                                    uint32_t* __restrict__ hist, uint32_t* __restrict__ cnt) {
+                                                    uint64_t* __restrict__ keys, uint32_t* __restrict__ hist,
+                                                    uint32_t* __restrict__ cnt) {
   __shared__ uint32_t sh[4][kRadix];
   for (int i = threadIdx.x; i < 4 * kRadix; i += blockDim.x) (&sh[0][0])[i] = 0;
   __syncthreads();
@@ -935,7 +977,6 @@ __global__ __launch_bounds__(256) void k_label_keys(const int32_t* __restrict__ 
     const uint32_t key = in ? (uint32_t)(lab64 >= 0 && lab64 <= n ? lab64 : n) : 0u;
     if (in) {
       keys[i] = key;
-      vals[i] = (uint32_t)i;
       for (int p = 0; p < npass; p++) atomicAdd(&sh[p][(key >> (8 * p)) & 255u], 1u);
     }
     // runs of equal counted labels in consecutive lanes: the first lane of a run adds its length
@@ -965,13 +1006,12 @@ __global__ void k_label_counts(const uint32_t* __restrict__ isort, const uint32_
 
 struct OrderLayout {
   size_t keys0, keys1, vals0, vals1, cnt, hist, meta, lookback, total;
-  int64_t ntiles;
 };
 
 OrderLayout order_layout(int64_t n) {
   OrderLayout L;
   size_t o = 0;
-  L.ntiles = div_up(n > 0 ? n : 1, kSortThreads * kKPTMin);
+  const int64_t ntiles = div_up(n > 0 ? n : 1, kSortTileMin);
   L.keys0 = o; o = align256(o + 8 * (size_t)n);
   L.keys1 = o; o = align256(o + 8 * (size_t)n);
   L.vals0 = o; o = align256(o + 4 * (size_t)n);
@@ -980,7 +1020,7 @@ OrderLayout order_layout(int64_t n) {
   L.cnt = o; o += 4 * (size_t)(n + 1);
   L.hist = o; o += 4 * (size_t)kPasses * kRadix;
   L.meta = o; o += 4 * 16;
-  L.lookback = o; o = align256(o + 4 * (size_t)4 * L.ntiles * kRadix);
+  L.lookback = o; o = align256(o + 4 * (size_t)4 * ntiles * kRadix);
   L.total = o;
   return L;
 }
@@ -996,25 +1036,42 @@ int fof_order_impl(hipStream_t s, const int32_t* igroup, const int32_t* npart, i
   uint32_t* hist = (uint32_t*)(tmp + L.hist);
   uint32_t* meta = (uint32_t*)(tmp + L.meta);
   uint32_t* lookback = (uint32_t*)(tmp + L.lookback);
-  if (fill_u32(s, cnt, 0u, (int64_t)((L.total - L.cnt) / 4))) return 1;
   int bits = 0;
   while (bits < 32 && ((uint64_t)n >> bits) != 0) bits++;  // keys are <= n
   const int npass = std::max(1, (bits + 7) / 8);
+  const SortTile st = sort_tile(n);
+  if (fill_u32(s, cnt, 0u, (int64_t)((L.lookback - L.cnt) / 4) + npass * st.tiles * kRadix)) return 1;
   const unsigned gb = (unsigned)std::min(div_up(n, 256), (int64_t)2048);
-  hipLaunchKernelGGL(k_label_keys, dim3(gb), dim3(256), 0, s, igroup, npart, n, npass, k0, v0, hist, cnt);
+  hipLaunchKernelGGL(k_label_keys, dim3(gb), dim3(256), 0, s, igroup, npart, n, npass, k0, hist, cnt);
   hipLaunchKernelGGL(k_hist_scan, dim3(1), dim3(256), 0, s, hist);
   if (check_launch("FofOrder keys")) return 1;
   for (int p = 0; p < npass; p++) {
     const uint64_t* ki = (p & 1) ? k1 : k0;
-    const uint32_t* vi = (p & 1) ? v1 : v0;
+    const uint32_t* vi = p == 0 ? nullptr : (p & 1) ? v1 : v0;
     uint64_t* ko = (p & 1) ? k0 : k1;
     // the last pass writes the permutation straight into isort
     uint32_t* vo = (p == npass - 1) ? (uint32_t*)isort : ((p & 1) ? v0 : v1);
-    onesweep(s, ki, vi, ko, vo, n, 8 * p, hist + p * kRadix, lookback + (int64_t)p * L.ntiles * kRadix, meta + 8 + p);
+    onesweep(s, st, ki, vi, ko, vo, n, 8 * p, hist + p * kRadix, lookback + p * st.tiles * kRadix, meta + 8 + p);
   }
   hipLaunchKernelGGL(k_label_counts, dim3((unsigned)div_up(n, 256)), dim3(256), 0, s, (const uint32_t*)isort, cnt, n,
                      counts);
   return check_launch("FofOrder");
+}
+
+// ---------------------------------------------------------------------------------------------
+// 8b. rows back to input order (the gradient of the sort)
+// ---------------------------------------------------------------------------------------------
+// out[id[i]] = rows[i], rows of `width` elements, one element per thread: the threads of a row are
+// neighbours, so its scattered write is one piece.  As an inverse permutation (zeros, arange, scatter)
+// and a gather on 64-bit indices this took 7 launches and 200 us for 2^22 rows of 3 floats.
+template <typename U, typename I>
+__global__ __launch_bounds__(256) void k_unsort_rows(const U* __restrict__ rows, const I* __restrict__ id, int64_t n,
+                                                     int width, U* __restrict__ out) {
+  const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (e >= n * width) return;
+  const int64_t i = e / width;
+  const int64_t dst = (int64_t)id[i];
+  if (dst >= 0 && dst < n) out[dst * width + (e - i * width)] = rows[e];
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -1110,6 +1167,25 @@ extern "C" int jzt_search_sorted_z(jzt_stream_t stream, const void* posz_have, c
   return check_launch("SearchSortedZ");
 }
 
+extern "C" int jzt_unsort_rows(jzt_stream_t stream, const void* rows, const void* id, int64_t n, int width,
+                               int elem_bytes, void* out) {
+  if (n < 0 || width < 0) return fail("jzt_unsort_rows: negative size");
+  if (n == 0 || width == 0) return 0;
+  const int64_t blocks = div_up(n * width, 256);
+  if (blocks > INT32_MAX) return fail("jzt_unsort_rows: too many elements");
+  const dim3 g((unsigned)blocks), b(256);
+  hipStream_t s = (hipStream_t)stream;
+  if (elem_bytes == 4)
+    hipLaunchKernelGGL((k_unsort_rows<uint32_t, int32_t>), g, b, 0, s, (const uint32_t*)rows, (const int32_t*)id, n,
+                       width, (uint32_t*)out);
+  else if (elem_bytes == 8)
+    hipLaunchKernelGGL((k_unsort_rows<uint64_t, int64_t>), g, b, 0, s, (const uint64_t*)rows, (const int64_t*)id, n,
+                       width, (uint64_t*)out);
+  else
+    return fail("jzt_unsort_rows: elements of 4 or 8 bytes");
+  return check_launch("UnsortRows");
+}
+
 extern "C" size_t jzt_fof_order_tmp_bytes(int64_t n) { return order_layout(n).total; }
 
 extern "C" int jzt_fof_order(jzt_stream_t stream, const int32_t* igroup, const int32_t* npart, int64_t n,
@@ -1168,6 +1244,18 @@ namespace jzt {
 namespace {
 constexpr size_t kNoAllocScratchBytes = 64ull << 20;
 constexpr int kMaxDevices = 64;
+// The sizes this entry takes are part of its interface (1,427,456 points for float 3-D): those whose pairs,
+// position copy, look-back state for 2048-point tiles and a compaction of runs fit into the array, though
+// the sort needs less now.
+size_t noalloc_limit_bytes(int64_t n, int dim, int dtype) {
+  size_t o = 0;
+  for (const size_t words : {2 * (size_t)n, (size_t)n, 2 * (size_t)n, (size_t)n,
+                             kRadix * kPasses + 16 + (size_t)kPasses * div_up(n, 2048) * kRadix,
+                             (size_t)n * dim * (dtype == JZT_F64 ? 2 : 1), (size_t)(n + 3) / 4,
+                             (size_t)(div_up(n, 2048) + 1 + n), (size_t)n / 2 + 1, (size_t)1})
+    o = align256(o + 4 * words);
+  return o;
+}
 }  // namespace
 }  // namespace jzt
 
@@ -1206,8 +1294,8 @@ extern "C" int jzt_pos_zorder_sort_noalloc(jzt_stream_t stream, const void* pos_
     return fail("jzt_pos_zorder_sort_noalloc: unsupported dim/dtype (dim " + std::to_string(dim) + ")");
   if (n >= (int64_t)kCountMask) return fail("jzt_pos_zorder_sort_noalloc: n must be < 2^30");
   const size_t need = sort_layout(n, dim, dtype).total;
-  if (need > kNoAllocScratchBytes)
-    return fail("jzt_pos_zorder_sort_noalloc: " + std::to_string(n) + " points need " + std::to_string(need) +
+  if (noalloc_limit_bytes(n, dim, dtype) > kNoAllocScratchBytes || need > kNoAllocScratchBytes)
+    return fail("jzt_pos_zorder_sort_noalloc: " + std::to_string(n) + " points need " + std::to_string(std::max(need, noalloc_limit_bytes(n, dim, dtype))) +
                 " bytes of scratch, more than the fixed " + std::to_string(kNoAllocScratchBytes) +
                 " bytes (use jzt_pos_zorder_sort with a caller workspace)");
   void* tmp = scratch_for_current_device();

@@ -67,6 +67,35 @@ def _zsort_impl(x: torch.Tensor, block_size: int = 64):
     return pos, ids
 
 
+class _Unsort(torch.autograd.Function):
+    """Rows (n, width) of the sorted order back to input order: out[idz] = rows.  Linear in rows; its
+    gradient is the gather by idz, so gradients of any order work."""
+
+    @staticmethod
+    def forward(ctx, rows, idz):
+        ctx.save_for_backward(idz)
+        n, width = rows.shape
+        rows = rows.contiguous()
+        out = torch.empty_like(rows)
+        L.call("jzt_unsort_rows", L.stream(), L.ptr(rows), L.ptr(idz.contiguous()), n, width, rows.element_size(),
+               L.ptr(out))
+        return out
+
+    @staticmethod
+    def backward(ctx, g):
+        (idz,) = ctx.saved_tensors
+        return g[idz.long()], None
+
+
+def _has_storage(t: torch.Tensor) -> bool:
+    """False for the tensors that batching and tracing put in a tensor's place."""
+    try:
+        t.data_ptr()
+    except RuntimeError:
+        return False
+    return True
+
+
 class _ZSort(torch.autograd.Function):
     """Custom VJP of tree.py:111-138: gradients scatter back through the inverse permutation."""
 
@@ -80,6 +109,8 @@ class _ZSort(torch.autograd.Function):
     @staticmethod
     def backward(ctx, gpos, gidz):
         (idz,) = ctx.saved_tensors
+        if _has_storage(gpos):
+            return _Unsort.apply(gpos, idz)
         idinv = torch.zeros_like(idz)
         idinv[idz.long()] = torch.arange(len(idz), dtype=idz.dtype, device=idz.device)
         return gpos[idinv.long()]

@@ -107,3 +107,53 @@ def test_zsort_tile_sizes(dev, oracle, kpt):
     p0, i0 = jz.tree.zsort(t)
     assert torch.equal(iz, i0) and torch.equal(pz, p0)
     assert np.array_equal(iz.cpu().numpy().astype(np.int64), oracle.zsort(x)[1])
+
+
+# one tile of each shape and its neighbours (2048, 4096, 8192, 12288 keys), the changes of shape
+# (2^18, 2^21, 2^23) and more tiles than one look-back step reads
+@pytest.mark.parametrize("n", [1, 2, 16, 17, 2047, 2048, 2049, 18433, (1 << 18) - 1, (1 << 18) + 1, (1 << 21) + 3,
+                               (1 << 23) + 5])
+def test_zsort_tiles(dev, oracle, n):
+    x = clustered(n, nhalos=64, seed=n) if n > 4096 else uniform(n, seed=n)
+    pz, idz = _gpu_zsort(x, dev)
+    opz, oidz = oracle.zsort(x)
+    assert np.array_equal(idz, oidz) and np.array_equal(pz, opz)
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+def test_zsort_equal_key_runs(dev, oracle, dtype):
+    """Runs of equal keys around the length that one thread per row orders (16): copies of a point, and
+    points that differ below the key's resolution."""
+    rng = np.random.default_rng(5)
+    parts = [rng.random((3000, 3)).astype(dtype), np.array([[1e6, 1., 1.]], dtype)]
+    for length in (2, 3, 15, 16, 17, 18, 33, 34, 300):
+        for _ in range(3):
+            c = rng.random(3)
+            parts.append(np.repeat(c[None], length, 0).astype(dtype))
+            parts.append((c + 1e-3 * rng.random((length, 3))).astype(dtype))
+    x = np.concatenate(parts)
+    x = np.ascontiguousarray(x[rng.permutation(len(x))])
+    pz, idz = _gpu_zsort(x, dev)
+    opz, oidz = oracle.zsort(x)
+    assert np.array_equal(idz, oidz) and np.array_equal(pz, opz)
+
+
+@pytest.mark.parametrize("dtype,dim", [(torch.float32, 3), (torch.float64, 2)])
+def test_zsort_gradient(dev, dtype, dim):
+    """The gradient is the given one in input order; also of a strided one, of second order and batched."""
+    import jztree_amd as jz
+    g = torch.Generator(device=dev).manual_seed(1)
+    x = torch.rand((1001, dim), dtype=dtype, device=dev, generator=g).requires_grad_()
+    posz, idz = jz.tree.zsort(x)
+    w = torch.randn((dim, 1001), dtype=dtype, device=dev, generator=g).T  # not contiguous
+    ref = torch.empty_like(x)
+    ref[idz.long()] = w
+    (gx,) = torch.autograd.grad(posz, x, w, retain_graph=True)
+    assert torch.equal(gx, ref)
+    wr = w.clone().requires_grad_()
+    (gx,) = torch.autograd.grad(posz, x, wr, create_graph=True)
+    (gw,) = torch.autograd.grad(gx, wr, x.detach())
+    assert torch.equal(gw, x.detach()[idz.long()])
+    wb = torch.stack([w, 2 * w, -w])
+    (gb,) = torch.autograd.grad(posz, x, wb, is_grads_batched=True)
+    assert torch.equal(gb, torch.stack([ref, 2 * ref, -ref]))
