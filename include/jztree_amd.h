@@ -325,6 +325,19 @@ int jzt_knn_leaf2leaf_ex(jzt_stream_t stream, const int32_t* ilist_spl, const in
                          size_t tmp_bytes, int64_t size_leaves_query, int64_t size_part_query, int64_t out_rows,
                          int k, float boxsize, int dim, int dtype);
 
+/* jzt_knn_leaf2leaf_ex with the bounding boxes of the source leaves (or null), which let it drop list
+ * entries that no query can reach; the results are the same.  leaf_boxes: 8 floats a leaf (lo, -, hi, -),
+ * 16-byte aligned, written by jzt_leaf_boxes for float32 positions in 2-3 dims (leaves without
+ * particles are left alone); other positions take no boxes and ignore them. */
+int jzt_knn_leaf2leaf_boxes(jzt_stream_t stream, const int32_t* ilist_spl, const int32_t* ilist_isrc,
+                         const float* ilist_r2, int64_t ilist_size, const int32_t* splT, const void* xT,
+                         const int32_t* splQ, const void* xQ, const int32_t* src_ids, const int32_t* dst_rows,
+                         const float* init_r2, int32_t* retry, void* knn_rad, int32_t* knn_id, void* tmp,
+                         size_t tmp_bytes, int64_t size_leaves_query, int64_t size_part_query, int64_t out_rows,
+                         int k, float boxsize, int dim, int dtype, const float* leaf_boxes);
+int jzt_leaf_boxes(jzt_stream_t stream, const int32_t* spl, const float* x, int64_t nleaves, int dim,
+                   float* leaf_boxes);
+
 /* KnnFused -- no single reference counterpart: replaces the leaf-plane KnnNode2Node together with
  * KnnLeaf2Leaf (knn.cuh:309-356, :602-694; callers knn.py:186 and :325) by one kernel that walks
  * the plane-1 lists (parent_ilist_*, r2-sorted, as produced by jzt_knn_node2node for plane 1) and

@@ -75,6 +75,9 @@ _SIGNATURES = {
                            _i32, _i32], _i32),
     "jzt_knn_leaf2leaf_ex": ([_p, _p, _p, _p, _i64, _p, _p, _p, _p, _p, _p, _p, _p, _p, _p, _p, _sz, _i64, _i64,
                               _i64, _i32, _f32, _i32, _i32], _i32),
+    "jzt_knn_leaf2leaf_boxes": ([_p, _p, _p, _p, _i64, _p, _p, _p, _p, _p, _p, _p, _p, _p, _p, _p, _sz, _i64, _i64,
+                              _i64, _i32, _f32, _i32, _i32, _p], _i32),
+    "jzt_leaf_boxes": ([_p, _p, _p, _i64, _i32, _p], _i32),
     "jzt_knn_fused": ([_p, _p, _p, _p, _i64, _p, _p, _p, _p, _p, _p, _p, _p, _p, _p, _p, _i64, _i64, _i32, _f32,
                        _i32, _i32], _i32),
     "jzt_knn_fused_retry": ([_p, _p, _p, _p, _i64, _p, _p, _p, _p, _p, _p, _p, _p, _p, _p, _p, _i64, _i64, _i32,

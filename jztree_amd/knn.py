@@ -48,8 +48,18 @@ class PosLvlNum:
         return torch.cat([self.pos, lvl_t[:, None]], dim=-1).contiguous()
 
 
+def _leaf_boxes(spl, x):
+    """Bounding boxes of the leaves' particles for the float32 leaf kernel (None where it does not run)."""
+    if x.dtype != torch.float32 or x.shape[-1] > 3:
+        return None
+    boxes = torch.empty((len(spl) - 1, 8), dtype=torch.float32, device=x.device)
+    L.call("jzt_leaf_boxes", L.stream(), L.ptr(spl), L.ptr(x.contiguous()), len(spl) - 1, x.shape[-1], L.ptr(boxes))
+    return boxes
+
+
 def _knn_leaf2leaf(ilist: InteractionList, splT, xT, splQ=None, xQ=None, k=32, boxsize=0., src_ids=None,
-                   dst_rows=None, out_rows: int | None = None, init_r2=None, out=None, balance: bool = True):
+                   dst_rows=None, out_rows: int | None = None, init_r2=None, out=None, balance: bool = True,
+                   boxes=None):
     """knn.py:28-60 -> KnnLeaf2Leaf.  Returns (rnn (rows,k), inn (rows,k) int32), plus the retry
     flags (nq int32) when init_r2 is given.
 
@@ -60,7 +70,8 @@ def _knn_leaf2leaf(ilist: InteractionList, splT, xT, splQ=None, xQ=None, k=32, b
     negative bound are skipped.  out = (rnn, inn[, retry]) writes into existing buffers.
     balance: hand the query leaves to the waves through the kernel's work queue (one atomic per
     leaf); False keeps the fixed order, for passes in which most leaves are skipped (negative
-    bounds), where the per-leaf atomics would cost more than the pass itself."""
+    bounds), where the per-leaf atomics would cost more than the pass itself.  boxes: the source
+    leaves' bounding boxes (_leaf_boxes), if the caller has them already."""
     if xQ is None:
         xQ = xT
     if splQ is None:
@@ -91,10 +102,13 @@ def _knn_leaf2leaf(ilist: InteractionList, splT, xT, splQ=None, xQ=None, k=32, b
     if init_r2 is not None and retry is None:
         retry = torch.empty(nq, dtype=torch.int32, device=dev)
     assert retry is None or (retry.shape == (nq,) and retry.dtype == torch.int32)
-    L.call("jzt_knn_leaf2leaf_ex", L.stream(), L.ptr(ilist.ispl), L.ptr(ilist.isrc), L.ptr(ilist.rad2),
-           ilist.size(), L.ptr(splT), L.ptr(xT.contiguous()), L.ptr(splQ), L.ptr(xQ.contiguous()), L.ptr(sid),
+    xT = xT.contiguous()
+    if boxes is None:
+        boxes = _leaf_boxes(splT, xT)
+    L.call("jzt_knn_leaf2leaf_boxes", L.stream(), L.ptr(ilist.ispl), L.ptr(ilist.isrc), L.ptr(ilist.rad2),
+           ilist.size(), L.ptr(splT), L.ptr(xT), L.ptr(splQ), L.ptr(xQ.contiguous()), L.ptr(sid),
            L.ptr(drow), L.ptr(ir2), L.ptr(retry), L.ptr(rnn), L.ptr(inn), L.ptr(tmp), nb, len(splQ) - 1, nq, rows,
-           int(k), float(boxsize or 0.), xT.shape[-1], dt)
+           int(k), float(boxsize or 0.), xT.shape[-1], dt, L.ptr(boxes))
     if init_r2 is not None:
         return rnn, inn, retry
     return rnn, inn
@@ -413,8 +427,9 @@ def _knn_leaf_start_bound(ilist: InteractionList, spl, posz, k: int, boxsize, le
     nq = len(xQ)
     size = len(splQ) - 1
     init = leaf_r2.to(torch.float32).contiguous() * (1.0 + 2.0 ** -10)  # a float32 factor: rounded once
+    boxes = _leaf_boxes(spl, posz)
     rnn, inn, retry = _knn_leaf2leaf(ilist, spl, posz, k=k, boxsize=boxsize, splQ=splQ, xQ=xQ, src_ids=src_ids,
-                                     dst_rows=dst_rows, init_r2=init)
+                                     dst_rows=dst_rows, init_r2=init, boxes=boxes)
     # eagerly the redo runs only when a query came up short (read back with the recorded conditions); under graph capture
     # it always runs, and every leaf without a short query skips it (negative radius)
     if checks.is_deferred() or checks.flush_with(retry.any()):
@@ -425,7 +440,7 @@ def _knn_leaf_start_bound(ilist: InteractionList, spl, posz, k: int, boxsize, le
                L.ptr(short), size, 0.0)
         redo = torch.where(short > 0, torch.full_like(init, float("inf")), torch.full_like(init, -1.0))
         _knn_leaf2leaf(ilist, spl, posz, k=k, boxsize=boxsize, splQ=splQ, xQ=xQ, src_ids=src_ids,
-                       dst_rows=dst_rows, init_r2=redo.contiguous(), out=(rnn, inn, retry), balance=False)
+                       dst_rows=dst_rows, init_r2=redo.contiguous(), out=(rnn, inn, retry), balance=False, boxes=boxes)
     return rnn, inn
 
 

@@ -301,3 +301,20 @@ def test_guaranteed_leaf_r2_matches_ancestor_walk(dev, n, leaf, k):
     got = _guaranteed_leaf_r2(th, k)
     nl = int(th.num(0))
     assert torch.equal(got[:nl], ref[:nl])
+
+
+@pytest.mark.parametrize("k,boxsize,dim", [(8, 1.0, 3), (64, 1.0, 3), (40, 0.0, 3), (12, 1.0, 2), (70, 1.0, 3)])
+def test_void_next_to_halo(dev, oracle, k, boxsize, dim):
+    """Dense clumps on the box faces and in its corner, in a thin background: background leaves list whole
+    clumps of which most or all particles are out of every query's reach, with and without the wrap."""
+    import jztree_amd as jz
+    rng = np.random.default_rng(11)
+    cent = np.array([[0.0, 0.0, 0.0], [0.5, 0.999, 0.3], [0.25, 0.5, 0.5], [0.9995, 0.5, 0.7]])[:, :dim]
+    x = np.concatenate([np.mod(c + 1e-3 * rng.standard_normal((2500, dim)), 1.0) for c in cent] + [rng.random((1500, dim))])
+    x = np.minimum(x.astype(np.float32), np.float32(1) - np.float32(2.0 ** -24))
+    x = np.ascontiguousarray(x[rng.permutation(len(x))])
+    cfg = jz.config.KNNConfig(alloc_fac_ilist=512.)
+    rnn, inn = jz.knn.knn(torch.from_numpy(x).to(dev), k, boxsize=boxsize or None, cfg=cfg)
+    r2o, io = oracle.knn(x, k, boxsize=boxsize)
+    assert np.array_equal(inn.cpu().numpy().astype(np.int64), io)
+    assert np.array_equal(rnn.cpu().numpy(), np.sqrt(r2o))
