@@ -313,7 +313,8 @@ def test_void_next_to_halo(dev, oracle, k, boxsize, dim):
     x = np.concatenate([np.mod(c + 1e-3 * rng.standard_normal((2500, dim)), 1.0) for c in cent] + [rng.random((1500, dim))])
     x = np.minimum(x.astype(np.float32), np.float32(1) - np.float32(2.0 ** -24))
     x = np.ascontiguousarray(x[rng.permutation(len(x))])
-    cfg = jz.config.KNNConfig(alloc_fac_ilist=512.)
+    cfg = jz.config.KNNConfig(alloc_fac_ilist=1024.)
+    cfg = dataclasses.replace(cfg, tree=dataclasses.replace(cfg.tree, alloc_fac_nodes=4.))
     rnn, inn = jz.knn.knn(torch.from_numpy(x).to(dev), k, boxsize=boxsize or None, cfg=cfg)
     r2o, io = oracle.knn(x, k, boxsize=boxsize)
     assert np.array_equal(inn.cpu().numpy().astype(np.int64), io)
