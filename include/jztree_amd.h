@@ -46,7 +46,8 @@ int jzt_abi_version(void);
 /* Tuning knobs (no counterpart in the reference, which has no autotuner): process-wide settings
  * read at each launch; results never depend on them.  Set them between calls, not while another
  * host thread launches.
- *   JZT_TUNE_LEAF_WAVES  waves per EU the leaf kNN kernel is compiled for when k <= 32 (1, 2, 4;
+ *   JZT_TUNE_LEAF_WAVES  waves per EU the leaf kNN kernel is compiled for when k <= 32 (1, 2, 4,
+ *                        which means 3 above k = 16;
  *                        default 4): the register budget per lane against occupancy
  *   JZT_TUNE_SORT_KPT    keys per thread of the onesweep radix passes (8, 12, 16; default 12, which
  *                        means 8 below 2^23 keys): tile = threads * kpt keys

@@ -214,14 +214,10 @@ template <int D, typename T> struct alignas(sizeof(T) == 4 ? 16 : 8) FofRec {
 };
 
 template <typename T> __device__ __forceinline__ T wave_min_t(T v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v = min(v, __shfl_xor(v, o, 64));
-  return v;
+  return wave_reduce(v, [](T a, T b) { return min(a, b); });
 }
 template <typename T> __device__ __forceinline__ T wave_max_t(T v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v = max(v, __shfl_xor(v, o, 64));
-  return v;
+  return wave_reduce(v, [](T a, T b) { return max(a, b); });
 }
 
 // Particle links inside each 64-particle chunk of a leaf, resolved before the leaf pairs (the

@@ -555,9 +555,6 @@ struct GlobalKV {
 // the lane strides go through DPP and, from 16 on, permlane swaps, so nothing waits for LDS
 // (exchanged with ds_bpermute, entry i*64 + lane, the sort was bound by LDS: 2.0 ms for the
 // 548,000 lists of 257 entries of 2^24 clustered points at leaf 48, 0.97 now).
-template <int CTRL> __device__ __forceinline__ uint32_t dpp(uint32_t x) {
-  return (uint32_t)__builtin_amdgcn_mov_dpp((int)x, CTRL, 0xf, 0xf, true);
-}
 // lane l's value of lane l ^ M, for M = 1, 2, 4, 8, 16, 32 (strides) and 3, 7, 15, 31, 63 (mirrors)
 template <int M> __device__ __forceinline__ uint32_t lane_xor(uint32_t x) {
   if constexpr (M == 1) return dpp<0xB1>(x);         // quad_perm 1,0,3,2
@@ -807,7 +804,13 @@ __device__ __forceinline__ float box_gap2(const Vec<D, float>& qlo, const Vec<D,
 // 224,000 particles for one wave of 10^6 clustered points at k = 64 (now 2,122; 1,903 -> 866 on
 // average), and that wave set the time of the launch.
 //
-// Query leaves come from a per-XCD item queue (xcd_queue) when the caller's tmp holds its eight
+// Two lanes per query while 32 queries or fewer are left of the leaf (half of the leaves at the default
+// size of 48: a leaf holds 30 points on average): each half of the wave takes every other source into
+// a list of its own, both accept up to what bounds the k nearest of the union, and the lists are merged
+// at the end.  Half of the lanes idled before, and the work for a source is the same for any number of
+// active lanes.
+//
+// Query leaves come from a per-XCD item queue (ItemWalk) when the caller's tmp holds its eight
 // counters (jzt_knn_leaf2leaf_tmp_bytes includes them), else in the fixed xcd_items order: the
 // leaves' costs vary widely, and with a fixed stride the last waves of the launch ran long after
 // the others had finished (plain kNN at 2^26: 92.4 -> 87.8 ms with the queue).
@@ -830,15 +833,13 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(W))) void k_
                                                  int64_t il_size, int64_t out_rows, int64_t nitems, int xcd,
                                                  uint32_t* __restrict__ queue, const LeafBox* __restrict__ boxes) {
   __shared__ SrcRec s_rec[64];
-  __shared__ uint64_t s_buf[kBufWords];
+  __shared__ uint64_t s_buf[64 * kBufStride<K>];
   const int lane = threadIdx.x;
   const int64_t nact = active_items(splQ, nitems);
-  const ItemRange items = xcd_items(nact, xcd != 0);
-  const ItemQueue iq_ = xcd_queue(nact, xcd != 0, queue);
-  const int64_t lq_end = queue ? iq_.end : items.end;
-  for (int64_t lq = queue ? queue_next(iq_) : items.first; lq < lq_end;
-       lq = queue ? queue_next(iq_) : lq + items.step) {
-    uint64_t* const row = s_buf + lane * kBufStride;
+  for (ItemWalk walk(nact, xcd != 0, queue); walk.more(); walk.advance()) {
+    const int64_t lq = walk.at;
+    walk.started();
+    uint64_t* const row = s_buf + lane * kBufStride<K>;
     const uint64_t lt_mask = (1ull << lane) - 1ull;
     const int q0 = splQ[lq], q1 = splQ[lq + 1];
     const int e0 = il_spl[lq], e1 = (int)min((int64_t)il_spl[lq + 1], il_size);
@@ -847,22 +848,35 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(W))) void k_
     const float r2_0 = init_r2 ? init_r2[lq] : 0.f;
     if (init_r2 && !(r2_0 >= 0.f)) continue;
     const uint64_t start_key = init_r2 ? (((uint64_t)__float_as_uint(r2_0) << 32) | 0xffffffffull) : kEmptyKey;
-    for (int qoff = q0; qoff < q1; qoff += 64) {
-      const int iq = min(qoff + lane, q1 - 1);
+    for (int qoff = q0, g = 1; qoff < q1; qoff += 64 / g) {
+      g = q1 - qoff <= 32 ? 2 : 1;  // lanes per query
+      const int sub = g == 2 ? lane >> 5 : 0, ql = qoff + (g == 2 ? lane & 31 : lane);
+      const int iq = min(ql, q1 - 1);
       const Vec<D, float> q = load_vec<D, float>(xQ, iq);
+      const int64_t orow = dst_rows ? (int64_t)dst_rows[iq] : (int64_t)iq;
       const uint64_t floor_key = FLOOR ? resume[iq] : 0ull;
-      Vec<D, float> qlo, qhi;  // bounding box of the query chunk
+      Vec<D, float> qlo, qhi;  // bounding box of the query chunk, in scalar registers
   #pragma unroll
       for (int d = 0; d < D; d++) {
-        qlo[d] = wave_minf(q[d]);
-        qhi[d] = wave_maxf(q[d]);
+        qlo[d] = rdlane(wave_minf(q[d]), 0);
+        qhi[d] = rdlane(wave_maxf(q[d]), 0);
       }
       uint64_t best[K];
   #pragma unroll
       for (int i = 0; i < K; i++) best[i] = start_key;
       int cnt = 0;  // entries in this lane's buffer row
-      // largest k-th distance of the wave (slack included); best[] changes only on flushes
-      float kmax = wave_maxf(key_r2(best[K - 1])) * kRmaxSlack;
+      // largest r2 that can still be among the query's k nearest; best[] changes only on flushes
+      auto bound = [&]() -> float {
+        // two lists: K of the union are within either's last, and within both their K/2-th (no branch:
+        // one here cost 27 registers)
+        const float r = key_r2(best[K - 1]), m = key_r2(best[K / 2 - 1]);
+        const float ro = __uint_as_float(other_half(__float_as_uint(r)));
+        const float mo = __uint_as_float(other_half(__float_as_uint(m)));
+        const float both = fminf(fminf(r, ro), fmaxf(m, mo));
+        return g == 2 ? both : r;
+      };
+      float kr = key_r2(start_key);
+      float kmax = wave_maxf(kr) * kRmaxSlack;  // of the wave, slack included
       float n_r2 = INFINITY;
       int n_src = 0;
       if (e0 + lane < e1) {
@@ -900,14 +914,11 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(W))) void k_
         uint64_t em = __ballot(m_in);
         const uint64_t wm = __ballot(m_wrap);
         int E = -1, t0 = 0, t1 = 0;  // the entry and the range of its particles that are left
-        // next chunk of at most 64 particles of the entries that some lane's k-th distance reaches
-        auto advance = [&]() -> bool {
-          t0 += 64;
-          while (t0 >= t1) {
-            if (!em) return false;
+        // the next entry that some lane's k-th distance reaches
+        auto next_entry = [&]() -> bool {
+          while (em) {
             E = __builtin_ctzll(em);
             em &= em - 1ull;
-            const float kr = key_r2(best[K - 1]);
             bool want = rdlane(m_r2, E) <= kr * kRmaxSlack;
             if (boxes) {
               LeafBox bx;
@@ -922,26 +933,33 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(W))) void k_
               else g2 = box_gap2<false, D>(q, q, bx, boxsize, half, w);
               want = want && g2 <= kr;
             }
-            if (!wave_any(want)) continue;
-            t0 = rdlane(m_t0, E);
-            t1 = rdlane(m_t1, E);
+            if (wave_any(want)) {
+              t0 = rdlane(m_t0, E);
+              t1 = rdlane(m_t1, E);
+              return true;
+            }
           }
-          return true;
+          return false;
         };
+        // the next chunk: up to 64 particles of as many entries as that takes, one per lane
         SrcRec cr;
-        int cn;
-        auto load_chunk = [&]() {
-          cn = min(64, t1 - t0);
-          if (lane < cn) {
-            const Vec<D, float> p = load_vec<D, float>(xT, t0 + lane);
+        auto load_chunk = [&]() -> int {
+          int n = 0, it = 0;
+          while (n < 64 && (t0 < t1 || next_entry())) {
+            if (lane >= n) it = t0 + lane - n;
+            const int c = min(64 - n, t1 - t0);
+            n += c;
+            t0 += c;
+          }
+          if (lane < n) {
+            const Vec<D, float> p = load_vec<D, float>(xT, it);
   #pragma unroll
             for (int d = 0; d < D; d++) cr.p[d] = p[d];
-            cr.id = src_ids ? (uint32_t)src_ids[t0 + lane] : (uint32_t)(t0 + lane);
+            cr.id = src_ids ? (uint32_t)src_ids[it] : (uint32_t)it;
           }
+          return n;
         };
-        bool more = advance();
-        if (more) load_chunk();
-        while (more) {
+        for (int cn = load_chunk(); cn;) {
           const int n_cur = cn;
           // Source filter: p can enter some lane's top-k only if its gap to the query box is within
           // the largest current k-th distance of the wave (or a periodic wrap is possible); the
@@ -961,19 +979,23 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(W))) void k_
           }
           const uint64_t keep = __ballot(reach);
           const bool wrap = PER && wave_any(need);
-          const int n_keep = __popcll(keep);
-          if (reach) s_rec[__popcll(keep & lt_mask)] = cr;
+          // the halves of the wave take every other source: those of odd rank from slot 32 on.  Slots
+          // past the last source hold NaN positions (a wave's LDS writes keep their order)
+          const int n_keep = (__popcll(keep) + g - 1) / g;
+          const int rank = __popcll(keep & lt_mask);
+          s_rec[lane].p[0] = __builtin_nanf("");
+          if (reach) s_rec[g == 2 ? (rank >> 1) + ((rank & 1) << 5) : rank] = cr;
           __syncthreads();
-          more = advance();
-          if (more) load_chunk();  // in flight while this chunk is consumed
-          if (consume_chunk<K, PER, FLOOR, D>(best, q, s_rec, n_keep, wrap, boxsize, half, floor_key, row, cnt))
-            kmax = wave_maxf(key_r2(best[K - 1])) * kRmaxSlack;
+          cn = load_chunk();  // in flight while this chunk is consumed
+          if (consume_chunk<K, PER, FLOOR, D>(best, q, s_rec + 32 * sub, n_keep, wrap, boxsize, half, floor_key, row,
+                                              cnt, kr, bound))
+            kmax = wave_maxf(kr) * kRmaxSlack;
           __syncthreads();
         }
       }
       if (wave_any(cnt > 0)) topk_flush<K>(best, row, cnt);
-      if (qoff + lane < q1) {
-        const int64_t orow = dst_rows ? (int64_t)dst_rows[iq] : (int64_t)iq;
+      if (g == 2) merge_halves<K>(best);
+      if (sub == 0 && ql < q1) {
         if (orow >= 0 && orow < out_rows) write_row<K>(best, rad_out, id_out, orow * ktot + koff, ktot - koff);
         // the last slot this pass reports (k need not be a power of two: slots past it may
         // keep the start key even when the query has all its neighbours)
@@ -1129,7 +1151,7 @@ int leaf2leaf_impl(hipStream_t s, const int32_t* il_spl, const int32_t* il_src, 
   // item queue counters after the resume keys, when the caller's tmp holds them
   const size_t qoff = align256(knn_leaf_nd_tmp_bytes(npart_q, k, false));
   uint32_t* queue = tmp && tmp_bytes >= qoff + 256 ? (uint32_t*)((char*)tmp + qoff) : nullptr;
-  dim3 g(grid_for8(nleaves_q)), b(64);
+  const dim3 b(64);
   const float* xt = (const float*)xT;
   const float* xq = (const float*)xQ;
   const int waves = tune_get(kTuneLeafWaves);
@@ -1137,27 +1159,30 @@ int leaf2leaf_impl(hipStream_t s, const int32_t* il_spl, const int32_t* il_src, 
   for (int koff = 0; koff < k; koff += 64) {
     const int kn = min(k - koff, 64);
     const bool floor = resume && koff > 0;
-    if (queue && fill_u32(s, queue, 0u, 8)) return 1;
+    if (queue && fill_u32(s, queue, 0u, 8 * kQueueStride)) return 1;
+    // waves that a compute unit holds: by registers for k > 8, by LDS for k <= 8
+    const dim3 g(queue ? queue_grid(nleaves_q, kn <= 8 ? 20 : kn <= 16 ? 16 : kn <= 32 ? 12 : 8) : grid_for8(nleaves_q));
 #define JZT_KNN_LAUNCH(KK, PER, FLOOR, W)                                                                              \
   hipLaunchKernelGGL((k_knn_leaf<KK, PER, FLOOR, D, W>), g, b, 0, s, il_spl, il_src, il_r2, splT, xt, splQ, xq, src_ids, \
                      dst_rows, init_r2, retry, (float*)rad, ids, resume, koff, k, boxsize, il_size, out_rows, nleaves_q, xcd, \
                      queue, boxes)
-  // waves per EU (the register budget of the kernel): tunable for K <= 32; the multi-pass tail
-  // (FLOOR) and K = 64 keep their fixed choice
-#define JZT_KNN_LAUNCH_W(KK, PER)                                                  \
-  do {                                                                             \
-    constexpr int w2 = KK > 32 ? 1 : 2, w4 = KK > 32 ? 1 : JZT_LEAF_WAVES;         \
-    if (KK > 32 || waves == 1) JZT_KNN_LAUNCH(KK, PER, false, 1);                  \
-    else if (waves == 2) JZT_KNN_LAUNCH(KK, PER, false, w2);                       \
-    else JZT_KNN_LAUNCH(KK, PER, false, w4);                                       \
+  // waves per EU (the register budget of the kernel): tunable for K <= 32.  4 spilled 29 registers at
+  // K = 32, in the flush (2^26 points, learned: 65.6 ms against 61.9 at 3); at K = 64, 2 spill 12 and
+  // hide more than 1 (1,000,003 points, k = 64: 4.5 ms against 5.1)
+#define JZT_KNN_LAUNCH_W(KK, PER)                                                            \
+  do {                                                                                       \
+    constexpr int w4 = KK > 32 ? 2 : KK > 16 ? 3 : JZT_LEAF_WAVES;                           \
+    if (KK <= 32 && waves == 1) JZT_KNN_LAUNCH(KK, PER, false, (KK > 32 ? 2 : 1));           \
+    else if (waves == 2) JZT_KNN_LAUNCH(KK, PER, false, 2);                                  \
+    else JZT_KNN_LAUNCH(KK, PER, false, w4);                                                 \
   } while (0)
 #define JZT_KNN_LAUNCH_K(KK)                                                            \
   do {                                                                                  \
     if (boxsize > 0.f) {                                                                \
-      if (floor) JZT_KNN_LAUNCH(KK, true, true, (KK > 32 ? 1 : JZT_LEAF_WAVES));        \
+      if (floor) JZT_KNN_LAUNCH(KK, true, true, (KK > 32 ? 1 : KK > 16 ? 3 : JZT_LEAF_WAVES));  \
       else JZT_KNN_LAUNCH_W(KK, true);                                                  \
     } else {                                                                            \
-      if (floor) JZT_KNN_LAUNCH(KK, false, true, (KK > 32 ? 1 : JZT_LEAF_WAVES));       \
+      if (floor) JZT_KNN_LAUNCH(KK, false, true, (KK > 32 ? 1 : KK > 16 ? 3 : JZT_LEAF_WAVES)); \
       else JZT_KNN_LAUNCH_W(KK, false);                                                 \
     }                                                                                   \
   } while (0)

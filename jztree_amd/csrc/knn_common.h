@@ -46,14 +46,10 @@ __device__ __forceinline__ float rdlane(float v, int i) {
   return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), i));
 }
 __device__ __forceinline__ float wave_minf(float v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v = fminf(v, __shfl_xor(v, o, 64));
-  return v;
+  return wave_reduce(v, [](float a, float b) { return fminf(a, b); });
 }
 __device__ __forceinline__ float wave_maxf(float v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o, 64));
-  return v;
+  return wave_reduce(v, [](float a, float b) { return fmaxf(a, b); });
 }
 
 // One source particle as staged in LDS: position and reported id in one 16-byte record.
@@ -75,8 +71,7 @@ struct alignas(16) SrcRec {
 #define JZT_TOPK_BUF 16
 #endif
 template <int K> constexpr int kBufCap = K < JZT_TOPK_BUF ? K : JZT_TOPK_BUF;
-constexpr int kBufStride = 17;
-constexpr int kBufWords = 64 * kBufStride;  // u64 per wave
+template <int K> constexpr int kBufStride = kBufCap<K> | 1;
 
 // Keys compared as doubles: the high word of a key is the bit pattern of a non-negative float r2
 // (at most +inf, 0x7f800000), so read as an IEEE double every key is non-negative, never NaN or
@@ -112,6 +107,42 @@ __device__ __forceinline__ void oddeven_sort_regs(uint64_t (&v)[N]) {
   }
 }
 
+// ascending order of a bitonic register array
+template <int K>
+__device__ __forceinline__ void bitonic_merge_regs(uint64_t (&v)[K]) {
+#pragma unroll
+  for (int stride = K / 2; stride > 0; stride >>= 1) {
+#pragma unroll
+    for (int i = 0; i < K; i++) {
+      const int j = i ^ stride;
+      if (j > i) ce_asc(v[i], v[j]);
+    }
+  }
+}
+
+// the value of the lane 32 away
+__device__ __forceinline__ uint32_t other_half(uint32_t x) {
+  const auto r = __builtin_amdgcn_permlane32_swap(x, x, false, false);
+  return (__lane_id() & 32) ? r[0] : r[1];
+}
+__device__ __forceinline__ uint64_t other_half(uint64_t x) {
+  return ((uint64_t)other_half((uint32_t)(x >> 32)) << 32) | other_half((uint32_t)x);
+}
+
+// Two ascending lists of the same query, in lanes 32 apart: both lanes get the K smallest of the union.
+template <int K>
+__device__ __forceinline__ void merge_halves(uint64_t (&best)[K]) {
+#pragma unroll
+  for (int i = 0; i < K / 2; i++) {
+    const uint64_t a = best[i], b = best[K - 1 - i], pa = other_half(a), pb = other_half(b);
+    best[i] = f64_as_key(__builtin_fmin(key_as_f64(a), key_as_f64(pb)));
+    best[K - 1 - i] = f64_as_key(__builtin_fmin(key_as_f64(b), key_as_f64(pa)));
+    // a pair at a time: all exchanges at once would need another K registers
+    if (i & 1) __builtin_amdgcn_sched_barrier(0);
+  }
+  bitonic_merge_regs<K>(best);
+}
+
 // Merge the lane's buffered keys row[0..cnt) into the ascending best[0..K): best becomes the K
 // smallest of the union, ascending.  cnt is reset.  The row is read whole (slots past cnt hold
 // stale keys, replaced by empty ones), so the reads need no per-slot branch.
@@ -130,21 +161,16 @@ __device__ __forceinline__ void topk_flush(uint64_t (&best)[K], const uint64_t* 
   for (int i = 0; i < M; i++) {
     best[K - M + i] = f64_as_key(__builtin_fmin(key_as_f64(best[K - M + i]), key_as_f64(b[M - 1 - i])));
   }
-  // bitonic merge to ascending order
-#pragma unroll
-  for (int stride = K / 2; stride > 0; stride >>= 1) {
-#pragma unroll
-    for (int i = 0; i < K; i++) {
-      const int j = i ^ stride;
-      if (j > i) ce_asc(best[i], best[j]);
-    }
-  }
+  bitonic_merge_regs<K>(best);
 }
 
 // Stream n staged source particles into the lane's buffer (and the top-k on flushes).  `wrap`
 // (wave-uniform) applies the periodic wrap; the caller clears it only when no difference of the
-// chunk needs it.  row = this lane's buffer row, cnt = its fill (at most kBufCap on entry and on
-// return).  Sources go JZT_CONSUME_UNROLL at a time: their LDS reads are issued together and the
+// chunk needs it.  recs = the lane's first source (the same for all lanes, or one for each half of the
+// wave); the sources that fill n up to a multiple of JZT_CONSUME_UNROLL have NaN positions, which
+// nothing accepts.  row = this lane's buffer row, cnt = its fill (at most kBufCap on entry and on
+// return), kr = the largest r2 it still accepts, which bound() gives anew after a flush.  Sources
+// go JZT_CONSUME_UNROLL at a time: their LDS reads are issued together and the
 // wave flushes before a group whenever some lane has less room than a whole group.  Returns
 // whether best[] changed (a flush happened).
 //
@@ -156,25 +182,25 @@ __device__ __forceinline__ void topk_flush(uint64_t (&best)[K], const uint64_t* 
 #ifndef JZT_CONSUME_UNROLL
 #define JZT_CONSUME_UNROLL 4
 #endif
-template <int K, bool PER, bool FLOOR, int D>
-__device__ __forceinline__ bool consume_chunk(uint64_t (&best)[K], const Vec<D, float>& q, const SrcRec* s_rec,
+template <int K, bool PER, bool FLOOR, int D, typename Bound>
+__device__ __forceinline__ bool consume_chunk(uint64_t (&best)[K], const Vec<D, float>& q, const SrcRec* recs,
                                               int n, bool wrap, float boxsize, float half, uint64_t floor_key,
-                                              uint64_t* row, int& cnt) {
+                                              uint64_t* row, int& cnt, float& kr, Bound bound) {
   constexpr int U = JZT_CONSUME_UNROLL;
   constexpr int CAP = kBufCap<K>;
   static_assert(U >= 1 && U <= CAP, "unroll must fit a buffer row");
   bool flushed = false;
-  float kr = key_r2(best[K - 1]);
   uint32_t* const row32 = reinterpret_cast<uint32_t*>(row);
+#pragma unroll 1
   for (int j = 0; j < n; j += U) {  // one flush site: the network is inlined once
     if (wave_any(cnt > CAP - U)) {
       topk_flush<K>(best, row, cnt);
       flushed = true;
-      kr = key_r2(best[K - 1]);
+      kr = bound();
     }
     SrcRec c[U];
 #pragma unroll
-    for (int u = 0; u < U; u++) c[u] = s_rec[j + u < n ? j + u : j];
+    for (int u = 0; u < U; u++) c[u] = recs[j + u];
     float r2[U];
 #pragma unroll
     for (int u = 0; u < U; u++) {
@@ -186,7 +212,7 @@ __device__ __forceinline__ bool consume_chunk(uint64_t (&best)[K], const Vec<D, 
     }
 #pragma unroll
     for (int u = 0; u < U; u++) {
-      bool acc = j + u < n && r2[u] <= kr;
+      bool acc = r2[u] <= kr;
       if (FLOOR) acc = acc && (((uint64_t)__float_as_uint(r2[u]) << 32) | c[u].id) > floor_key;
       row32[2 * cnt] = c[u].id;
       row32[2 * cnt + 1] = __float_as_uint(r2[u]);

@@ -123,10 +123,13 @@ __device__ __forceinline__ void consume_list(uint64_t (&best)[K], const Vec<D, f
         noff = 0;
       }
     }
-    if (lane < n_cur) s_rec[lane] = cr;
+    if (lane >= n_cur) cr.p[0] = __builtin_nanf("");  // fills the chunk's last group of sources
+    s_rec[lane] = cr;
     __syncthreads();
     if (ne < n) load(ne, noff);
-    consume_chunk<K, PER, false, D>(best, q, s_rec, n_cur, w_cur, boxsize, half, 0ull, row, cnt);
+    float kr = key_r2(best[K - 1]);
+    consume_chunk<K, PER, false, D>(best, q, s_rec, n_cur, w_cur, boxsize, half, 0ull, row, cnt, kr,
+                                    [&] { return key_r2(best[K - 1]); });
     __syncthreads();
     e = ne;
     off = noff;
@@ -143,8 +146,8 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(K <= 32 ? 4 
     int32_t* __restrict__ id_out, int ktot, T boxsize, int64_t nitems, int64_t npart) {
   __shared__ SrcRec s_rec[64];
   __shared__ uint64_t s_list[kListCap];
-  __shared__ uint64_t s_buf[kBufWords];
-  uint64_t* const row = s_buf + threadIdx.x * kBufStride;
+  __shared__ uint64_t s_buf[64 * kBufStride<K>];
+  uint64_t* const row = s_buf + threadIdx.x * kBufStride<K>;
   const int lane = threadIdx.x;
   const int64_t nact_ = active_items(l2p, nitems);
   const T half = (T)(float)(T(0.5) * boxsize);

@@ -12,7 +12,7 @@
 // all lanes from LDS.  Exactness of the filter: by monotone rounding, every canonical r2 from the
 // box is >= the gap^2 computed with the same FMA chain.
 //
-// Query leaves are taken from a per-XCD item queue (xcd_queue) when the caller's tmp holds its
+// Query leaves are taken from a per-XCD item queue (ItemWalk) when the caller's tmp holds its
 // counters, else in the fixed xcd_items order.
 //
 // k above the per-pass slot count KMAX (64 for float, 32 for double) runs ceil(k / KMAX) passes;
@@ -26,20 +26,10 @@
 namespace jzt {
 
 template <typename T> __device__ __forceinline__ T wave_min_t(T v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) {
-    const T w = __shfl_xor(v, o, 64);
-    v = w < v ? w : v;
-  }
-  return v;
+  return wave_reduce(v, [](T a, T b) { return b < a ? b : a; });
 }
 template <typename T> __device__ __forceinline__ T wave_max_t(T v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) {
-    const T w = __shfl_xor(v, o, 64);
-    v = w > v ? w : v;
-  }
-  return v;
+  return wave_reduce(v, [](T a, T b) { return b > a ? b : a; });
 }
 
 // (r2a, ia) < (r2b, ib) in the (r2, id) order; false whenever r2a is NaN
@@ -88,11 +78,9 @@ __global__ __launch_bounds__(64) void k_knn_leaf_nd(const int32_t* __restrict__ 
   const T slack = (T)(1.0f + kBoundSlack);
   const bool floor = res_r2 != nullptr && koff > 0;
   const int64_t nact = active_items(splQ, nitems);
-  const ItemRange items = xcd_items(nact, xcd != 0);
-  const ItemQueue iq_ = xcd_queue(nact, xcd != 0, queue);
-  const int64_t lq_end = queue ? iq_.end : items.end;
-  for (int64_t lq = queue ? queue_next(iq_) : items.first; lq < lq_end;
-       lq = queue ? queue_next(iq_) : lq + items.step) {
+  for (ItemWalk walk(nact, xcd != 0, queue); walk.more(); walk.advance()) {
+    const int64_t lq = walk.at;
+    walk.started();
     const int q0 = splQ[lq], q1 = splQ[lq + 1];
     const int e0 = il_spl[lq], e1 = (int)min((int64_t)il_spl[lq + 1], il_size);
     // a negative (or NaN) start bound marks a leaf that this launch leaves untouched
@@ -236,11 +224,11 @@ int knn_leaf_nd_impl(hipStream_t s, const int32_t* il_spl, const int32_t* il_src
   // item-queue counters after the resume pairs, when the caller's tmp holds them
   const size_t qoff = align256(knn_leaf_nd_tmp_bytes(npart_q, k, sizeof(T) == 8));
   uint32_t* queue = tmp && tmp_bytes >= qoff + 256 ? (uint32_t*)((char*)tmp + qoff) : nullptr;
-  const dim3 g(grid_for8(nleaves_q)), b(64);
+  const dim3 g(queue ? queue_grid(nleaves_q, 32) : grid_for8(nleaves_q)), b(64);
   const int xcd = tune_get(kTuneXcd);
   for (int koff = 0; koff < k; koff += KMAX) {
     const int kn = min(k - koff, KMAX);
-    if (queue && fill_u32(s, queue, 0u, 8)) return 1;
+    if (queue && fill_u32(s, queue, 0u, 8 * kQueueStride)) return 1;
 #define JZT_ND_LAUNCH(KK, PER)                                                                                     \
   hipLaunchKernelGGL((k_knn_leaf_nd<KK, PER, D, T>), g, b, 0, s, il_spl, il_src, il_r2, splT, (const T*)xT, splQ, \
                      (const T*)xQ, src_ids, dst_rows, init_r2, retry, (T*)rad, ids, res_r2, res_id, koff, k,       \

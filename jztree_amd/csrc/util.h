@@ -104,26 +104,70 @@ __device__ __forceinline__ ItemRange xcd_items(int64_t n, bool on) {
   const int64_t x = blockIdx.x & 7, per = (n + 7) >> 3;
   return {x * per + (int64_t)(blockIdx.x >> 3), n < (x + 1) * per ? n : (x + 1) * per, g >> 3};
 }
-// Dynamic form of xcd_items for one-wave blocks: the blocks of an XCD take the items of its eighth
-// one at a time from a shared counter (counters[x], zeroed before the launch), so the XCD's blocks
-// finish together however uneven the items are; the item set and the XCD-contiguous order are
-// those of xcd_items.  It pays where items are expensive and uneven (kNN query leaves: -5% kernel
-// time at 2^26); for the cheap, even FoF leaves every fetch order tried was slower than the static
-// one.  queue_next is called by all 64 lanes (wave-uniform result).
-struct ItemQueue {
-  int64_t begin, end;
+// Walk over the items of xcd_items by one-wave workgroups, in that fixed order or (counters given, zeroed
+// before the launch) dynamically: the blocks of an XCD take the items of its eighth from a shared
+// counter, so they finish together however uneven the items are; the item set and the XCD-contiguous
+// order are the same.  It pays where items are expensive and uneven (kNN query leaves); for the cheap,
+// even FoF leaves every fetch order tried was slower than the static one.
+//
+// An atomic on a counter that all waves share takes about 11 ns, one after the other on all XCDs: item by
+// item, with 50,000 waves that each make one more to find the queue empty, 32,000 leaves of k = 8 waited
+// 0.9 ms for it (1.13 ms the kernel, 0.70 now).  queue_grid therefore launches no more waves than the
+// chip holds, and where there are 16 pairs of items for each wave they are taken in pairs over the first
+// three quarters (eights cost more in L2 hits and balance than they saved: 2^26 points, learned kNN,
+// 63.7 ms against 62.6).
+constexpr int kQueueStride = 8;  // words from counter to counter
+struct ItemWalk {
+  int64_t at, end;  // the item in hand; all 64 lanes call the functions (wave-uniform results)
+  int64_t step, begin, big, stop, fresh;
   uint32_t* ctr;
+  uint32_t chunk, got, count;
+  __device__ __forceinline__ ItemWalk(int64_t n, bool on, uint32_t* counters) {
+    const ItemRange r = xcd_items(n, on);
+    at = r.first;
+    end = r.end;
+    step = r.step;
+    ctr = counters;
+    if (ctr) {
+      const int64_t g = gridDim.x;
+      const bool split = on && (g & 7) == 0;
+      const int64_t per = split ? (n + 7) >> 3 : n, waves = split ? g >> 3 : g;
+      begin = split ? (blockIdx.x & 7) * per : 0;
+      if (split) ctr += (blockIdx.x & 7) * kQueueStride;
+      big = begin + per / 4 * 3;
+      chunk = (uint32_t)min(max(per / (16 * waves), (int64_t)1), (int64_t)2);
+      take(begin);
+      next();
+    }
+  }
+  __device__ __forceinline__ bool more() const { return at < end; }
+  // to be called when the work on an item begins: the next ones are asked for meanwhile
+  __device__ __forceinline__ void started() {
+    if (ctr && at >= fresh) {
+      fresh = stop;
+      take(at);
+    }
+  }
+  __device__ __forceinline__ void advance() {
+    if (!ctr) at += step;
+    else if (++at >= stop) next();
+  }
+
+ private:
+  __device__ __forceinline__ void take(int64_t pos) {
+    count = pos < big ? chunk : 1u;
+    got = 0;
+    if (threadIdx.x == 0) got = atomicAdd(ctr, count);
+  }
+  __device__ __forceinline__ void next() {
+    at = fresh = begin + (int64_t)(uint32_t)__builtin_amdgcn_readfirstlane(got);
+    stop = at + (int64_t)count;
+  }
 };
-__device__ __forceinline__ ItemQueue xcd_queue(int64_t n, bool on, uint32_t* counters) {
-  const int64_t g = gridDim.x;
-  if (!on || (g & 7) != 0) return {0, n, counters};
-  const int64_t x = blockIdx.x & 7, per = (n + 7) >> 3;
-  return {x * per, n < (x + 1) * per ? n : (x + 1) * per, counters + x};
-}
-__device__ __forceinline__ int64_t queue_next(const ItemQueue& q) {
-  uint32_t v = 0;
-  if (threadIdx.x == 0) v = atomicAdd(q.ctr, 1u);
-  return q.begin + (int64_t)__builtin_amdgcn_readfirstlane(v);
+// grid of a kernel of one-wave workgroups that walk a queue, `per_cu` of which a compute unit holds
+inline unsigned queue_grid(int64_t n, int per_cu) {
+  const int64_t most = 256 * (int64_t)per_cu;
+  return (unsigned)(((n <= 0 ? 8 : n < most ? n : most) + 7) & ~(int64_t)7);
 }
 // grid for xcd_items: at most kMaxGrid blocks, a multiple of 8
 inline unsigned grid_for8(int64_t n) {

@@ -319,3 +319,16 @@ def test_void_next_to_halo(dev, oracle, k, boxsize, dim):
     r2o, io = oracle.knn(x, k, boxsize=boxsize)
     assert np.array_equal(inn.cpu().numpy().astype(np.int64), io)
     assert np.array_equal(rnn.cpu().numpy(), np.sqrt(r2o))
+
+
+@pytest.mark.parametrize("leaf", [16, 31, 32, 33, 48, 63, 64, 65, 96, 97, 130])
+@pytest.mark.parametrize("k,boxsize", [(1, 1.0), (8, 0.0), (33, 1.0), (70, 0.0)])
+def test_leaf_query_chunks(dev, oracle, leaf, k, boxsize):
+    """Leaf sizes around the 32 queries from which on two lanes share a query, and around whole chunks of
+    64; chunks of sources that span several leaves."""
+    import jztree_amd as jz
+    x = uniform(3001, seed=leaf)
+    cfg = jz.config.KNNConfig(alloc_fac_ilist=1024.)
+    cfg = dataclasses.replace(cfg, tree=dataclasses.replace(cfg.tree, max_leaf_size=leaf, alloc_fac_nodes=3.))
+    rnn, inn = _knn(x, k, dev, boxsize=boxsize or None, cfg=cfg)
+    _check(x, k, rnn, inn, oracle, boxsize=boxsize)
