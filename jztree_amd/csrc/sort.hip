@@ -503,17 +503,15 @@ __device__ __forceinline__ void finish_row(const T* __restrict__ pos, uint32_t v
 // wrote and read a flag per row: 120 us instead of 95 at 4.2e6 points.
 constexpr int kShortRun = 16;
 
+// low: bits of the keys that the rows are not sorted by (runs are equal in the bits above them).
 template <int D, typename T>
-__global__ __launch_bounds__(256) void k_finish(const uint64_t* __restrict__ keys, const uint32_t* __restrict__ vals,
-                                                const int32_t* __restrict__ setk, int64_t n,
-                                                const T* __restrict__ pos, T* __restrict__ pos_out,
-                                                typename IntOf<T>::type* __restrict__ id_out,
-                                                int32_t* __restrict__ runs, int32_t* nruns, int64_t max_runs) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
+__device__ __forceinline__ void finish_at(int64_t i, int low, const uint64_t* keys, const uint32_t* vals,
+                                          const int32_t* __restrict__ setk, int64_t n, const T* __restrict__ pos,
+                                          T* __restrict__ pos_out, typename IntOf<T>::type* __restrict__ id_out,
+                                          int32_t* __restrict__ runs, int32_t* nruns, int64_t max_runs) {
   const uint64_t k = keys[i];
   const int32_t sk = setk ? setk[i] : 0;
-  auto same = [&](int64_t j) { return keys[j] == k && (!setk || setk[j] == sk); };
+  auto same = [&](int64_t j) { return (keys[j] ^ k) >> low == 0 && (!setk || setk[j] == sk); };
   const uint32_t v = vals[i];
   int64_t dst = i;
   const bool prev = i > 0 && same(i - 1), next = i + 1 < n && same(i + 1);
@@ -529,9 +527,22 @@ __global__ __launch_bounds__(256) void k_finish(const uint64_t* __restrict__ key
       return;
     }
     dst = a;
-    for (int64_t j = a; j < b; j++) dst += j != i && idx_less<D, T>(pos, vals[j], v);
+    for (int64_t j = a; j < b; j++) {
+      const uint64_t kj = keys[j];
+      dst += kj < k || (kj == k && j != i && idx_less<D, T>(pos, vals[j], v));
+    }
   }
   finish_row<D, T>(pos, v, dst, n, pos_out, id_out);
+}
+
+template <int D, typename T>
+__global__ __launch_bounds__(256) void k_finish(const uint64_t* __restrict__ keys, const uint32_t* __restrict__ vals,
+                                                const int32_t* __restrict__ setk, int64_t n,
+                                                const T* __restrict__ pos, T* __restrict__ pos_out,
+                                                typename IntOf<T>::type* __restrict__ id_out,
+                                                int32_t* __restrict__ runs, int32_t* nruns, int64_t max_runs) {
+  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < n) finish_at<D, T>(i, 0, keys, vals, setk, n, pos, pos_out, id_out, runs, nruns, max_runs);
 }
 
 // One workgroup per listed run (grid-stride over the list).  The run's end is found by
@@ -605,15 +616,163 @@ __global__ __launch_bounds__(256) void k_long_runs(const uint64_t* __restrict__ 
 }
 
 template <int D, typename T>
-int finish(hipStream_t s, const uint64_t* keys, uint32_t* vals, const int32_t* setk, int64_t n, const T* pos,
-           T* pos_out, typename IntOf<T>::type* id_out, int32_t* runs, int32_t* nruns) {
+int long_runs(hipStream_t s, const uint64_t* keys, uint32_t* vals, const int32_t* setk, int64_t n, const T* pos,
+              T* pos_out, typename IntOf<T>::type* id_out, int32_t* runs, int32_t* nruns) {
   const int64_t max_runs = n / (kShortRun + 1) + 1;  // none shorter is listed
-  hipLaunchKernelGGL((k_finish<D, T>), dim3((unsigned)div_up(n, 256)), dim3(256), 0, s, keys, vals, setk, n, pos,
-                     pos_out, id_out, runs, nruns, max_runs);
   if (n > kShortRun)
     hipLaunchKernelGGL((k_long_runs<D, T>), dim3((unsigned)std::min(max_runs, (int64_t)512)), dim3(256), 0, s, keys,
                        vals, n, pos, pos_out, id_out, runs, nruns, max_runs, setk);
   return check_launch("zsort finish");
+}
+template <int D, typename T>
+int finish(hipStream_t s, const uint64_t* keys, uint32_t* vals, const int32_t* setk, int64_t n, const T* pos,
+           T* pos_out, typename IntOf<T>::type* id_out, int32_t* runs, int32_t* nruns) {
+  hipLaunchKernelGGL((k_finish<D, T>), dim3((unsigned)div_up(n, 256)), dim3(256), 0, s, keys, vals, setk, n, pos,
+                     pos_out, id_out, runs, nruns, n / (kShortRun + 1) + 1);
+  return long_runs<D, T>(s, keys, vals, setk, n, pos, pos_out, id_out, runs, nruns);
+}
+
+// ---------------------------------------------------------------------------------------------
+// 7. small arrays: the whole sort by one workgroup
+// ---------------------------------------------------------------------------------------------
+// Steps 1 to 5 for up to kSmallSort points: keys and indices in registers (a wave's are consecutive, so
+// the passes are stable), exchanged through LDS pass by pass.  Small sorts are bound by their
+// launches; one workgroup is bound by the ranking (8 ballots a key and pass).  A sort alone, us, by one
+// workgroup / over many: 1000 points 23 / 59, 4096 42 / 62, 8192 68 / 70, 16,384 120 / 80.  In a call
+// that goes on to build the tree, the 12 launches saved are worth another 50 us (FoF of 12,800 points
+// 398 -> 350), which is where the limit comes from.  Other positions than the instantiated ones take
+// the passes over many workgroups at any size.
+constexpr int kSmallThreads = 1024;
+constexpr int kSmallKeys = 16;  // a thread's
+constexpr int64_t kSmallSort = kSmallThreads * kSmallKeys;
+template <int D, typename T> constexpr bool kHasSmallSort = D <= 3 && std::is_floating_point<T>::value;
+
+template <int D, typename T>
+__global__ __launch_bounds__(kSmallThreads) void k_small_sort(const T* __restrict__ pos, int n, uint64_t* keys,
+                                                              uint32_t* vals, T* __restrict__ pos_out,
+                                                              typename IntOf<T>::type* __restrict__ id_out,
+                                                              int32_t* __restrict__ runs, int32_t* nruns) {
+  constexpr int W = kSmallThreads / 64;
+  __shared__ uint64_t s_keys[kSmallSort];
+  __shared__ uint32_t s_wcnt[W][kRadix];
+  __shared__ uint32_t s_base[kRadix];
+  __shared__ int s_scan[W];
+  __shared__ uint32_t s_emax[W];
+  const int tid = threadIdx.x, w = tid >> 6, lane = tid & 63;
+  const uint64_t lt_mask = (1ull << lane) - 1ull;
+  const int rounds = (n + kSmallThreads - 1) / kSmallThreads;  // keys per thread that are needed
+  const int first = w * 64 * rounds + lane;                    // the thread's are first + 64 * r
+  if (tid == 0) *nruns = 0;
+
+  // bounds (as k_bounds)
+  uint32_t emax = 0, neg = 0, inf = 0;
+  for (int i = tid; i < n * D; i += kSmallThreads) bounds_value<T>(pos[i], emax, neg, inf);
+  emax = wave_reduce(emax, [](uint32_t a, uint32_t b) { return max(a, b); });
+  if (lane == 0) s_emax[w] = emax;
+  const bool general = (__syncthreads_or((int)neg) | __syncthreads_or((int)inf)) != 0;
+  for (int i = 0; i < W; i++) emax = max(emax, s_emax[i]);
+  const int Lt = top_level_from_meta<T>(&emax);
+
+  uint64_t key[kSmallKeys];
+  uint32_t val[kSmallKeys], rank[kSmallKeys];
+#pragma unroll
+  for (int r = 0; r < kSmallKeys; r++) {
+    if (r < rounds) {
+      const int i = first + 64 * r;
+      key[r] = ~0ull;  // past the end: after every point, NaN rows included (equal keys, later index)
+      val[r] = (uint32_t)i;
+      if (i < n) {
+        T x[D];
+#pragma unroll
+        for (int d = 0; d < D; d++) x[d] = pos[i * D + d];
+        key[r] = morton_key<D, T>(x, Lt, general);
+      }
+    }
+  }
+
+  uint32_t* const s_vals = reinterpret_cast<uint32_t*>(s_keys);
+  auto pass = [&](int shift) {
+    for (int i = tid; i < W * kRadix; i += kSmallThreads) (&s_wcnt[0][0])[i] = 0;
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < kSmallKeys; r++) {
+      if (r < rounds) {
+        const uint32_t d = (uint32_t)(key[r] >> shift) & 255u;
+        uint64_t m = ~0ull;
+#pragma unroll
+        for (int b = 0; b < 8; b++) {
+          const bool bit = (d >> b) & 1u;
+          const uint64_t bal = __ballot(bit);
+          m &= bit ? bal : ~bal;
+        }
+        const uint32_t pre = s_wcnt[w][d], below = (uint32_t)__popcll(m & lt_mask);
+        rank[r] = pre + below;
+        if (below == 0) s_wcnt[w][d] = pre + (uint32_t)__popcll(m);
+      }
+    }
+    __syncthreads();
+    uint32_t total = 0;
+    if (tid < kRadix) {
+#pragma unroll
+      for (int i = 0; i < W; i++) {
+        const uint32_t c = s_wcnt[i][tid];
+        s_wcnt[i][tid] = total;
+        total += c;
+      }
+    }
+    int sum;
+    const int base = block_excl_scan<kSmallThreads>((int)total, s_scan, &sum);
+    if (tid < kRadix) s_base[tid] = (uint32_t)base;
+    // a digit that all keys share moves nothing
+    if (__syncthreads_or(tid < kRadix && (int)total == rounds * kSmallThreads)) return;
+#pragma unroll
+    for (int r = 0; r < kSmallKeys; r++) {
+      if (r < rounds) {
+        const uint32_t d = (uint32_t)(key[r] >> shift) & 255u;
+        rank[r] += s_base[d] + s_wcnt[w][d];
+        s_keys[rank[r]] = key[r];
+      }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < kSmallKeys; r++)
+      if (r < rounds) key[r] = s_keys[first + 64 * r];
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < kSmallKeys; r++)
+      if (r < rounds) s_vals[rank[r]] = val[r];
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < kSmallKeys; r++)
+      if (r < rounds) val[r] = s_vals[first + 64 * r];
+    __syncthreads();
+    };
+  // the passes from bit `low` on; then the rows, in global memory for their neighbours
+  auto sort_from = [&](int low) {
+#pragma unroll 1
+    for (int shift = low; shift < 63; shift += 8) pass(shift);
+#pragma unroll
+    for (int r = 0; r < kSmallKeys; r++) {
+      const int i = first + 64 * r;
+      if (r < rounds && i < n) {
+        keys[i] = key[r];
+        vals[i] = val[r];
+      }
+    }
+    __syncthreads();
+  };
+  // the top 40 bits part the points of nearly every set this small, up to short runs
+  int low = 23;
+#pragma unroll 1
+  while (true) {
+    sort_from(low);
+    bool is_long = false;
+    for (int i = tid; i + kShortRun < n; i += kSmallThreads) is_long |= (keys[i] ^ keys[i + kShortRun]) >> low == 0;
+    if (low == 0 || !__syncthreads_or(is_long)) break;
+    low = 0;
+  }
+  for (int i = tid; i < n; i += kSmallThreads)
+    finish_at<D, T>(i, low, keys, vals, nullptr, n, pos, pos_out, id_out, runs, nruns, n / (kShortRun + 1) + 1);
 }
 
 // Tile of a pass over n pairs.  More threads per tile mean fewer look-back rows and longer writes,
@@ -685,9 +844,6 @@ int zsort_impl(hipStream_t s, const T* pos_in, T* pos_out, typename IntOf<T>::ty
   uint32_t* hist = (uint32_t*)(tmp + L.hist);
   uint32_t* meta = (uint32_t*)(tmp + L.meta);
   uint32_t* lookback = (uint32_t*)(tmp + L.lookback);
-  const SortTile st = sort_tile(n);
-  // zero histograms, meta (incl. tile counters) and look-back state in one fill
-  if (fill_u32(s, hist, 0u, (int64_t)((L.lookback - L.hist) / 4) + kPasses * st.tiles * kRadix)) return 1;
   const T* src = pos_in;
   if ((const void*)pos_in == (const void*)pos_out) {
     T* cp = (T*)(tmp + L.poscopy);
@@ -695,6 +851,18 @@ int zsort_impl(hipStream_t s, const T* pos_in, T* pos_out, typename IntOf<T>::ty
       return fail("zsort: copy of aliased input failed");
     src = cp;
   }
+  if constexpr (kHasSmallSort<D, T>) {
+    if (n <= kSmallSort) {
+      int32_t* runs = (int32_t*)(tmp + L.runs);
+      hipLaunchKernelGGL((k_small_sort<D, T>), dim3(1), dim3(kSmallThreads), 0, s, src, (int)n, k0, v0, pos_out, id_out,
+                         runs, (int32_t*)meta + 4);
+      if (check_launch("zsort small")) return 1;
+      return long_runs<D, T>(s, k0, v0, nullptr, n, src, pos_out, id_out, runs, (int32_t*)meta + 4);
+    }
+  }
+  const SortTile st = sort_tile(n);
+  // zero histograms, meta (incl. tile counters) and look-back state in one fill
+  if (fill_u32(s, hist, 0u, (int64_t)((L.lookback - L.hist) / 4) + kPasses * st.tiles * kRadix)) return 1;
   int64_t blocks = div_up(n * D, 256 * 16);
   if (blocks > 2048) blocks = 2048;
   if constexpr (std::is_integral<T>::value)
@@ -718,7 +886,7 @@ int zsort_impl(hipStream_t s, const T* pos_in, T* pos_out, typename IntOf<T>::ty
 }
 
 // ---------------------------------------------------------------------------------------------
-// 7. segmented sort (many independent point sets, one pipeline)
+// 8. segmented sort (many independent point sets, one pipeline)
 // ---------------------------------------------------------------------------------------------
 // Points of set s occupy [off[s], off[s+1]) of the input; the output keeps every set in its range,
 // z-ordered inside it exactly as a single-set sort of that set would order it (the Morton window
@@ -948,7 +1116,7 @@ int zsort_seg_impl(hipStream_t s, const T* pos_in, T* pos_out, typename IntOf<T>
 }
 
 // ---------------------------------------------------------------------------------------------
-// 8. group order (FoF catalogue): stable sort of the particles by their group label
+// 9. group order (FoF catalogue): stable sort of the particles by their group label
 // ---------------------------------------------------------------------------------------------
 // _fof_order (fof.py:510-519): igr[i] = igroup[i] for the filled particles (i < npart), n for the
 // rest; isort = stable argsort of igr; counts[i] = number of filled particles labelled isort[i]
@@ -1059,7 +1227,7 @@ int fof_order_impl(hipStream_t s, const int32_t* igroup, const int32_t* npart, i
 }
 
 // ---------------------------------------------------------------------------------------------
-// 8b. rows back to input order (the gradient of the sort)
+// 10. rows back to input order (the gradient of the sort)
 // ---------------------------------------------------------------------------------------------
 // out[id[i]] = rows[i], rows of `width` elements, one element per thread: the threads of a row are
 // neighbours, so its scattered write is one piece.  As an inverse permutation (zeros, arange, scatter)
@@ -1075,7 +1243,7 @@ __global__ __launch_bounds__(256) void k_unsort_rows(const U* __restrict__ rows,
 }
 
 // ---------------------------------------------------------------------------------------------
-// 9. SearchSortedZ (sort.cuh:82-132): insertion indices into a z-sorted array
+// 11. SearchSortedZ (sort.cuh:82-132): insertion indices into a z-sorted array
 // ---------------------------------------------------------------------------------------------
 // For each query x: the index i with have[i-1] < x <= have[i] in the exact z-order of this sort
 // (binary search with the exact comparator), i.e. the left insertion point; n_have past the end.

@@ -109,9 +109,9 @@ def test_zsort_tile_sizes(dev, oracle, kpt):
     assert np.array_equal(iz.cpu().numpy().astype(np.int64), oracle.zsort(x)[1])
 
 
-# one tile of each shape and its neighbours (2048, 4096, 8192, 12288 keys), the changes of shape
+# rounds of the one-workgroup sort (1024 keys each, up to 16384), tiles, the changes of tile shape
 # (2^18, 2^21, 2^23) and more tiles than one look-back step reads
-@pytest.mark.parametrize("n", [1, 2, 16, 17, 2047, 2048, 2049, 18433, (1 << 18) - 1, (1 << 18) + 1, (1 << 21) + 3,
+@pytest.mark.parametrize("n", [1, 2, 16, 17, 1023, 1024, 1025, 2047, 2049, 5000, 16383, 16384, 16385, 18433, (1 << 18) - 1, (1 << 18) + 1, (1 << 21) + 3,
                                (1 << 23) + 5])
 def test_zsort_tiles(dev, oracle, n):
     x = clustered(n, nhalos=64, seed=n) if n > 4096 else uniform(n, seed=n)
@@ -157,3 +157,29 @@ def test_zsort_gradient(dev, dtype, dim):
     wb = torch.stack([w, 2 * w, -w])
     (gb,) = torch.autograd.grad(posz, x, wb, is_grads_batched=True)
     assert torch.equal(gb, torch.stack([ref, 2 * ref, -ref]))
+
+
+@pytest.mark.parametrize("dim,dtype", [(2, np.float32), (3, np.float32), (2, np.float64), (3, np.float64)])
+@pytest.mark.parametrize("kind", ["tight", "signed", "equal", "nan"])
+def test_zsort_small(dev, oracle, dim, dtype, kind):
+    """Sets for one workgroup whose points the top bits of the keys do not part, with signs, all equal,
+    and with NaN rows next to the largest key."""
+    rng = np.random.default_rng(9)
+    x = rng.random((3000, dim))
+    if kind == "tight":
+        x = 0.3 + 1e-4 * x
+        x[0] = 1.0
+    elif kind == "signed":
+        x = 2 * x - 1
+        x[::17] = np.inf
+        x[::19, 0] = -np.inf
+    elif kind == "equal":
+        x[:] = 0.25
+    x = x.astype(dtype)
+    if kind == "nan":
+        x[::7] = np.nextafter(dtype(1), dtype(0))
+        x[::11, 1] = np.nan
+    x = np.ascontiguousarray(x)
+    pz, idz = _gpu_zsort(x, dev)
+    opz, oidz = oracle.zsort(x)
+    assert np.array_equal(idz, oidz) and np.array_equal(pz, opz, equal_nan=True)
