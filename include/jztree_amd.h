@@ -107,6 +107,17 @@ int jzt_search_sorted_z(jzt_stream_t stream, const void* posz_have, const void* 
 int jzt_unsort_rows(jzt_stream_t stream, const void* rows, const void* id, int64_t n, int width, int elem_bytes,
                     void* out);
 
+/* Distances for the dense top-plane list (jzt_dense_ilist_top) of 2-3 dims: with r2, every entry gets the
+ * squared distance of the two super-nodes' bounding boxes, from below (negative where they touch, -inf
+ * for the node itself), and every row is sorted by it; without r2, entries farther than `limit`
+ * are replaced by -1, which FofNode2Node skips.  nodes: the top plane's (centre, level) rows; nsuper:
+ * device count. */
+size_t jzt_dense_ilist_r2_tmp_bytes(int64_t size_super, int dim, int dtype);
+int jzt_dense_ilist_r2(jzt_stream_t stream, const void* nodes, int64_t nnodes, const int32_t* spl_super,
+                       const int32_t* ispl, int64_t size_super, const int32_t* nsuper, int32_t* ilist, float* r2,
+                       int64_t size_ilist, float boxsize, float limit, int dim, int dtype, void* tmp,
+                       size_t tmp_bytes);
+
 /* SegmentSort -- replaces ffi target "SegmentSort" (generated/ffi_knn.cu:412-423, knn.cuh:700-722,
  * caller knn.py:112-127).  Sorts (key, val) within segments spl[i]..spl[i+1] by (key, val). */
 int jzt_segment_sort(jzt_stream_t stream, const int32_t* spl, const float* key, const int32_t* val,

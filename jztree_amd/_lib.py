@@ -33,6 +33,8 @@ _SIGNATURES = {
     "jzt_pos_zorder_sort_noalloc": ([_p, _p, _p, _p, _i64, _i32, _i32], _i32),
     "jzt_zsort_segmented_tmp_bytes": ([_i64, _i64, _i32, _i32], _sz),
     "jzt_pos_zorder_sort_segmented": ([_p, _p, _p, _p, _p, _i64, _p, _sz, _i64, _i32, _i32], _i32),
+    "jzt_dense_ilist_r2_tmp_bytes": ([_i64, _i32, _i32], _sz),
+    "jzt_dense_ilist_r2": ([_p, _p, _i64, _p, _p, _i64, _p, _p, _p, _i64, _f32, _f32, _i32, _i32, _p, _sz], _i32),
     "jzt_unsort_rows": ([_p, _p, _p, _i64, _i32, _i32, _p], _i32),
     "jzt_segment_sort": ([_p, _p, _p, _p, _p, _p, _i64, _i64], _i32),
     "jzt_search_sorted_z": ([_p, _p, _p, _i64, _i64, _i32, _i32, _i32, _p], _i32),

@@ -1038,6 +1038,84 @@ int segment_sort(hipStream_t s, const int32_t* spl, float* key, int32_t* val, co
   return check_launch(what);
 }
 
+// ------------------------------------------------------------------------------------------------
+// distances for the dense top-plane list
+// ------------------------------------------------------------------------------------------------
+// The dense list pairs every super-node (about 32 consecutive top-plane nodes) with every other, at no
+// distance: each of the three passes over the top plane tested all pairs of its nodes (2048 to 13,000),
+// and the radius search met the node's own neighbourhood only when the list came to it.  With the
+// distances of the super-nodes' bounding boxes, sorted, the passes stop where the radius ends.  A
+// distance is lowered by 2^-15 of itself and the boxes are widened by 2^-20 of their coordinates, which
+// covers the rounding of the nodes' own distances: the nodes' lists are the same.
+template <int D, typename T>
+__global__ __launch_bounds__(256) void k_super_boxes(const T* __restrict__ nodes, const int32_t* __restrict__ spl,
+                                                     const int32_t* __restrict__ nsuper, int64_t nmax, int64_t nnodes,
+                                                     T* __restrict__ boxes) {
+  const int sub = threadIdx.x & 31;
+  const int64_t ns = min((int64_t)nsuper[0], nmax);
+  for (int64_t i = (int64_t)blockIdx.x * (blockDim.x / 32) + (threadIdx.x >> 5); i < ns;
+       i += (int64_t)gridDim.x * (blockDim.x / 32)) {
+    const int64_t a = spl[i], b = min((int64_t)spl[i + 1], nnodes);
+    T lo[D], hi[D];
+#pragma unroll
+    for (int d = 0; d < D; d++) {
+      lo[d] = (T)INFINITY;
+      hi[d] = -(T)INFINITY;
+    }
+    for (int64_t j = a + sub; j < b; j += 32) {
+      const NodeT<D, T> n = load_node<D, T>(nodes, j);
+      const Vec<D, T> e = lvl_half_ext<D, T>(n.level);
+#pragma unroll
+      for (int d = 0; d < D; d++) {
+        lo[d] = min(lo[d], n.cent[d] - e[d]);
+        hi[d] = max(hi[d], n.cent[d] + e[d]);
+      }
+    }
+    for (int o = 16; o > 0; o >>= 1) {
+#pragma unroll
+      for (int d = 0; d < D; d++) {
+        lo[d] = min(lo[d], __shfl_xor(lo[d], o, 32));
+        hi[d] = max(hi[d], __shfl_xor(hi[d], o, 32));
+      }
+    }
+    if (sub == 0) {
+#pragma unroll
+      for (int d = 0; d < D; d++) {
+        const T c = T(0.5) * lo[d] + T(0.5) * hi[d];
+        boxes[i * 2 * D + d] = c;
+        boxes[i * 2 * D + D + d] = (T(0.5) * hi[d] - T(0.5) * lo[d]) + (abs(lo[d]) + abs(hi[d])) * T(1.0 / 1048576.0);
+      }
+    }
+  }
+}
+
+// r2 given: the distance of every entry (negative for touching super-nodes, nearest first, as in
+// k_node_insert); else entries beyond `limit` are replaced by -1, which the FoF passes skip.
+template <int D, typename T>
+__global__ __launch_bounds__(256) void k_dense_r2(const T* __restrict__ boxes, const int32_t* __restrict__ nsuper,
+                                                  int64_t nmax, int64_t size_ilist, T boxsize, float limit,
+                                                  int32_t* __restrict__ ilist, float* __restrict__ r2) {
+  const int64_t ns = nsuper[0];
+  if (ns > nmax) return;  // reported by the list's own check
+  const int64_t m = min(ns * ns, size_ilist);
+  for (int64_t j = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; j < m; j += (int64_t)gridDim.x * blockDim.x) {
+    const int64_t a = j / ns, b = j - a * ns;
+    Vec<D, T> ca, cb, w;
+#pragma unroll
+    for (int d = 0; d < D; d++) {
+      ca[d] = boxes[a * 2 * D + d];
+      cb[d] = boxes[b * 2 * D + d];
+      w[d] = boxes[a * 2 * D + D + d] + boxes[b * 2 * D + D + d];
+    }
+    const float g2 = (float)mindist2<D, T>(ca, cb, w, boxsize) * (1.0f - 2.f * kBoundSlack);
+    if (!r2) {
+      if (g2 > limit) ilist[j] = -1;
+    } else {
+      r2[j] = g2 > 0.f ? g2 : a == b ? -INFINITY : -1.0f / fmaxf((float)maxdist2<D, T>(ca, cb, w, boxsize), 1e-30f);
+    }
+  }
+}
+
 __global__ void k_scale_rmax2(const float* __restrict__ in, float* __restrict__ out, int64_t n) {
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i < n) out[i] = in[i] * kRmaxSlack;
@@ -1260,6 +1338,35 @@ extern "C" int jzt_knn_node2node_tmp(jzt_stream_t stream, const int32_t* parent_
 #undef JZT_N2N_DIM
 #undef JZT_N2N
   return fail("KnnNode2Node: unsupported dim/dtype");
+}
+
+extern "C" size_t jzt_dense_ilist_r2_tmp_bytes(int64_t size_super, int dim, int dtype) {
+  return (size_t)size_super * 2 * dim * (dtype == JZT_F64 ? 8 : 4);
+}
+
+extern "C" int jzt_dense_ilist_r2(jzt_stream_t stream, const void* nodes, int64_t nnodes, const int32_t* spl_super,
+                                  const int32_t* ispl, int64_t size_super, const int32_t* nsuper, int32_t* ilist,
+                                  float* r2, int64_t size_ilist, float boxsize, float limit, int dim, int dtype,
+                                  void* tmp, size_t tmp_bytes) {
+  hipStream_t s = (hipStream_t)stream;
+  if (size_super <= 0 || nnodes <= 0) return 0;
+  if (nnodes >= INT32_MAX) return fail("DenseIlistR2: too many nodes");
+  if (tmp_bytes < jzt_dense_ilist_r2_tmp_bytes(size_super, dim, dtype)) return fail("DenseIlistR2: tmp buffer too small");
+#define JZT_DENSE_R2(D, T)                                                                                          \
+  hipLaunchKernelGGL((k_super_boxes<D, T>), dim3((unsigned)std::min(div_up(size_super, 8), (int64_t)256)), dim3(256), \
+                     0, s, (const T*)nodes, spl_super, nsuper, size_super, nnodes, (T*)tmp);                         \
+  hipLaunchKernelGGL((k_dense_r2<D, T>), dim3((unsigned)std::min(div_up(size_ilist, 256), (int64_t)1024)), dim3(256), \
+                     0, s, (const T*)tmp, nsuper, size_super, size_ilist, (T)boxsize, limit, ilist, r2)
+  if (dim == 3 && dtype == JZT_F32) { JZT_DENSE_R2(3, float); }
+  else if (dim == 3 && dtype == JZT_F64) { JZT_DENSE_R2(3, double); }
+  else if (dim == 2 && dtype == JZT_F32) { JZT_DENSE_R2(2, float); }
+  else if (dim == 2 && dtype == JZT_F64) { JZT_DENSE_R2(2, double); }
+  else return fail("DenseIlistR2: unsupported dim/dtype");
+#undef JZT_DENSE_R2
+  if (check_launch("DenseIlistR2")) return 1;
+  if (!r2) return 0;
+  // rows past the last super-node are empty
+  return segment_sort(s, ispl, r2, ilist, r2, ilist, size_super, size_ilist, size_super, nullptr, "DenseIlistR2 sort");
 }
 
 extern "C" int jzt_segment_max_f32(jzt_stream_t stream, const int32_t* spl, const float* vals, int64_t nvals,

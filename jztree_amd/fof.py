@@ -130,12 +130,14 @@ def _fof_dual_walk(th: TreeHierarchy, rlink: float, boxsize: float = 0., alloc_f
     r2link_set (extension, batch forests): float32 r2link of every set, used in place of rlink."""
     nplanes = th.num_planes()
     size = th.size()
-    spl, ilist = top_plane_lists(th, int(th.size_leaves * alloc_fac_ilist))
+    tables = plane_tables(th)
+    # beyond 2^-10 more than the linking length no pair of nodes is looked at (their own test allows 2^-16)
+    limit = None if r2link_set is not None else float(rlink) ** 2 * (1. + 2. ** -10)
+    spl, ilist = top_plane_lists(th, int(th.size_leaves * alloc_fac_ilist), tables, boxsize, r2_limit=limit)
     if r2link_set is not None:
         assert th.leaf_set is not None
         r2_plane = [r2link_set[s.long()].contiguous() for s in _plane_node_sets(th, spl)]
     dev = spl.device
-    tables = plane_tables(th)
     n2c = tables.spl + [spl]
     igroup = torch.arange(size, dtype=torch.int32, device=dev)
     lvl = torch.full_like(igroup, th.info().max_lvl())  # of the super-nodes

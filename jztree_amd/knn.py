@@ -166,8 +166,8 @@ def _knn_dual_walk(th: TreeHierarchy, k: int, boxsize: float | None = None,
     With return_parents, also returns (rmax2 of the plane's nodes or None at the top, the
     node-to-child splits of that plane)."""
     nlevels = th.num_planes()
-    spl, ilist = top_plane_lists(th, int(th.size_leaves * alloc_fac_ilist), with_r2=True)
     tables = plane_tables(th)
+    spl, ilist = top_plane_lists(th, int(th.size_leaves * alloc_fac_ilist), tables, boxsize, with_r2=True)
     n2c = tables.spl + [spl]
     rmax2 = None
     for level in reversed(range(stop_level, nlevels)):
@@ -277,8 +277,8 @@ def _knn_radius_walk(th: TreeHierarchy, k: int, radii: list, boxsize: float = 0.
     keep_plane1: also return (the plane-1 lists, plane-1 -> leaf splits) -- with a one-plane tree
     the dense top-level list and its super-node splits."""
     nlevels = th.num_planes()
-    spl, ilist = top_plane_lists(th, int(th.size_leaves * alloc_fac_ilist), with_r2=True)
     tables = plane_tables(th)
+    spl, ilist = top_plane_lists(th, int(th.size_leaves * alloc_fac_ilist), tables, boxsize, with_r2=True)
     n2c = tables.spl + [spl]
     plane1 = None
     for level in reversed(range(nlevels)):

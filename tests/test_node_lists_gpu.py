@@ -7,6 +7,8 @@ FofNode2Node: joined nodes and lists against all pairs, at every number of child
 Node lists: every child's radius against the exact weighted selection and every list against all pairs,
 with parents whose lists are short (one wave) and long (queued), fewer and more than 64 particles of
 candidates per child, one and several children per work item."""
+import dataclasses
+
 import numpy as np
 import pytest
 import torch
@@ -186,3 +188,27 @@ def test_fof_node_passes_against_all_pairs(dev, nparents, kids):
         got[i, src[ispl[i]:ispl[i + 1]]] = True
     assert not (need & ~got).any() and not (got & ~may).any()
     assert need.any()
+
+
+@pytest.mark.parametrize("n,dim,dtype,boxsize", [(200003, 3, "f32", 1.0), (150001, 2, "f32", 0.0),
+                                                 (120001, 3, "f64", 1.0), (130001, 2, "f64", 1.0)])
+def test_dense_top_distances(dev, monkeypatch, n, dim, dtype, boxsize):
+    """Neighbours and groups with the super-nodes' distances in the dense list equal those without; the
+    points are clustered towards the faces of the box."""
+    import jztree_amd as jz
+    rng = np.random.default_rng(n)
+    x = np.concatenate([rng.random((n // 2, dim)), np.mod(0.02 * rng.standard_normal((n - n // 2, dim)), 1.0)])
+    x = np.minimum(x, 1 - 2.0 ** -24).astype(np.float32 if dtype == "f32" else np.float64)
+    t = torch.from_numpy(np.ascontiguousarray(x[rng.permutation(n)])).to(dev)
+    kcfg, fcfg = jz.config.KNNConfig(alloc_fac_ilist=512.), jz.config.FofConfig(alloc_fac_ilist=256.)
+    tree = lambda c: dataclasses.replace(c, tree=dataclasses.replace(c.tree, max_leaf_size=32, alloc_fac_nodes=2.5))
+    kcfg, fcfg = tree(kcfg), tree(fcfg)
+    rl = 0.2 * n ** (-1.0 / dim)
+    out = []
+    for least in (0, 1 << 40):
+        monkeypatch.setattr(jz.tree, "_DENSE_R2_LEAVES", least)
+        rnn, inn = jz.knn.knn(t, 10, boxsize=boxsize or None, cfg=kcfg)
+        pz, ig = jz.fof.fof_labels(t, rl, boxsize=boxsize, cfg=fcfg)
+        out.append((rnn, inn, pz, ig))
+    for a, b in zip(*out):
+        assert torch.equal(a, b)
