@@ -615,8 +615,7 @@ def zsort_and_tree_multi_type(part: Tuple, cfg_tree: TreeConfig = TreeConfig(), 
     # filled rows of each type first (rows with a NaN position last), as concatenate_pytrees does
     valid = torch.cat([~torch.isnan(get_pos(p)[:, 0]) for p in part])
     compress = torch.argsort((~valid).to(torch.int8), stable=True)
-    ptype = torch.repeat_interleave(torch.arange(num_types, dtype=torch.uint8, device=dev),
-                                    torch.tensor(sizes, device=dev))[compress]
+    ptype = torch.cat([torch.full((m,), t, dtype=torch.uint8, device=dev) for t, m in enumerate(sizes)])[compress]
 
     def stack(items):
         first = items[0]
