@@ -37,25 +37,57 @@ template <typename T> __device__ __forceinline__ bool pair_less(T r2a, uint32_t 
   return r2a < r2b || (r2a == r2b && ia < ib);
 }
 
-// Insert (r2, id) into the ascending pairs (caller guarantees it is below the last one); top-down
-// compare/select network with statically indexed registers, leaving every 8 slots once no lane
-// still shifts.
+// ascending compare-exchange of two (r2, id) pairs
+template <typename T> __device__ __forceinline__ void pair_ce(T& ra, uint32_t& ia, T& rb, uint32_t& ib) {
+  const bool sw = pair_less(rb, ib, ra, ia);
+  const T r = sw ? rb : ra;
+  const uint32_t i = sw ? ib : ia;
+  rb = sw ? ra : rb;
+  ib = sw ? ia : ib;
+  ra = r;
+  ia = i;
+}
+
+// Merge the lane's buffered pairs [0, cnt) of its LDS row into the ascending (br, bi)[0..K): both become the
+// K smallest of the union (Batcher's odd-even merge sort of the row, half-cleaner, bitonic merge).
+// Inserting every candidate by itself ran a network of K steps for nearly every source, as some lane
+// accepts it; a flush costs about six of those and takes up to kNdBuf candidates of every lane.
+template <int K> constexpr int kNdBuf = K < 16 ? K : 16;
 template <int K, typename T>
-__device__ __forceinline__ void pair_insert(T (&br)[K], uint32_t (&bi)[K], T r2, uint32_t id) {
-  bool hi = true;  // (r2, id) < slot i
+__device__ __forceinline__ void pair_flush(T (&br)[K], uint32_t (&bi)[K], const T* row_r, const uint32_t* row_i, int& cnt) {
+  constexpr int M = kNdBuf<K>;
+  T r[M];
+  uint32_t id[M];
 #pragma unroll
-  for (int i = K - 1; i >= 1; i--) {
-    const bool lo = pair_less(r2, id, br[i - 1], bi[i - 1]);
-    const T tr = hi ? r2 : br[i];
-    const uint32_t ti = hi ? id : bi[i];
-    br[i] = lo ? br[i - 1] : tr;
-    bi[i] = lo ? bi[i - 1] : ti;
-    hi = lo;
-    if ((i & 7) == 0 && !wave_any(lo)) return;
+  for (int i = 0; i < M; i++) {
+    r[i] = i < cnt ? row_r[i] : (T)INFINITY;
+    id[i] = i < cnt ? row_i[i] : 0xffffffffu;
   }
-  if (hi) {
-    br[0] = r2;
-    bi[0] = id;
+  cnt = 0;
+#pragma unroll
+  for (int p = 1; p < M; p <<= 1) {
+#pragma unroll
+    for (int k = p; k >= 1; k >>= 1) {
+#pragma unroll
+      for (int j = k % p; j <= M - 1 - k; j += 2 * k) {
+#pragma unroll
+        for (int i = 0; i < M; i++)
+          if (i <= k - 1 && i <= M - j - k - 1 && (i + j) / (2 * p) == (i + j + k) / (2 * p))
+            pair_ce(r[i + j], id[i + j], r[i + j + k], id[i + j + k]);
+      }
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < M; i++) {
+    const bool take = pair_less(r[M - 1 - i], id[M - 1 - i], br[K - M + i], bi[K - M + i]);
+    br[K - M + i] = take ? r[M - 1 - i] : br[K - M + i];
+    bi[K - M + i] = take ? id[M - 1 - i] : bi[K - M + i];
+  }
+#pragma unroll
+  for (int stride = K / 2; stride > 0; stride >>= 1) {
+#pragma unroll
+    for (int i = 0; i < K; i++)
+      if ((i ^ stride) > i) pair_ce(br[i], bi[i], br[i ^ stride], bi[i ^ stride]);
   }
 }
 
@@ -72,7 +104,12 @@ __global__ __launch_bounds__(64) void k_knn_leaf_nd(const int32_t* __restrict__ 
                                                     int64_t nitems, int xcd, uint32_t* __restrict__ queue) {
   __shared__ Vec<D, T> s_p[64];
   __shared__ uint32_t s_id[64];
+  constexpr int kRow = kNdBuf<K> | 1;  // odd: the lanes' rows start in different banks
+  __shared__ T s_br[64 * kRow];
+  __shared__ uint32_t s_bi[64 * kRow];
   const int lane = threadIdx.x;
+  T* const row_r = s_br + lane * kRow;
+  uint32_t* const row_i = s_bi + lane * kRow;
   const uint64_t lt_mask = (1ull << lane) - 1ull;
   const T box = (T)boxsize, half = (T)(0.5f * boxsize);
   const T slack = (T)(1.0f + kBoundSlack);
@@ -109,6 +146,7 @@ __global__ __launch_bounds__(64) void k_knn_leaf_nd(const int32_t* __restrict__ 
         br[i] = start_r2;
         bi[i] = 0xffffffffu;
       }
+      int cnt = 0;  // pairs in the lane's row
       T kmax = wave_max_t(br[K - 1]) * slack;
       bool done = false;
       for (int eb = e0; eb < e1 && !done; eb += 64) {
@@ -156,22 +194,26 @@ __global__ __launch_bounds__(64) void k_knn_leaf_nd(const int32_t* __restrict__ 
               s_id[slot] = pid;
             }
             __syncthreads();
-            bool inserted = false;
+            // an accepted candidate goes into the lane's row, any other is overwritten by the next
+#pragma unroll 1
             for (int j = 0; j < n_keep; j++) {
+              if (wave_any(cnt == kNdBuf<K>)) {
+                pair_flush<K, T>(br, bi, row_r, row_i, cnt);
+                kmax = wave_max_t(br[K - 1]) * slack;
+              }
               const Vec<D, T> s = s_p[j];
               const uint32_t sid = s_id[j];
               const T r2 = (PER && wrap) ? dist2P<true, D, T>(q, s, box, half) : dist2P<false, D, T>(q, s, box, half);
               const bool acc = pair_less(r2, sid, br[K - 1], bi[K - 1]) && (!floor || pair_less(fr2, fid, r2, sid));
-              if (wave_any(acc)) {
-                inserted = true;
-                if (acc) pair_insert<K, T>(br, bi, r2, sid);
-              }
+              row_r[cnt] = r2;
+              row_i[cnt] = sid;
+              cnt += acc ? 1 : 0;
             }
-            if (inserted) kmax = wave_max_t(br[K - 1]) * slack;
             __syncthreads();
           }
         }
       }
+      if (wave_any(cnt > 0)) pair_flush<K, T>(br, bi, row_r, row_i, cnt);
       if (qoff + lane < q1) {
         const int nk = min(K, ktot - koff);
         const int64_t orow = dst_rows ? (int64_t)dst_rows[iq] : (int64_t)iq;
