@@ -679,7 +679,7 @@ __global__ __launch_bounds__(kSmallThreads) void k_small_sort(const T* __restric
   for (int r = 0; r < kSmallKeys; r++) {
     if (r < rounds) {
       const int i = first + 64 * r;
-      key[r] = ~0ull;  // past the end: after every point, NaN rows included (equal keys, later index)
+      key[r] = ~0ull;  // past the end: after every row (NaN rows have the same key and come earlier)
       val[r] = (uint32_t)i;
       if (i < n) {
         T x[D];
@@ -750,7 +750,7 @@ __global__ __launch_bounds__(kSmallThreads) void k_small_sort(const T* __restric
   // the passes from bit `low` on; then the rows, in global memory for their neighbours
   auto sort_from = [&](int low) {
 #pragma unroll 1
-    for (int shift = low; shift < 63; shift += 8) pass(shift);
+    for (int shift = low; shift < 64; shift += 8) pass(shift);
 #pragma unroll
     for (int r = 0; r < kSmallKeys; r++) {
       const int i = first + 64 * r;
@@ -761,8 +761,9 @@ __global__ __launch_bounds__(kSmallThreads) void k_small_sort(const T* __restric
     }
     __syncthreads();
   };
-  // the top 40 bits part the points of nearly every set this small, up to short runs
-  int low = 23;
+  // The top 40 bits part the points of nearly every set this small, up to short runs.  Bit 63 is one of
+  // them: it is all that tells a NaN row (~0) from a point in the top corner of a non-negative 3-D set.
+  int low = 24;
 #pragma unroll 1
   while (true) {
     sort_from(low);

@@ -183,3 +183,22 @@ def test_zsort_small(dev, oracle, dim, dtype, kind):
     pz, idz = _gpu_zsort(x, dev)
     opz, oidz = oracle.zsort(x)
     assert np.array_equal(idz, oidz) and np.array_equal(pz, opz, equal_nan=True)
+
+
+@pytest.mark.parametrize("dim,dtype", [(2, np.float32), (3, np.float32), (2, np.float64), (3, np.float64)])
+@pytest.mark.parametrize("n,few", [(6, 1), (1000, 1), (1000, 8), (9001, 3)])
+def test_zsort_small_nan_rows_next_to_the_top_corner(dev, oracle, dim, dtype, n, few):
+    """A few NaN rows before and between points whose key bits are all ones (too few for a long run):
+    the NaN rows come last, and a tree of the set counts the others."""
+    import jztree_amd as jz
+    rng = np.random.default_rng(n)
+    x = rng.random((n, dim)).astype(dtype)
+    rows = np.sort(rng.permutation(n)[:2 * few])
+    x[rows[::2], 0] = np.nan  # every point of the corner has a NaN row before it
+    x[rows[1::2]] = np.nextafter(dtype(1), dtype(0))
+    pz, idz = _gpu_zsort(x, dev)
+    opz, oidz = oracle.zsort(x)
+    assert np.array_equal(idz, oidz) and np.array_equal(pz, opz, equal_nan=True)
+    _, _, th = jz.tree.zsort_and_tree_origin(torch.from_numpy(x).to(dev), jz.config.TreeConfig(alloc_fac_nodes=2.))
+    jz.checks.flush()
+    assert int(th.splits_leaf_to_part(0).max()) == n - few
