@@ -469,30 +469,41 @@ __global__ __launch_bounds__(NT) void k_node_insert(
 // ------------------------------------------------------------------------------------------------
 // segmented sort by (key, val)
 // ------------------------------------------------------------------------------------------------
-// A (key, val) pair is one double whose high word is the key's own bits: keys are floats, so the
-// exponent field of the double never reaches 0x7ff (float infinity and NaN patterns are ordinary
-// doubles), and the double order is the float total order; below zero the order of the low word is
-// reversed, so val is stored complemented there.  Denormal doubles are kept by the FP64 mode.  A
-// compare-exchange is then one FP64 compare (or v_min_f64 + v_max_f64) instead of a 64-bit integer one.
+// A (key, val) pair P of a node list, whose keys are distances and never NaN, is one double with the key's
+// own bits as its high word: up to float infinity (0x7f800000) the double's exponent field stays below 0x7ff,
+// and the double order is the float total order; below zero the order of the low word is reversed, so
+// val is stored complemented there.  Denormal doubles are kept by the FP64 mode.  A compare-exchange is
+// then one FP64 compare (or v_min_f64 + v_max_f64) instead of a 64-bit integer one.
+// Keys of a caller (jzt_segment_sort) can be any bits: NaN patterns from 0x7ff00000 on would make the
+// double a NaN, and -0 with val -1 would be -0.0, equal to +0 with val 0.  Their pairs are 64-bit integers in
+// the same order.
 constexpr int kSegThreads = 256;
 constexpr int kSegLds = 4096;        // entries a workgroup of kSegThreads sorts in LDS (32 KB)
 constexpr int kSegBigThreads = 1024;
 constexpr int kSegBigLds = 16384;    // entries a workgroup of kSegBigThreads sorts in LDS (128 KB)
 constexpr int kWaveSortMax = 1024;   // entries one wave sorts in registers
 
-__device__ __forceinline__ double kv_pack(float k, int32_t v) {
+template <typename P> constexpr bool kAnyKey = std::is_same<P, uint64_t>::value;
+template <typename P> __device__ __forceinline__ P kv_pack(float k, int32_t v) {
   const uint32_t kb = __float_as_uint(k);
-  const uint32_t lo = (kb >> 31) ? ~(uint32_t)v : (uint32_t)v;
-  return __longlong_as_double((long long)(((uint64_t)kb << 32) | lo));
+  if constexpr (kAnyKey<P>) return ((uint64_t)((kb >> 31) ? ~kb : kb | 0x80000000u) << 32) | (uint32_t)v;
+  else return __longlong_as_double((long long)(((uint64_t)kb << 32) | ((kb >> 31) ? ~(uint32_t)v : (uint32_t)v)));
 }
-__device__ __forceinline__ float kv_key(double p) {
-  return __uint_as_float((uint32_t)((uint64_t)__double_as_longlong(p) >> 32));
+template <typename P> __device__ __forceinline__ float kv_key(P p) {
+  const uint32_t h = (uint32_t)(__builtin_bit_cast(uint64_t, p) >> 32);
+  if constexpr (kAnyKey<P>) return __uint_as_float((h >> 31) ? h & 0x7fffffffu : ~h);
+  else return __uint_as_float(h);
 }
-__device__ __forceinline__ int32_t kv_val(double p) {
-  const uint64_t b = (uint64_t)__double_as_longlong(p);
-  return (int32_t)((b >> 63) ? ~(uint32_t)b : (uint32_t)b);
+template <typename P> __device__ __forceinline__ int32_t kv_val(P p) {
+  const uint64_t b = __builtin_bit_cast(uint64_t, p);
+  if constexpr (kAnyKey<P>) return (int32_t)(uint32_t)b;
+  else return (int32_t)((b >> 63) ? ~(uint32_t)b : (uint32_t)b);
 }
-__device__ __forceinline__ double kv_last() { return __longlong_as_double(0x7fefffffffffffffll); }  // above every pair
+// no pair is above it
+template <typename P> __device__ __forceinline__ P kv_last() {
+  if constexpr (kAnyKey<P>) return ~0ull;
+  else return __longlong_as_double(0x7fefffffffffffffll);
+}
 
 // Bitonic network with only ascending comparators (the first stage of each merge compares mirrored
 // pairs), so lengths need not be powers of two (virtual +inf tail).
@@ -507,7 +518,7 @@ __device__ __forceinline__ void bitonic_sort_asc(Arr a, int len) {
       int i = blk * size + off;
       int j = blk * size + size - 1 - off;
       if (j < len) {
-        const double x = a.load(i), y = a.load(j);
+        const auto x = a.load(i), y = a.load(j);
         if (y < x) {
           a.store(i, y);
           a.store(j, x);
@@ -521,7 +532,7 @@ __device__ __forceinline__ void bitonic_sort_asc(Arr a, int len) {
         int i = blk * 2 * stride + off;
         int j = i + stride;
         if (j < len) {
-          const double x = a.load(i), y = a.load(j);
+          const auto x = a.load(i), y = a.load(j);
           if (y < x) {
             a.store(i, y);
             a.store(j, x);
@@ -533,17 +544,17 @@ __device__ __forceinline__ void bitonic_sort_asc(Arr a, int len) {
   }
 }
 
-struct LdsArr {
-  double* p;
-  __device__ __forceinline__ double load(int i) const { return p[i]; }
-  __device__ __forceinline__ void store(int i, double x) const { p[i] = x; }
+template <typename P> struct LdsArr {
+  P* p;
+  __device__ __forceinline__ P load(int i) const { return p[i]; }
+  __device__ __forceinline__ void store(int i, P x) const { p[i] = x; }
 };
 // (key, val) pairs sorted in place in global memory
-struct GlobalKV {
+template <typename P> struct GlobalKV {
   float* k;
   int32_t* v;
-  __device__ __forceinline__ double load(int i) const { return kv_pack(k[i], v[i]); }
-  __device__ __forceinline__ void store(int i, double x) const {
+  __device__ __forceinline__ P load(int i) const { return kv_pack<P>(k[i], v[i]); }
+  __device__ __forceinline__ void store(int i, P x) const {
     k[i] = kv_key(x);
     v[i] = kv_val(x);
   }
@@ -573,22 +584,25 @@ template <int M> __device__ __forceinline__ uint32_t lane_xor(uint32_t x) {
   } else if constexpr (M == 31) return lane_xor<16>(lane_xor<15>(x));
   else return lane_xor<32>(lane_xor<31>(x));  // 63
 }
-template <int M> __device__ __forceinline__ double lane_xor(double v) {
-  const uint64_t b = (uint64_t)__double_as_longlong(v);
-  const uint32_t lo = lane_xor<M>((uint32_t)b), hi = lane_xor<M>((uint32_t)(b >> 32));
-  return __longlong_as_double((long long)(((uint64_t)hi << 32) | lo));
+template <int M, typename P> __device__ __forceinline__ P pair_xor(P v) {
+  return on_words(v, [](uint32_t x) { return lane_xor<M>(x); });
 }
-// keeps the smaller of v and o where `low`, else the larger (v and o differ or are both padding)
-__device__ __forceinline__ double keep_side(double v, double o, bool low) { return (o < v) == low ? o : v; }
+// keeps the smaller of v and o where `low`, else the larger (of equal ones either)
+template <typename P> __device__ __forceinline__ P keep_side(P v, P o, bool low) { return (o < v) == low ? o : v; }
 
 __device__ __forceinline__ void kv_order(double& a, double& b) {
   const double lo = __builtin_fmin(a, b), hi = __builtin_fmax(a, b);
   a = lo;
   b = hi;
 }
+__device__ __forceinline__ void kv_order(uint64_t& a, uint64_t& b) {
+  const uint64_t lo = a < b ? a : b, hi = a < b ? b : a;
+  a = lo;
+  b = hi;
+}
 
 // entries x ^ S for register strides S < E (the whole wave is in blocks of 2S)
-template <int E, int S> __device__ __forceinline__ void half_clean(double (&v)[E], int lane) {
+template <int E, int S, typename P> __device__ __forceinline__ void half_clean(P (&v)[E], int lane) {
   if constexpr (S < E) {
 #pragma unroll
     for (int i = 0; i < E; i++)
@@ -596,12 +610,12 @@ template <int E, int S> __device__ __forceinline__ void half_clean(double (&v)[E
   } else {
     const bool low = (lane & (S / E)) == 0;
 #pragma unroll
-    for (int i = 0; i < E; i++) v[i] = keep_side(v[i], lane_xor<S / E>(v[i]), low);
+    for (int i = 0; i < E; i++) v[i] = keep_side(v[i], pair_xor<S / E>(v[i]), low);
   }
   if constexpr (S > 1) half_clean<E, S / 2>(v, lane);
 }
 // merges sorted blocks of SIZE/2 entries into sorted blocks of SIZE, from SIZE = 2 up to 64 * E
-template <int E, int SIZE> __device__ __forceinline__ void wave_merge(double (&v)[E], int lane) {
+template <int E, int SIZE, typename P> __device__ __forceinline__ void wave_merge(P (&v)[E], int lane) {
   if constexpr (SIZE <= E) {
 #pragma unroll
     for (int i = 0; i < E; i++) {
@@ -611,9 +625,9 @@ template <int E, int SIZE> __device__ __forceinline__ void wave_merge(double (&v
   } else {
     constexpr int M = SIZE / E - 1;  // mirrored partner: lane ^ M, register E - 1 - i
     const bool low = (lane & (SIZE / E / 2)) == 0;
-    double o[E];
+    P o[E];
 #pragma unroll
-    for (int i = 0; i < E; i++) o[i] = lane_xor<M>(v[E - 1 - i]);
+    for (int i = 0; i < E; i++) o[i] = pair_xor<M>(v[E - 1 - i]);
 #pragma unroll
     for (int i = 0; i < E; i++) v[i] = keep_side(v[i], o[i], low);
   }
@@ -621,14 +635,14 @@ template <int E, int SIZE> __device__ __forceinline__ void wave_merge(double (&v
   if constexpr (SIZE < 64 * E) wave_merge<E, SIZE * 2>(v, lane);
 }
 
-template <int E>
+template <int E, typename P>
 __device__ __forceinline__ void wave_sort_segment(float* key, int32_t* val, const float* key_in, const int32_t* val_in,
                                                   int64_t b, int len, int lane) {
-  double v[E];
+  P v[E];
 #pragma unroll
   for (int i = 0; i < E; i++) {
     const int idx = i * 64 + lane;  // any assignment will do before the sort: the coalesced one
-    v[i] = idx < len ? kv_pack(key_in[b + idx], val_in[b + idx]) : kv_last();
+    v[i] = idx < len ? kv_pack<P>(key_in[b + idx], val_in[b + idx]) : kv_last<P>();
   }
   wave_merge<E, 2>(v, lane);
 #pragma unroll
@@ -647,6 +661,7 @@ inline int64_t seg_queue_words(int64_t nmax) { return nmax / kWaveSortMax + 1; }
 
 // Segments of up to kWaveSortMax entries, one wave each (in place allowed: a wave reads its whole
 // segment into registers before writing); longer ones are queued for k_segment_sort.
+template <typename P>
 __global__ __launch_bounds__(64) void k_segment_sort_wave(const int32_t* __restrict__ spl, float* key, int32_t* val,
                                                           const float* key_in, const int32_t* val_in, int64_t nmax,
                                                           int64_t nitems, int32_t* __restrict__ queue) {
@@ -661,21 +676,21 @@ __global__ __launch_bounds__(64) void k_segment_sort_wave(const int32_t* __restr
       if (queue && lane == 0) queue[1 + atomicAdd(queue, 1)] = (int32_t)seg;
       continue;
     }
-    if (len <= 64) wave_sort_segment<1>(key, val, key_in, val_in, b, (int)len, lane);
-    else if (len <= 128) wave_sort_segment<2>(key, val, key_in, val_in, b, (int)len, lane);
-    else if (len <= 256) wave_sort_segment<4>(key, val, key_in, val_in, b, (int)len, lane);
-    else if (len <= 512) wave_sort_segment<8>(key, val, key_in, val_in, b, (int)len, lane);
-    else wave_sort_segment<16>(key, val, key_in, val_in, b, (int)len, lane);
+    if (len <= 64) wave_sort_segment<1, P>(key, val, key_in, val_in, b, (int)len, lane);
+    else if (len <= 128) wave_sort_segment<2, P>(key, val, key_in, val_in, b, (int)len, lane);
+    else if (len <= 256) wave_sort_segment<4, P>(key, val, key_in, val_in, b, (int)len, lane);
+    else if (len <= 512) wave_sort_segment<8, P>(key, val, key_in, val_in, b, (int)len, lane);
+    else wave_sort_segment<16, P>(key, val, key_in, val_in, b, (int)len, lane);
   }
 }
 
 // One workgroup per segment of more than LO entries: up to CAP in LDS; longer ones, where BIG, in
 // place in the output arrays (global memory, visible within the workgroup across barriers).
-template <int NT, int LO, int CAP, bool BIG>
+template <typename P, int NT, int LO, int CAP, bool BIG>
 __global__ __launch_bounds__(NT) void k_segment_sort(const int32_t* __restrict__ spl, float* key, int32_t* val,
                                                      const float* key_in, const int32_t* val_in, int64_t nmax,
                                                      int64_t nitems, const int32_t* __restrict__ queue) {
-  __shared__ double s_a[CAP];
+  __shared__ P s_a[CAP];
   const int64_t nseg = queue ? (int64_t)queue[0] : active_items(spl, nitems);
   for (int64_t it = blockIdx.x; it < nseg; it += gridDim.x) {
     const int64_t seg = queue ? (int64_t)queue[1 + it] : it;
@@ -684,9 +699,9 @@ __global__ __launch_bounds__(NT) void k_segment_sort(const int32_t* __restrict__
     if (e - b <= LO || (!BIG && e - b > CAP)) continue;
     const int len = (int)(e - b);
     if (len <= CAP) {
-      for (int i = threadIdx.x; i < len; i += NT) s_a[i] = kv_pack(key_in[b + i], val_in[b + i]);
+      for (int i = threadIdx.x; i < len; i += NT) s_a[i] = kv_pack<P>(key_in[b + i], val_in[b + i]);
       __syncthreads();
-      bitonic_sort_asc(LdsArr{s_a}, len);
+      bitonic_sort_asc(LdsArr<P>{s_a}, len);
       for (int i = threadIdx.x; i < len; i += NT) {
         key[b + i] = kv_key(s_a[i]);
         val[b + i] = kv_val(s_a[i]);
@@ -699,7 +714,7 @@ __global__ __launch_bounds__(NT) void k_segment_sort(const int32_t* __restrict__
         }
         __syncthreads();
       }
-      bitonic_sort_asc(GlobalKV{key + b, val + b}, len);
+      bitonic_sort_asc(GlobalKV<P>{key + b, val + b}, len);
     }
     __syncthreads();  // the next segment reuses s_a
   }
@@ -1017,22 +1032,23 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(W))) void k_
 // has no more than max_len entries, so kernels for longer ones than that are not launched.  Lists of 4096
 // to 16384 entries (the nodes around a void; 200 of 548,000 at 2^24, leaf 48) are sorted in 128 KB of LDS:
 // in global memory they took 3.1 ms together, 0.9 now.
+template <typename P>
 int segment_sort(hipStream_t s, const int32_t* spl, float* key, int32_t* val, const float* key_in,
                  const int32_t* val_in, int64_t nseg, int64_t nmax, int64_t max_len, int32_t* queue, const char* what) {
   if (nseg <= 0) return 0;
   if (queue && max_len > kWaveSortMax && fill_u32(s, queue, 0u, 1)) return 1;
   // four times the waves that the chip holds: workgroups stride over the segments
   const unsigned gw = (unsigned)(nseg < 32768 ? nseg : 32768);
-  hipLaunchKernelGGL(k_segment_sort_wave, dim3(gw), dim3(64), 0, s, spl, key, val, key_in, val_in, nmax, nseg,
+  hipLaunchKernelGGL(k_segment_sort_wave<P>, dim3(gw), dim3(64), 0, s, spl, key, val, key_in, val_in, nmax, nseg,
                      max_len > kWaveSortMax ? queue : nullptr);
   if (check_launch(what)) return 1;
   // the kernels touch disjoint segments; without a queue their workgroups go over all of them
   if (max_len > kWaveSortMax)
-    hipLaunchKernelGGL((k_segment_sort<kSegThreads, kWaveSortMax, kSegLds, false>),
+    hipLaunchKernelGGL((k_segment_sort<P, kSegThreads, kWaveSortMax, kSegLds, false>),
                        dim3((unsigned)(nseg < 4096 ? nseg : 4096)), dim3(kSegThreads), 0, s, spl, key, val, key_in,
                        val_in, nmax, nseg, queue);
   if (max_len > kSegLds)
-    hipLaunchKernelGGL((k_segment_sort<kSegBigThreads, kSegLds, kSegBigLds, true>),
+    hipLaunchKernelGGL((k_segment_sort<P, kSegBigThreads, kSegLds, kSegBigLds, true>),
                        dim3((unsigned)(nseg < 1024 ? nseg : 1024)), dim3(kSegBigThreads), 0, s, spl, key, val, key_in,
                        val_in, nmax, nseg, queue);
   return check_launch(what);
@@ -1214,7 +1230,7 @@ int node2node_impl(hipStream_t s, const int32_t* pil_spl, const int32_t* pil_src
   // (a list names every node at most once)
   const size_t qoff = align256(4 * (size_t)node_queue_words(size_parents));
   int32_t* sq = tmp && tmp_bytes >= qoff + 4 * (size_t)seg_queue_words(il_size) ? (int32_t*)((char*)tmp + qoff) : nullptr;
-  return segment_sort(s, il_spl, il_r2, il_src, il_r2, il_src, size_nodes, il_size, size_nodes, sq, "KnnNode2Node sort");
+  return segment_sort<double>(s, il_spl, il_r2, il_src, il_r2, il_src, size_nodes, il_size, size_nodes, sq, "KnnNode2Node sort");
 }
 
 template <int D>
@@ -1366,7 +1382,7 @@ extern "C" int jzt_dense_ilist_r2(jzt_stream_t stream, const void* nodes, int64_
   if (check_launch("DenseIlistR2")) return 1;
   if (!r2) return 0;
   // rows past the last super-node are empty
-  return segment_sort(s, ispl, r2, ilist, r2, ilist, size_super, size_ilist, size_super, nullptr, "DenseIlistR2 sort");
+  return segment_sort<double>(s, ispl, r2, ilist, r2, ilist, size_super, size_ilist, size_super, nullptr, "DenseIlistR2 sort");
 }
 
 extern "C" int jzt_segment_max_f32(jzt_stream_t stream, const int32_t* spl, const float* vals, int64_t nvals,
@@ -1463,6 +1479,6 @@ extern "C" int jzt_segment_sort(jzt_stream_t stream, const int32_t* spl, const f
                                 float* key_out, int32_t* val_out, int64_t size_segs, int64_t size_keys) {
   hipStream_t s = (hipStream_t)stream;
   if (size_segs <= 0) return 0;
-  return segment_sort(s, spl, key_out, val_out, key, val, size_segs, size_keys, size_keys, nullptr,
+  return segment_sort<uint64_t>(s, spl, key_out, val_out, key, val, size_segs, size_keys, size_keys, nullptr,
                       "SegmentSort");
 }

@@ -39,6 +39,30 @@ def test_segment_sort_lengths(dev, lens):
         assert np.array_equal(ko[a:b], key[a:b][o]) and np.array_equal(vo[a:b], val[a:b][o]), (a, b)
 
 
+@pytest.mark.parametrize("lens", [[3, 64, 65, 300, 1000, 1024], [1500, 5000, 17000]])
+def test_segment_sort_any_key_bits(dev, lens):
+    """Keys of every bit pattern, NaN ones and both zeros among them, in the float total order (by val among
+    equal ones): every pair comes out once."""
+    import jztree_amd._lib as L
+    rng = np.random.default_rng(sum(lens))
+    n = sum(lens)
+    bits = rng.integers(0, 1 << 32, size=n, dtype=np.uint64).astype(np.uint32)
+    bits[::5] = rng.integers(0x7f800000, 0x80000000, size=len(bits[::5]), dtype=np.uint64).astype(np.uint32)
+    bits[1::5] = rng.integers(0xff800000, 1 << 32, size=len(bits[1::5]), dtype=np.uint64).astype(np.uint32)
+    bits[::7], bits[1::7] = 0, 0x80000000
+    bits[2::7], bits[3::7] = 0xffffffff, 0x7fffffff
+    val = rng.integers(-2, 2, size=n).astype(np.int32)
+    spl = np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)
+    t = [torch.from_numpy(a).to(dev) for a in (spl, bits.view(np.float32), val)]
+    ko, vo = torch.empty_like(t[1]), torch.empty_like(t[2])
+    L.call("jzt_segment_sort", L.stream(), L.ptr(t[0]), L.ptr(t[1]), L.ptr(t[2]), L.ptr(ko), L.ptr(vo), len(lens), n)
+    ko, vo = ko.cpu().numpy().view(np.uint32), vo.cpu().numpy()
+    order = np.where(bits >> 31, ~bits, bits | np.uint32(0x80000000))
+    for a, b in zip(spl[:-1], spl[1:]):
+        o = np.lexsort((val[a:b].view(np.uint32), order[a:b]))
+        assert np.array_equal(ko[a:b], bits[a:b][o]) and np.array_equal(vo[a:b], val[a:b][o]), (a, b)
+
+
 def _half_ext(lvl, dim):
     o = (lvl + 2000 * dim) // dim - 2000
     r = lvl - o * dim
