@@ -11,7 +11,8 @@
 //      the first pass reads no indices)
 //   5. finish: pos_out = pos_in[idx], id_out = idx; members of a short run of equal keys write to
 //      their place by the exact comparator                                   (r12+12 w12+4 B/pt)
-//   6. long runs of equal keys, sorted and written by a workgroup each (rare)
+//   6. long runs of equal keys whose points differ below the key, sorted and written by a workgroup
+//      each (rare)
 //
 // Key construction.  For coordinates whose largest finite exponent is Lt, each dim contributes a
 // B-bit code (B = 63/dim, i.e. 21 for 3D): the fixed-point bits of |x| at levels Lt-B+1 .. Lt.
@@ -497,46 +498,62 @@ __device__ __forceinline__ void finish_row(const T* __restrict__ pos, uint32_t v
 }
 
 // One row per thread.  A row whose key no neighbour has goes where it stands; the members of a run of
-// up to kShortRun equal keys (of the same set, with setk) each count those before them; the starts of
-// longer runs are listed for k_long_runs.  Bound by the random reads of pos (a cache line for every
-// 12 or 24 bytes).  Flags, compaction, fix-up and gather as steps of their own took 6 launches and
-// wrote and read a flag per row: 120 us instead of 95 at 4.2e6 points.
+// up to kShortRun equal keys (of the same set, with setk) each count those before them.  The members of a
+// longer run go where they stand too: the passes are stable, so copies of a point and NaN rows are in
+// order; a member that is not after the one before it lists the run's start, once, for k_long_runs (the
+// mark is a bit of its value: values are below 2^30).  With all members left to that kernel, one workgroup
+// copied the run: 2^24 points in two places 73 ms, a third of them NaN 48; now 1.65 and 1.61, as when
+// all are apart.
+// Bound by the random reads of pos (a cache line for every 12 or 24 bytes).  Flags, compaction, fix-up and
+// gather as steps of their own took 6 launches and wrote and read a flag per row: 120 us instead of 95 at
+// 4.2e6 points.
 constexpr int kShortRun = 16;
+constexpr uint32_t kListed = 1u << 31;
 
 // low: bits of the keys that the rows are not sorted by (runs are equal in the bits above them).
 template <int D, typename T>
-__device__ __forceinline__ void finish_at(int64_t i, int low, const uint64_t* keys, const uint32_t* vals,
+__device__ __forceinline__ void finish_at(int64_t i, int low, const uint64_t* keys, uint32_t* vals,
                                           const int32_t* __restrict__ setk, int64_t n, const T* __restrict__ pos,
                                           T* __restrict__ pos_out, typename IntOf<T>::type* __restrict__ id_out,
                                           int32_t* __restrict__ runs, int32_t* nruns, int64_t max_runs) {
   const uint64_t k = keys[i];
   const int32_t sk = setk ? setk[i] : 0;
   auto same = [&](int64_t j) { return (keys[j] ^ k) >> low == 0 && (!setk || setk[j] == sk); };
-  const uint32_t v = vals[i];
+  const uint32_t v = vals[i] & ~kListed;
   int64_t dst = i;
   const bool prev = i > 0 && same(i - 1), next = i + 1 < n && same(i + 1);
   if (prev || next) {
-    int64_t a = i, b = i + 1;  // the run is [a, b), looked at up to kShortRun rows either way
-    while (a > 0 && i - a < kShortRun && same(a - 1)) a--;
-    while (b < n && b - i <= kShortRun && same(b)) b++;
-    if (b - a > kShortRun) {
-      if (!prev) {
-        const int32_t at = atomicAdd(nruns, 1);
-        if (at < max_runs) runs[at] = (int32_t)i;
-      }
-      return;
+    int64_t a = i, b = i + 1;  // the run is [a, b)
+    bool is_long = (i >= kShortRun && same(i - kShortRun)) || (i + kShortRun < n && same(i + kShortRun));
+    if (!is_long) {
+      while (a > 0 && same(a - 1)) a--;
+      while (b < n && same(b)) b++;
+      is_long = b - a > kShortRun;
     }
-    dst = a;
-    for (int64_t j = a; j < b; j++) {
-      const uint64_t kj = keys[j];
-      dst += kj < k || (kj == k && j != i && idx_less<D, T>(pos, vals[j], v));
+    if (!is_long) {
+      dst = a;
+      for (int64_t j = a; j < b; j++) {
+        const uint64_t kj = keys[j];
+        dst += kj < k || (kj == k && j != i && idx_less<D, T>(pos, vals[j], v));
+      }
+    } else if (prev && idx_less<D, T>(pos, v, vals[i - 1] & ~kListed)) {
+      int64_t lo = 0, hi = i - 1;  // the run's start: rows with the same key are consecutive
+      while (lo < hi) {
+        const int64_t mid = (lo + hi) >> 1;
+        if (same(mid)) hi = mid;
+        else lo = mid + 1;
+      }
+      if (!(ld_acq(&vals[lo]) & kListed) && !(atomicOr(&vals[lo], kListed) & kListed)) {
+        const int32_t at = atomicAdd(nruns, 1);
+        if (at < max_runs) runs[at] = (int32_t)lo;
+      }
     }
   }
   finish_row<D, T>(pos, v, dst, n, pos_out, id_out);
 }
 
 template <int D, typename T>
-__global__ __launch_bounds__(256) void k_finish(const uint64_t* __restrict__ keys, const uint32_t* __restrict__ vals,
+__global__ __launch_bounds__(256) void k_finish(const uint64_t* __restrict__ keys, uint32_t* vals,
                                                 const int32_t* __restrict__ setk, int64_t n,
                                                 const T* __restrict__ pos, T* __restrict__ pos_out,
                                                 typename IntOf<T>::type* __restrict__ id_out,
@@ -545,10 +562,9 @@ __global__ __launch_bounds__(256) void k_finish(const uint64_t* __restrict__ key
   if (i < n) finish_at<D, T>(i, 0, keys, vals, setk, n, pos, pos_out, id_out, runs, nruns, max_runs);
 }
 
-// One workgroup per listed run (grid-stride over the list).  The run's end is found by
-// a strided parallel search, sortedness by (exact order, index) is checked pairwise, and unsorted
-// runs are put in order by a bitonic network (ascending comparators only, so any length works)
-// applied in place to the run's indices in global memory.
+// One workgroup per listed run (grid-stride over the list).  The run's end is found by a strided
+// parallel search, and the run is put in order by a bitonic network (ascending comparators only, so any
+// length works) applied in place to its indices in global memory.
 template <int D, typename T>
 __global__ __launch_bounds__(256) void k_long_runs(const uint64_t* __restrict__ keys, uint32_t* vals, int64_t n,
                                                    const T* __restrict__ pos, T* __restrict__ pos_out,
@@ -561,7 +577,10 @@ __global__ __launch_bounds__(256) void k_long_runs(const uint64_t* __restrict__ 
   for (int64_t r = blockIdx.x; r < nruns; r += gridDim.x) {
     const int64_t start = runs[r];
     const uint64_t k = keys[start];
-    if (threadIdx.x == 0) s_end = (unsigned long long)n;
+    if (threadIdx.x == 0) {
+      s_end = (unsigned long long)n;
+      vals[start] &= ~kListed;
+    }
     __syncthreads();
     const int32_t sk = setk ? setk[start] : 0;
     for (int64_t j = start + 1 + threadIdx.x; j < n; j += blockDim.x) {
@@ -572,18 +591,27 @@ __global__ __launch_bounds__(256) void k_long_runs(const uint64_t* __restrict__ 
     }
     __syncthreads();
     const int64_t end = (int64_t)s_end;
-    bool bad = false;
-    for (int64_t j = start + threadIdx.x; j + 1 < end; j += blockDim.x)
-      bad |= !idx_less<D, T>(pos, vals[j], vals[j + 1]);
-    if (__syncthreads_or(bad)) {
-      const int64_t len = end - start;
-      uint32_t* a = vals + start;
-      int64_t np2 = 1;
-      while (np2 < len) np2 <<= 1;
-      for (int64_t size = 2; size <= np2; size <<= 1) {
+    const int64_t len = end - start;
+    uint32_t* a = vals + start;
+    int64_t np2 = 1;
+    while (np2 < len) np2 <<= 1;
+    for (int64_t size = 2; size <= np2; size <<= 1) {
+      for (int64_t t = threadIdx.x; t < np2 / 2; t += blockDim.x) {
+        int64_t blk = t / (size / 2), off = t % (size / 2);
+        int64_t i = blk * size + off, j = blk * size + size - 1 - off;
+        if (j < len) {
+          uint32_t x = a[i], y = a[j];
+          if (idx_less<D, T>(pos, y, x)) {
+            a[i] = y;
+            a[j] = x;
+          }
+        }
+      }
+      __syncthreads();
+      for (int64_t stride = size / 4; stride > 0; stride >>= 1) {
         for (int64_t t = threadIdx.x; t < np2 / 2; t += blockDim.x) {
-          int64_t blk = t / (size / 2), off = t % (size / 2);
-          int64_t i = blk * size + off, j = blk * size + size - 1 - off;
+          int64_t blk = t / stride, off = t % stride;
+          int64_t i = blk * 2 * stride + off, j = i + stride;
           if (j < len) {
             uint32_t x = a[i], y = a[j];
             if (idx_less<D, T>(pos, y, x)) {
@@ -593,20 +621,6 @@ __global__ __launch_bounds__(256) void k_long_runs(const uint64_t* __restrict__ 
           }
         }
         __syncthreads();
-        for (int64_t stride = size / 4; stride > 0; stride >>= 1) {
-          for (int64_t t = threadIdx.x; t < np2 / 2; t += blockDim.x) {
-            int64_t blk = t / stride, off = t % stride;
-            int64_t i = blk * 2 * stride + off, j = i + stride;
-            if (j < len) {
-              uint32_t x = a[i], y = a[j];
-              if (idx_less<D, T>(pos, y, x)) {
-                a[i] = y;
-                a[j] = x;
-              }
-            }
-          }
-          __syncthreads();
-        }
       }
     }
     for (int64_t j = start + threadIdx.x; j < end; j += blockDim.x)

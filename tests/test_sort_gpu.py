@@ -202,3 +202,46 @@ def test_zsort_small_nan_rows_next_to_the_top_corner(dev, oracle, dim, dtype, n,
     _, _, th = jz.tree.zsort_and_tree_origin(torch.from_numpy(x).to(dev), jz.config.TreeConfig(alloc_fac_nodes=2.))
     jz.checks.flush()
     assert int(th.splits_leaf_to_part(0).max()) == n - few
+
+
+def _runs_set(rng, n, dim, dtype):
+    """n rows in random order: runs of equal keys around the length that one thread per row orders (16) and far
+    beyond, as copies of a point and as points that differ below the key's resolution, NaN rows, and
+    single points."""
+    parts = [np.full((1, dim), 1e6), np.full((n // 5, dim), np.nan)]
+    for length in (2, 15, 16, 17, 18, 33, 300, 1500):
+        for _ in range(2):
+            c = rng.random(dim)
+            parts.append(np.repeat(c[None], length, 0))
+            parts.append(c + 1e-3 * rng.random((length, dim)))
+            mixed = c + 1e-3 * rng.random((length, dim))  # copies and others in one run
+            parts.append(mixed[rng.integers(0, min(3, length), length)])
+    x = np.concatenate(parts)
+    x = np.concatenate([x, rng.random((n - len(x), dim))])
+    return np.ascontiguousarray(x[rng.permutation(n)].astype(dtype))
+
+
+@pytest.mark.parametrize("dtype,dim", [(np.float32, 3), (np.float64, 3), (np.float32, 2), (np.float32, 5)])
+@pytest.mark.parametrize("n", [16000, 20011, 150001])
+def test_zsort_long_runs(dev, oracle, dtype, dim, n):
+    """Long runs by one workgroup (n <= 16384) and by the passes over many."""
+    x = _runs_set(np.random.default_rng(n), n, dim, dtype)
+    pz, idz = _gpu_zsort(x, dev)
+    opz, oidz = oracle.zsort(x)
+    assert np.array_equal(idz, oidz) and np.array_equal(pz, opz, equal_nan=True)
+
+
+@pytest.mark.parametrize("sizes", [[13000, 5, 14001, 1, 16000], [13000] * 3 + [1] * 300])
+def test_zsort_sets_long_runs(dev, oracle, sizes):
+    """The same runs in a batch, the same points in several sets: a run ends where its set does."""
+    import jztree_amd as jz
+    one = _runs_set(np.random.default_rng(3), 16000, 3, np.float32)
+    x = np.concatenate([one[:s] for s in sizes])
+    off = np.concatenate([[0], np.cumsum(sizes)])
+    print(f"[zsort sets] {len(sizes)} sets, {len(x)} rows", flush=True)
+    pz, idz = jz.batch.zsort_sets(torch.from_numpy(x).to(dev), jz.batch.set_offsets(sizes, dev))
+    pz, idz = pz.cpu().numpy(), idz.cpu().numpy()
+    for a, b in zip(off[:-1], off[1:]):
+        _, oidz = oracle.zsort(x[a:b])
+        assert np.array_equal(idz[a:b] - a, oidz), (a, b)
+    assert np.array_equal(pz, x[idz], equal_nan=True)
