@@ -101,3 +101,21 @@ def test_build_overflow_is_reported(dev):
     ok = jz.config.KNNConfig(alloc_fac_ilist=1024., tree=dataclasses.replace(cfg, alloc_fac_nodes=8.))
     r, _ = jz.knn.knn(x, 8, cfg=ok)  # usable after
     assert torch.isfinite(r).all()
+
+
+@pytest.mark.parametrize("dim,dtype", [(3, torch.float32), (2, torch.float64)])
+@pytest.mark.parametrize("n", [16384, 16385, 200_003])
+@pytest.mark.parametrize("tail", [0, 1, 300, 0.6])
+def test_points_of_padded_positions(dev, n, dim, dtype, tail):
+    """Points of a set whose last rows in z-order hold NaN: those with a NaN first coordinate are padding."""
+    import jztree_amd as jz
+    g = torch.Generator(device=dev).manual_seed(n)
+    x = torch.rand((n, dim), generator=g, dtype=dtype, device=dev)
+    m = tail if tail >= 1 else int(tail * n)
+    x[:m] = float("nan")
+    x[:m:5, 0] = 0.5  # a NaN in other coordinates only: a point
+    posz, _ = jz.tree.zsort(x[torch.randperm(n, generator=g, device=dev)])
+    print(f"[tail] n={n} dim={dim} {dtype} tail={m}", flush=True)
+    th = jz.tree.build_tree_hierarchy(posz, jz.config.TreeConfig(max_leaf_size=48, alloc_fac_nodes=3.))
+    jz.checks.flush()
+    assert int(th.splits_leaf_to_part(0).max()) == int((~torch.isnan(x[:, 0])).sum())
