@@ -510,7 +510,8 @@ __device__ __forceinline__ void finish_row(const T* __restrict__ pos, uint32_t v
 constexpr int kShortRun = 16;
 constexpr uint32_t kListed = 1u << 31;
 
-// low: bits of the keys that the rows are not sorted by (runs are equal in the bits above them).
+// low: bits of the keys that the rows are not sorted by, but in runs of more than kShortRun rows that are
+// equal in the bits above them.
 template <int D, typename T>
 __device__ __forceinline__ void finish_at(int64_t i, int low, const uint64_t* keys, uint32_t* vals,
                                           const int32_t* __restrict__ setk, int64_t n, const T* __restrict__ pos,
@@ -520,33 +521,38 @@ __device__ __forceinline__ void finish_at(int64_t i, int low, const uint64_t* ke
   const int32_t sk = setk ? setk[i] : 0;
   auto same = [&](int64_t j) { return (keys[j] ^ k) >> low == 0 && (!setk || setk[j] == sk); };
   const uint32_t v = vals[i] & ~kListed;
-  int64_t dst = i;
-  const bool prev = i > 0 && same(i - 1), next = i + 1 < n && same(i + 1);
-  if (prev || next) {
-    int64_t a = i, b = i + 1;  // the run is [a, b)
-    bool is_long = (i >= kShortRun && same(i - kShortRun)) || (i + kShortRun < n && same(i + kShortRun));
-    if (!is_long) {
-      while (a > 0 && same(a - 1)) a--;
-      while (b < n && same(b)) b++;
-      is_long = b - a > kShortRun;
+  int64_t dst = i, a, b;  // the run is [a, b)
+  auto find_run = [&]() -> bool {
+    a = i;
+    b = i + 1;
+    if (!(i > 0 && same(i - 1)) && !(i + 1 < n && same(i + 1))) return true;
+    if ((i >= kShortRun && same(i - kShortRun)) || (i + kShortRun < n && same(i + kShortRun))) return false;
+    while (a > 0 && same(a - 1)) a--;
+    while (b < n && same(b)) b++;
+    return b - a <= kShortRun;
+  };
+  bool is_short = find_run();
+  if (!is_short && low) {
+    low = 0;
+    is_short = find_run();
+  }
+  if (is_short) {
+    dst = a;
+    for (int64_t j = a; j < b; j++) {
+      if (j == i) continue;
+      const uint64_t kj = keys[j];
+      dst += kj < k || (kj == k && idx_less<D, T>(pos, vals[j], v));
     }
-    if (!is_long) {
-      dst = a;
-      for (int64_t j = a; j < b; j++) {
-        const uint64_t kj = keys[j];
-        dst += kj < k || (kj == k && j != i && idx_less<D, T>(pos, vals[j], v));
-      }
-    } else if (prev && idx_less<D, T>(pos, v, vals[i - 1] & ~kListed)) {
-      int64_t lo = 0, hi = i - 1;  // the run's start: rows with the same key are consecutive
-      while (lo < hi) {
-        const int64_t mid = (lo + hi) >> 1;
-        if (same(mid)) hi = mid;
-        else lo = mid + 1;
-      }
-      if (!(ld_acq(&vals[lo]) & kListed) && !(atomicOr(&vals[lo], kListed) & kListed)) {
-        const int32_t at = atomicAdd(nruns, 1);
-        if (at < max_runs) runs[at] = (int32_t)lo;
-      }
+  } else if (i > 0 && same(i - 1) && idx_less<D, T>(pos, v, vals[i - 1] & ~kListed)) {
+    int64_t lo = 0, hi = i - 1;  // the run's start: rows with the same key are consecutive
+    while (lo < hi) {
+      const int64_t mid = (lo + hi) >> 1;
+      if (same(mid)) hi = mid;
+      else lo = mid + 1;
+    }
+    if (!(ld_acq(&vals[lo]) & kListed) && !(atomicOr(&vals[lo], kListed) & kListed)) {
+      const int32_t at = atomicAdd(nruns, 1);
+      if (at < max_runs) runs[at] = (int32_t)lo;
     }
   }
   finish_row<D, T>(pos, v, dst, n, pos_out, id_out);
@@ -651,14 +657,21 @@ int finish(hipStream_t s, const uint64_t* keys, uint32_t* vals, const int32_t* s
 // ---------------------------------------------------------------------------------------------
 // Steps 1 to 5 for up to kSmallSort points: keys and indices in registers (a wave's are consecutive, so
 // the passes are stable), exchanged through LDS pass by pass.  Small sorts are bound by their
-// launches; one workgroup is bound by the ranking (8 ballots a key and pass).  A sort alone, us, by one
-// workgroup / over many: 1000 points 23 / 59, 4096 42 / 62, 8192 68 / 70, 16,384 120 / 80.  In a call
-// that goes on to build the tree, the 12 launches saved are worth another 50 us (FoF of 12,800 points
-// 398 -> 350), which is where the limit comes from.  Other positions than the instantiated ones take
-// the passes over many workgroups at any size.
+// launches; one workgroup is bound by the ranking (8 ballots a key and pass).  Float 3-D points, us, by
+// one workgroup / over many, replayed from a graph and (eager call, with its host work):
+//   1000  29 / 63 (48 / 96)      4096  48 / 78 (66 / 111)      8192  73 / 81 (92 / 111)
+//   10,240  89 / 82 (107 / 113)  12,288  102 / 83 (121 / 115)  16,384  129 / 83 (148 / 116)
+// kSmallAlone is where a sort by itself stops gaining.  A call that goes on to build a tree keeps its host
+// ahead with fewer launches (FoF of 12,800 points 460 us eager by one workgroup, 500 over many) and asks for
+// kSmallSort (few_launches).
+// Five passes sort by the top 40 bits, which part the points of nearly every set this small, up to short
+// runs and runs that stand in order (copies, NaN rows); others take all eight passes, at once if a sample
+// shows such a run, else after the five.  8192 points, eager: one far outlier 170 us (123 over many, 207
+// with thirteen passes), a clump of 40 points 126 or 180, a third NaN 91 (173 when that took thirteen).
+// Other positions than the instantiated ones take the passes over many workgroups at any size.
 constexpr int kSmallThreads = 1024;
 constexpr int kSmallKeys = 16;  // a thread's
-constexpr int64_t kSmallSort = kSmallThreads * kSmallKeys;
+constexpr int64_t kSmallSort = kSmallThreads * kSmallKeys, kSmallAlone = kSmallSort / 2;
 template <int D, typename T> constexpr bool kHasSmallSort = D <= 3 && std::is_floating_point<T>::value;
 
 template <int D, typename T>
@@ -775,15 +788,36 @@ __global__ __launch_bounds__(kSmallThreads) void k_small_sort(const T* __restric
     }
     __syncthreads();
   };
-  // The top 40 bits part the points of nearly every set this small, up to short runs.  Bit 63 is one of
-  // them: it is all that tells a NaN row (~0) from a point in the top corner of a non-negative 3-D set.
+  // Bit 63 is among the top 40: it is all that tells a NaN row (~0) from a point in the top corner of a
+  // non-negative 3-D set.
   int low = 24;
+  {  // rows that only the lower bits part, among the first of every wave's: long runs are likely
+    const uint32_t hi = (uint32_t)(key[0] >> 32), lo = (uint32_t)key[0];
+    bool met = false;
+#pragma unroll
+    for (int l = 0; l < 64; l += 4) {
+      const uint32_t h = hi ^ (uint32_t)__builtin_amdgcn_readlane((int)hi, l);
+      const uint32_t w = lo ^ (uint32_t)__builtin_amdgcn_readlane((int)lo, l);
+      met |= h == 0 && w - 1u < (1u << low) - 1u;
+    }
+    if (__syncthreads_or(met)) low = 0;
+  }
 #pragma unroll 1
   while (true) {
     sort_from(low);
-    bool is_long = false;
-    for (int i = tid; i + kShortRun < n; i += kSmallThreads) is_long |= (keys[i] ^ keys[i + kShortRun]) >> low == 0;
-    if (low == 0 || !__syncthreads_or(is_long)) break;
+    if (low == 0) break;
+    // a row of a longer run whose key is not after the one before it (rows of one key are in order)
+    bool again = false;
+    for (int i = tid + 1; i < n; i += kSmallThreads) {
+      auto same = [&](int j) { return j >= 0 && j < n && (keys[j] ^ keys[i]) >> low == 0; };
+      if (keys[i] < keys[i - 1] && same(i - 1)) {
+        int a = i - 1, b = i + 1;
+        while (b - a <= kShortRun && same(a - 1)) a--;
+        while (b - a <= kShortRun && same(b)) b++;
+        again |= b - a > kShortRun;
+      }
+    }
+    if (!__syncthreads_or(again)) break;
     low = 0;
   }
   for (int i = tid; i < n; i += kSmallThreads)
@@ -850,7 +884,8 @@ SortLayout sort_layout(int64_t n, int dim, int dtype) {
 }
 
 template <int D, typename T>
-int zsort_impl(hipStream_t s, const T* pos_in, T* pos_out, typename IntOf<T>::type* id_out, char* tmp, int64_t n) {
+int zsort_impl(hipStream_t s, const T* pos_in, T* pos_out, typename IntOf<T>::type* id_out, char* tmp, int64_t n,
+               bool few_launches) {
   SortLayout L = sort_layout(n, D, sizeof(T) == 8 ? JZT_F64 : JZT_F32);
   uint64_t* k0 = (uint64_t*)(tmp + L.keys0);
   uint64_t* k1 = (uint64_t*)(tmp + L.keys1);
@@ -867,7 +902,7 @@ int zsort_impl(hipStream_t s, const T* pos_in, T* pos_out, typename IntOf<T>::ty
     src = cp;
   }
   if constexpr (kHasSmallSort<D, T>) {
-    if (n <= kSmallSort) {
+    if (n <= (few_launches ? kSmallSort : kSmallAlone)) {
       int32_t* runs = (int32_t*)(tmp + L.runs);
       hipLaunchKernelGGL((k_small_sort<D, T>), dim3(1), dim3(kSmallThreads), 0, s, src, (int)n, k0, v0, pos_out, id_out,
                          runs, (int32_t*)meta + 4);
@@ -1382,8 +1417,8 @@ extern "C" int jzt_fof_order(jzt_stream_t stream, const int32_t* igroup, const i
 
 extern "C" size_t jzt_zsort_tmp_bytes(int64_t n, int dim, int dtype) { return sort_layout(n, dim, dtype).total; }
 
-extern "C" int jzt_pos_zorder_sort(jzt_stream_t stream, const void* pos_in, void* pos_out, void* id_out, void* tmp,
-                                   size_t tmp_bytes, int64_t n, int dim, int dtype) {
+extern "C" int jzt_pos_zorder_sort_ex(jzt_stream_t stream, const void* pos_in, void* pos_out, void* id_out, void* tmp,
+                                      size_t tmp_bytes, int64_t n, int dim, int dtype, int few_launches) {
   hipStream_t s = (hipStream_t)stream;
   if (n < 0) return fail("jzt_pos_zorder_sort: negative n");
   if (n == 0) return 0;
@@ -1393,17 +1428,18 @@ extern "C" int jzt_pos_zorder_sort(jzt_stream_t stream, const void* pos_in, void
     return fail("jzt_pos_zorder_sort: tmp buffer too small (have " + std::to_string(tmp_bytes) + ", need " +
                 std::to_string(need) + ")");
   char* t = (char*)tmp;
+  const bool few = few_launches != 0;
   // dims 2-10, as the reference instantiates PosZorderSort (_generate_ffi.py:9-21)
 #define JZT_ZS(D)                                                                                                \
   case D:                                                                                                        \
     switch (dtype) {                                                                                             \
-      case JZT_F32: return zsort_impl<D, float>(s, (const float*)pos_in, (float*)pos_out, (int32_t*)id_out, t, n); \
+      case JZT_F32: return zsort_impl<D, float>(s, (const float*)pos_in, (float*)pos_out, (int32_t*)id_out, t, n, few); \
       case JZT_F64:                                                                                              \
-        return zsort_impl<D, double>(s, (const double*)pos_in, (double*)pos_out, (int64_t*)id_out, t, n);        \
+        return zsort_impl<D, double>(s, (const double*)pos_in, (double*)pos_out, (int64_t*)id_out, t, n, few);   \
       case JZT_I32:                                                                                              \
-        return zsort_impl<D, int32_t>(s, (const int32_t*)pos_in, (int32_t*)pos_out, (int32_t*)id_out, t, n);     \
+        return zsort_impl<D, int32_t>(s, (const int32_t*)pos_in, (int32_t*)pos_out, (int32_t*)id_out, t, n, few); \
       default:                                                                                                   \
-        return zsort_impl<D, int64_t>(s, (const int64_t*)pos_in, (int64_t*)pos_out, (int64_t*)id_out, t, n);     \
+        return zsort_impl<D, int64_t>(s, (const int64_t*)pos_in, (int64_t*)pos_out, (int64_t*)id_out, t, n, few); \
     }
   if (dtype == JZT_F32 || dtype == JZT_F64 || dtype == JZT_I32 || dtype == JZT_I64) {
     switch (dim) {
@@ -1413,6 +1449,11 @@ extern "C" int jzt_pos_zorder_sort(jzt_stream_t stream, const void* pos_in, void
   }
 #undef JZT_ZS
   return fail("jzt_pos_zorder_sort: unsupported dim/dtype (dim " + std::to_string(dim) + ")");
+}
+
+extern "C" int jzt_pos_zorder_sort(jzt_stream_t stream, const void* pos_in, void* pos_out, void* id_out, void* tmp,
+                                   size_t tmp_bytes, int64_t n, int dim, int dtype) {
+  return jzt_pos_zorder_sort_ex(stream, pos_in, pos_out, id_out, tmp, tmp_bytes, n, dim, dtype, 0);
 }
 
 // ---------------------------------------------------------------------------------------------

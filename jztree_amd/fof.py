@@ -16,11 +16,11 @@ import torch
 
 from . import _lib as L
 from . import checks
-from .checks import raise_if
+from .checks import is_deferred, raise_if
 from .config import FofCatalogueConfig, FofConfig
 from .data import (FofCatalogue, InteractionList, PackedArray, TreeHierarchy, count_not_nan, get_pos,
                    tree_map_by_len, verify_ilist)
-from .tree import _tmp, build_tree_hierarchy, plane_tables, top_plane_lists, zsort
+from .tree import _tmp, _zsort, build_tree_hierarchy, plane_tables, top_plane_lists
 
 
 @dataclass
@@ -205,7 +205,7 @@ def fof_labels(part, rlink: float, boxsize: float = 0., cfg: FofConfig = FofConf
     kernels over the float64 tree (z-order from the float64 keys)."""
     try:
         if th is None:
-            partz, idz = zsort(part)
+            partz, idz = _zsort(part, not is_deferred())
             th = build_tree_hierarchy(partz, cfg_tree=cfg.tree)
         else:
             partz, idz = part, None

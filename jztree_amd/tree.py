@@ -15,7 +15,7 @@ import numpy as np
 import torch
 
 from . import _lib as L
-from .checks import raise_if
+from .checks import is_deferred, raise_if
 from .config import TreeConfig, RegularizationConfig
 from .data import (InteractionList, RankIdx, LevelInfo, PackedArray, Pos, TreeHierarchy, get_num, get_num_total, get_pos,
                    same_width_int, tree_map_by_len, verify_ilist)
@@ -50,7 +50,7 @@ def _tmp(nbytes: int, device) -> torch.Tensor:
 # z-order sort (tree.py:75-141)
 # ------------------------------------------------------------------------------------------------
 
-def _zsort_impl(x: torch.Tensor, block_size: int = 64):
+def _zsort_impl(x: torch.Tensor, block_size: int = 64, few_launches: bool = False):
     """tree.py:75-93 -> PosZorderSort."""
     assert x.ndim == 2
     n, dim = x.shape
@@ -63,7 +63,8 @@ def _zsort_impl(x: torch.Tensor, block_size: int = 64):
     dt = L.sort_dtype_code(x.dtype)
     nb = L.LIB.jzt_zsort_tmp_bytes(n, dim, dt)
     tmp = _tmp(nb, x.device)
-    L.call("jzt_pos_zorder_sort", L.stream(), L.ptr(x), L.ptr(pos), L.ptr(ids), L.ptr(tmp), nb, n, dim, dt)
+    L.call("jzt_pos_zorder_sort_ex", L.stream(), L.ptr(x), L.ptr(pos), L.ptr(ids), L.ptr(tmp), nb, n, dim, dt,
+           int(few_launches))
     return pos, ids
 
 
@@ -100,8 +101,8 @@ class _ZSort(torch.autograd.Function):
     """Custom VJP of tree.py:111-138: gradients scatter back through the inverse permutation."""
 
     @staticmethod
-    def forward(ctx, x):
-        pos, idz = _zsort_impl(x.detach())
+    def forward(ctx, x, few_launches):
+        pos, idz = _zsort_impl(x.detach(), few_launches=few_launches)
         ctx.save_for_backward(idz)
         ctx.mark_non_differentiable(idz)
         return pos, idz
@@ -110,10 +111,10 @@ class _ZSort(torch.autograd.Function):
     def backward(ctx, gpos, gidz):
         (idz,) = ctx.saved_tensors
         if _has_storage(gpos):
-            return _Unsort.apply(gpos, idz)
+            return _Unsort.apply(gpos, idz), None
         idinv = torch.zeros_like(idz)
         idinv[idz.long()] = torch.arange(len(idz), dtype=idz.dtype, device=idz.device)
-        return gpos[idinv.long()]
+        return gpos[idinv.long()], None
 
 
 def zsort(pos):
@@ -125,10 +126,15 @@ def zsort(pos):
     Returns:
         (posz, idz) with posz = pos[idz].
     """
+    return _zsort(pos, False)
+
+
+def _zsort(pos, few_launches: bool):
+    """zsort, with few_launches on behalf of an eager call that goes on to queue more work."""
     assert get_pos(pos).ndim == 2, "positions must have shape (N,3)"
     if torch.is_tensor(pos):
-        return _ZSort.apply(pos)
-    posz, idz = _ZSort.apply(pos.pos)
+        return _ZSort.apply(pos, few_launches)
+    posz, idz = _ZSort.apply(pos.pos, few_launches)
     out = tree_map_by_len(lambda v: v[idz.long()], pos, len(posz))
     try:
         out.pos = posz
@@ -588,7 +594,7 @@ def zsort_and_tree(part, cfg_tree: TreeConfig = TreeConfig(), data: Any | None =
     """tree.py:363-421 (single GPU): z-sort (carrying `data`) and build the hierarchy.
 
     Returns (partz, th), or (partz, dataz, th) when data is given."""
-    partz, isort = zsort(part)
+    partz, isort = _zsort(part, not is_deferred())
     dtz = tree_map_by_len(lambda v: v[isort.long()], (data, ptype), len(get_pos(partz)))
     th = build_tree_hierarchy(partz, cfg_tree, ptype=dtz[1], num_types=num_types)
     out = [partz]
@@ -678,7 +684,7 @@ def zsort_and_tree_origin(part, cfg_tree: TreeConfig = TreeConfig()):
     """zsort_and_tree(part, cfg_tree, data=RankIdx(rank=None, idx=arange(n) int32)), without the
     gather of the arange: its z-ordered copy is the sort permutation itself.
     Returns (partz, originz, th)."""
-    partz, isort = zsort(part)
+    partz, isort = _zsort(part, not is_deferred())
     th = build_tree_hierarchy(partz, cfg_tree)
     return partz, RankIdx(rank=None, idx=isort.to(torch.int32)), th
 

@@ -245,3 +245,33 @@ def test_zsort_sets_long_runs(dev, oracle, sizes):
         _, oidz = oracle.zsort(x[a:b])
         assert np.array_equal(idz[a:b] - a, oidz), (a, b)
     assert np.array_equal(pz, x[idz], equal_nan=True)
+
+
+def _lower_bits_sets(rng, n, dim):
+    """Sets for the one-workgroup sort whose top key bits leave runs of more than 16 rows: in order, out of order
+    by the lower bits, by less than the key, all but one row in one run, and a clump of few rows."""
+    x = rng.random((n, dim))
+    copies, near, below, far, clump = x.copy(), x.copy(), x.copy(), x.copy(), x.copy()
+    copies[:n // 3] = x[0]
+    copies[n // 3:n // 2] = x[1]
+    c = rng.random((max(n // 60, 1), dim))
+    near = (c[rng.integers(0, len(c), n)] + 1e-7 * rng.random((n, dim))) / 2
+    below = np.concatenate([c[rng.integers(0, len(c), n - 1)] + 1e-9 * rng.random((n - 1, dim)), [[1e3] * dim]])
+    far[n // 2] = 1e5
+    clump[n // 2:n // 2 + 40] = 0.3 + 1e-7 * rng.random((40, dim))
+    return dict(copies=copies, near=near, below=below, far=far, clump=clump)
+
+
+@pytest.mark.parametrize("kind", ["copies", "near", "below", "far", "clump"])
+@pytest.mark.parametrize("n", [100, 1025, 8192, 8193, 16384])
+def test_zsort_small_lower_bits(dev, oracle, kind, n):
+    """By itself (one workgroup up to 8192 rows) and for a call that asks for few launches (up to 16,384)."""
+    import jztree_amd as jz
+    for dim, dtype in ((3, np.float32), (3, np.float64), (2, np.float32)):
+        x = np.ascontiguousarray(_lower_bits_sets(np.random.default_rng(n), n, dim)[kind].astype(dtype))
+        _, oidz = oracle.zsort(x)
+        t = torch.from_numpy(x).to(dev)
+        for few in (False, True):
+            pz, idz = jz.tree._zsort(t, few)
+            assert np.array_equal(idz.cpu().numpy(), oidz), (dim, dtype, few)
+            assert np.array_equal(pz.cpu().numpy(), x[oidz]), (dim, dtype, few)
