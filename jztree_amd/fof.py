@@ -132,7 +132,7 @@ def _fof_dual_walk(th: TreeHierarchy, rlink: float, boxsize: float = 0., alloc_f
     size = th.size()
     tables = plane_tables(th)
     # beyond 2^-10 more than the linking length no pair of nodes is looked at (their own test allows 2^-16)
-    limit = None if r2link_set is not None else float(rlink) ** 2 * (1. + 2. ** -10)
+    limit = None if r2link_set is not None else _r2link(rlink) * (1. + 2. ** -10)
     spl, ilist = top_plane_lists(th, int(th.size_leaves * alloc_fac_ilist), tables, boxsize, r2_limit=limit)
     if r2link_set is not None:
         assert th.leaf_set is not None

@@ -97,3 +97,24 @@ def test_fof_float64(dev, boxsize):
         return np.array([first.setdefault(v, k) for k, v in enumerate(l)])
     assert np.array_equal(canon(lab), canon(comp))
     assert ncomp < len(x)
+
+
+@pytest.mark.parametrize("n", [300, 300_000])  # 300,000: enough leaves for distances in the dense list
+@pytest.mark.parametrize("rlink", [1e200, np.float16(1e-3), np.float16(0.5)])
+def test_fof_linking_length_of_any_size(dev, n, rlink):
+    """A length whose square overflows links everything; a half-precision length is squared as it is given."""
+    import jztree_amd as jz
+    import dataclasses
+    x = torch.from_numpy(np.random.default_rng(n).random((n, 3), dtype=np.float32)).to(dev)
+    if n > 300:  # few neighbours within the lengths below 1
+        x *= 20.
+    cfg = jz.config.FofConfig(alloc_fac_ilist=400.)
+    cfg = dataclasses.replace(cfg, tree=dataclasses.replace(cfg.tree, alloc_fac_nodes=2.))
+    with np.errstate(over="ignore"):
+        _, lab = jz.fof.fof_labels(x, rlink, cfg=cfg)
+        if rlink == 1e200:
+            assert not bool(lab.any())
+        else:
+            r = float(np.sqrt(np.float64(np.float32(rlink * rlink))))  # the float32 r2 that the call uses
+            _, ref = jz.fof.fof_labels(x, r, cfg=cfg)
+            assert torch.equal(lab, ref)
