@@ -69,12 +69,13 @@ def _zsort_impl(x: torch.Tensor, block_size: int = 64, few_launches: bool = Fals
 
 
 class _Unsort(torch.autograd.Function):
-    """Rows (n, width) of the sorted order back to input order: out[idz] = rows.  Linear in rows; its
-    gradient is the gather by idz, so gradients of any order work."""
+    """Rows (n, width) of the sorted order back to input order: out[idz] = rows.  Linear in rows: the
+    tangent goes the same way, and the gradient is the gather by idz, so gradients of any order work."""
 
     @staticmethod
     def forward(ctx, rows, idz):
         ctx.save_for_backward(idz)
+        ctx.save_for_forward(idz)
         n, width = rows.shape
         rows = rows.contiguous()
         out = torch.empty_like(rows)
@@ -86,6 +87,18 @@ class _Unsort(torch.autograd.Function):
     def backward(ctx, g):
         (idz,) = ctx.saved_tensors
         return g[idz.long()], None
+
+    @staticmethod
+    def jvp(ctx, t, _):
+        return _unsort(t, ctx.saved_tensors[0])
+
+
+def _unsort(rows, idz):
+    if _has_storage(rows):
+        return _Unsort.apply(rows, idz)
+    idinv = torch.zeros_like(idz)
+    idinv[idz.long()] = torch.arange(len(idz), dtype=idz.dtype, device=idz.device)
+    return rows[idinv.long()]
 
 
 def _has_storage(t: torch.Tensor) -> bool:
@@ -110,11 +123,7 @@ class _ZSort(torch.autograd.Function):
     @staticmethod
     def backward(ctx, gpos, gidz):
         (idz,) = ctx.saved_tensors
-        if _has_storage(gpos):
-            return _Unsort.apply(gpos, idz), None
-        idinv = torch.zeros_like(idz)
-        idinv[idz.long()] = torch.arange(len(idz), dtype=idz.dtype, device=idz.device)
-        return gpos[idinv.long()], None
+        return _unsort(gpos, idz), None
 
 
 def zsort(pos):

@@ -275,3 +275,23 @@ def test_zsort_small_lower_bits(dev, oracle, kind, n):
             pz, idz = jz.tree._zsort(t, few)
             assert np.array_equal(idz.cpu().numpy(), oidz), (dim, dtype, few)
             assert np.array_equal(pz.cpu().numpy(), x[oidz]), (dim, dtype, few)
+
+
+@pytest.mark.parametrize("dtype,dim", [(torch.float32, 3), (torch.float64, 2)])
+def test_zsort_gradient_forward_over_reverse(dev, dtype, dim):
+    """A gradient that carries a tangent: both come back in input order, also through saved-tensor hooks, and
+    batched."""
+    import torch.autograd.forward_ad as fw
+    import jztree_amd as jz
+    g = torch.Generator(device=dev).manual_seed(2)
+    x = torch.rand((1001, dim), dtype=dtype, device=dev, generator=g).requires_grad_()
+    w, t = (torch.randn((1001, dim), dtype=dtype, device=dev, generator=g) for _ in range(2))
+    with torch.autograd.graph.saved_tensors_hooks(lambda v: v.cpu(), lambda v: v.to(dev)):
+        posz, idz = jz.tree.zsort(x)
+    back = lambda v: torch.empty_like(v).index_copy_(0, idz.long(), v)
+    with fw.dual_level():
+        (gx,) = torch.autograd.grad(posz, x, fw.make_dual(w, t), retain_graph=True)
+        p, dp = fw.unpack_dual(gx)
+        assert torch.equal(p, back(w)) and torch.equal(dp, back(t))
+    (gb,) = torch.autograd.grad(posz, x, torch.stack([w, t]), is_grads_batched=True)
+    assert torch.equal(gb, torch.stack([back(w), back(t)]))
