@@ -75,7 +75,7 @@ def test_zsort_large_is_permutation_and_sorted(dev, oracle):
     assert all(oracle.z_exact_cmp(pz[i], pz[i + 1]) <= 0 for i in sample)
 
 
-def test_zsort_gradient(dev):
+def test_zsort_gradient_backward(dev):
     """custom VJP (tree.py:111-138): the gradient scatters back through the permutation."""
     import jztree_amd as jz
     x = torch.from_numpy(uniform(1000, seed=8)).to(dev).requires_grad_(True)
