@@ -573,7 +573,7 @@ int fof_node_impl(hipStream_t s, const int32_t* pil_spl, const int32_t* pil, con
                   int64_t pil_size, int64_t il_size, float r2link, const float* r2v, float boxsize, bool zero_list,
                   uint8_t* overflow) {
   const T* nd = (const T*)nodes;
-  if (size_parent <= 0 && overflow) return fail("FofNode2Node: no parents");
+  if (size_parent <= 0 && overflow && clear_flag(s, overflow)) return 1;  // empty lists
   if (fill_u32(s, il_spl, 0u, size_node + 1)) return 1;
   if (zero_list && fill_u32(s, il, 0u, il_size)) return 1;
   if (size_node >= INT32_MAX) return fail("FofNode2Node: too many nodes");

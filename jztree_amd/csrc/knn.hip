@@ -1191,7 +1191,7 @@ int node2node_impl(hipStream_t s, const int32_t* pil_spl, const int32_t* pil_src
   const T* nd = (const T*)nodes;
   if (fill_u32(s, il_spl, 0u, size_nodes + 1)) return 1;
   if (size_nodes >= INT32_MAX) return fail("KnnNode2Node: too many nodes");
-  if (size_parents <= 0) return overflow ? fail("KnnNode2Node: no parents") : 0;
+  if (size_parents <= 0) return overflow ? clear_flag(s, overflow) : 0;  // empty lists
   const dim3 g(node_grid(size_parents, 64)), b(64), gl(node_grid(size_parents, kNodeThreads)), bl(kNodeThreads);
   // without room for the queue, one-wave workgroups run the long lists too
   const bool split = tmp && tmp_bytes >= 4 * (size_t)node_queue_words(size_parents);

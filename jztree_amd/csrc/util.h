@@ -27,6 +27,7 @@ inline size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
 
 // fill n 32-bit words with v
 int fill_u32(hipStream_t s, void* p, uint32_t v, int64_t n);
+int clear_flag(hipStream_t s, uint8_t* p);
 
 // Stable compaction: out[j] = index of the j-th nonzero flag (j < size), remaining out = fill
 // (or *fill_dev when given);

@@ -36,6 +36,12 @@ int fill_u32(hipStream_t s, void* p, uint32_t v, int64_t n) {
   return check_launch("fill_u32");
 }
 
+__global__ void k_clear_flag(uint8_t* p) { *p = 0; }
+int clear_flag(hipStream_t s, uint8_t* p) {
+  hipLaunchKernelGGL(k_clear_flag, dim3(1), dim3(1), 0, s, p);
+  return check_launch("clear_flag");
+}
+
 // pass 1: per-tile sums
 __global__ __launch_bounds__(kScanThreads) void k_scan_reduce(const int32_t* __restrict__ in, int64_t n,
                                                               int32_t* __restrict__ tile_sums) {

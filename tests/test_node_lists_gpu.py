@@ -236,3 +236,20 @@ def test_dense_top_distances(dev, monkeypatch, n, dim, dtype, boxsize):
         out.append((rnn, inn, pz, ig))
     for a, b in zip(*out):
         assert torch.equal(a, b)
+
+
+def test_no_parents_give_empty_lists(dev):
+    """Nodes without parents: lists of no entries, labels as given, nothing raised."""
+    import jztree_amd as jz
+    from jztree_amd.data import InteractionList
+    from jztree_amd.fof import PosLvl, _fof_node2node
+    from jztree_amd.knn import PosLvlNum, _knn_node2node_ilist
+    i32 = lambda *v: torch.tensor(v, dtype=torch.int32, device=dev)
+    pos = torch.rand((5, 3), device=dev)
+    il = InteractionList(i32(0), torch.zeros(64, dtype=torch.int32, device=dev), rad2=torch.zeros(64, device=dev))
+    out = _knn_node2node_ilist(il, i32(0), PosLvlNum(pos=pos, lvl=i32(*[-12] * 5), npart=i32(*[1] * 5)), k=2)
+    assert out.ispl.tolist() == [0] * 6
+    ig, out = _fof_node2node(InteractionList(il.ispl, il.isrc), i32(0), PosLvl(pos=pos, lvl=i32(*[-12] * 5)),
+                             i32(0, 1, 2, 3, 4), rlink=0.1)
+    assert out.ispl.tolist() == [0] * 6 and ig.tolist() == [0, 1, 2, 3, 4]
+    jz.checks.flush()
