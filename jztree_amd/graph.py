@@ -15,13 +15,40 @@ tensors the callable closes over: copy new data into them (same shapes) between 
 """
 from __future__ import annotations
 
+import contextlib
 import gc
+import threading
 from typing import Any, Callable
 
 import torch
 
 from . import _lib as L
 from . import checks
+
+
+_gc_lock = threading.Lock()
+_gc_paused = 0       # captures under way, in all threads
+_gc_resume = False   # whether the last of them turns the collector on again
+
+
+@contextlib.contextmanager
+def _no_collection():
+    """No garbage collection until every thread has left this block; then as it was before the first
+    entered.  The collector is one for the process: a thread that restored what it had found would turn
+    it on under another one's capture, or leave it off."""
+    global _gc_paused, _gc_resume
+    with _gc_lock:
+        if _gc_paused == 0:
+            _gc_resume = gc.isenabled()
+            gc.disable()
+        _gc_paused += 1
+    try:
+        yield
+    finally:
+        with _gc_lock:
+            _gc_paused -= 1
+            if _gc_paused == 0 and _gc_resume:
+                gc.enable()
 
 
 class Captured:
@@ -46,17 +73,12 @@ class Captured:
         # No garbage collection while the stream is capturing: freeing another graph then (one held by
         # a reference cycle) synchronises the device in its destructor, which a capture does not
         # permit, and the error ends the process.
-        collecting = gc.isenabled()
-        gc.disable()
         try:
-            with checks.deferred(), torch.cuda.graph(self.graph):
+            with _no_collection(), checks.deferred(), torch.cuda.graph(self.graph):
                 self.out = fn()
         except BaseException:
             checks.clear()
             raise
-        finally:
-            if collecting:
-                gc.enable()
         self._conds = checks.take()
         counts = torch.zeros(4, dtype=torch.int64)
         L.call("jzt_graph_count_nodes", self.graph.raw_cuda_graph(), counts.data_ptr())
