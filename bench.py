@@ -240,7 +240,7 @@ def bench_batch(jz, torch, dev, nsets, k, steps, warmup, timer):
     off = np.concatenate([[0], np.cumsum(sizes)])
     box = 1.0
     ctree, tres = jz.autotune.tune_pipeline_sets(x, sizes, k, rl, boxsize=box, leaf_sizes=(16, 24, 32, 48),
-                                                 leaf_waves=(2, 4), sort_kpts=(12, 16), reps=2)
+                                                 leaf_waves=(4,), sort_kpts=(12, 16), reps=2)
     eager = lambda: jz.batch.pipeline_sets(x, sizes, k, rl, boxsize=box, cfg_tree=ctree)
     ref = [t.clone() for t in eager()]
     g = jz.batch.CapturedSets(x, sizes, k, rl, boxsize=box, cfg_tree=ctree)
@@ -428,7 +428,7 @@ def main():
         fcfg, ftune = jz.autotune.tune_fof(x, rlink, boxsize=box, cfg=fcfg, leaf_sizes=(32, 64, 96, 128),
                                            sort_kpts=(12, 16), reps=2)
         kcfg, ktune = jz.autotune.tune_knn(x, k, boxsize=box, cfg=kcfg, leaf_sizes=(64, 96, 128, 160),
-                                           leaf_waves=(2, 4), sort_kpts=(12, 16), reps=2)
+                                           leaf_waves=(4,), sort_kpts=(12, 16), reps=2)
         tune_info = {"leaf_size_knn": ktune.leaf_size, "leaf_waves": ktune.leaf_waves, "sort_kpt": ktune.sort_kpt,
                      "leaf_size_fof": ftune.leaf_size, "fof_sort_kpt": ftune.sort_kpt, "xcd": best_xcd,
                      "knn_ms_by_xcd_order": xcd_ms, "knn_candidates": len(ktune.table),

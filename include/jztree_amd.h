@@ -46,9 +46,8 @@ int jzt_abi_version(void);
 /* Tuning knobs (no counterpart in the reference, which has no autotuner): process-wide settings
  * read at each launch; results never depend on them.  Set them between calls, not while another
  * host thread launches.
- *   JZT_TUNE_LEAF_WAVES  waves per EU the leaf kNN kernel is compiled for when k <= 32 (1, 2, 4,
- *                        which means 3 above k = 16;
- *                        default 4): the register budget per lane against occupancy
+ *   JZT_TUNE_LEAF_WAVES  (1, 2, 4; default 4) without effect: the leaf kNN kernel's register need no
+ *                        longer depends on the waves it is compiled for.  Accepted and returned as before
  *   JZT_TUNE_SORT_KPT    keys per thread of the onesweep radix passes (8, 12, 16; default 12, which
  *                        means 8 below 2^23 keys): tile = threads * kpt keys
  *   JZT_TUNE_XCD         order of the query leaves in the kNN and FoF leaf kernels (0, 1; default

@@ -3,8 +3,8 @@
 Picks, by timing candidates on the caller's own points:
 
   leaf_size   TreeConfig.max_leaf_size: the query and source granularity of the leaf kernels
-  leaf_waves  waves per EU the leaf kNN kernel is compiled for (k <= 32): its register budget
-              against occupancy (library knob JZT_TUNE_LEAF_WAVES)
+  leaf_waves  a knob that has no effect any more (library knob JZT_TUNE_LEAF_WAVES), kept for
+              settings and caches that name it: one candidate by default
   sort_kpt    keys per thread of the onesweep radix passes, i.e. the sort's tile of 256 * kpt
               keys (library knob JZT_TUNE_SORT_KPT)
 
@@ -160,7 +160,7 @@ def _tune(kind, n, k, dtype, dim, boxsize, nsets, run, cache, reps, sort_kpts, l
 
 
 def tune_knn(pos: torch.Tensor, k: int, boxsize: float | None = None, cfg: KNNConfig = KNNConfig(),
-             leaf_sizes: Sequence[int] = (32, 48, 64), leaf_waves: Sequence[int] = (1, 2, 4),
+             leaf_sizes: Sequence[int] = (32, 48, 64), leaf_waves: Sequence[int] = (4,),
              sort_kpts: Sequence[int] = (8, 12, 16), reps: int = 3, cache: str | None = None):
     """Tune knn() on these points.  Returns (cfg with the chosen leaf size, TuneResult); the chosen
     knobs are applied to the library."""
@@ -177,7 +177,7 @@ def tune_knn(pos: torch.Tensor, k: int, boxsize: float | None = None, cfg: KNNCo
 
 
 def tune_pipeline_sets(pos: torch.Tensor, sizes, k: int, rlink, boxsize: float = 0., cfg_tree=None,
-                       leaf_sizes: Sequence[int] = (16, 24, 32, 48), leaf_waves: Sequence[int] = (1, 2, 4),
+                       leaf_sizes: Sequence[int] = (16, 24, 32, 48), leaf_waves: Sequence[int] = (4,),
                        sort_kpts: Sequence[int] = (8, 12, 16), reps: int = 3, cache: str | None = None):
     """Tune batch.pipeline_sets (sort, forest, kNN, FoF of a batch of sets).  Returns (tree config
     with the chosen leaf size, TuneResult); the chosen knobs are applied to the library."""

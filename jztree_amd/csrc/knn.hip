@@ -28,9 +28,6 @@ namespace jzt {
 namespace {
 
 constexpr float kRmaxSlack = 1.0f + kBoundSlack;
-#ifndef JZT_LEAF_WAVES
-#define JZT_LEAF_WAVES 4
-#endif
 
 template <int D, typename T> struct NodeT {
   Vec<D, T> cent;
@@ -1248,44 +1245,36 @@ int leaf2leaf_impl(hipStream_t s, const int32_t* il_spl, const int32_t* il_src, 
   const dim3 b(64);
   const float* xt = (const float*)xT;
   const float* xq = (const float*)xQ;
-  const int waves = tune_get(kTuneLeafWaves);
   const int xcd = tune_get(kTuneXcd);
   for (int koff = 0; koff < k; koff += 64) {
     const int kn = min(k - koff, 64);
     const bool floor = resume && koff > 0;
     if (queue && fill_u32(s, queue, 0u, 8 * kQueueStride)) return 1;
-    // waves that a compute unit holds: by registers for k > 8, by LDS for k <= 8
+    // waves that a compute unit holds, by registers
     const dim3 g(queue ? queue_grid(nleaves_q, kn <= 8 ? 20 : kn <= 16 ? 16 : kn <= 32 ? 12 : 8) : grid_for8(nleaves_q));
 #define JZT_KNN_LAUNCH(KK, PER, FLOOR, W)                                                                              \
   hipLaunchKernelGGL((k_knn_leaf<KK, PER, FLOOR, D, W>), g, b, 0, s, il_spl, il_src, il_r2, splT, xt, splQ, xq, src_ids, \
                      dst_rows, init_r2, retry, (float*)rad, ids, resume, koff, k, boxsize, il_size, out_rows, nleaves_q, xcd, \
                      queue, boxes)
-  // waves per EU (the register budget of the kernel): tunable for K <= 32.  4 spilled 29 registers at
-  // K = 32, in the flush (2^26 points, learned: 65.6 ms against 61.9 at 3); at K = 64, 2 spill 12 and
-  // hide more than 1 (1,000,003 points, k = 64: 4.5 ms against 5.1)
-#define JZT_KNN_LAUNCH_W(KK, PER)                                                            \
-  do {                                                                                       \
-    constexpr int w4 = KK > 32 ? 2 : KK > 16 ? 3 : JZT_LEAF_WAVES;                           \
-    if (KK <= 32 && waves == 1) JZT_KNN_LAUNCH(KK, PER, false, (KK > 32 ? 2 : 1));           \
-    else if (waves == 2) JZT_KNN_LAUNCH(KK, PER, false, 2);                                  \
-    else JZT_KNN_LAUNCH(KK, PER, false, w4);                                                 \
-  } while (0)
-#define JZT_KNN_LAUNCH_K(KK)                                                            \
-  do {                                                                                  \
-    if (boxsize > 0.f) {                                                                \
-      if (floor) JZT_KNN_LAUNCH(KK, true, true, (KK > 32 ? 1 : KK > 16 ? 3 : JZT_LEAF_WAVES));  \
-      else JZT_KNN_LAUNCH_W(KK, true);                                                  \
-    } else {                                                                            \
-      if (floor) JZT_KNN_LAUNCH(KK, false, true, (KK > 32 ? 1 : KK > 16 ? 3 : JZT_LEAF_WAVES)); \
-      else JZT_KNN_LAUNCH_W(KK, false);                                                 \
-    }                                                                                   \
+  // waves per EU (the register budget of the kernel).  K <= 8 takes 89 registers and K <= 16 122 with any
+  // budget that holds them; at K = 32, 4 waves spilled 29, in the flush (2^26 points, learned: 65.6 ms against
+  // 61.9 at 3); at K = 64, 2 spill 12 and hide more than 1 (1,000,003 points, k = 64: 4.5 ms against 5.1)
+#define JZT_KNN_LAUNCH_K(KK)                                                      \
+  do {                                                                            \
+    constexpr int w = KK > 32 ? 2 : KK > 16 ? 3 : 4, wf = KK > 32 ? 1 : w;        \
+    if (boxsize > 0.f) {                                                          \
+      if (floor) JZT_KNN_LAUNCH(KK, true, true, wf);                              \
+      else JZT_KNN_LAUNCH(KK, true, false, w);                                    \
+    } else {                                                                      \
+      if (floor) JZT_KNN_LAUNCH(KK, false, true, wf);                             \
+      else JZT_KNN_LAUNCH(KK, false, false, w);                                   \
+    }                                                                             \
   } while (0)
     if (kn <= 8) JZT_KNN_LAUNCH_K(8);
     else if (kn <= 16) JZT_KNN_LAUNCH_K(16);
     else if (kn <= 32) JZT_KNN_LAUNCH_K(32);
     else JZT_KNN_LAUNCH_K(64);
 #undef JZT_KNN_LAUNCH_K
-#undef JZT_KNN_LAUNCH_W
 #undef JZT_KNN_LAUNCH
     if (check_launch("KnnLeaf2Leaf")) return 1;
   }

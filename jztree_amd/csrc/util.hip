@@ -329,7 +329,7 @@ int flags_or_level_i8(hipStream_t s, int8_t* flags, const int32_t* lvl, int64_t 
   return check_launch("FlagsOrLevel");
 }
 
-// leaf kNN waves per EU (K <= 32), onesweep keys per thread, XCD-aware order of the leaf kernels
+// leaf kNN waves per EU (without effect), onesweep keys per thread, XCD-aware order of the leaf kernels
 static int g_tune[kTuneCount] = {4, 12, 1};
 int tune_get(int knob) { return (knob >= 0 && knob < kTuneCount) ? __atomic_load_n(&g_tune[knob], __ATOMIC_RELAXED) : 0; }
 
