@@ -414,8 +414,8 @@ def main():
     if args.no_tune:
         kcfg = dataclasses.replace(kcfg, tree=dataclasses.replace(kcfg.tree, max_leaf_size=128))
         fcfg = dataclasses.replace(fcfg, tree=dataclasses.replace(fcfg.tree, max_leaf_size=128))
-        jz.autotune.set_knobs(leaf_waves=4, sort_kpt=16, xcd=1)
-        tune_info = {"skipped": True, "leaf_size_knn": 128, "leaf_size_fof": 128, "leaf_waves": 4, "sort_kpt": 16,
+        jz.autotune.set_knobs(leaf_waves=4, sort_kpt=12, xcd=1)
+        tune_info = {"skipped": True, "leaf_size_knn": 128, "leaf_size_fof": 128, "leaf_waves": 4, "sort_kpt": 12,
                      "xcd": 1}
     else:
         xcd_ms = {}

@@ -49,7 +49,8 @@ int jzt_abi_version(void);
  *   JZT_TUNE_LEAF_WAVES  (1, 2, 4; default 4) without effect: the leaf kNN kernel's register need no
  *                        longer depends on the waves it is compiled for.  Accepted and returned as before
  *   JZT_TUNE_SORT_KPT    keys per thread of the onesweep radix passes (8, 12, 16; default 12, which
- *                        means 8 below 2^23 keys): tile = threads * kpt keys
+ *                        means 8 below 2^23 keys; 16 means the default from 2^21 keys on): a tile is 256 threads
+ *                        below 2^18 keys, 512 below 2^21, else 1024, times the keys per thread
  *   JZT_TUNE_XCD         order of the query leaves in the kNN and FoF leaf kernels (0, 1; default
  *                        1): 1 gives each of the 8 XCDs a contiguous eighth of the z-ordered
  *                        leaves, so that neighbouring leaves share an L2; 0 deals consecutive

@@ -5,8 +5,9 @@ Picks, by timing candidates on the caller's own points:
   leaf_size   TreeConfig.max_leaf_size: the query and source granularity of the leaf kernels
   leaf_waves  a knob that has no effect any more (library knob JZT_TUNE_LEAF_WAVES), kept for
               settings and caches that name it: one candidate by default
-  sort_kpt    keys per thread of the onesweep radix passes, i.e. the sort's tile of 256 * kpt
-              keys (library knob JZT_TUNE_SORT_KPT)
+  sort_kpt    keys per thread of the onesweep radix passes, i.e. the sort's tile of that many keys for
+              each of 256 to 1024 threads, by size; the default 12 means 8 below 2^23 keys, and 16
+              means the default from 2^21 on (library knob JZT_TUNE_SORT_KPT)
 
 None of them changes a result: the tuner checks that every candidate's output equals the first
 candidate's, bit for bit, and raises otherwise.  The chosen knobs are applied to the library, the

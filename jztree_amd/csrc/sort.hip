@@ -830,15 +830,17 @@ __global__ __launch_bounds__(kSmallThreads) void k_small_sort(const T* __restric
 //   65,536 points 94 / 101 / 128 / 158      2^20 255 / 219 / 235 / 260      2^22 623 / 502 / 481 / 499
 //   2^24 2077 / 1713 / 1601 / 1573          2^26 8200 / 6820 / 6348 / 5847
 // (256 x 12 with one look-back row at a time: 130, 530, 810, 2600, 7800.)  A tuned number of keys per
-// thread other than the default takes the place of 8 and 12.
+// thread other than the default takes the place of 8 and 12, but for 1024 x 16, which spilled 22 registers and
+// was nowhere faster than the default that runs instead: 2^21 361 / 291, 2^22 473 / 473, 2^24 1740 / 1572,
+// 2^26 6515 / 5860.
 struct SortTile {
   int threads, kpt;
   int64_t tiles;
 };
 SortTile sort_tile(int64_t n) {
   const int tuned = tune_get(kTuneSortKpt);
-  const int kpt = tuned != 12 ? tuned : n < (int64_t)1 << 23 ? 8 : 12;
   const int threads = n < (int64_t)1 << 18 ? 256 : n < (int64_t)1 << 21 ? 512 : 1024;
+  const int kpt = tuned == 8 || (tuned == 16 && threads < 1024) ? tuned : n < (int64_t)1 << 23 ? 8 : 12;
   return {threads, kpt, div_up(n, (int64_t)threads * kpt)};
 }
 
@@ -850,14 +852,11 @@ int onesweep(hipStream_t s, const SortTile& st, const uint64_t* ki, const uint32
     hipLaunchKernelGGL((k_onesweep<TH, K>), dim3((unsigned)st.tiles), dim3(TH), 0, s, ki, vi, ko, vo, n, shift, \
                        bucket, lookback, counter)
   JZT_SWEEP(256, 8);
-  JZT_SWEEP(256, 12);
   JZT_SWEEP(256, 16);
   JZT_SWEEP(512, 8);
-  JZT_SWEEP(512, 12);
   JZT_SWEEP(512, 16);
   JZT_SWEEP(1024, 8);
   JZT_SWEEP(1024, 12);
-  JZT_SWEEP(1024, 16);
 #undef JZT_SWEEP
   return 0;
 }

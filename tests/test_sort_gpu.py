@@ -295,3 +295,21 @@ def test_zsort_gradient_forward_over_reverse(dev, dtype, dim):
         assert torch.equal(p, back(w)) and torch.equal(dp, back(t))
     (gb,) = torch.autograd.grad(posz, x, torch.stack([w, t]), is_grads_batched=True)
     assert torch.equal(gb, torch.stack([back(w), back(t)]))
+
+
+@pytest.mark.parametrize("kpt", [8, 16])
+@pytest.mark.parametrize("n", [(1 << 18) + 1, (1 << 21) - 1, (1 << 21) + 3])
+def test_zsort_tuned_tiles_of_larger_sets(dev, n, kpt):
+    """The tuned number of keys per thread with 512 and 1024 threads a tile."""
+    import jztree_amd as jz
+    x = torch.rand((n, 3), device=dev, generator=torch.Generator(device=dev).manual_seed(n))
+    p0, i0 = jz.tree.zsort(x)
+    before = jz.autotune.get_knobs()
+    try:
+        jz.autotune.set_knobs(sort_kpt=kpt)
+        print(f"[zsort tile] n={n} kpt={kpt}", flush=True)
+        pz, iz = jz.tree.zsort(x)
+        torch.cuda.synchronize()
+    finally:
+        jz.autotune.set_knobs(**before)
+    assert torch.equal(iz, i0) and torch.equal(pz, p0)
