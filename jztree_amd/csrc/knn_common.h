@@ -11,34 +11,6 @@ namespace jzt {
 
 __device__ __forceinline__ float key_r2(uint64_t k) { return __uint_as_float((uint32_t)(k >> 32)); }
 
-// Insert `key` into the ascending list best[0..K) (caller guarantees key < best[K-1]; keys are
-// unique).  Top-down: slot i takes best[i-1] where key < best[i-1], takes key where
-// best[i-1] <= key < best[i], and keeps its value otherwise; each comparison serves two
-// neighbouring slots.  Every 8 slots the wave leaves the (fully unrolled, statically indexed)
-// network once no active lane still shifts.
-template <int K>
-__device__ __forceinline__ void topk_insert(uint64_t (&best)[K], uint64_t key) {
-  if constexpr (K == 1) {
-    best[0] = key;
-  } else {
-    bool hi = true;                     // key < best[i]
-    bool lo_next = key < best[K - 2];   // compare issued one step ahead of its selects
-#pragma unroll
-    for (int i = K - 1; i >= 1; i--) {
-      const bool lo = lo_next;          // key < best[i-1]
-      if (i >= 2) lo_next = key < best[i - 2];
-      const uint64_t t = hi ? key : best[i];
-      best[i] = lo ? best[i - 1] : t;
-      hi = lo;
-      // materialise the slot before the next exit test: otherwise the selects sink below the
-      // exits and the compare masks of several blocks stay live in (spilled) SGPRs
-      asm volatile("" : "+v"(best[i]));
-      if ((i & 7) == 0 && !wave_any(lo)) return;
-    }
-    best[0] = hi ? key : best[0];
-  }
-}
-
 constexpr uint64_t kEmptyKey = (0x7f800000ull << 32) | 0xffffffffull;  // (r2 = +inf, id = -1)
 
 __device__ __forceinline__ int rdlane(int v, int i) { return __builtin_amdgcn_readlane(v, i); }
