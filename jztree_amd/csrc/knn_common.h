@@ -62,8 +62,8 @@ __device__ __forceinline__ void ce_asc(uint64_t& a, uint64_t& b) {
 // ascending sort of a register array by Batcher's odd-even merge sort (N a power of two; 63
 // compare-exchanges for N = 16 against 80 for the bitonic network): for each merge width 2p, merge
 // steps of distance k = p, p/2, ..., 1 compare i+j with i+j+k inside one 2p-block.
-template <int N>
-__device__ __forceinline__ void oddeven_sort_regs(uint64_t (&v)[N]) {
+// ce(a, b) orders entries a < b.
+template <int N, typename CE> __device__ __forceinline__ void oddeven_network(CE ce) {
 #pragma unroll
   for (int p = 1; p < N; p <<= 1) {
 #pragma unroll
@@ -72,7 +72,7 @@ __device__ __forceinline__ void oddeven_sort_regs(uint64_t (&v)[N]) {
       for (int j = k % p; j <= N - 1 - k; j += 2 * k) {
 #pragma unroll
         for (int i = 0; i < N; i++) {
-          if (i <= k - 1 && i <= N - j - k - 1 && (i + j) / (2 * p) == (i + j + k) / (2 * p)) ce_asc(v[i + j], v[i + j + k]);
+          if (i <= k - 1 && i <= N - j - k - 1 && (i + j) / (2 * p) == (i + j + k) / (2 * p)) ce(i + j, i + j + k);
         }
       }
     }
@@ -127,7 +127,7 @@ __device__ __forceinline__ void topk_flush(uint64_t (&best)[K], const uint64_t* 
 #pragma unroll
   for (int i = 0; i < M; i++) b[i] = i < cnt ? b[i] : kEmptyKey;
   cnt = 0;
-  oddeven_sort_regs<M>(b);
+  oddeven_network<M>([&](int x, int y) { ce_asc(b[x], b[y]); });
   // half-cleaner of best ++ reverse(b padded to K): the low half holds the K smallest, bitonic
 #pragma unroll
   for (int i = 0; i < M; i++) {

@@ -64,19 +64,7 @@ __device__ __forceinline__ void pair_flush(T (&br)[K], uint32_t (&bi)[K], const 
     id[i] = i < cnt ? row_i[i] : 0xffffffffu;
   }
   cnt = 0;
-#pragma unroll
-  for (int p = 1; p < M; p <<= 1) {
-#pragma unroll
-    for (int k = p; k >= 1; k >>= 1) {
-#pragma unroll
-      for (int j = k % p; j <= M - 1 - k; j += 2 * k) {
-#pragma unroll
-        for (int i = 0; i < M; i++)
-          if (i <= k - 1 && i <= M - j - k - 1 && (i + j) / (2 * p) == (i + j + k) / (2 * p))
-            pair_ce(r[i + j], id[i + j], r[i + j + k], id[i + j + k]);
-      }
-    }
-  }
+  oddeven_network<M>([&](int x, int y) { pair_ce(r[x], id[x], r[y], id[y]); });
 #pragma unroll
   for (int i = 0; i < M; i++) {
     const bool take = pair_less(r[M - 1 - i], id[M - 1 - i], br[K - M + i], bi[K - M + i]);
