@@ -135,7 +135,8 @@ def stream() -> int:
 
 
 def ptr(t) -> int | None:
-    """Device pointer of a tensor (None for None)."""
+    """Device pointer of a tensor (None for None).  It does not keep the tensor: the memory of a temporary
+    is handed to the next one made, so a call takes pointers of held tensors."""
     if t is None:
         return None
     return t.data_ptr()

@@ -75,8 +75,9 @@ def _fof_node2node(ilist: InteractionList, spl_parent, node_data: PosLvl, node_i
     over = torch.empty(1, dtype=torch.bool, device=dev)
     per_parent = torch.is_tensor(rlink)  # r2link per parent node (batches of sets)
     r2v = _r2_items(rlink, spl_parent.shape[0] - 1) if per_parent else None
-    L.call("jzt_fof_node2node_ex", L.stream(), L.ptr(ilist.ispl), L.ptr(ilist.isrc), L.ptr(spl_parent.contiguous()),
-           L.ptr(r2v), L.ptr(node_data.pos_lvl()), L.ptr(ig), L.ptr(ig), L.ptr(il_spl), L.ptr(il),
+    spl_c, rows = spl_parent.contiguous(), node_data.pos_lvl()
+    L.call("jzt_fof_node2node_ex", L.stream(), L.ptr(ilist.ispl), L.ptr(ilist.isrc), L.ptr(spl_c),
+           L.ptr(r2v), L.ptr(rows), L.ptr(ig), L.ptr(ig), L.ptr(il_spl), L.ptr(il),
            spl_parent.shape[0] - 1, size, ilist.size(), ilist.size(), 0. if per_parent else _r2link(rlink),
            float(boxsize or 0.), node_data.pos.shape[-1], L.dtype_code(node_data.pos.dtype), L.ptr(over))
     node_ilist = verify_ilist(InteractionList(il_spl, il))
@@ -95,15 +96,14 @@ def _node_to_child_label(igroup, lvl, spl, rlink: float, dim: int, num=None, siz
         size_child = igroup.numel()
     out = torch.empty(size_child, dtype=torch.int32, device=dev)
     loc = None if flag_local is None else flag_local.to(torch.uint8).contiguous()
+    ig, lv, sp = (t.to(torch.int32).contiguous() for t in (igroup, lvl, spl))
     if torch.is_tensor(rlink):  # r2link per parent node (batches of sets)
         assert flag_local is None
-        L.call("jzt_node_to_child_label_sets", L.stream(), L.ptr(igroup.to(torch.int32).contiguous()),
-               L.ptr(lvl.to(torch.int32).contiguous()), L.ptr(spl.to(torch.int32).contiguous()),
-               L.ptr(_r2_items(rlink, igroup.numel())), L.ptr(out), igroup.numel(), size_child, int(dim),
-               L.dtype_code(dtype))
+        r2v = _r2_items(rlink, igroup.numel())
+        L.call("jzt_node_to_child_label_sets", L.stream(), L.ptr(ig), L.ptr(lv), L.ptr(sp), L.ptr(r2v), L.ptr(out),
+               igroup.numel(), size_child, int(dim), L.dtype_code(dtype))
     else:
-        L.call("jzt_node_to_child_label", L.stream(), L.ptr(igroup.to(torch.int32).contiguous()), L.ptr(loc),
-               L.ptr(lvl.to(torch.int32).contiguous()), L.ptr(spl.to(torch.int32).contiguous()), L.ptr(out),
+        L.call("jzt_node_to_child_label", L.stream(), L.ptr(ig), L.ptr(loc), L.ptr(lv), L.ptr(sp), L.ptr(out),
                igroup.numel(), size_child, _r2link(rlink), int(dim), L.dtype_code(dtype))
     if num is not None:
         out = torch.where(torch.arange(size_child, device=dev) < num, out, torch.zeros_like(out))
@@ -165,21 +165,21 @@ def _fof_leaf2leaf(leaf_data: FofNodeData, ilist: InteractionList, posz, rlink: 
     part_igroup = _node_to_child_label(leaf_data.igroup, leaf_data.lvl, leaf_data.spl, rlink=rl,
                                        size_child=len(posz), dim=posz.shape[-1], dtype=posz.dtype)
     out = part_igroup  # linked in place
+    spl, posz = leaf_data.spl.contiguous(), posz.contiguous()
     if leaf_r2link is not None:
+        r2v = _r2_items(leaf_r2link, len(spl) - 1)
         L.call("jzt_fof_leaf2leaf_sets", L.stream(), L.ptr(ilist.ispl), L.ptr(ilist.isrc), ilist.size(),
-               L.ptr(leaf_data.spl.contiguous()), L.ptr(_r2_items(leaf_r2link, len(leaf_data.spl) - 1)),
-               L.ptr(posz.contiguous()), L.ptr(part_igroup), L.ptr(out), len(leaf_data.spl) - 1, len(posz),
+               L.ptr(spl), L.ptr(r2v), L.ptr(posz), L.ptr(part_igroup), L.ptr(out), len(spl) - 1, len(posz),
                float(boxsize or 0.), posz.shape[-1], L.dtype_code(posz.dtype))
     elif leaf_data.cent is not None and leaf_data.cent.dtype == posz.dtype:
         cells = PosLvl(pos=leaf_data.cent, lvl=leaf_data.lvl, rows=leaf_data.rows).pos_lvl()
         L.call("jzt_fof_leaf2leaf_cells", L.stream(), L.ptr(ilist.ispl), L.ptr(ilist.isrc), ilist.size(),
-               L.ptr(leaf_data.spl.contiguous()), L.ptr(posz.contiguous()), L.ptr(cells), L.ptr(part_igroup),
-               L.ptr(out), len(leaf_data.spl) - 1, len(posz), _r2link(rlink), float(boxsize or 0.), posz.shape[-1],
+               L.ptr(spl), L.ptr(posz), L.ptr(cells), L.ptr(part_igroup),
+               L.ptr(out), len(spl) - 1, len(posz), _r2link(rlink), float(boxsize or 0.), posz.shape[-1],
                L.dtype_code(posz.dtype))
     else:
         L.call("jzt_fof_leaf2leaf", L.stream(), L.ptr(ilist.ispl), L.ptr(ilist.isrc), ilist.size(),
-               L.ptr(leaf_data.spl.contiguous()),
-               L.ptr(posz.contiguous()), L.ptr(part_igroup), L.ptr(out), len(leaf_data.spl) - 1, len(posz),
+               L.ptr(spl), L.ptr(posz), L.ptr(part_igroup), L.ptr(out), len(spl) - 1, len(posz),
                _r2link(rlink), float(boxsize or 0.), posz.shape[-1], L.dtype_code(posz.dtype))
     return out
 

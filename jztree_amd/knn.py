@@ -218,9 +218,10 @@ def _knn_fused(th: TreeHierarchy, posz, k: int, boxsize: float | None = None, al
     sid = None if src_ids is None else src_ids.to(torch.int32).contiguous()
     drow = None if dst_rows is None else dst_rows.to(torch.int32).contiguous()
     ir2 = None if init_r2 is None else init_r2.to(torch.float32).contiguous()
+    n2c, posz = n2c.contiguous(), posz.contiguous()
     L.call("jzt_knn_fused", L.stream(), L.ptr(ilist_p.ispl), L.ptr(ilist_p.isrc), L.ptr(ilist_p.rad2),
-           ilist_p.size(), L.ptr(n2c.contiguous()), L.ptr(leaf_parent), L.ptr(leaf_nodes), L.ptr(l2p),
-           L.ptr(posz.contiguous()), L.ptr(sid), L.ptr(drow), L.ptr(ir2), L.ptr(retry), L.ptr(rnn), L.ptr(inn),
+           ilist_p.size(), L.ptr(n2c), L.ptr(leaf_parent), L.ptr(leaf_nodes), L.ptr(l2p),
+           L.ptr(posz), L.ptr(sid), L.ptr(drow), L.ptr(ir2), L.ptr(retry), L.ptr(rnn), L.ptr(inn),
            size, n, int(k), float(boxsize or 0.), posz.shape[-1], L.dtype_code(posz.dtype))
     return rnn, inn, retry
 
@@ -407,9 +408,10 @@ def _fused_retry(th: TreeHierarchy, ilist_p: InteractionList, n2c, posz, k: int,
     leaf_parent, leaf_nodes, l2p = _leaf_plane_args(th, n2c)
     sid = None if src_ids is None else src_ids.to(torch.int32).contiguous()
     drow = None if dst_rows is None else dst_rows.to(torch.int32).contiguous()
+    n2c, posz, cap = n2c.contiguous(), posz.contiguous(), cap.contiguous()
     L.call("jzt_knn_fused_retry", L.stream(), L.ptr(ilist_p.ispl), L.ptr(ilist_p.isrc), L.ptr(ilist_p.rad2),
-           ilist_p.size(), L.ptr(n2c.contiguous()), L.ptr(leaf_parent), L.ptr(leaf_nodes), L.ptr(l2p),
-           L.ptr(posz.contiguous()), L.ptr(sid), L.ptr(drow), L.ptr(cap.contiguous()), L.ptr(retry), L.ptr(rnn),
+           ilist_p.size(), L.ptr(n2c), L.ptr(leaf_parent), L.ptr(leaf_nodes), L.ptr(l2p),
+           L.ptr(posz), L.ptr(sid), L.ptr(drow), L.ptr(cap), L.ptr(retry), L.ptr(rnn),
            L.ptr(inn), th.size(), len(posz), int(k), float(boxsize), posz.shape[-1], L.dtype_code(posz.dtype))
 
 
@@ -436,8 +438,8 @@ def _knn_leaf_start_bound(ilist: InteractionList, spl, posz, k: int, boxsize, le
         # per leaf: does it hold a flagged query (a segment maximum over the query splits; a
         # scatter of every flag onto its leaf costs an atomic per query)
         short = torch.empty(size, dtype=torch.float32, device=xQ.device)
-        L.call("jzt_segment_max_f32", L.stream(), L.ptr(splQ.contiguous()), L.ptr(retry.to(torch.float32)), nq,
-               L.ptr(short), size, 0.0)
+        spl_c, flags = splQ.contiguous(), retry.to(torch.float32)
+        L.call("jzt_segment_max_f32", L.stream(), L.ptr(spl_c), L.ptr(flags), nq, L.ptr(short), size, 0.0)
         redo = torch.where(short > 0, torch.full_like(init, float("inf")), torch.full_like(init, -1.0))
         _knn_leaf2leaf(ilist, spl, posz, k=k, boxsize=boxsize, splQ=splQ, xQ=xQ, src_ids=src_ids,
                        dst_rows=dst_rows, init_r2=redo.contiguous(), out=(rnn, inn, retry), balance=False, boxes=boxes)

@@ -134,7 +134,8 @@ class RadiusProposer:
         """(loss, gradient) of the mean squared error on standardised (x, t), from jzt_mlp_grad."""
         grad = torch.empty(NPARAM, dtype=torch.float32, device=self.device)
         loss = torch.empty(1, dtype=torch.float32, device=self.device)
-        L.call("jzt_mlp_grad", L.stream(), L.ptr(self.wq), L.ptr(x.contiguous()), L.ptr(t.contiguous()), len(t),
+        x, t = x.contiguous(), t.contiguous()
+        L.call("jzt_mlp_grad", L.stream(), L.ptr(self.wq), L.ptr(x), L.ptr(t), len(t),
                L.ptr(grad), L.ptr(loss))
         return loss, grad
 

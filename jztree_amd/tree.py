@@ -221,7 +221,8 @@ def detect_leaf_boundaries(posz: torch.Tensor, ptype: torch.Tensor | None = None
     if set_id is not None:
         assert num_types == 1 and cfg_reg is None, "batches of sets use one particle type and no regularization"
         assert set_id.dtype == torch.int32 and len(set_id) == n
-        L.call("jzt_flag_leaf_boundaries_sets", L.stream(), L.ptr(posz.contiguous()), L.ptr(set_id.contiguous()),
+        posz, set_id = posz.contiguous(), set_id.contiguous()
+        L.call("jzt_flag_leaf_boundaries_sets", L.stream(), L.ptr(posz), L.ptr(set_id),
                L.ptr(lvl_bound_t), L.ptr(npart_t), L.ptr(flags), L.ptr(lvl), n, dim, L.dtype_code(posz.dtype),
                int(leaf_size), int(leaf_size + 1))
     else:
@@ -265,7 +266,8 @@ def determine_znode_boundaries(posz: torch.Tensor, block_size: int = 64, nleaves
     lvl, lb, rb = (torch.empty(size + 1, dtype=torch.int32, device=dev) for _ in range(3))
     if set_id is not None:
         assert set_id.dtype == torch.int32 and len(set_id) == size
-        L.call("jzt_find_node_boundaries_sets", L.stream(), L.ptr(posz.contiguous()), L.ptr(set_id.contiguous()),
+        posz, set_id = posz.contiguous(), set_id.contiguous()
+        L.call("jzt_find_node_boundaries_sets", L.stream(), L.ptr(posz), L.ptr(set_id),
                L.ptr(pos_bound), L.ptr(nl), L.ptr(lvl), L.ptr(lb), L.ptr(rb), size + 1, dim,
                L.dtype_code(posz.dtype), -2000)
     else:
@@ -292,8 +294,8 @@ def get_node_geometry(posz: torch.Tensor, lbound: torch.Tensor, rbound: torch.Te
     lvl = torch.empty(size if mode & 1 else 1, dtype=torch.int32, device=dev)
     cent = torch.empty((size if mode & 2 else 1, dim), dtype=posz.dtype, device=dev)
     ext = torch.empty((size if mode & 4 else 1, dim), dtype=posz.dtype, device=dev)
-    L.call("jzt_get_node_geometry", L.stream(), L.ptr(posz.contiguous()), L.ptr(lbound.contiguous()),
-           L.ptr(rbound.contiguous()), L.ptr(num_t), L.ptr(lvl), L.ptr(cent), L.ptr(ext), size, n, dim,
+    posz, lbound, rbound = posz.contiguous(), lbound.contiguous(), rbound.contiguous()
+    L.call("jzt_get_node_geometry", L.stream(), L.ptr(posz), L.ptr(lbound), L.ptr(rbound), L.ptr(num_t), L.ptr(lvl), L.ptr(cent), L.ptr(ext), size, n, dim,
            L.dtype_code(posz.dtype), -2000, mode, int(bool(upper_extent)))
     rdict = {"lvl": lvl, "cent": cent, "ext": ext}
     res = [rdict[k] for k in result.split("_")]
@@ -497,9 +499,11 @@ def plane_tables(th: TreeHierarchy) -> PlaneTables:
     spl = c32(th.splits_leaf_to_part(0))
     out = torch.empty((3, nl, size + 1), dtype=torch.int32, device=dev)
     nodes = torch.empty((nl, size + 1, dim + 1), dtype=cent.dtype, device=dev)
-    L.call("jzt_plane_tables", L.stream(), L.ptr(c32(th.ispl_n2n.data)), L.ptr(c32(th.ispl_n2l.data)),
-           L.ptr(c32(th.ispl_n2n.ispl)), L.ptr(c32(th.ispl_n2n.fill_values)), L.ptr(c32(th.ispl_n2l.fill_values)),
-           L.ptr(c32(th.lvl.data)), L.ptr(cent), L.ptr(c32(th.lvl.ispl)), L.ptr(spl), spl.numel(), nl, size, dim,
+    n2n, n2l, level_spl, n2n_fill, n2l_fill, lvl, prop_spl = (
+        c32(t) for t in (th.ispl_n2n.data, th.ispl_n2l.data, th.ispl_n2n.ispl, th.ispl_n2n.fill_values,
+                         th.ispl_n2l.fill_values, th.lvl.data, th.lvl.ispl))
+    L.call("jzt_plane_tables", L.stream(), L.ptr(n2n), L.ptr(n2l), L.ptr(level_spl), L.ptr(n2n_fill), L.ptr(n2l_fill),
+           L.ptr(lvl), L.ptr(cent), L.ptr(prop_spl), L.ptr(spl), spl.numel(), nl, size, dim,
            L.dtype_code(cent.dtype), L.ptr(out[0]), L.ptr(nodes), L.ptr(out[1]), L.ptr(out[2]))
     return PlaneTables(list(out[0].unbind(0)), list(nodes[:, :size].unbind(0)), list(out[1, :, :size].unbind(0)),
                        list(out[2, :, :size].unbind(0)))
@@ -515,7 +519,8 @@ def center_of_mass(ispl: torch.Tensor, pos: torch.Tensor, mass, kahan_summation:
     m = torch.as_tensor(mass, dtype=pos.dtype, device=dev)
     m = torch.broadcast_to(m, pos.shape[:-1]).contiguous()
     out = torch.empty((max(n, 0), pos.shape[-1] + 1), dtype=pos.dtype, device=dev)
-    L.call("jzt_center_of_mass", L.stream(), L.ptr(ispl.contiguous()), L.ptr(pos.contiguous()), L.ptr(m),
+    ispl, pos = ispl.contiguous(), pos.contiguous()
+    L.call("jzt_center_of_mass", L.stream(), L.ptr(ispl), L.ptr(pos), L.ptr(m),
            L.ptr(out), n, int(bool(kahan_summation)), pos.shape[-1], L.dtype_code(pos.dtype))
     return out[:, :-1], out[:, -1]
 
@@ -681,7 +686,8 @@ def search_sorted_z(posz: torch.Tensor, posz_query: torch.Tensor, block_size: in
     assert posz.dtype == posz_query.dtype
     assert posz.shape[-1] == posz_query.shape[-1]
     out = torch.empty(len(posz_query), dtype=torch.int32, device=posz.device)
-    L.call("jzt_search_sorted_z", L.stream(), L.ptr(posz.contiguous()), L.ptr(posz_query.contiguous()), len(posz),
+    posz, posz_query = posz.contiguous(), posz_query.contiguous()
+    L.call("jzt_search_sorted_z", L.stream(), L.ptr(posz), L.ptr(posz_query), len(posz),
            len(posz_query), posz.shape[-1], L.sort_dtype_code(posz.dtype), int(bool(leaf_search)), L.ptr(out))
     return out
 
