@@ -337,7 +337,8 @@ def _delete_rows(x: torch.Tensor, idx: torch.Tensor) -> torch.Tensor:
     # in range even when an (already recorded) allocation overflow made the indices meaningless
     mark.index_fill_(0, torch.clamp(idx.long(), 0, n - 1).reshape(-1), 1)  # scalar as kernel argument
     dest = torch.arange(n, device=x.device) - (torch.cumsum(mark, 0) - mark)
-    dest = torch.where(mark.bool(), torch.full_like(dest, n - m), dest)
+    # (then several can be the same one: rows past the n - m that are kept go with the deleted ones)
+    dest = torch.where(mark.bool(), torch.full_like(dest, n - m), torch.clamp(dest, max=n - m))
     out = torch.empty((n - m + 1,) + tuple(x.shape[1:]), dtype=x.dtype, device=x.device)
     out[dest] = x
     return out[:n - m]
