@@ -444,6 +444,7 @@ def _build_hierarchy(posz, node_sizes, alloc_size, npart, cfg_reg: Regularizatio
     first coordinate is not NaN.  Returns (leaf splits, n2l, n2n, lvl, geom_cent, leaf_set)."""
     n, dim = posz.shape
     dev = posz.device
+    assert set_id is None or (set_id.dtype == torch.int32 and len(set_id) == n)
     posz = posz.contiguous()
     nl = len(node_sizes)
     A = alloc_size

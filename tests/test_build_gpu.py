@@ -119,3 +119,15 @@ def test_points_of_padded_positions(dev, n, dim, dtype, tail):
     th = jz.tree.build_tree_hierarchy(posz, jz.config.TreeConfig(max_leaf_size=48, alloc_fac_nodes=3.))
     jz.checks.flush()
     assert int(th.splits_leaf_to_part(0).max()) == int((~torch.isnan(x[:, 0])).sum())
+
+
+@pytest.mark.parametrize("bad", ["int64", "short"])
+def test_set_ids_are_checked(dev, bad):
+    """The set of every row is int32, one a row; anything else is refused before a kernel reads it."""
+    import jztree_amd as jz
+    posz, _ = jz.tree.zsort(torch.rand((500, 3), device=dev))
+    seg = torch.zeros(500, dtype=torch.int32, device=dev)
+    seg = seg.long() if bad == "int64" else seg[:-1]
+    with pytest.raises(AssertionError):
+        jz.tree.build_tree_hierarchy(posz, jz.config.TreeConfig(alloc_fac_nodes=2.), set_id=seg, nsets=1)
+    jz.checks.clear()
