@@ -52,6 +52,7 @@ def _leaf_boxes(spl, x):
     """Bounding boxes of the leaves' particles for the float32 leaf kernel (None where it does not run)."""
     if x.dtype != torch.float32 or x.shape[-1] > 3:
         return None
+    assert spl.dtype == torch.int32
     boxes = torch.empty((len(spl) - 1, 8), dtype=torch.float32, device=x.device)
     L.call("jzt_leaf_boxes", L.stream(), L.ptr(spl), L.ptr(x.contiguous()), len(spl) - 1, x.shape[-1], L.ptr(boxes))
     return boxes
