@@ -1284,11 +1284,11 @@ int fof_order_impl(hipStream_t s, const int32_t* igroup, const int32_t* npart, i
 template <typename U, typename I>
 __global__ __launch_bounds__(256) void k_unsort_rows(const U* __restrict__ rows, const I* __restrict__ id, int64_t n,
                                                      int width, U* __restrict__ out) {
-  const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (e >= n * width) return;
-  const int64_t i = e / width;
-  const int64_t dst = (int64_t)id[i];
-  if (dst >= 0 && dst < n) out[dst * width + (e - i * width)] = rows[e];
+  for (int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; e < n * width; e += (int64_t)gridDim.x * blockDim.x) {
+    const int64_t i = e / width;
+    const int64_t dst = (int64_t)id[i];
+    if (dst >= 0 && dst < n) out[dst * width + (e - i * width)] = rows[e];
+  }
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -1388,9 +1388,8 @@ extern "C" int jzt_unsort_rows(jzt_stream_t stream, const void* rows, const void
                                int elem_bytes, void* out) {
   if (n < 0 || width < 0) return fail("jzt_unsort_rows: negative size");
   if (n == 0 || width == 0) return 0;
-  const int64_t blocks = div_up(n * width, 256);
-  if (blocks > INT32_MAX) return fail("jzt_unsort_rows: too many elements");
-  const dim3 g((unsigned)blocks), b(256);
+  // a launch holds less than 2^32 threads
+  const dim3 g((unsigned)std::min(div_up(n * width, 256), (int64_t)1 << 22)), b(256);
   hipStream_t s = (hipStream_t)stream;
   if (elem_bytes == 4)
     hipLaunchKernelGGL((k_unsort_rows<uint32_t, int32_t>), g, b, 0, s, (const uint32_t*)rows, (const int32_t*)id, n,

@@ -313,3 +313,20 @@ def test_zsort_tuned_tiles_of_larger_sets(dev, n, kpt):
     finally:
         jz.autotune.set_knobs(**before)
     assert torch.equal(iz, i0) and torch.equal(pz, p0)
+
+
+def test_unsort_rows_of_many_elements(dev):
+    """More elements than one launch holds threads."""
+    import jztree_amd._lib as L
+    n, width = 1031, 4_200_000
+    assert n * width > 1 << 32
+    rows = torch.empty((n, width), dtype=torch.int32, device=dev)
+    rows.copy_(torch.arange(n, dtype=torch.int32, device=dev)[:, None])
+    idz = torch.randperm(n, device=dev, generator=torch.Generator(device=dev).manual_seed(0)).to(torch.int32)
+    out = torch.full_like(rows, -1)
+    print("[unsort] 4.3e9 elements", flush=True)
+    L.call("jzt_unsort_rows", L.stream(), L.ptr(rows), L.ptr(idz), n, width, 4, L.ptr(out))
+    inv = torch.empty_like(idz)
+    inv[idz.long()] = torch.arange(n, dtype=torch.int32, device=dev)
+    for a in range(0, n, 100):
+        assert bool((out[a:a + 100] == inv[a:a + 100, None]).all()), a
