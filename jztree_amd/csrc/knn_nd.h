@@ -254,6 +254,8 @@ int knn_leaf_nd_impl(hipStream_t s, const int32_t* il_spl, const int32_t* il_src
   // item-queue counters after the resume pairs, when the caller's tmp holds them
   const size_t qoff = align256(knn_leaf_nd_tmp_bytes(npart_q, k, sizeof(T) == 8));
   uint32_t* queue = tmp && tmp_bytes >= qoff + 256 ? (uint32_t*)((char*)tmp + qoff) : nullptr;
+  // 32 waves a compute unit for every instance; it holds 4 (K = 32, many dims) to 16 of them, so the others
+  // find the queue empty when they start
   const dim3 g(queue ? queue_grid(nleaves_q, 32) : grid_for8(nleaves_q)), b(64);
   const int xcd = tune_get(kTuneXcd);
   for (int koff = 0; koff < k; koff += KMAX) {

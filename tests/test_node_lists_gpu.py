@@ -1,8 +1,7 @@
 """Kernels of KnnNode2Node and its list sort, at the sizes where their split changes.
 
 Segment sort: lengths around the powers of two of the one-wave sort (64 to 1024 entries), of the LDS sorts
-(4096, 16384) and beyond, negative keys, equal keys, against numpy's lexicographic order.
-FofNode2Node at every number of children per work item, against the oracle.
+(4096, 16384) and beyond, negative keys, equal keys, keys of any bits, against numpy's lexicographic order.
 FofNode2Node: joined nodes and lists against all pairs, at every number of children per work item.
 Node lists: every child's radius against the exact weighted selection and every list against all pairs,
 with parents whose lists are short (one wave) and long (queued), fewer and more than 64 particles of
