@@ -83,3 +83,24 @@ def test_captured_objects_are_freed_without_garbage_collection(dev):
     seen = []
     jz.graph.Captured(lambda: seen.append(gc.isenabled()) or torch.zeros(4, device=dev))
     assert seen == [was, False] and gc.isenabled() == was  # the eager run, then the capture
+
+
+@pytest.mark.parametrize("n", [8192, 12000, 16384])
+def test_captured_small_sets(dev, n):
+    """Sizes at which a captured call sorts another way than an eager one (few launches there, few passes here)."""
+    import jztree_amd as jz
+    g = torch.Generator(device=dev).manual_seed(n)
+    inputs = [torch.rand((n, 3), device=dev, generator=g) for _ in range(2)]
+    x = inputs[0].clone()
+    step = lambda: (jz.tree.zsort(x), jz.knn.knn(x, 8, boxsize=1.0), jz.fof.fof_labels(x, 0.01, boxsize=1.0))
+    print(f"[capture] n={n}", flush=True)
+    cap = jz.graph.Captured(step)
+    for rep in range(3):
+        x.copy_(inputs[rep % 2])
+        (pz, iz), (r, i), (fz, lab) = cap.run()
+        torch.cuda.synchronize()
+        cap.check()
+        got = [t.clone() for t in (pz, iz, r, i, fz, lab)]
+        (pz, iz), (r, i), (fz, lab) = step()
+        for a, b in zip(got, (pz, iz, r, i, fz, lab)):
+            assert torch.equal(a, b), rep
