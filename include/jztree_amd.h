@@ -68,7 +68,7 @@ int jzt_get_tuning(int knob);
 /* PosZorderSort -- replaces ffi target "PosZorderSort" (generated/ffi_sort.cu:62-164, host
  * sort.cuh:40-76, caller tree.py:75-93).  pos_out[i] = pos_in[id_out[i]] in z-order; pos_out may
  * alias pos_in (the reference aliases {0:0}).  Order: exact Morton order of the float bits, ties by
- * input index.  NaN rows last.  dim in [2, 3]. */
+ * input index.  NaN rows last.  dim 2 to 10; JZT_F32, JZT_F64, JZT_I32 or JZT_I64. */
 size_t jzt_zsort_tmp_bytes(int64_t n, int dim, int dtype);
 int jzt_pos_zorder_sort(jzt_stream_t stream, const void* pos_in, void* pos_out, void* id_out, void* tmp,
                         size_t tmp_bytes, int64_t n, int dim, int dtype);
@@ -124,7 +124,8 @@ int jzt_dense_ilist_r2(jzt_stream_t stream, const void* nodes, int64_t nnodes, c
                        size_t tmp_bytes);
 
 /* SegmentSort -- replaces ffi target "SegmentSort" (generated/ffi_knn.cu:412-423, knn.cuh:700-722,
- * caller knn.py:112-127).  Sorts (key, val) within segments spl[i]..spl[i+1] by (key, val). */
+ * caller knn.py:112-127).  Sorts (key, val) within segments spl[i]..spl[i+1] by (key, val): keys in the total
+ * order of their bits (-0 before 0, NaN at either end by sign), vals as unsigned words. */
 int jzt_segment_sort(jzt_stream_t stream, const int32_t* spl, const float* key, const int32_t* val,
                      float* key_out, int32_t* val_out, int64_t size_segs, int64_t size_keys);
 
